@@ -104,6 +104,20 @@ struct Operand {
   int ld;               // elements between rows (multiple of 8)
   int row0;             // first row of this tile
   int rows;             // total valid rows (> row0); rows past the end are clamped (their results are masked later)
+  // K-contiguous operand: the tile's rows 128 .. 255 are taken this many rows earlier (VocabTail below; 0 elsewhere).
+  int upper_back = 0;
+  // K-major operand: the last pair of k-tiles is taken this many k-rows earlier (VocabTail below; 0 elsewhere).
+  int last_pair_back = 0;
+};
+
+// A vocabulary that is not a multiple of two k-tiles, in a contraction over the vocabulary.  The products run over whole
+// groups of 128 vocab columns (two k-tiles); the last group would reach past the weight's last row.  It is therefore moved
+// back by `back` rows so that it ends with the vocabulary: group columns 0 .. back - 1 repeat columns of the group before it and
+// carry zeros, columns back .. 127 are the vocabulary's last ones.  Every row the products read exists, so no zero-padded
+// copy of the weight is needed.  `from` is the first column of that group in the unshifted numbering.
+struct VocabTail {
+  int from;  // V / 128 * 128; columns at or beyond it belong to the last, moved group
+  int back;  // 0 when the vocabulary is a multiple of 128
 };
 // A B operand may instead be "K-major": the same matrix stored transposed, ptr[k * ld + n], so that a 16-byte chunk
 // holds eight consecutive n of one k (what a producer writes when n is its contiguous axis).  Then row0 is the first
@@ -177,7 +191,8 @@ __device__ __forceinline__ void make_plan(CopyPlan& p, const Operand& a, const O
     const int c = (j * NWAVES + wave) * 64 + lane;  // chunk index inside the slot
     const int row = c >> 3;
     const int kc = (c & 7) ^ swz(row);
-    int ra = a.row0 + row < a.rows ? row : a.rows - 1 - a.row0;  // row inside the tile; rows past the end re-read the last one
+    int ra = row >= BM / 2 ? row - a.upper_back : row;
+    ra = a.row0 + ra < a.rows ? ra : a.rows - 1 - a.row0;  // row inside the tile; rows past the end re-read the last one
     p.a_src[j] = (uint32_t)ra * (uint32_t)a.ld * 2u + (uint32_t)(kc * 16);
     if (BKM) {
       const int block = j * NWAVES + wave;             // rows 2 * block, 2 * block + 1 of the k-tile
@@ -197,6 +212,12 @@ __device__ __forceinline__ void make_plan(CopyPlan& p, const Operand& a, const O
   p.a_bytes = (const char*)a.ptr + (a_row0 * (size_t)a.ld + (size_t)k_begin) * 2;
   p.b_bytes = (const char*)b.ptr +
               (BKM ? ((size_t)k_begin * (size_t)b.ld + b_row0) * 2 : (b_row0 * (size_t)b.ld + (size_t)k_begin) * 2);
+}
+
+// Bytes by which the last pair of k-tiles of the B operand starts earlier than its place in the sequence.
+template <bool BKM>
+__device__ __forceinline__ size_t last_pair_back_bytes(const Operand& b) {
+  return BKM ? (size_t)b.last_pair_back * (size_t)b.ld * 2u : 0u;
 }
 
 // Bytes between consecutive k-tiles of the B operand.
@@ -236,6 +257,7 @@ template <bool BKM = false>
 __device__ __forceinline__ void prefetch_first_tiles(const Operand& a, const Operand& b, int k_begin, int nk, char* lds) {
   CopyPlan p;  // rebuilt by mainloop(): keeping it in registers across an epilogue costs more than recomputing it
   make_plan<BKM>(p, a, b, k_begin);
+  if (BKM && nk == 2) p.b_bytes -= last_pair_back_bytes<BKM>(b);
   const uint32_t w0 = wave_copy_base(lds);
   copy_part(p.a_bytes, p.a_src, w0 + 0 * OPERAND_BYTES, 0, COPIES_PER_OPERAND);
   copy_part(p.b_bytes, p.b_src, w0 + 1 * OPERAND_BYTES, 0, COPIES_PER_OPERAND);
@@ -608,6 +630,7 @@ __device__ __forceinline__ void mainloop_pairs(const Operand& a, const Operand& 
   std::false_type no;
   // nk is even: tiles alternate even, odd and the sequence is a straight line.
   for (int kt = 0; kt + 3 < nk; kt += 2) {
+    if (BKM && kt + 4 == nk) gb -= last_pair_back_bytes<BKM>(b);  // this pass copies the last pair
     tile_step(even, yes, yes, X, Y);
     tile_step(odd, yes, yes, Y, X);
   }

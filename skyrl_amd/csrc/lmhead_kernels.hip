@@ -8,7 +8,7 @@
 //   lmhead_fwd_merge   per block of 64 tokens: merges the partials (online log-sum-exp), gathers the label logit with an
 //                      fp32 dot product hidden[t] . weight[label], writes logprob / entropy / lse / pz.
 // Backward (6*T*V*H flop), looped over vocab chunks of `vocab_chunk` columns:
-//   transpose_bf16     hidden^T once per call (and weight^T only when V is not a multiple of 64).
+//   transpose_bf16     hidden^T once per call (and weight^T only for small vocabularies that are not multiples of 128).
 //   lmhead_bwd_dz      recompute a logits tile, form dz in registers and write it (bf16) into one token-major panel of
 //                      the chunk.
 //   lmhead_bwd_gemm    dHidden (+)= dz . weight and dW[chunk] = dz^T . hidden with fp32 accumulation, both from that
@@ -330,6 +330,7 @@ struct DzArgs {
   const float* dlogprobs;
   const float* dentropy;
   int vc0, tiles_m, tiles_n;  // first vocab row of the chunk; tiles of the chunk panel along vocab and tokens
+  VocabTail tail;
   uint16_t* D;                // [tiles_n * 256, ldd]  dz, token-major
   int ldd;
   // When not NULL: the number of tokens, <= T, as a value in device memory (what a compaction kernel counted).  T then
@@ -343,6 +344,26 @@ struct DzArgs {
   // 0, or 126 - n: softmax probabilities below 2^-n are treated as zero (SKYRL_BWD_FLUSH_TINY_DZ).
   float p_shift;
 };
+
+// Which vocabulary rows the 128 panel columns of a wave (columns panel0 .. panel0 + 127 in the full numbering) stand for:
+// column vl is vocabulary row v0 + vl for lo <= vl < hi and carries zeros elsewhere.
+struct WaveRows {
+  int v0, lo, hi;
+};
+__device__ __forceinline__ WaveRows wave_vocab_rows(int panel0, int V, const VocabTail& tail) {
+  const bool moved = tail.back > 0 && panel0 == tail.from;
+  const int v0 = panel0 - (moved ? tail.back : 0);
+  const int left = (tail.back > 0 && panel0 > tail.from) ? 0 : V - v0;  // no rows at all behind the moved group
+  return WaveRows{v0, moved ? tail.back : 0, left < 0 ? 0 : (left < WM ? left : WM)};
+}
+
+// The A operand of a dz tile: weight rows of panel columns panel0 .. panel0 + 255, the moved group included.
+__device__ __forceinline__ Operand dz_weight_rows(const uint16_t* W, int ldw, int panel0, int V, const VocabTail& tail) {
+  Operand a{W, ldw, panel0, V};
+  if (tail.back > 0 && panel0 == tail.from) a.row0 -= tail.back;
+  if (tail.back > 0 && panel0 + WM == tail.from) a.upper_back = tail.back;
+  return a;
+}
 
 template <bool ENTGRAD, bool EVEN>
 __device__ __forceinline__ void dz_tile(const DzArgs& z, int id, char* lds) {
@@ -367,10 +388,11 @@ __device__ __forceinline__ void dz_tile(const DzArgs& z, int id, char* lds) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
   const int lrow = lane & 15, kq = lane >> 4;
-  const int vloc_base = tm * BM + wm * WM;    // first vocab row of this wave inside the chunk panel
-  const int vbase = vc0 + vloc_base;          // ... and in the full vocab
+  const int vloc_base = tm * BM + wm * WM;    // first column of this wave inside the chunk panel
+  const WaveRows rows = wave_vocab_rows(vc0 + vloc_base, V, z.tail);
+  const int vbase = rows.v0;                  // the vocabulary row of its first column
   const int tbase = tn * BN + wn * WN;        // first token of this wave (always inside the padded panels)
-  const bool full = vbase + WM <= V;
+  const bool full = rows.lo == 0 && rows.hi == WM;
   const float scale2 = rcp_temp * kLog2e;
 
   // Per-token inputs of the epilogue.  The loads are issued here, before the mainloop, and their values are first touched
@@ -395,7 +417,7 @@ __device__ __forceinline__ void dz_tile(const DzArgs& z, int id, char* lds) {
   Operand a{W, ldw, vc0 + (tm % 4) * BM, V};
   Operand b{Hd, ldh, (tn % 8) * BN, T};
 #else
-  Operand a{W, ldw, vc0 + tm * BM, V};
+  const Operand a = dz_weight_rows(W, ldw, vc0 + tm * BM, V, z.tail);
   Operand b{Hd, ldh, tn * BN, T};
 #endif
   acc_t acc;
@@ -431,7 +453,7 @@ __device__ __forceinline__ void dz_tile(const DzArgs& z, int id, char* lds) {
     const float pz = (ENTGRAD && valid) ? v[3] : 0.f;
     const int64_t y = valid ? *(const int64_t*)(tokv + WN * 16 + (j * MT + lrow) * 8) : (int64_t)-1;
     const int64_t yrel64 = y - (int64_t)vbase;
-    yrel_[j] = (y >= 0 && y < (int64_t)V && yrel64 >= 0 && yrel64 < WM) ? (int)yrel64 : -1;
+    yrel_[j] = (y >= 0 && y < (int64_t)V && yrel64 >= rows.lo && yrel64 < rows.hi) ? (int)yrel64 : -1;
     gs_[j] = g * rcp_temp;
     c0_[j] = -(g - q * pz) * rcp_temp;
     c1_[j] = -q * rcp_temp * rcp_temp;
@@ -504,7 +526,7 @@ __device__ __forceinline__ void dz_tile(const DzArgs& z, int id, char* lds) {
       if (RAGGED) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (vbase + vl + r >= V) d[r] = 0.f;
+          if (vl + r < rows.lo || vl + r >= rows.hi) d[r] = 0.f;
       }
       f32x4 v4 = {d[0], d[1], d[2], d[3]};
       const bf16x4 b4 = __builtin_convertvector(v4, bf16x4);
@@ -607,6 +629,7 @@ struct SoftCeDzArgs {
   const float* lse_teacher;
   const float* dloss;
   int vc0, tiles_m, tiles_n;  // first vocab row of the chunk; tiles along the chunk's vocab rows and the stacked rows
+  VocabTail tail;
   uint16_t* D;                // [Tp, ldd]  dz of the student rows, token-major
   int ldd;
 };
@@ -625,9 +648,9 @@ __global__ __launch_bounds__(NTHREADS) void softce_dz_tiles(const SoftCeDzArgs z
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
   const int lrow = lane & 15, kq = lane >> 4;
   const int vloc_base = tm * BM + wm * WM;
-  const int vbase = vc0 + vloc_base;
+  const WaveRows rows = wave_vocab_rows(vc0 + vloc_base, V, z.tail);
   const int tokbase = (tn * WAVES_N + wn) * kPairRows;  // first token of this wave
-  const bool full = vbase + WM <= V;
+  const bool full = rows.lo == 0 && rows.hi == WM;
   const float scale2 = z.rcp_temp * kLog2e;
 
   // Per-token inputs: unconditional loads from a clamped index, issued before the mainloop and first touched behind it (as
@@ -642,7 +665,7 @@ __global__ __launch_bounds__(NTHREADS) void softce_dz_tiles(const SoftCeDzArgs z
     lt2_[j] = z.lse_teacher[tc];
   }
 
-  Operand a{W, z.ldw, vc0 + tm * BM, V};
+  const Operand a = dz_weight_rows(W, z.ldw, vc0 + tm * BM, V, z.tail);
   Operand b{S, H, tn * BN, 2 * z.Tp};
   acc_t acc;
   prefetch_first_tiles(a, b, 0, H / BK, lds);  // the first copies travel while the accumulators are cleared
@@ -686,7 +709,7 @@ __global__ __launch_bounds__(NTHREADS) void softce_dz_tiles(const SoftCeDzArgs z
       if (!full) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (vbase + vl + r >= V) d[r] = 0.f;
+          if (vl + r < rows.lo || vl + r >= rows.hi) d[r] = 0.f;
       }
       f32x4 v4 = {d[0], d[1], d[2], d[3]};
       const bf16x4 b4 = __builtin_convertvector(v4, bf16x4);
@@ -729,6 +752,10 @@ struct GemmArgs {
   // value of that extent is an upper bound that sizes the grid and the scratch; tiles beyond the count return at once.
   const int* T_dev;
   int t_role;
+  // The moved last group of a vocabulary that is not a multiple of 128 (VocabTail), relative to the chunk.  dHidden contracts
+  // over it: the last pair of its k-tiles reads the weight k_back rows earlier.  dW has it as output rows: row n at or beyond
+  // n_tail is row n - n_back, and the first n_back of those belong to the group before it.
+  int k_back, n_tail, n_back;
 };
 enum { kTokensOnM = 1, kTokensOnN = 2, kTokensOnK = 3 };
 
@@ -758,7 +785,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bid, char* lds)
   Operand b{p.B, p.ldb, (tn % 8) * BN, p.b_rows};
 #else
   Operand a{p.A, p.lda, tm * BM, p.a_rows};
-  Operand b{p.B, p.ldb, tn * BN, p.b_rows};
+  Operand b{p.B, p.ldb, tn * BN, p.b_rows, 0, p.k_back};
 #endif
   acc_t acc;
   if (nk > 0) prefetch_first_tiles<BKM>(a, b, 0, nk, lds);
@@ -818,8 +845,12 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bid, char* lds)
 
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    const int n = tn * BN + wn * WN + j * MT + lrow;
+    int n = tn * BN + wn * WN + j * MT + lrow;
     if (n >= N) continue;
+    if (n >= p.n_tail) {
+      n -= p.n_back;
+      if (n < p.n_tail) continue;
+    }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int m = tm * BM + wm * WM + i * MT + kq * 4;  // this lane holds m .. m+3
@@ -849,7 +880,7 @@ __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_gemm(const GemmArgs p0, c
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
   const int id = blockIdx.x;
   // dW always reads the dz panel K-major (K = tokens); dHidden either reads the weight itself K-major (K = vocab) or,
-  // when the vocabulary is not a multiple of two k-tiles, a transposed, zero-padded copy of it with K contiguous.
+  // for a small vocabulary that is not a multiple of two k-tiles, a transposed, zero-padded copy of it with K contiguous.
   const bool second = id >= tiles0;
   if (second || p0.b_kmajor) gemm_tile<true>(second ? p1 : p0, second ? id - tiles0 : id, lds);
   else gemm_tile<false>(p0, id, lds);
@@ -1369,10 +1400,19 @@ struct BwdWorkspace {
   size_t bytes;
 };
 
-// The dHidden GEMM contracts over the vocabulary.  When V is a multiple of two k-tiles (the gradient GEMMs run whole pairs
-// of k-tiles) it reads the weight rows where they are (K-major B operand); otherwise the last pair would reach past the
-// weight's last row, and a transposed copy, zero-padded to whole tiles, is made in the workspace instead.
-inline bool reads_weight_in_place(int64_t V) { return V % (2 * BK) == 0; }
+// The dHidden GEMM contracts over the vocabulary, in whole pairs of k-tiles, and reads the weight rows where they are
+// (K-major B operand); the last, incomplete group of a vocabulary that is not a multiple of 128 is moved back (VocabTail).
+// A transposed, zero-padded copy in the workspace stays below 1024 rows only: a vocabulary below 128 has no group to move
+// back, and there the copy is the cheaper side -- whole backward, copy against in place: 42.3 / 44.0 us at T=300, H=128,
+// V=1000; 60.7 / 59.4 at T=512, H=1024, V=1000; 79.8 / 75.9 at V=2001; 515 / 499 at V=32001.  A pass over the weight saved:
+// 0.38 of 5.9 ms at T=2654, H=4096, V=128261.
+constexpr int64_t kInPlaceMinVocab = 1024;
+inline bool reads_weight_in_place(int64_t V) { return V % (2 * BK) == 0 || V >= kInPlaceMinVocab; }
+inline VocabTail vocab_tail(int64_t V) {
+  const int64_t rest = V % (2 * BK);
+  if (rest == 0 || !reads_weight_in_place(V)) return VocabTail{0x7fffffff, 0};
+  return VocabTail{(int)(V - rest), (int)(2 * BK - rest)};
+}
 
 inline int64_t bwd_block_tokens(int64_t T) { return T < kBwdTokenBlock ? T : kBwdTokenBlock; }
 inline int64_t bwd_num_blocks(int64_t T) { return (T + kBwdTokenBlock - 1) / kBwdTokenBlock; }
@@ -1383,7 +1423,9 @@ BwdWorkspace carve_bwd(void* ws, int64_t T, int64_t H, int64_t Hk, int64_t V, in
   const int64_t Tb = bwd_block_tokens(T), Tpad = round_up(Tb, 256), Vpad = round_up(V, 256);
   Carver c(ws);
   BwdWorkspace w{};
-  w.Wt = reads_weight_in_place(V) ? nullptr : c.take<uint16_t>((size_t)H * (Vpad + kLdPad));
+  // The size a transposed weight would take stays part of the query for every vocabulary that is not a multiple of 128:
+  // callers may have sized their scratch by the documented formula.  It is only written below kInPlaceMinVocab.
+  w.Wt = V % (2 * BK) == 0 ? nullptr : c.take<uint16_t>((size_t)H * (Vpad + kLdPad));
   w.Ht = c.take<uint16_t>((size_t)H * (Tpad + kLdPad));
   w.dHacc = c.take<float>((size_t)Tpad * round_up(H, 256));  // accumulator order, whole tiles
   w.D = c.take<uint16_t>((size_t)Tpad * (vc + kLdPad));
@@ -1409,7 +1451,7 @@ GemmArgs make_gemm(const uint16_t* A, int64_t lda, int64_t a_rows, const uint16_
                    bool c_rows_m, int64_t nk, int64_t M, int64_t N, const float* Cin, float* Cf, uint16_t* Cb, int64_t ldc,
                    const float* Pin = nullptr, float* Pout = nullptr, const int* T_dev = nullptr, int t_role = 0) {
   return GemmArgs{A,       (int)lda, (int)a_rows, B,  (int)ldb, (int)b_rows, b_kmajor ? 1 : 0, c_rows_m ? 1 : 0, (int)nk,
-                  (int)M,  (int)N,   Cin,         Cf, Cb,       (int)ldc,    Pin,              Pout, T_dev, t_role};
+                  (int)M,  (int)N,   Cin,         Cf, Cb,       (int)ldc,    Pin,              Pout, T_dev, t_role, 0, 0x7fffffff, 0};
 }
 
 unsigned gemm_tiles(const GemmArgs& g) { return (unsigned)(((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN)); }
@@ -1473,7 +1515,7 @@ SoftCeBwdWorkspace carve_softce_bwd(void* ws, int64_t T, int64_t H, int64_t V, i
   Carver c(ws);
   SoftCeBwdWorkspace w;
   w.S = c.take<uint16_t>((size_t)(2 * Tp) * (size_t)H);
-  w.Wt = reads_weight_in_place(V) ? nullptr : c.take<uint16_t>((size_t)H * (Vpad + kLdPad));
+  w.Wt = V % (2 * BK) == 0 ? nullptr : c.take<uint16_t>((size_t)H * (Vpad + kLdPad));  // as in carve_bwd
   w.dHacc = c.take<float>((size_t)round_up(T, 256) * round_up(H, 256));
   w.D = c.take<uint16_t>((size_t)Tp * (vc + kLdPad));
   w.bytes = (size_t)round_up((int64_t)c.off, 256);
@@ -1564,6 +1606,7 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
     if ((e = hipGetLastError()) != hipSuccess) return (int)e;
   }
   const int tiles_t = (int)(Tpad / 256);
+  const VocabTail tail = vocab_tail(V);
   const int64_t nchunks = (Vpad + vc - 1) / vc;
   auto chunk_width = [&](int64_t ci) { return (Vpad - ci * vc) < vc ? (Vpad - ci * vc) : vc; };  // multiple of 256
   const GemmArgs none{};
@@ -1573,7 +1616,7 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
     // width, and it needs a second panel.
     const int64_t vc0 = ci * vc, vcw = chunk_width(ci);
     const DzArgs z{Wp, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)Hk, (int)V, rcp_temperature, labels, row_lse, row_pz,
-                   dlogprobs, dentropy, (int)vc0, (int)(vcw / 256), tiles_t, w.D, (int)(vcw + kLdPad), T_dev, resid, p_shift};
+                   dlogprobs, dentropy, (int)vc0, (int)(vcw / 256), tiles_t, tail, w.D, (int)(vcw + kLdPad), T_dev, resid, p_shift};
     e = launch_bwd_dz(s, dentropy != nullptr, z, (unsigned)(vcw / 256 * tiles_t));
     if (e != hipSuccess) return (int)e;
     // dHidden[t, h] (+)= sum_v D[t, v] . weight^T[h, vc0 + v]        (A = weight^T rows at k offset vc0, B = D rows)
@@ -1585,21 +1628,25 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
     uint16_t* dh_out = last ? d_hidden : (uint16_t*)nullptr;
     const float* dh_in = first ? (const float*)nullptr : (const float*)w.dHacc;
     float* dh_keep = last ? (float*)nullptr : w.dHacc;
-    // In place: C[t, h] with A = D rows (K = vocab, contiguous), B = weight rows vc0.. read K-major; the k extent stops at V.
-    // Otherwise: C[h, t] with A = weight^T rows, B = D rows.  The partial sums are in accumulator order either way.
-    const int64_t kext = (V - vc0) < vcw ? (V - vc0) : vcw;
-    const GemmArgs gh =
+    // In place: C[t, h] with A = D rows (K = vocab, contiguous), B = weight rows vc0.. read K-major; the k extent stops at the
+    // end of V's last group of 128.  Otherwise: C[h, t] with A = weight^T rows, B = D rows.  The partial sums are in accumulator
+    // order either way.
+    const int64_t kext = round_up(rows, 2 * BK);
+    GemmArgs gh =
         w_in_place ? make_gemm(w.D, vcw + kLdPad, Tpad, Wp + (size_t)vc0 * (size_t)ld_weight, ld_weight, H, true, true, kext / BK, Tb,
                                H, nullptr, nullptr, dh_out, H, dh_in, dh_keep, T_dev, kTokensOnM)
                    : make_gemm(w.Wt + vc0, Vpad + kLdPad, H, w.D, vcw + kLdPad, Tpad, false, false, vcw / BK, H, Tb, nullptr,
                                nullptr, dh_out, H, dh_in, dh_keep, T_dev, kTokensOnN);
     // A frozen LM head needs no dW: the launch then carries the dHidden tiles alone.
-    const GemmArgs gw = want_dw ? make_gemm(w.Ht, Tpad + kLdPad, H, w.D, vcw + kLdPad, vcw, true, false, Tpad / BK, H, rows,
+    const bool moved = last && tail.back > 0;  // the chunk ends with a moved group
+    if (moved) gh.k_back = tail.back;
+    GemmArgs gw = want_dw ? make_gemm(w.Ht, Tpad + kLdPad, H, w.D, vcw + kLdPad, vcw, true, false, Tpad / BK, H, moved ? kext : rows,
                                             dw_in ? dw_in + dw_off : (const float*)nullptr,
                                             dw_f32 ? dw_f32 + dw_off : (float*)nullptr,
                                             dw_bf16 ? dw_bf16 + dw_off : (uint16_t*)nullptr, H, nullptr, nullptr, T_dev,
                                             kTokensOnK)
                                 : none;
+    if (moved && want_dw) gw.n_tail = (int)(tail.from - vc0), gw.n_back = tail.back;
     e = launch_bwd_gemm(s, gh, gw);
     if (e != hipSuccess) return (int)e;
   }
@@ -1908,6 +1955,7 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
   hipError_t e = launch_softce_pack(s, student_hidden, ld_student, teacher_hidden, ld_teacher, T, seq_len, shift, H, w.S);
   if (e != hipSuccess) return (int)e;
   const bool w_in_place = reads_weight_in_place(V);
+  const VocabTail tail = vocab_tail(V);
   if (!w_in_place) {
     Timed timed(kTranspose, s);
     hipLaunchKernelGGL(transpose_bf16, dim3((unsigned)(Vpad / 64), (unsigned)(H / 64)), dim3(256), 0, s, Wp, (int)ld_weight,
@@ -1919,7 +1967,7 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
   for (int64_t ci = 0; ci < nchunks; ++ci) {
     const int64_t vc0 = ci * vc, vcw = (Vpad - vc0) < vc ? (Vpad - vc0) : vc;
     const SoftCeDzArgs z{Wp, (int)ld_weight, w.S, (int)T, (int)Tp, (int)H, (int)V, rcp_temperature, lse_student, lse_teacher,
-                         dloss, (int)vc0, (int)(vcw / 256), (int)(2 * Tp / BN), w.D, (int)(vcw + kLdPad)};
+                         dloss, (int)vc0, (int)(vcw / 256), (int)(2 * Tp / BN), tail, w.D, (int)(vcw + kLdPad)};
     {
       Timed timed(kSoftCeDz, s);
       auto kernel = even_ktiles(H) ? softce_dz_tiles<true> : softce_dz_tiles<false>;
@@ -1932,12 +1980,13 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
     uint16_t* dh_out = last ? (uint16_t*)d_student_hidden : (uint16_t*)nullptr;
     const float* dh_in = first ? (const float*)nullptr : (const float*)w.dHacc;
     float* dh_keep = last ? (float*)nullptr : w.dHacc;
-    const int64_t kext = (V - vc0) < vcw ? (V - vc0) : vcw;
-    const GemmArgs gh =
+    const int64_t kext = round_up((V - vc0) < vcw ? (V - vc0) : vcw, 2 * BK);
+    GemmArgs gh =
         w_in_place ? make_gemm(w.D, vcw + kLdPad, Tp, Wp + (size_t)vc0 * (size_t)ld_weight, ld_weight, H, true, true, kext / BK, T,
                                H, nullptr, nullptr, dh_out, H, dh_in, dh_keep)
                    : make_gemm(w.Wt + vc0, Vpad + kLdPad, H, w.D, vcw + kLdPad, Tp, false, false, vcw / BK, H, T, nullptr,
                                nullptr, dh_out, H, dh_in, dh_keep);
+    if (last && tail.back > 0) gh.k_back = tail.back;
     e = launch_bwd_gemm(s, gh, none);
     if (e != hipSuccess) return (int)e;
   }

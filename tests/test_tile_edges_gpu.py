@@ -1,0 +1,67 @@
+"""The sizes at which the tile kernels' dispatch rules change or a tile, group or split is incomplete, against the oracle.
+
+Bounds: d_hidden and d_weight are bf16-rounded products of a dz that is itself rounded to bf16 once, 2^-9 / sqrt(3) relative
+each and independent of the sizes: 3e-3 in the 2-norm, a single row at most four times that where its norm is of the order of the
+others'."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import lmhead_oracle as O
+from skyrl_amd import ops
+from skyrl_amd.mtp_soft_ce import soft_ce_from_hidden
+
+pytestmark = pytest.mark.gpu
+
+GRAD_REL_L2 = 5e-3
+GRAD_ROW_REL_L2 = 2e-2
+
+
+def _operands(T, H, V, seed, dtype=torch.bfloat16):
+    gen = torch.Generator().manual_seed(seed)
+    hidden = torch.randn(T, H, generator=gen).to(torch.bfloat16)
+    weight = (torch.randn(V, H, generator=gen) * 3 / H**0.5).to(dtype)
+    labels = torch.randint(0, V, (T,), generator=gen)
+    g, q = torch.randn(T, generator=gen), torch.randn(T, generator=gen) * 0.2
+    return hidden, weight, labels, g, q
+
+
+def _close(got, want, tag):
+    got, want = got.detach().double().cpu(), want.double()
+    rel = float((got - want).norm() / want.norm())
+    norms = want.norm(dim=1)
+    row = float(((got - want).norm(dim=1) / norms.clamp_min(0.1 * float(norms.mean()))).max())
+    assert rel < GRAD_REL_L2 and row < GRAD_ROW_REL_L2, f"{tag}: {rel:.2e}, worst row {row:.2e}"
+
+
+# The last group of 128 vocabulary rows is moved back from V = 1024 on: one row left over, one missing, the group in the lower
+# and in the upper half of a tile, alone in its chunk, and the sizes around the rule's line.
+@pytest.mark.parametrize("V,vc", [(1023, 0), (1025, 0), (1025, 256), (1151, 256), (1152, 256), (1153, 256), (1279, 512), (5001, 0)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_vocabulary_that_ends_inside_a_group(V, vc, dtype, cuda_device):
+    T, H, t = 300, 192, 0.8
+    hidden, weight, labels, g, q = _operands(T, H, V, seed=V + vc, dtype=dtype)
+    labels[:6] = torch.tensor([V - 1, V - 128, V // 128 * 128 - 1, min(V - 1, V // 128 * 128), V - 127, 0])
+    g[7::5], q[7::5] = 0.0, 0.0
+    h, w, y, gd, qd = (x.to(cuda_device) for x in (hidden, weight, labels, g, q))
+    _, _, lse, pz = ops.lmhead_fwd(h, w, y, 1.0 / t, True)
+    ex = O.exact_fwd_bwd(hidden, weight, labels, t, g, q)
+    for active in (False, True):
+        dh, dw = ops.lmhead_bwd(h, w, y, lse, pz, gd, qd, 1.0 / t, vc, active)
+        _close(dh, ex["d_hidden"], f"dHidden V={V} chunk={vc}")
+        _close(dw, ex["d_weight"], f"dW V={V} chunk={vc}")
+    assert torch.equal(ops.lmhead_bwd_hidden(h, w, y, lse, pz, gd, qd, 1.0 / t, vc, True), dh)
+    if dtype == torch.bfloat16:
+        acc = torch.full((V, H), 0.5, device=cuda_device)
+        ops.lmhead_bwd_accumulate(h, w, y, lse, pz, gd, qd, 1.0 / t, acc, vc)
+        _close(acc - 0.5, ex["d_weight"], f"accumulated dW V={V}")
+        # the draft loss contracts over the same vocabulary
+        s = hidden.reshape(2, 150, H).to(cuda_device).requires_grad_(True)
+        teacher = torch.randn(2, 150, H, generator=torch.Generator().manual_seed(V)).to(torch.bfloat16)
+        up = g.reshape(2, 150)
+        (soft_ce_from_hidden(s, teacher.to(cuda_device), w, shift=1, vocab_chunk=vc) * up.to(cuda_device)).sum().backward()
+        zs, zt = hidden.double() @ weight.double().t(), teacher.roll(-1, dims=1).reshape(T, H).double() @ weight.double().t()
+        want = (g.double()[:, None] * (zs.softmax(-1) - zt.softmax(-1))) @ weight.double()
+        _close(s.grad.reshape(T, H), want, f"draft loss V={V}")
