@@ -659,11 +659,11 @@ __device__ __forceinline__ void mainloop(const Operand& a, const Operand& b, int
 //  2. Walk the logical order in bands of `group_m` tiles along M, N-major inside a band, so the ~32 workgroups
 //     concurrently resident on one XCD cover a compact group_m x (32/group_m) patch and share operand panels in that
 //     XCD's L2.
-__device__ __forceinline__ void tile_coords(int id, int tiles_m, int tiles_n, int group_m, int& tm, int& tn) {
-  const int total = tiles_m * tiles_n;
+__device__ __forceinline__ int xcd_contiguous(int id, int total) {
   const int per_xcd = total >> 3;
-  int logical = id;
-  if (id < (per_xcd << 3)) logical = (id & 7) * per_xcd + (id >> 3);
+  return id < (per_xcd << 3) ? (id & 7) * per_xcd + (id >> 3) : id;
+}
+__device__ __forceinline__ void banded_tile(int logical, int tiles_m, int tiles_n, int group_m, int& tm, int& tn) {
   const int band_sz = group_m * tiles_n;
   const int band = logical / band_sz;
   const int in_band = logical - band * band_sz;
@@ -672,6 +672,9 @@ __device__ __forceinline__ void tile_coords(int id, int tiles_m, int tiles_n, in
   gm = gm < group_m ? gm : group_m;
   tn = in_band / gm;
   tm = m_first + (in_band - tn * gm);
+}
+__device__ __forceinline__ void tile_coords(int id, int tiles_m, int tiles_n, int group_m, int& tm, int& tn) {
+  banded_tile(xcd_contiguous(id, tiles_m * tiles_n), tiles_m, tiles_n, group_m, tm, tn);
 }
 
 // Sum / maximum over the four lanes (l, l^16, l^32, l^48) that hold the same accumulator column, result in all four.

@@ -35,6 +35,8 @@ using namespace lmhead;
 
 namespace {
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 #ifndef LMHEAD_GROUP_M
@@ -475,7 +477,6 @@ __device__ __forceinline__ void dz_tile(const DzArgs& z, int id, char* lds) {
   // non-temporal: the panel is a gigabyte that is read back only by the next launch, and letting it displace the operand
   // panels from L2 costs the mainloops of the neighbouring tiles more than the stores themselves.
   char* stage = lds + wave * kStage;
-  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   // Every staging address is one per-lane base plus a compile-time constant (an immediate of the LDS instruction), and the
   // panel rows are walked with one running pointer: written as (j * 16 + row) * pitch the compiler keeps eight row indices
   // alive across the whole epilogue and spills them, and a spill reload waits for vmcnt(0) -- i.e. for every panel store in flight.
@@ -683,7 +684,6 @@ __global__ __launch_bounds__(NTHREADS) void softce_dz_tiles(const SoftCeDzArgs z
   constexpr int kTokRow = WM * 2 + 16;
   constexpr int kStage = WN * kTokRow;
   char* stage = lds + wave * kStage;
-  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   auto flush_block = [&](int j) {  // as in dz_tile: a finished token block leaves while the next one is computed
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
@@ -730,6 +730,8 @@ __global__ __launch_bounds__(NTHREADS) void softce_dz_tiles(const SoftCeDzArgs z
 // and dWeight products of a vocab chunk have no dependency on each other, and together they fill the 256 CUs in whole
 // rounds where each alone leaves a partial last round.
 // ------------------------------------------------------------------------------------------------------------
+constexpr int kSlabWaveFloats = TM * TN * 64 * 4;            // one wave's accumulators
+constexpr int64_t kSlabTileFloats = NWAVES * kSlabWaveFloats;  // one tile's: 256 KiB
 struct GemmArgs {
   const uint16_t* A;
   int lda, a_rows;
@@ -742,11 +744,19 @@ struct GemmArgs {
   float* Cf;
   uint16_t* Cb;
   int ldc;
-  // Partial sums carried from launch to launch (dHidden across vocab chunks) live in "accumulator order": tile by tile,
-  // wave by wave, MFMA block by MFMA block, each lane's 4 registers contiguous.  Reading and writing them is 16 bytes
-  // per lane and 1 KiB contiguous per wave instruction, with no address arithmetic beyond a constant offset.
-  const float* Pin;
-  float* Pout;
+  // Partial sums that leave a launch (dHidden: from vocab chunk to vocab chunk, and from the splits of its contraction) live in
+  // "accumulator order": split by split, tile by tile, wave by wave, MFMA block by MFMA block, each lane's 4 registers
+  // contiguous.  Reading and writing them is 16 bytes per lane and 1 KiB contiguous per wave instruction, with no address
+  // arithmetic beyond a constant offset.  p_first: nothing to add yet; p_last: the sum is complete with this launch, and without
+  // splits it leaves as C.
+  float* P;
+  int p_first, p_last;
+  // Number of splits of the contraction: workgroups per C tile, each with its share of the k-tile pairs and its own slab of P,
+  // summed by lmhead_dh_reduce.  splits_dev, when not NULL, replaces it (what compact_active_rows chose for its token count).
+  int splits;
+  const int* splits_dev;
+  // When not NULL: row m of the bf16 output is row row_map[m] of C.
+  const int* row_map;
   // When not NULL: a token count in device memory that replaces one extent of the problem, chosen by t_role: the rows M
   // (kTokensOnM), the columns N (kTokensOnN) or the contraction length, nk = ceil(count / 64) (kTokensOnK).  The host-side
   // value of that extent is an upper bound that sizes the grid and the scratch; tiles beyond the count return at once.
@@ -758,6 +768,35 @@ struct GemmArgs {
   int k_back, n_tail, n_back;
 };
 enum { kTokensOnM = 1, kTokensOnN = 2, kTokensOnK = 3 };
+
+// How many workgroups share the vocabulary of one dHidden tile.  There are tokens/256 x H/256 such tiles with a contraction of a
+// whole chunk of the vocabulary: 18 tiles of 2374 k-tiles at T=611, H=1536, V=151936, which one workgroup each leaves on 18
+// of 256 CUs for 2.5 ms.  Rated in k-tiles of mainloop: the dHidden tiles alone in whole rounds of the CUs, or everything the
+// launch carries spread evenly plus half a dW tile of tail, plus what the slabs cost to write, read and add (a 256 KiB slab
+// tile about a seventeenth of a k-tile of the whole chip).  At least 1024 vocabulary rows per split.  Integer arithmetic: the
+// host and compact_active_rows, which rates one candidate per lane for the token count it found, must agree.
+// Measured, GEMM launches of the backward, one workgroup per tile -> split: 2750 -> 560 us at T=428 (active), H=1536, V=151936
+// (12 tiles x 8 splits); 544 -> 168 us at T=1050, H=1024, V=32000, fp32 weight; 2714 -> 1509 us at T=4096, H=2048, V=151936 and
+// 2304 -> 1317 us at T=1592, H=4096, V=128261, both without dW; 3030 -> 2700 us at T=4096, H=1536, V=151936.  With 192 tiles and
+// more the dW tiles fill the CUs and the launch is not split.
+constexpr int kMinSplitPairs = 8;
+constexpr int kMaxSplits = 64;
+struct SplitProblem {
+  int tiles_h;    // dHidden tiles per 256 tokens
+  int pairs;      // k-tile pairs of a chunk's vocabulary
+  int dw_tiles;   // dW tiles of the same launch (0: frozen weight)
+  int slots;      // slab tiles there is room for
+  int ncu;
+};
+__host__ __device__ inline int64_t split_cost(const SplitProblem& p, int tokens, int splits) {
+  const int tiles = (tokens + BM - 1) / BM * p.tiles_h;
+  if (splits > 1 && ((int64_t)tiles * splits > p.slots || p.pairs / splits < kMinSplitPairs)) return INT64_MAX;
+  const int64_t len = 2 * ((p.pairs + splits - 1) / splits) + (splits > 1 ? 10 : 8);
+  const int64_t items = (int64_t)tiles * splits, dw_len = (tokens + 2 * BK - 1) / (2 * BK) * 2 + 6;
+  const int64_t alone = (int64_t)(((int)items + p.ncu - 1) / p.ncu) * len * p.ncu;
+  const int64_t spread = items * len + p.dw_tiles * dw_len + (p.dw_tiles ? dw_len * p.ncu / 2 : 0);
+  return (alone > spread ? alone : spread) + (splits > 1 ? items * 15 + 4 * p.ncu : 0);
+}
 
 // BKM: the B operand is K-major.  The two variants are separate instantiations of the whole tile (mainloop and
 // epilogue) so that their accumulators never meet at a join, where the register allocator would shuffle all 256 of them.
@@ -772,26 +811,37 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bid, char* lds)
     // Nothing to contract: C += 0 needs no work; a C that is overwritten or converted still goes through the epilogue.
     if (nk == 0 && !p.Cb && p.Cin == p.Cf) return;
   }
+  const int splits = p.splits_dev ? __builtin_amdgcn_readfirstlane(*p.splits_dev) : p.splits;
   // Tiles of the extents in force: with a device-side count the tiles that hold tokens are numbered from 0, so that the
   // round-robin of workgroup ids over the XCDs spreads exactly those, and the rest of the (static) grid returns at once.  The
   // partial sums that cross vocab chunks are laid out by the same numbering (the count does not change between chunks).
   const int tiles_m = (M + BM - 1) / BM;
   const int tiles_n = (N + BN - 1) / BN;
-  if (bid >= tiles_m * tiles_n) return;
-  int tm, tn;
-  tile_coords(bid, tiles_m, tiles_n, kGroupM, tm, tn);
+  const int tiles = tiles_m * tiles_n;
+  if (bid >= tiles * splits) return;
+  int tm, tn, k0 = 0, k_back = p.k_back, split = 0;
+  int logical = xcd_contiguous(bid, tiles * splits);
+  if (splits > 1) {  // split by split, so that the workgroups resident on an XCD read the same range of both operands
+    split = logical / tiles;
+    logical -= split * tiles;
+    const int pairs = nk / 2, p0 = pairs * split / splits, p1 = pairs * (split + 1) / splits;
+    k0 = __builtin_amdgcn_readfirstlane(2 * p0), nk = __builtin_amdgcn_readfirstlane(2 * (p1 - p0));
+    if (split != splits - 1) k_back = 0;
+    if (nk == 0 && !p.p_first) return;  // a narrow last chunk: this split adds nothing to its slab
+  }
+  banded_tile(logical, tiles_m, tiles_n, kGroupM, tm, tn);
 #if LMHEAD_ABLATE & 16
   Operand a{p.A, p.lda, (tm % 4) * BM, p.a_rows};
   Operand b{p.B, p.ldb, (tn % 8) * BN, p.b_rows};
 #else
   Operand a{p.A, p.lda, tm * BM, p.a_rows};
-  Operand b{p.B, p.ldb, tn * BN, p.b_rows, 0, p.k_back};
+  Operand b{p.B, p.ldb, tn * BN, p.b_rows, 0, k_back};
 #endif
   acc_t acc;
-  if (nk > 0) prefetch_first_tiles<BKM>(a, b, 0, nk, lds);
+  if (nk > 0) prefetch_first_tiles<BKM>(a, b, k0 * BK, nk, lds);
   zero_acc(acc);
   if (nk > 0) {
-    mainloop<BKM, true>(a, b, 0, nk, lds, acc);  // nk is even for every gradient GEMM (make_gemm checks)
+    mainloop<BKM, true>(a, b, k0 * BK, nk, lds, acc);  // nk is even for every gradient GEMM (make_gemm checks)
   }
 
   const float* __restrict__ Cin = p.Cin;
@@ -802,43 +852,69 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bid, char* lds)
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
   const int lrow = lane & 15, kq = lane >> 4;
 
-  if (p.Pin || p.Pout) {
-    const size_t base = ((size_t)(tm * tiles_n + tn) * NWAVES + wave) * (TM * TN * 64 * 4) + (size_t)lane * 4;
-    if (p.Pin) {  // sixteen loads in flight at a time: one at a time costs a round trip to HBM each (36 us per tile)
+  if (p.P) {
+    float* part = p.P + ((size_t)(split * tiles + tm * tiles_n + tn) * NWAVES + wave) * kSlabWaveFloats + (size_t)lane * 4;
+    if (!p.p_first) {  // sixteen loads in flight at a time: one at a time costs a round trip to HBM each (36 us per tile)
 #pragma unroll
       for (int i = 0; i < TM; i += 2) {
         f32x4 t[2 * TN];
 #pragma unroll
-        for (int x = 0; x < 2 * TN; ++x) t[x] = *(const f32x4*)(p.Pin + base + (size_t)(i * TN + x) * (64 * 4));
+        for (int x = 0; x < 2 * TN; ++x) t[x] = *(const f32x4*)(part + (size_t)(i * TN + x) * (64 * 4));
 #pragma unroll
         for (int x = 0; x < 2 * TN; ++x) acc[i + x / TN][x % TN] += t[x];
       }
     }
-    if (p.Pout) {
+    if (!p.p_last || splits > 1) {
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) *(f32x4*)(p.Pout + base + (size_t)(i * TN + j) * (64 * 4)) = acc[i][j];
+        for (int j = 0; j < TN; ++j) *(f32x4*)(part + (size_t)(i * TN + j) * (64 * 4)) = acc[i][j];
+      return;
     }
   }
-  if (!Cf && !Cb) return;
 
-  if (BKM && p.c_rows_m) {
-    // Output rows run along M: a lane's four values belong to four different rows; sixteen lanes (n = lrow) cover 32
-    // contiguous bytes of each.  Only the last vocab chunk's dHidden tiles come through here.
+  if (Cb && !Cin && !Cf) {
+    // bf16 rows leave through LDS: in the accumulator layout a store instruction writes 32 contiguous bytes of sixteen rows (c_rows_m:
+    // two bytes per lane), staged it writes 256 of four: 1110 -> 1046 us for a whole training pass at T=611, H=1536, V=151936,
+    // whose dW tiles have eight k-tiles each.  The mainloop has left LDS free and every wave uses a region of its
+    // own, so no barrier is needed.  Staged rows run along M with c_rows_m (the tokens of dHidden), along N otherwise.
+    constexpr int kRow = WM * 2 + 16;
+    static_assert(WM == WN && NWAVES * WN * kRow <= LDS_BYTES, "output staging does not fit LDS");
+    char* stage = lds + wave * (WN * kRow);
+    const bool along_m = BKM && p.c_rows_m;
+    if (along_m) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int n = tn * BN + wn * WN + j * MT + lrow;
-      if (n >= N) continue;
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int m = tm * BM + wm * WM + i * MT + kq * 4;
-        const bf16x4 b4 = __builtin_convertvector(acc[i][j], bf16x4);
-        const uint16_t* h4 = (const uint16_t*)&b4;
+        for (int j = 0; j < TN; ++j) {
+          const bf16x4 b4 = __builtin_convertvector(acc[i][j], bf16x4);
+          const uint16_t* h4 = (const uint16_t*)&b4;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (m + r < M) Cb[(size_t)(m + r) * (size_t)ldc + n] = h4[r];
+          for (int r = 0; r < 4; ++r) *(uint16_t*)(stage + (i * MT + kq * 4 + r) * kRow + (j * MT + lrow) * 2) = h4[r];
+        }
+    } else {
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const bf16x4 b4 = __builtin_convertvector(acc[i][j], bf16x4);
+          *(uint2*)(stage + (j * MT + lrow) * kRow + (i * MT + kq * 4) * 2) = *(const uint2*)&b4;
+        }
+    }
+    const int row0 = along_m ? tm * BM + wm * WM : tn * BN + wn * WN, rows = along_m ? M : N;
+    const int col = (along_m ? tn * BN + wn * WN : tm * BM + wm * WM) + lrow * 8, cols = along_m ? N : M;
+    if (col >= cols) return;  // whole 16-byte pieces: both extents that run along rows are multiples of 64
+#pragma unroll
+    for (int it = 0; it < WN / 4; ++it) {
+      const u32x4 v = *(const u32x4*)(stage + (it * 4 + kq) * kRow + lrow * 16);
+      int r = row0 + it * 4 + kq;
+      if (r >= rows) continue;
+      if (r >= p.n_tail) {
+        r -= p.n_back;
+        if (r < p.n_tail) continue;
       }
+      if (p.row_map) r = p.row_map[r];
+      *(u32x4*)(Cb + (size_t)r * (size_t)ldc + col) = v;
     }
     return;
   }
@@ -879,11 +955,64 @@ __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_dz(const DzArgs z) {
 __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_gemm(const GemmArgs p0, const GemmArgs p1, int tiles0) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
   const int id = blockIdx.x;
+  // With a device-side token count the dW tiles start right behind the dHidden tiles in force; what is left of the (static) grid
+  // returns at once.
+  if (p0.T_dev) {
+    const int count = __builtin_amdgcn_readfirstlane(*p0.T_dev);
+    const int other = p0.t_role == kTokensOnM ? p0.N : p0.M;
+    tiles0 = (count + BM - 1) / BM * ((other + BN - 1) / BN) *
+             (p0.splits_dev ? __builtin_amdgcn_readfirstlane(*p0.splits_dev) : p0.splits);
+  }
   // dW always reads the dz panel K-major (K = tokens); dHidden either reads the weight itself K-major (K = vocab) or,
   // for a small vocabulary that is not a multiple of two k-tiles, a transposed, zero-padded copy of it with K contiguous.
   const bool second = id >= tiles0;
   if (second || p0.b_kmajor) gemm_tile<true>(second ? p1 : p0, second ? id - tiles0 : id, lds);
   else gemm_tile<false>(p0, id, lds);
+}
+
+// dHidden rows from the slabs of a split contraction: C[m, n] = bf16(sum of the slabs), added in split order.  One workgroup per
+// 16 tokens x 128 columns (an MFMA row block of a wave): 16-byte loads of contiguous slab pieces, 16-byte row pieces out
+// through LDS.  HBM-bound, splits x tokens x H x 4 bytes: 8 us at 240 slab tiles (60 MB).
+struct DhReduceArgs {
+  const float* P;
+  int M, H, splits;
+  const int *T_dev, *splits_dev, *row_map;  // as in GemmArgs
+  uint16_t* C;
+  int ldc;
+};
+constexpr int kReduceGroups = NWAVES * TM;  // workgroups per tile
+
+__global__ __launch_bounds__(256) void lmhead_dh_reduce(const DhReduceArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t rows[MT][WN + 8];
+  const int splits = a.splits_dev ? *a.splits_dev : a.splits;
+  const int M = a.T_dev ? *a.T_dev : a.M;
+  const int tiles_n = (a.H + BN - 1) / BN, tiles = (M + BM - 1) / BM * tiles_n;
+  const int tile = blockIdx.x / kReduceGroups, wave = blockIdx.x / TM % NWAVES, i = blockIdx.x % TM;
+  if (splits < 2 || tile >= tiles) return;  // without splits the GEMM epilogue has written C
+  const int m0 = tile / tiles_n * BM + wave / WAVES_N * WM + i * MT;
+  const int n0 = tile % tiles_n * BN + wave % WAVES_N * WN;
+  if (m0 >= M || n0 >= a.H) return;
+  const int tid = threadIdx.x;
+  const float* part = a.P + ((size_t)tile * NWAVES + wave) * kSlabWaveFloats + (size_t)(i * TN) * (64 * 4) + (size_t)tid * 4;
+  const size_t slab = (size_t)tiles * kSlabTileFloats;
+  f32x4 sum[2] = {*(const f32x4*)part, *(const f32x4*)(part + 1024)};
+#pragma unroll 4
+  for (int s = 1; s < splits; ++s) {
+    sum[0] += *(const f32x4*)(part + (size_t)s * slab);
+    sum[1] += *(const f32x4*)(part + (size_t)s * slab + 1024);
+  }
+  const int lane = tid & 63, lrow = lane & 15, kq = lane >> 4;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const bf16x4 b4 = __builtin_convertvector(sum[u], bf16x4);
+    const uint16_t* h4 = (const uint16_t*)&b4;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) rows[kq * 4 + r][(u * 4 + (tid >> 6)) * MT + lrow] = h4[r];
+  }
+  __syncthreads();
+  const int r = tid >> 4, c = (tid & 15) * 8, m = m0 + r;
+  if (m < M && n0 + c < a.H)
+    *(uint4*)(a.C + (size_t)(a.row_map ? a.row_map[m] : m) * (size_t)a.ldc + n0 + c) = *(const uint4*)&rows[r][c];
 }
 
 // Measurement aid: the mainloop's MFMA sequence (two 32-k steps of 64 MFMAs, same order, accumulators in AGPRs) with
@@ -1040,19 +1169,20 @@ __global__ __launch_bounds__(256) void split_operand_rows(const void* __restrict
 // ------------------------------------------------------------------------------------------------------------
 // Row compaction for the backward.  A token whose upstream gradients are both zero has a zero dz row: it adds nothing to
 // dW and its dHidden row is zero.  In RL micro-batches those are the prompt and padding tokens the loss mask removes, often
-// more than half of the batch.  Three small kernels let the backward run on the remaining rows without the host ever
+// more than half of the batch.  Two small kernels let the backward run on the remaining rows without the host ever
 // learning how many there are (no synchronisation, so the call can be captured in a HIP graph):
 //   compact_active_rows   one workgroup: idx[i] = i-th token with g != 0 or q != 0 (ascending), counts[0] = their number n,
-//                         counts[1 + b] = how many of them fall into block b of `block` compacted rows
+//                         counts[1 + b] = how many of them fall into block b of `block` compacted rows,
+//                         counts[1 + nblocks + b] = the splits of that block's dHidden contraction (split_cost)
 //   gather_active_rows    compacted copies of hidden rows and of the per-token inputs; zero dHidden rows for the inactive
-//   scatter_active_rows   dHidden rows of the compacted problem back to their tokens
-// The GEMM kernels take the counts from device memory (T_dev) and run on the static upper-bound grid.
+// The GEMM kernels take the counts from device memory (T_dev), run on the static upper-bound grid and write the dHidden rows
+// through the index list.
 // ------------------------------------------------------------------------------------------------------------
 constexpr int kCompactThreads = 1024;
 
 __global__ __launch_bounds__(kCompactThreads) void compact_active_rows(const float* __restrict__ g, const float* __restrict__ q,
-                                                                       int T, int block, int nblocks, int* __restrict__ idx,
-                                                                       int* __restrict__ counts) {
+                                                                       int T, int block, int nblocks, SplitProblem split,
+                                                                       int* __restrict__ idx, int* __restrict__ counts) {
   __shared__ int wave_sum[kCompactThreads / 64];
   __shared__ int carry;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1085,10 +1215,23 @@ __global__ __launch_bounds__(kCompactThreads) void compact_active_rows(const flo
       counts[b] = left < 0 ? 0 : (left > block ? block : (int)left);
     }
   }
+  for (int b = wave; b < nblocks; b += kCompactThreads / 64) {  // lane l rates l + 1 splits; the cheapest, of equals the fewest, wins
+    const long long left = (long long)n - (long long)b * block;
+    const int tokens = left < 0 ? 0 : (left > block ? block : (int)left);
+    long long best = split_cost(split, tokens, lane + 1);
+    int splits = lane + 1;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const long long c = __shfl_xor(best, o, 64);
+      const int k = __shfl_xor(splits, o, 64);
+      if (c < best || (c == best && k < splits)) best = c, splits = k;
+    }
+    if (lane == 0) counts[1 + nblocks + b] = splits;
+  }
 }
 
 // One workgroup per row r < T: as compacted row r (when r < n) it copies the inputs of token idx[r]; as token r it clears
-// d_hidden[r] -- active tokens get their row from scatter_active_rows afterwards.
+// d_hidden[r] -- active tokens get their row from the dHidden GEMM (or the sum over its splits) afterwards.
 __global__ __launch_bounds__(256) void gather_active_rows(const int* __restrict__ idx, const int* __restrict__ counts,
                                                           const uint16_t* __restrict__ hidden, int ldh, int Hk, int H,
                                                           const int64_t* __restrict__ labels, const float* __restrict__ lse,
@@ -1111,16 +1254,6 @@ __global__ __launch_bounds__(256) void gather_active_rows(const int* __restrict_
     g_c[r] = g[t];
     if (q) q_c[r] = q[t], pz_c[r] = pz[t];
   }
-}
-
-__global__ __launch_bounds__(256) void scatter_active_rows(const int* __restrict__ idx, const int* __restrict__ counts,
-                                                           const uint16_t* __restrict__ d_hidden_c, int H,
-                                                           uint16_t* __restrict__ d_hidden) {
-  const int r = blockIdx.x;
-  if (r >= counts[0]) return;
-  const uint16_t* src = d_hidden_c + (size_t)r * (size_t)H;
-  uint16_t* dst = d_hidden + (size_t)idx[r] * (size_t)H;
-  for (int c = threadIdx.x * 8; c < H; c += 256 * 8) *(uint4*)(dst + c) = *(const uint4*)(src + c);
 }
 
 // What the bf16 product dropped of the label's dz value d (see DzArgs::label_resid), added to the weight gradient in fp32:
@@ -1158,15 +1291,15 @@ __global__ __launch_bounds__(256) void zero_f32(float* __restrict__ p, int n) {
 // HIP events on the launch stream.  Closed profiles cost one thread-local load per launch.
 enum KernelKind {
   kFwdTiles = 0, kFwdMerge, kTranspose, kBwdChunkDz, kBwdChunkGemm, kSoftCePack, kSoftCeFwdTiles, kSoftCeFinish, kSoftCeDz,
-  kCompactRows, kSplitOperand, kTopkFilter, kTopkSelect, kTopkRows, kTopkBwdRows,
+  kCompactRows, kSplitOperand, kTopkFilter, kTopkSelect, kTopkRows, kTopkBwdRows, kDhReduce,
   kNumKernelKinds
 };
 const char* const kKernelNames[kNumKernelKinds] = {"lmhead_fwd_tiles", "lmhead_fwd_merge", "transpose_bf16",
                                                    "lmhead_bwd_dz", "lmhead_bwd_gemm", "softce_pack_rows",
                                                    "softce_fwd_tiles", "softce_finish", "softce_dz_tiles",
-                                                   "active_rows[compact+gather+scatter]", "split_operand_rows",
+                                                   "active_rows[compact+gather]", "split_operand_rows",
                                                    "topk_filter_tiles", "topk_select", "topk_softce_rows",
-                                                   "topk_softce_bwd_rows"};
+                                                   "topk_softce_bwd_rows", "lmhead_dh_reduce"};
 struct Profile {
   struct Rec {
     int kind;
@@ -1279,12 +1412,44 @@ int64_t list_schedule(int64_t count_a, int64_t len_a, int64_t count_b, int64_t l
 // chunk -- dz tiles of H/64 k-tiles plus an epilogue, then dHidden tiles of chunk/64 and dW tiles of T'/64 k-tiles,
 // list-scheduled over the CUs, plus a fixed cost per launch -- and the cheapest wins.  At the 7B shape (T = 16384, H = 3584)
 // that is 49152 columns: 4096 x 3 dz tiles and 896 + 2688 GEMM tiles per launch, both multiples of 256 CUs.
+SplitProblem split_problem(int64_t T, int64_t H, int64_t vc, bool want_dw, int64_t slots, int ncu) {
+  const int64_t tiles_h = (H + BN - 1) / BN;
+  return SplitProblem{(int)tiles_h, (int)(vc / (2 * BK)), want_dw ? (int)(tiles_h * (vc / BM)) : 0, (int)slots, ncu};
+}
+
+// Slab tiles of dHidden partial sums for at most T tokens and chunks of vc columns.  A launch with 192 dHidden tiles or more keeps
+// three quarters of the CUs busy with them and is not given more; below that there is room for one tile per CU.
+constexpr int64_t kSplitBelowTiles = 192;
+int64_t slab_slots(int64_t T, int64_t H, int64_t vc) {
+  const int64_t tiles = (T + BM - 1) / BM * ((H + BN - 1) / BN), most = vc / (2 * BK) / kMinSplitPairs;
+  if (tiles >= kSplitBelowTiles || most < 2) return tiles;
+  const int64_t room = 2 * tiles > 256 ? 2 * tiles : 256;
+  const int64_t used = tiles * (most < kMaxSplits ? most : kMaxSplits);
+  return room < used ? room : used;
+}
+
+int best_splits(const SplitProblem& p, int64_t tokens) {
+  int best = 1;
+  int64_t best_cost = split_cost(p, (int)tokens, 1);
+  for (int k = 2; k <= kMaxSplits; ++k) {
+    const int64_t c = split_cost(p, (int)tokens, k);
+    if (c < best_cost) best = k, best_cost = c;
+  }
+  return best;
+}
+
 int64_t default_vocab_chunk(int64_t T, int64_t H, int64_t V) {
   const int64_t Tpad = round_up(T, 256), Vpad = round_up(V, 256), Hpad = round_up(H, 256);
   const int ncu = compute_units();
   const int64_t tiles_t = Tpad / 256, tiles_h = Hpad / 256;
   const int64_t kDzEpilogue = 8, kGemmEpilogue = 6, kLaunch = 24;  // in k-tiles (about 1.3 us each)
   const int64_t kMaxPanelBytes = (int64_t)3 << 29;  // of dz values, before the row padding
+  // Few dHidden tiles: their contraction is split over the CUs (split_cost), whole rounds no longer depend on the width, and the
+  // fewest chunks are the cheapest.
+  if (tiles_h * tiles_t < kSplitBelowTiles) {
+    const int64_t widest = kMaxPanelBytes / (Tpad * 2) / 2048 * 2048, chunks = (Vpad + widest - 1) / widest;
+    return round_up((Vpad + chunks - 1) / chunks, 256);
+  }
   int64_t best_vc = 0, best_cost = 0;
   for (int64_t vc = 2048;; vc += 2048) {
     if (vc > Vpad) vc = Vpad;
@@ -1393,10 +1558,11 @@ struct BwdWorkspace {
   uint16_t *Wt, *Ht, *D;
   float *dHacc, *dWsum, *label_resid;
   // only with row compaction (skyrl_lmhead_bwd_active_rows):
-  uint16_t *hidden_c, *d_hidden_c;
+  uint16_t* hidden_c;
   int64_t* labels_c;
   float *lse_c, *pz_c, *g_c, *q_c;
   int *idx, *counts;
+  int64_t slots;  // slab tiles dHacc holds
   size_t bytes;
 };
 
@@ -1427,21 +1593,24 @@ BwdWorkspace carve_bwd(void* ws, int64_t T, int64_t H, int64_t Hk, int64_t V, in
   // callers may have sized their scratch by the documented formula.  It is only written below kInPlaceMinVocab.
   w.Wt = V % (2 * BK) == 0 ? nullptr : c.take<uint16_t>((size_t)H * (Vpad + kLdPad));
   w.Ht = c.take<uint16_t>((size_t)H * (Tpad + kLdPad));
-  w.dHacc = c.take<float>((size_t)Tpad * round_up(H, 256));  // accumulator order, whole tiles
+  // dHidden partial sums in accumulator order, whole tiles.  The row-compacting entry point has more room for them: its token
+  // count, and with it the number of tiles, may be far below T.
+  const int64_t slab_floats = slab_slots(Tb, H, vc) * kSlabTileFloats + (compact ? T * H / 2 : 0);
+  w.slots = slab_floats / kSlabTileFloats;
+  w.dHacc = c.take<float>((size_t)slab_floats);
   w.D = c.take<uint16_t>((size_t)Tpad * (vc + kLdPad));
   // Several blocks and a bf16 dW: the sum over the blocks is kept in fp32 here and rounded once, by the last block.
   w.dWsum = bwd_num_blocks(T) > 1 ? c.take<float>((size_t)V * (size_t)H) : nullptr;
   w.label_resid = Hk > H ? c.take<float>((size_t)Tpad) : nullptr;  // stacked terms: fp32 operands
   if (compact) {
     w.hidden_c = c.take<uint16_t>((size_t)T * (size_t)Hk);
-    w.d_hidden_c = c.take<uint16_t>((size_t)T * (size_t)H);
     w.labels_c = c.take<int64_t>((size_t)T);
     w.lse_c = c.take<float>((size_t)T);
     w.pz_c = c.take<float>((size_t)T);
     w.g_c = c.take<float>((size_t)T);
     w.q_c = c.take<float>((size_t)T);
     w.idx = c.take<int>((size_t)T);
-    w.counts = c.take<int>((size_t)bwd_num_blocks(T) + 1);
+    w.counts = c.take<int>((size_t)bwd_num_blocks(T) * 2 + 1);
   }
   w.bytes = (size_t)round_up((int64_t)c.off, 256);
   return w;
@@ -1449,12 +1618,33 @@ BwdWorkspace carve_bwd(void* ws, int64_t T, int64_t H, int64_t Hk, int64_t V, in
 
 GemmArgs make_gemm(const uint16_t* A, int64_t lda, int64_t a_rows, const uint16_t* B, int64_t ldb, int64_t b_rows, bool b_kmajor,
                    bool c_rows_m, int64_t nk, int64_t M, int64_t N, const float* Cin, float* Cf, uint16_t* Cb, int64_t ldc,
-                   const float* Pin = nullptr, float* Pout = nullptr, const int* T_dev = nullptr, int t_role = 0) {
-  return GemmArgs{A,       (int)lda, (int)a_rows, B,  (int)ldb, (int)b_rows, b_kmajor ? 1 : 0, c_rows_m ? 1 : 0, (int)nk,
-                  (int)M,  (int)N,   Cin,         Cf, Cb,       (int)ldc,    Pin,              Pout, T_dev, t_role, 0, 0x7fffffff, 0};
+                   const int* T_dev = nullptr, int t_role = 0) {
+  GemmArgs g{};
+  g.A = A, g.lda = (int)lda, g.a_rows = (int)a_rows, g.B = B, g.ldb = (int)ldb, g.b_rows = (int)b_rows;
+  g.b_kmajor = b_kmajor ? 1 : 0, g.c_rows_m = c_rows_m ? 1 : 0, g.nk = (int)nk, g.M = (int)M, g.N = (int)N;
+  g.Cin = Cin, g.Cf = Cf, g.Cb = Cb, g.ldc = (int)ldc;
+  g.splits = 1, g.T_dev = T_dev, g.t_role = t_role, g.n_tail = 0x7fffffff;
+  return g;
 }
 
 unsigned gemm_tiles(const GemmArgs& g) { return (unsigned)(((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN)); }
+
+// dHidden of one vocab chunk, C[t, h] (+)= sum_v D[t, v] . weight[vc0 + v, h].  In place: A = D rows (K = vocab, contiguous), B =
+// weight rows vc0.. read K-major; the k extent stops at the end of V's last group of 128.  Otherwise (a small vocabulary with a
+// transposed copy): C[h, t] with A = weight^T rows, B = D rows, and no splits.
+GemmArgs dhidden_gemm(const uint16_t* D, int64_t ldd, int64_t d_rows, const uint16_t* W, int64_t ldw, const uint16_t* Wt,
+                      int64_t ldwt, int64_t vc0, int64_t vcw, int64_t V, int64_t T, int64_t H, uint16_t* d_hidden, float* slabs,
+                      bool first, bool last, const int* T_dev) {
+  const VocabTail tail = vocab_tail(V);
+  const int64_t kext = round_up((V - vc0) < vcw ? (V - vc0) : vcw, 2 * BK);
+  GemmArgs g = Wt ? make_gemm(Wt + vc0, ldwt, H, D, ldd, d_rows, false, false, vcw / BK, H, T, nullptr, nullptr, d_hidden, H, T_dev,
+                              kTokensOnN)
+                  : make_gemm(D, ldd, d_rows, W + (size_t)vc0 * (size_t)ldw, ldw, H, true, true, kext / BK, T, H, nullptr, nullptr,
+                              d_hidden, H, T_dev, kTokensOnM);
+  g.P = slabs, g.p_first = first, g.p_last = last;
+  if (last) g.k_back = tail.back;
+  return g;
+}
 
 hipError_t launch_bwd_dz(hipStream_t s, bool entgrad, const DzArgs& z, unsigned dz_tiles) {
   Timed timed(kBwdChunkDz, s);
@@ -1472,11 +1662,26 @@ hipError_t launch_bwd_dz(hipStream_t s, bool entgrad, const DzArgs& z, unsigned 
 
 // Both problems (p1 may be empty) must have an even number of k-tiles: every caller contracts over padded extents that
 // are multiples of 256, or over vocabulary rows that reads_weight_in_place() admits.
-hipError_t launch_bwd_gemm(hipStream_t s, const GemmArgs& p0, const GemmArgs& p1) {
+// slots: slab tiles there is room for, which bounds splits * tiles when the splits are chosen on the device.
+hipError_t launch_bwd_gemm(hipStream_t s, const GemmArgs& p0, const GemmArgs& p1, int64_t slots) {
   if ((p0.nk & 1) || (p1.nk & 1)) return hipErrorInvalidValue;
-  const unsigned t0 = gemm_tiles(p0), t1 = gemm_tiles(p1);
+  unsigned t0 = gemm_tiles(p0) * (unsigned)p0.splits;
+  if (p0.splits_dev && (int64_t)t0 < slots) t0 = (unsigned)slots;
+  const unsigned t1 = gemm_tiles(p1);
   Timed timed(kBwdChunkGemm, s);
   hipLaunchKernelGGL(lmhead_bwd_gemm, dim3(t0 + t1), dim3(NTHREADS), 0, s, p0, p1, (int)t0);
+  return hipGetLastError();
+}
+
+// The sum over the slabs of a split dHidden contraction; g is the GEMM of the last chunk.
+hipError_t launch_dh_reduce(hipStream_t s, const GemmArgs& g, int64_t slots) {
+  if (!g.splits_dev && g.splits < 2) return hipSuccess;
+  // only a problem with at most half as many tiles as slots is ever split
+  const int64_t tiles = gemm_tiles(g), most = g.splits_dev && slots / 2 < tiles ? slots / 2 : tiles;
+  if (most < 1) return hipSuccess;
+  Timed timed(kDhReduce, s);
+  hipLaunchKernelGGL(lmhead_dh_reduce, dim3((unsigned)(most * kReduceGroups)), dim3(256), 0, s,
+                     DhReduceArgs{g.P, g.M, g.N, g.splits, g.T_dev, g.splits_dev, g.row_map, g.Cb, g.ldc});
   return hipGetLastError();
 }
 
@@ -1507,6 +1712,7 @@ SoftCeFwdWorkspace carve_softce_fwd(void* ws, int64_t T, int64_t H, int64_t V) {
 struct SoftCeBwdWorkspace {
   uint16_t *S, *Wt, *D;
   float* dHacc;
+  int64_t slots;
   size_t bytes;
 };
 
@@ -1516,7 +1722,8 @@ SoftCeBwdWorkspace carve_softce_bwd(void* ws, int64_t T, int64_t H, int64_t V, i
   SoftCeBwdWorkspace w;
   w.S = c.take<uint16_t>((size_t)(2 * Tp) * (size_t)H);
   w.Wt = V % (2 * BK) == 0 ? nullptr : c.take<uint16_t>((size_t)H * (Vpad + kLdPad));  // as in carve_bwd
-  w.dHacc = c.take<float>((size_t)round_up(T, 256) * round_up(H, 256));
+  w.slots = slab_slots(T, H, vc);
+  w.dHacc = c.take<float>((size_t)(w.slots * kSlabTileFloats));
   w.D = c.take<uint16_t>((size_t)Tp * (vc + kLdPad));
   w.bytes = (size_t)round_up((int64_t)c.off, 256);
   return w;
@@ -1587,7 +1794,8 @@ size_t bwd_workspace_bytes(int64_t T, int64_t H, int64_t V, int64_t vocab_chunk,
 // epilogue as  (Cin ? Cin : 0) + product  ->  Cf (fp32) and / or Cb (bf16), each a [V, H] matrix or NULL.
 int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, int64_t ld_weight, const int64_t* labels,
                     const float* row_lse, const float* row_pz, const float* dlogprobs, const float* dentropy, int64_t Tb,
-                    const int* T_dev, int64_t H, int64_t Hk, int64_t V, float rcp_temperature, uint16_t* d_hidden, bool want_dw,
+                    const int* T_dev, const int* splits_dev, const int* row_map, int64_t H, int64_t Hk, int64_t V,
+                    float rcp_temperature, uint16_t* d_hidden, bool want_dw,
                     const float* dw_in, float* dw_f32, uint16_t* dw_bf16, int64_t vc, const BwdWorkspace& w, float p_shift,
                     hipStream_t s) {
   const int64_t Tpad = round_up(Tb, 256), Vpad = round_up(V, 256);
@@ -1607,6 +1815,9 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
   }
   const int tiles_t = (int)(Tpad / 256);
   const VocabTail tail = vocab_tail(V);
+  // The splits are those of a full chunk: the slabs are carried from chunk to chunk.
+  const int splits =
+      !T_dev && w_in_place ? best_splits(split_problem(Tb, H, vc < Vpad ? vc : Vpad, want_dw, w.slots, compute_units()), Tb) : 1;
   const int64_t nchunks = (Vpad + vc - 1) / vc;
   auto chunk_width = [&](int64_t ci) { return (Vpad - ci * vc) < vc ? (Vpad - ci * vc) : vc; };  // multiple of 256
   const GemmArgs none{};
@@ -1625,29 +1836,20 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
     const int64_t rows = (V - vc0) < vcw ? (V - vc0) : vcw;
     // dW rows are complete within their chunk (for this token block), so they can leave the GEMM epilogue in either precision.
     const size_t dw_off = (size_t)vc0 * (size_t)H;
-    uint16_t* dh_out = last ? d_hidden : (uint16_t*)nullptr;
-    const float* dh_in = first ? (const float*)nullptr : (const float*)w.dHacc;
-    float* dh_keep = last ? (float*)nullptr : w.dHacc;
-    // In place: C[t, h] with A = D rows (K = vocab, contiguous), B = weight rows vc0.. read K-major; the k extent stops at the
-    // end of V's last group of 128.  Otherwise: C[h, t] with A = weight^T rows, B = D rows.  The partial sums are in accumulator
-    // order either way.
-    const int64_t kext = round_up(rows, 2 * BK);
-    GemmArgs gh =
-        w_in_place ? make_gemm(w.D, vcw + kLdPad, Tpad, Wp + (size_t)vc0 * (size_t)ld_weight, ld_weight, H, true, true, kext / BK, Tb,
-                               H, nullptr, nullptr, dh_out, H, dh_in, dh_keep, T_dev, kTokensOnM)
-                   : make_gemm(w.Wt + vc0, Vpad + kLdPad, H, w.D, vcw + kLdPad, Tpad, false, false, vcw / BK, H, Tb, nullptr,
-                               nullptr, dh_out, H, dh_in, dh_keep, T_dev, kTokensOnN);
+    GemmArgs gh = dhidden_gemm(w.D, vcw + kLdPad, Tpad, Wp, ld_weight, w_in_place ? nullptr : w.Wt, Vpad + kLdPad, vc0, vcw, V, Tb, H,
+                               d_hidden, w.dHacc, first, last, T_dev);
+    gh.splits = splits, gh.splits_dev = w_in_place ? splits_dev : nullptr, gh.row_map = row_map;
     // A frozen LM head needs no dW: the launch then carries the dHidden tiles alone.
     const bool moved = last && tail.back > 0;  // the chunk ends with a moved group
-    if (moved) gh.k_back = tail.back;
-    GemmArgs gw = want_dw ? make_gemm(w.Ht, Tpad + kLdPad, H, w.D, vcw + kLdPad, vcw, true, false, Tpad / BK, H, moved ? kext : rows,
+    GemmArgs gw = want_dw ? make_gemm(w.Ht, Tpad + kLdPad, H, w.D, vcw + kLdPad, vcw, true, false, Tpad / BK, H,
+                                            moved ? round_up(rows, 2 * BK) : rows,
                                             dw_in ? dw_in + dw_off : (const float*)nullptr,
                                             dw_f32 ? dw_f32 + dw_off : (float*)nullptr,
-                                            dw_bf16 ? dw_bf16 + dw_off : (uint16_t*)nullptr, H, nullptr, nullptr, T_dev,
-                                            kTokensOnK)
+                                            dw_bf16 ? dw_bf16 + dw_off : (uint16_t*)nullptr, H, T_dev, kTokensOnK)
                                 : none;
     if (moved && want_dw) gw.n_tail = (int)(tail.from - vc0), gw.n_back = tail.back;
-    e = launch_bwd_gemm(s, gh, gw);
+    e = launch_bwd_gemm(s, gh, gw, w.slots);
+    if (e == hipSuccess && last) e = launch_dh_reduce(s, gh, w.slots);
     if (e != hipSuccess) return (int)e;
   }
   if (resid) {
@@ -1694,7 +1896,7 @@ int bwd_entry(const void* hidden, int64_t ld_hidden, const void* weight, int64_t
   if (compact) {
     Timed timed(kCompactRows, s);
     hipLaunchKernelGGL(compact_active_rows, dim3(1), dim3(kCompactThreads), 0, s, dlogprobs, dentropy, (int)T, (int)Tb,
-                       (int)nblocks, w.idx, w.counts);
+                       (int)nblocks, split_problem(Tb, H, vc, d_weight != nullptr, w.slots, compute_units()), w.idx, w.counts);
     hipLaunchKernelGGL(gather_active_rows, dim3((unsigned)T), dim3(256), 0, s, (const int*)w.idx, (const int*)w.counts, Hp,
                        (int)ld_hidden, (int)Hk, (int)H, labels, row_lse, row_pz, dlogprobs, dentropy, w.hidden_c, w.labels_c,
                        w.lse_c, w.pz_c, w.g_c, w.q_c, (uint16_t*)d_hidden);
@@ -1732,21 +1934,15 @@ int bwd_entry(const void* hidden, int64_t ld_hidden, const void* weight, int64_t
     if (compact) {
       st = bwd_token_block(w.hidden_c + (size_t)t0 * (size_t)Hk, Hk, Wp, ld_weight, w.labels_c + t0, w.lse_c + t0,
                            dentropy ? w.pz_c + t0 : nullptr, w.g_c + t0, dentropy ? w.q_c + t0 : nullptr, Tcur,
-                           w.counts + 1 + b, H, Hk, V, rcp_temperature, w.d_hidden_c + (size_t)t0 * (size_t)H, d_weight != nullptr,
-                           dw_in, dw_f32, dw_bf16, vc, w, p_shift, s);
+                           w.counts + 1 + b, w.counts + 1 + nblocks + b, w.idx + t0, H, Hk, V, rcp_temperature, (uint16_t*)d_hidden,
+                           d_weight != nullptr, dw_in, dw_f32, dw_bf16, vc, w, p_shift, s);
     } else {
       st = bwd_token_block(Hp + (size_t)t0 * (size_t)ld_hidden, ld_hidden, Wp, ld_weight, labels + t0, row_lse + t0,
-                           row_pz ? row_pz + t0 : nullptr, dlogprobs + t0, dentropy ? dentropy + t0 : nullptr, Tcur, nullptr, H,
-                           Hk, V, rcp_temperature, (uint16_t*)d_hidden + (size_t)t0 * (size_t)H, d_weight != nullptr, dw_in, dw_f32,
+                           row_pz ? row_pz + t0 : nullptr, dlogprobs + t0, dentropy ? dentropy + t0 : nullptr, Tcur, nullptr,
+                           nullptr, nullptr, H, Hk, V, rcp_temperature, (uint16_t*)d_hidden + (size_t)t0 * (size_t)H, d_weight != nullptr, dw_in, dw_f32,
                            dw_bf16, vc, w, p_shift, s);
     }
     if (st) return st;
-  }
-  if (compact) {
-    Timed timed(kCompactRows, s);
-    hipLaunchKernelGGL(scatter_active_rows, dim3((unsigned)T), dim3(256), 0, s, (const int*)w.idx, (const int*)w.counts,
-                       (const uint16_t*)w.d_hidden_c, (int)H, (uint16_t*)d_hidden);
-    if ((e = hipGetLastError()) != hipSuccess) return (int)e;
   }
   return SKYRL_LMHEAD_OK;
 }
@@ -1956,6 +2152,7 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
   if (e != hipSuccess) return (int)e;
   const bool w_in_place = reads_weight_in_place(V);
   const VocabTail tail = vocab_tail(V);
+  const int splits = w_in_place ? best_splits(split_problem(T, H, vc, false, w.slots, compute_units()), T) : 1;
   if (!w_in_place) {
     Timed timed(kTranspose, s);
     hipLaunchKernelGGL(transpose_bf16, dim3((unsigned)(Vpad / 64), (unsigned)(H / 64)), dim3(256), 0, s, Wp, (int)ld_weight,
@@ -1977,17 +2174,11 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
     // d student hidden [t, h] (+)= sum_v D[t, v] . weight[vc0 + v, h]: the dHidden GEMM of the log-probability backward,
     // partial sums carried from chunk to chunk in accumulator order, bf16 rows written by the last chunk.
     const bool first = ci == 0, last = ci == nchunks - 1;
-    uint16_t* dh_out = last ? (uint16_t*)d_student_hidden : (uint16_t*)nullptr;
-    const float* dh_in = first ? (const float*)nullptr : (const float*)w.dHacc;
-    float* dh_keep = last ? (float*)nullptr : w.dHacc;
-    const int64_t kext = round_up((V - vc0) < vcw ? (V - vc0) : vcw, 2 * BK);
-    GemmArgs gh =
-        w_in_place ? make_gemm(w.D, vcw + kLdPad, Tp, Wp + (size_t)vc0 * (size_t)ld_weight, ld_weight, H, true, true, kext / BK, T,
-                               H, nullptr, nullptr, dh_out, H, dh_in, dh_keep)
-                   : make_gemm(w.Wt + vc0, Vpad + kLdPad, H, w.D, vcw + kLdPad, Tp, false, false, vcw / BK, H, T, nullptr,
-                               nullptr, dh_out, H, dh_in, dh_keep);
-    if (last && tail.back > 0) gh.k_back = tail.back;
-    e = launch_bwd_gemm(s, gh, none);
+    GemmArgs gh = dhidden_gemm(w.D, vcw + kLdPad, Tp, Wp, ld_weight, w_in_place ? nullptr : w.Wt, Vpad + kLdPad, vc0, vcw, V, T, H,
+                               (uint16_t*)d_student_hidden, w.dHacc, first, last, nullptr);
+    gh.splits = splits;
+    e = launch_bwd_gemm(s, gh, none, w.slots);
+    if (e == hipSuccess && last) e = launch_dh_reduce(s, gh, w.slots);
     if (e != hipSuccess) return (int)e;
   }
   return SKYRL_LMHEAD_OK;

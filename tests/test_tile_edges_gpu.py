@@ -65,3 +65,29 @@ def test_vocabulary_that_ends_inside_a_group(V, vc, dtype, cuda_device):
         zs, zt = hidden.double() @ weight.double().t(), teacher.roll(-1, dims=1).reshape(T, H).double() @ weight.double().t()
         want = (g.double()[:, None] * (zs.softmax(-1) - zt.softmax(-1))) @ weight.double()
         _close(s.grad.reshape(T, H), want, f"draft loss V={V}")
+
+
+# The dHidden contraction is split over workgroups when there are few tiles: one token tile and as many splits as the vocabulary
+# allows, several chunks, a last chunk with fewer k-tile pairs than splits (one split has nothing to add), hidden columns that
+# overhang a tile, and a count of active rows far below the number of tokens (down to none).
+@pytest.mark.parametrize("T,H,V,vc", [(40, 64, 20000, 0), (700, 128, 4224, 2048), (257, 320, 8192, 0), (513, 192, 6001, 2048)])
+@pytest.mark.parametrize("keep", [1.0, 0.3, 0.0])
+def test_split_hidden_gradient(T, H, V, vc, keep, cuda_device):
+    hidden, weight, labels, g, q = _operands(T, H, V, seed=T + V)
+    keep_rows = torch.rand(T, generator=torch.Generator().manual_seed(T)) < keep
+    g, q = g * keep_rows, q * keep_rows
+    h, w, y, gd, qd = (x.to(cuda_device) for x in (hidden, weight, labels, g, q))
+    _, _, lse, pz = ops.lmhead_fwd(h, w, y, 1.0, True)
+    dense = ops.lmhead_bwd_bf16(h, w, y, lse, pz, gd, qd, 1.0, vc)
+    active = ops.lmhead_bwd_bf16(h, w, y, lse, pz, gd, qd, 1.0, vc, True)
+    frozen = ops.lmhead_bwd_hidden(h, w, y, lse, pz, gd, qd, 1.0, vc, True)
+    if keep == 0.0:
+        assert all(not t.any() for t in (*dense, *active, frozen))
+        return
+    ex = O.exact_fwd_bwd(hidden, weight, labels, 1.0, g, q)
+    for dh in (dense[0], active[0], frozen):
+        _close(dh, ex["d_hidden"], f"dHidden T={T} H={H} V={V} chunk={vc}")
+        assert not dh[(~keep_rows).to(cuda_device)].any()
+    for dw in (dense[1], active[1]):
+        _close(dw, ex["d_weight"], f"dW T={T} H={H} V={V} chunk={vc}")
+    assert torch.equal(active[0], ops.lmhead_bwd_bf16(h, w, y, lse, pz, gd, qd, 1.0, vc, True)[0])   # a fixed order of addition
