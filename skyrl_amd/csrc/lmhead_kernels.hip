@@ -5,7 +5,7 @@
 //                      scale by 1/temperature, per-token max / sum-exp / sum (z-max)*exp over the tile's vocab rows;
 //                      writes one (max, sum, pz) partial per token per 128-row half tile, in blocks of 64 tokens.  Logits
 //                      never leave VGPRs.
-//   lmhead_fwd_merge   per block of 64 tokens: merges the partials (online log-sum-exp), gathers the label logit with an
+//   lmhead_fwd_merge   per 16 tokens: merges the partials (online log-sum-exp), gathers the label logit with an
 //                      fp32 dot product hidden[t] . weight[label], writes logprob / entropy / lse / pz.
 // Backward (6*T*V*H flop), looped over vocab chunks of `vocab_chunk` columns:
 //   transpose_bf16     hidden^T once per call (and weight^T only for small vocabularies that are not multiples of 128).
@@ -193,36 +193,54 @@ __global__ __launch_bounds__(NTHREADS) void lmhead_fwd_tiles(const uint16_t* __r
 }
 
 // ------------------------------------------------------------------------------------------------------------
-// Forward merge.  One workgroup of 16 waves per block of 64 tokens: lane = token, wave w merges parts w, w + 16, ... of that
-// token (every load of a wave is 256 contiguous bytes), the sixteen running triples meet in LDS; then sixteen lanes per
-// token gather the label logit.
+// Forward merge.  One workgroup of 16 waves per 16 tokens: lane = (token, part mod 4), wave w merges parts 4w .. 4w + 3, then
+// every 64th of them (a load is 64 contiguous bytes of four parts), the running triples meet in shuffles and in LDS.  Wave w
+// also takes the label logit of token w, 64 lanes to the dot product.
+// What bounds it: 12 bytes per part and token and two rows per label from HBM for many tokens, the chain of load and merge steps
+// for few.  Sixty-four streams per token and 24 loads in flight per lane keep that chain at three steps for 1188 parts (16
+// streams of 64-token blocks: 19), and one exponential per part instead of two.  V=151936: 35 -> 11 us at T=137, 40 -> 13 at
+// T=611, 39 -> 14 at T=2048 with entropy, 50 -> 34 at T=8192 with entropy; 83 -> 81 us at T=16384, H=3584 (5.8 TB/s).
 // Merge algebra as in efficient_entropy_triton_kernel_epilogue (fused_linear_logprob_triton.py:417-467) except that
 // the running max starts at -inf (that kernel starts it at 0, which loses rows whose logits are all << 0).
 // Out-of-range labels give logprob 0 (model_utils.py:337; fused_linear_logprob_triton.py:1898-1905).
 // ------------------------------------------------------------------------------------------------------------
-constexpr int kMergeTokens = kPartTokens;
+constexpr int kMergeTokens = 16;
 constexpr int kMergeThreads = 1024;
 constexpr int kMergeWaves = kMergeThreads / 64;
-constexpr int kDotLanes = kMergeThreads / kMergeTokens;  // lanes per token in the label-logit phase
+static_assert(kMergeWaves == kMergeTokens && kPartTokens % kMergeTokens == 0, "one wave per token for the label logit");
 
-// Two partial triples (maximum, sum e^(z - max), third statistic) of one token become one.  RELATIVE: the third statistic
-// is sum (z - max) e^(z - max) and moves with the maximum, e' = c (e + (max - max') s); otherwise it is sum y e^(z - max) of
-// some y that does not depend on the maximum and only scales.
+// Partial triples (maximum, sum e^(z - max), third statistic) of one token become one.  RELATIVE: the third statistic is
+// sum (z - max) e^(z - max) and moves with the maximum, e' = c (e + (max - max') s); otherwise it is sum y e^(z - max) of some y that
+// does not depend on the maximum and only scales.  A part without a single vocabulary row has maximum -inf and adds nothing.
+// One exponential per part, taken relative to the largest maximum of the batch: the parts of a batch do not wait for each
+// other.  (2^(d log2 e) through v_exp_f32: its relative error grows with |d|, the part's weight falls faster; |d| e^d < 0.4.)
+template <bool RELATIVE, int N>
+__device__ __forceinline__ void merge_partials(float& M, float& S, float& E, const float (&m)[N], const float (&s)[N],
+                                               const float (&e)[N]) {
+  float top = M;
+#pragma unroll
+  for (int u = 0; u < N; ++u) top = fmaxf(top, m[u]);
+  if (!(top > -INFINITY)) return;
+  auto add = [&](float mu, float su, float eu, float& sum_s, float& sum_e) {
+    const float d = fmaxf(mu - top, -1.0e30f);  // finite: an empty part has s = e = 0
+    const float c = __builtin_amdgcn_exp2f(d * kLog2e);
+    // Explicit fused multiply-adds: which products the compiler would contract is its choice, and it need not make the same one
+    // in every build.
+    sum_s = fmaf(su, c, sum_s);
+    sum_e = fmaf(RELATIVE ? fmaf(d, su, eu) : eu, c, sum_e);
+  };
+  float sum_s = 0.f, sum_e = 0.f;
+  add(M, S, E, sum_s, sum_e);
+#pragma unroll
+  for (int u = 0; u < N; ++u) add(m[u], s[u], e[u], sum_s, sum_e);
+  M = top, S = sum_s, E = sum_e;
+}
+
+// The triple of lane ^ o joins this lane's.
 template <bool RELATIVE>
-__device__ __forceinline__ void merge_partial(float& M, float& S, float& E, float m, float s, float e) {
-  if (!(m > -INFINITY)) return;  // a part without a single vocabulary row
-  if (!(M > -INFINITY)) {
-    M = m, S = s, E = e;
-    return;
-  }
-  const float Mn = fmaxf(M, m);
-  const float da = M - Mn, db = m - Mn;
-  const float ca = expf(da), cb = expf(db);
-  // Explicit fused multiply-adds: which of the two products of a * b + c * d the compiler would contract is its choice, and it
-  // need not make the same one in every build.
-  E = RELATIVE ? fmaf(ca, fmaf(da, S, E), cb * fmaf(db, s, e)) : fmaf(E, ca, e * cb);
-  S = fmaf(S, ca, s * cb);
-  M = Mn;
+__device__ __forceinline__ void merge_lanes(float& M, float& S, float& E, int o) {
+  const float m[1] = {__shfl_xor(M, o, 64)}, s[1] = {__shfl_xor(S, o, 64)}, e[1] = {__shfl_xor(E, o, 64)};
+  merge_partials<RELATIVE>(M, S, E, m, s, e);
 }
 
 template <bool RELATIVE>
@@ -235,80 +253,83 @@ __global__ __launch_bounds__(kMergeThreads) void lmhead_fwd_merge(const float* _
                                                                   float* __restrict__ logprobs, float* __restrict__ entropy,
                                                                   float* __restrict__ row_lse, float* __restrict__ row_pz) {
   __shared__ float sm_m[kMergeWaves][kMergeTokens], sm_s[kMergeWaves][kMergeTokens], sm_e[kMergeWaves][kMergeTokens];
-  __shared__ float sm_lse[kMergeTokens], sm_pz[kMergeTokens];
-  const int tid = threadIdx.x;
+  __shared__ float sm_dot[kMergeTokens];
+  __shared__ int sm_has_label[kMergeTokens];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // Four consecutive workgroups read the same cache lines (16 of a block's 64 tokens each): keep them on one XCD.
+  const int t0 = xcd_contiguous(blockIdx.x, gridDim.x) * kMergeTokens;
+  const int64_t y = (labels && t0 + wave < T) ? labels[t0 + wave] : (int64_t)-1;
   {
-    const int lane = tid & 63, wave = tid >> 6;
-    const int t = blockIdx.x * kMergeTokens + lane;
-    const size_t base = (size_t)blockIdx.x * (size_t)nparts * kPartTokens + lane;
+    const int t = t0 + (lane & 15);
+    const size_t base = part_index(0, t, nparts);
     float M = -INFINITY, S = 0.f, E = 0.f;
     if (t < T) {
-      constexpr int kBatch = 4;  // loads in flight per array before the dependent merge chain
-      for (int p0 = wave; p0 < nparts; p0 += kMergeWaves * kBatch) {
+      constexpr int kBatch = 8, kStreams = kMergeWaves * 4;  // loads in flight per array before the dependent merge chain
+      for (int p0 = wave * 4 + (lane >> 4); p0 < nparts; p0 += kStreams * kBatch) {
         float m[kBatch], sv[kBatch], ev[kBatch];
 #pragma unroll
         for (int u = 0; u < kBatch; ++u) {
-          const int p = p0 + u * kMergeWaves;
+          const int p = p0 + u * kStreams;
           const bool in = p < nparts;
           const size_t idx = base + (size_t)(in ? p : p0) * kPartTokens;
-          m[u] = in ? part_max[idx] : -INFINITY;
+          m[u] = part_max[idx];
           sv[u] = part_sum[idx];
           ev[u] = part_pz ? part_pz[idx] : 0.f;
         }
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u) merge_partial<RELATIVE>(M, S, E, m[u], sv[u], ev[u]);
+        for (int u = 0; u < kBatch; ++u)
+          if (p0 + u * kStreams >= nparts) m[u] = -INFINITY, sv[u] = 0.f, ev[u] = 0.f;
+        merge_partials<RELATIVE>(M, S, E, m, sv, ev);
       }
     }
-    sm_m[wave][lane] = M;
-    sm_s[wave][lane] = S;
-    sm_e[wave][lane] = E;
-    __syncthreads();
-    if (wave == 0) {
-      float Mg = -INFINITY, Sg = 0.f, Eg = 0.f;
-      for (int g = 0; g < kMergeWaves; ++g) merge_partial<RELATIVE>(Mg, Sg, Eg, sm_m[g][lane], sm_s[g][lane], sm_e[g][lane]);
-      const float log_s = logf(Sg);
-      sm_lse[lane] = Mg + log_s;
-      // RELATIVE: sm_pz holds the entropy itself, ln s - e / s, and sum p z is recovered as lse - entropy (exactly what the
-      // absolute form would have subtracted the other way round).
-      sm_pz[lane] = RELATIVE ? log_s - Eg / Sg : Eg / Sg;
-    }
-    __syncthreads();
+    merge_lanes<RELATIVE>(M, S, E, 16);
+    merge_lanes<RELATIVE>(M, S, E, 32);
+    if (lane < kMergeTokens) sm_m[wave][lane] = M, sm_s[wave][lane] = S, sm_e[wave][lane] = E;
   }
-  // Label logit: 16 lanes per token, 16-byte loads, fp32 accumulation.
-  const int tl = tid / kDotLanes, sub = tid % kDotLanes;
-  const int t = blockIdx.x * kMergeTokens + tl;
+  // Label logit: 16-byte loads, fp32 accumulation.
   float dot = 0.f;
-  bool has_label = false;
-  if (t < T && labels) {
-    const int64_t y = labels[t];
-    has_label = (y >= 0 && y < (int64_t)V);
-    if (has_label) {
-      const uint16_t* hp = Hd + (size_t)t * (size_t)ldh;
-      const uint16_t* wp = W + (size_t)y * (size_t)ldw;
-      for (int c = sub * 8; c < H; c += kDotLanes * 8) {
-        const uint4 hv = *(const uint4*)(hp + c);
-        const uint4 wv = *(const uint4*)(wp + c);
-        const uint32_t hh[4] = {hv.x, hv.y, hv.z, hv.w};
-        const uint32_t ww[4] = {wv.x, wv.y, wv.z, wv.w};
+  const bool has_label = y >= 0 && y < (int64_t)V;
+  if (has_label) {
+    const uint16_t* hp = Hd + (size_t)(t0 + wave) * (size_t)ldh;
+    const uint16_t* wp = W + (size_t)y * (size_t)ldw;
+#pragma unroll 4
+    for (int c = lane * 8; c < H; c += 64 * 8) {
+      const uint4 hv = *(const uint4*)(hp + c);
+      const uint4 wv = *(const uint4*)(wp + c);
+      const uint32_t hh[4] = {hv.x, hv.y, hv.z, hv.w};
+      const uint32_t ww[4] = {wv.x, wv.y, wv.z, wv.w};
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          dot = fmaf(__uint_as_float(hh[k] << 16), __uint_as_float(ww[k] << 16), dot);
-          dot = fmaf(__uint_as_float(hh[k] & 0xffff0000u), __uint_as_float(ww[k] & 0xffff0000u), dot);
-        }
+      for (int k = 0; k < 4; ++k) {
+        dot = fmaf(__uint_as_float(hh[k] << 16), __uint_as_float(ww[k] << 16), dot);
+        dot = fmaf(__uint_as_float(hh[k] & 0xffff0000u), __uint_as_float(ww[k] & 0xffff0000u), dot);
       }
     }
   }
 #pragma unroll
-  for (int o = 1; o < kDotLanes; o <<= 1) dot += __shfl_xor(dot, o, 64);
-  if (sub == 0 && t < T) {
-    const float lse = sm_lse[tl];
-    const float ent = RELATIVE ? sm_pz[tl] : lse - sm_pz[tl];
-    const float pz = RELATIVE ? lse - sm_pz[tl] : sm_pz[tl];
-    if (logprobs) logprobs[t] = has_label ? dot * rcp_temp - lse : 0.f;
-    if (entropy) entropy[t] = ent;
-    if (row_lse) row_lse[t] = lse;
-    if (row_pz) row_pz[t] = pz;
+  for (int o = 1; o < 64; o <<= 1) dot += __shfl_xor(dot, o, 64);
+  if (lane == 0) sm_dot[wave] = dot, sm_has_label[wave] = has_label;
+  __syncthreads();
+  if (wave != 0) return;
+  const int tl = lane & 15, t = t0 + tl;
+  float M = -INFINITY, S = 0.f, E = 0.f;
+  float wm[kMergeWaves / 4], ws[kMergeWaves / 4], we[kMergeWaves / 4];
+#pragma unroll
+  for (int u = 0; u < kMergeWaves / 4; ++u) {
+    const int w = (lane >> 4) * (kMergeWaves / 4) + u;
+    wm[u] = sm_m[w][tl], ws[u] = sm_s[w][tl], we[u] = sm_e[w][tl];
   }
+  merge_partials<RELATIVE>(M, S, E, wm, ws, we);
+  merge_lanes<RELATIVE>(M, S, E, 16);
+  merge_lanes<RELATIVE>(M, S, E, 32);
+  if (lane >= kMergeTokens || t >= T) return;
+  const float log_s = logf(S), lse = M + log_s;
+  // RELATIVE: the entropy itself, ln s - e / s, comes out of the sums, and sum p z is recovered as lse - entropy (exactly what
+  // the absolute form subtracts the other way round).
+  const float third = RELATIVE ? log_s - E / S : E / S;
+  if (logprobs) logprobs[t] = sm_has_label[tl] ? sm_dot[tl] * rcp_temp - lse : 0.f;
+  if (entropy) entropy[t] = RELATIVE ? third : lse - third;
+  if (row_lse) row_lse[t] = lse;
+  if (row_pz) row_pz[t] = RELATIVE ? lse - third : third;
 }
 
 // ------------------------------------------------------------------------------------------------------------
