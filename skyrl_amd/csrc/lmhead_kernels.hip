@@ -1770,13 +1770,16 @@ hipError_t launch_softce_pack(hipStream_t s, const void* student, int64_t lds_, 
 }
 
 
-// Top-k logits from hidden states.  Tokens are walked in blocks of at most 16384 and the vocabulary in chunks of 1024, 2048,
-// 4096 and then 8192 columns: the first chunk passes every logit (no threshold yet), and from then on a logit passes with
-// probability k / (columns seen so far) on exchangeable columns, so that short early chunks keep the candidate lists short.
-// A candidate list holds a whole chunk (cap columns per token), which makes the filter exact for any data: in the worst
-// case -- logits ascending with the column -- every logit is a candidate and the select kernel does all the work.
+// Top-k logits from hidden states.  Tokens are walked in blocks of at most 16384, the vocabulary in chunks.  The first chunk's
+// logits are stored and searched (topk_init); from then on a logit passes with probability k / (columns seen so far) on
+// exchangeable columns, so a later chunk may be 512 / k times as wide as what was seen before it and still leaves half a bulk
+// round to topk_select.  A candidate list holds a whole chunk (cap columns per token), which makes the filter exact for any
+// data: in the worst case -- logits ascending with the column -- every logit is a candidate and the select kernel does all the
+// work.  What the lists may take, 1 GiB, is shared by the tokens of a block: few tokens mean few, wide chunks and so few launches
+// whose tiles fill whole rounds of the CUs (T=1800, H=2048, V=151936, k=32: 21 chunks, 1.20 + 0.30 ms of tiles and selection -> 3 chunks, 1.11 + 0.08 ms).
 constexpr int64_t kTopkTokenBlock = 16384;
-constexpr int64_t kTopkFirstChunk = 1024, kTopkMaxChunk = 8192;
+constexpr int64_t kTopkListColumns = 8192;  // per token of a full block
+constexpr int64_t kTopkDenseMin = 8192, kTopkDenseMax = 1024 * topk::kInitLogits;
 
 struct TopkWorkspace {
   unsigned *cnt, *have;
@@ -1789,8 +1792,8 @@ struct TopkWorkspace {
 TopkWorkspace carve_topk(void* ws, int64_t T, int64_t V, int64_t k) {
   TopkWorkspace w;
   w.block_tokens = T < kTopkTokenBlock ? T : kTopkTokenBlock;
-  const int64_t vpad = round_up(V, 256);
-  w.cap = vpad < kTopkMaxChunk ? vpad : kTopkMaxChunk;
+  const int64_t vpad = round_up(V, 256), room = kTopkTokenBlock * kTopkListColumns / w.block_tokens / 256 * 256;
+  w.cap = vpad < room ? vpad : room;
   Carver c(ws);
   w.cnt = c.take<unsigned>((size_t)w.block_tokens);
   w.have = c.take<unsigned>((size_t)w.block_tokens);
@@ -2232,22 +2235,41 @@ int skyrl_lmhead_topk_logits(const void* hidden, int64_t ld_hidden, const void* 
     const int64_t Tb = (T - t0) < block_tokens ? (T - t0) : block_tokens;
     const int tiles_n = (int)((Tb + BN - 1) / BN);
     const uint16_t* Hp = (const uint16_t*)hidden + (size_t)t0 * (size_t)ld_hidden;
-    hipLaunchKernelGGL(topk::topk_reset, dim3((unsigned)((Tb + 255) / 256)), dim3(256), 0, s, (int)Tb, w.have, w.thr, w.cnt);
-    if ((e = hipGetLastError()) != hipSuccess) return (int)e;
-    int64_t width = kTopkFirstChunk;
-    for (int64_t v0 = 0; v0 < V;) {
-      const int64_t chunk = width < w.cap ? width : w.cap;
-      const int64_t vrows = (V - v0) < chunk ? (V - v0) : chunk;
-      const bool last = v0 + vrows >= V;
-      topk::FilterArgs a{Wp + (size_t)v0 * (size_t)ld_weight, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)H, (int)vrows,
-                         (int)v0, rcp_temperature, (int)((vrows + BM - 1) / BM), tiles_n, kGroupM, w.thr, w.cnt, w.cand,
-                         (int)w.cap};
-      {
-        Timed timed(kTopkFilter, s);
-        auto kernel = even_ktiles(H) ? topk::topk_filter_tiles<true> : topk::topk_filter_tiles<false>;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(NTHREADS), 0, s, a);
-      }
+    auto chunk_args = [&](int64_t v0, int64_t vrows) {
+      return topk::FilterArgs{Wp + (size_t)v0 * (size_t)ld_weight, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)H, (int)vrows,
+                              (int)v0, rcp_temperature, (int)((vrows + BM - 1) / BM), tiles_n, kGroupM, w.thr, w.cnt, w.cand,
+                              (int)w.cap, (float*)w.cand};
+    };
+    auto launch_tiles = [&](auto kernel, const topk::FilterArgs& a) {
+      Timed timed(kTopkFilter, s);
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(NTHREADS), 0, s, a);
+      return hipGetLastError();
+    };
+    // First chunk: one tile per CU where the stored logits allow it.
+    int64_t dense = round_up(BM * ((256 + tiles_n - 1) / tiles_n), 256);
+    dense = dense < kTopkDenseMin ? kTopkDenseMin : (dense > kTopkDenseMax ? kTopkDenseMax : dense);
+    if (dense > w.cap) dense = w.cap;
+    if (dense > V) dense = V;
+    {
+      const topk::FilterArgs a = chunk_args(0, dense);
+      if ((e = launch_tiles(even_ktiles(H) ? topk::topk_first_tiles<true> : topk::topk_first_tiles<false>, a)) != hipSuccess) return (int)e;
+      Timed timed(kTopkSelect, s);
+      auto init = dense <= 256 * topk::kInitLogits ? topk::topk_init<256> : topk::topk_init<1024>;
+      hipLaunchKernelGGL(init, dim3((unsigned)Tb), dim3(dense <= 256 * topk::kInitLogits ? 256 : 1024), 0, s, (int)k,
+                         (const float*)w.cand, a.tiles_m * BM, (int)dense, w.best, w.have, w.thr, w.cnt);
       if ((e = hipGetLastError()) != hipSuccess) return (int)e;
+    }
+    const int64_t round_columns = tiles_n < 256 ? BM * (256 / tiles_n) : BM;  // columns of a chunk whose tiles fill the CUs once
+    for (int64_t v0 = dense;;) {
+      int64_t width = 512 / k > 1 ? v0 * (512 / k) : v0;
+      width = width < w.cap ? width : w.cap;
+      width = width > round_columns ? width / round_columns * round_columns : width / BM * BM;
+      if (width < BM) width = BM;
+      const int64_t vrows = (V - v0) < width ? (V - v0) : width;
+      const bool last = v0 + vrows >= V;
+      if (vrows > 0 && (e = launch_tiles(even_ktiles(H) ? topk::topk_filter_tiles<true> : topk::topk_filter_tiles<false>,
+                                         chunk_args(v0, vrows))) != hipSuccess)
+        return (int)e;
       {
         Timed timed(kTopkSelect, s);
         hipLaunchKernelGGL(topk::topk_select, dim3((unsigned)((Tb + topk::kSelectWaves - 1) / topk::kSelectWaves)),
@@ -2257,7 +2279,7 @@ int skyrl_lmhead_topk_logits(const void* hidden, int64_t ld_hidden, const void* 
       }
       if ((e = hipGetLastError()) != hipSuccess) return (int)e;
       v0 += vrows;
-      width *= 2;
+      if (last) break;
     }
   }
   return SKYRL_LMHEAD_OK;

@@ -2,9 +2,12 @@
 // _VocabParallelTopkSoftCE on one vocabulary shard): the k largest teacher logits of every token straight from the teacher's
 // hidden states -- no [T, V] logits tensor -- and the soft cross-entropy of the student over those k columns.
 //
-//   topk_filter_tiles   one 256(vocab) x 256(token) logits tile of a vocabulary chunk, the forward's GEMM; the epilogue compares
-//                       every logit with the token's threshold (the k-th largest logit among the columns of earlier chunks, a
-//                       lower bound of the final one) and appends the few that pass to the token's candidate list.
+//   topk_first_tiles    one 256(vocab) x 256(token) logits tile of the first vocabulary chunk, the forward's GEMM; the logits
+//                       themselves are stored, [T, chunk] fp32.
+//   topk_filter_tiles   the same of a later chunk; the epilogue compares every logit with the token's threshold (the k-th
+//                       largest logit among the columns of earlier chunks, a lower bound of the final one) and appends the few
+//                       that pass to the token's candidate list.
+//   topk_init           one workgroup per token: the k best of the first chunk's logits and the first threshold.
 //   topk_select         one wave per token: merges the chunk's candidates into the token's running k best, raises its
 //                       threshold, empties the candidate list.  After the last chunk it also writes the k logits and their
 //                       columns, best first.
@@ -54,11 +57,11 @@ struct FilterArgs {
   unsigned* cnt;       // [T] candidates appended in this launch
   key_t* cand;         // [T, cap]
   int cap;             // >= columns of a chunk, so that a list cannot overflow
+  float* dense;        // first chunk: its logits [T, tiles_m * 256]
 };
 
-template <bool EVEN>
-__global__ __launch_bounds__(NTHREADS) void topk_filter_tiles(const FilterArgs a) {
-  __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+template <bool DENSE, bool EVEN>
+__device__ __forceinline__ void topk_tile(const FilterArgs& a, char* lds) {
   int tm, tn;
   tile_coords(blockIdx.x, a.tiles_m, a.tiles_n, a.group_m, tm, tn);
 
@@ -71,7 +74,7 @@ __global__ __launch_bounds__(NTHREADS) void topk_filter_tiles(const FilterArgs a
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
     const int t = tn * BN + wn * WN + j * MT + lrow;
-    th[j] = a.thr[t < a.T ? t : a.T - 1];
+    th[j] = DENSE ? 0.f : a.thr[t < a.T ? t : a.T - 1];
   }
 
   Operand oa{a.W, a.ldw, tm * BM, a.vrows};
@@ -84,6 +87,18 @@ __global__ __launch_bounds__(NTHREADS) void topk_filter_tiles(const FilterArgs a
   const int vbase = tm * BM + wm * WM;  // first row of this wave inside the chunk
   if (vbase >= a.vrows) return;
   const float s = a.rcp_temp;
+  if (DENSE) {  // columns past vrows are stored as they come (copies of the last row) and not read
+    const size_t pitch = (size_t)a.tiles_m * BM;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int t = tn * BN + wn * WN + j * MT + lrow;
+      if (t >= a.T) continue;
+      float* row = a.dense + (size_t)t * pitch + vbase + kq * 4;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) *(f32x4*)(row + i * MT) = acc[i][j] * s;
+    }
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
     const int t = tn * BN + wn * WN + j * MT + lrow;
@@ -142,6 +157,18 @@ __global__ __launch_bounds__(NTHREADS) void topk_filter_tiles(const FilterArgs a
   }
 }
 
+template <bool EVEN>
+__global__ __launch_bounds__(NTHREADS) void topk_first_tiles(const FilterArgs a) {
+  __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+  topk_tile<true, EVEN>(a, lds);
+}
+
+template <bool EVEN>
+__global__ __launch_bounds__(NTHREADS) void topk_filter_tiles(const FilterArgs a) {
+  __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+  topk_tile<false, EVEN>(a, lds);
+}
+
 // Smallest key of the wave's values, in every lane.
 __device__ __forceinline__ key_t wave_min_key(key_t v) {
 #pragma unroll
@@ -154,14 +181,45 @@ __device__ __forceinline__ key_t wave_min_key(key_t v) {
 
 constexpr int kSelectWaves = 4;
 constexpr int kMaxK = 1024;
+
+// LDS operations of one wave execute in order; the fences only keep the compiler from caching entries that another lane has
+// rewritten.
+__device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
+// The k largest of the M > k keys in `list` (LDS, unique keys), moved to its front by the calling wave: a bisection over the key
+// bits finds a threshold that exactly k keys reach (a pass over the keys per bit, usually 20 to 30 bits until the count is exact).
+__device__ __forceinline__ void keep_largest(key_t* list, int M, int k, int lane) {
+  key_t reach = 0;  // grows bit by bit while at least k keys reach it; done when exactly k do
+  for (int b = 63; b >= 0; --b) {
+    const key_t trial = reach | ((key_t)1 << b);
+    int c = 0;
+    for (int e = lane; e < M; e += 64) c += list[e] >= trial ? 1 : 0;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) c += __shfl_xor(c, o, 64);
+    if (c >= k) {
+      reach = trial;
+      if (c == k) break;
+    }
+  }
+  int w = 0;  // in-place compaction: a step reads 64 entries and writes at or below where it read
+  for (int base = 0; base < M; base += 64) {
+    const int e = base + lane;
+    const key_t x = e < M ? list[e] : 0;
+    const bool keep = e < M && x >= reach;
+    const unsigned long long mask = __ballot(keep);
+    wave_lds_fence();
+    if (keep) list[w + __popcll(mask & (((key_t)1 << lane) - 1))] = x;
+    w += (int)__popcll(mask);
+    wave_lds_fence();
+  }
+}
+
 constexpr int kSelectStage = 1024;   // candidates one bulk round takes into LDS, behind the list
 constexpr int kSelectBulkMin = 96;   // fewer candidates than this are inserted one by one
 
 // best: [T, k] running lists (unordered), have: [T] entries of the list that are filled.  One wave per token; the list lives
 // in LDS while the wave works on it.  Many candidates (the first chunks, a large k, adversarial data) are merged in bulk: up to
-// kSelectStage of them are put behind the list, a bisection over the key bits finds a threshold that exactly k keys reach
-// (keys are unique, so one exists; a pass over the keys per bit, usually 20 to 30 bits until the count is exact), and the keys
-// that reach it are compacted to the front in place.  A few candidates are inserted one by one, each replacing the worst
+// kSelectStage of them are put behind the list and keep_largest() brings the best to the front.  A few candidates are inserted one by one, each replacing the worst
 // entry.  With `final_vals` the finished list is written out best first.
 __global__ __launch_bounds__(64 * kSelectWaves) void topk_select(int T, int k, key_t* __restrict__ best, unsigned* __restrict__ have,
                                                                  float* __restrict__ thr, unsigned* __restrict__ cnt,
@@ -175,9 +233,7 @@ __global__ __launch_bounds__(64 * kSelectWaves) void topk_select(int T, int k, k
   key_t* gl = best + (size_t)t * (size_t)k;
   int n_have = (int)have[t];
   for (int e = lane; e < n_have; e += 64) list[e] = gl[e];
-  // LDS operations of one wave execute in order; the fences below only keep the compiler from caching list entries that
-  // another lane has rewritten.
-  auto lds_fence = []() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+  auto lds_fence = []() { wave_lds_fence(); };
   lds_fence();
   const unsigned n_raw = cnt[t];
   const int n = (int)(n_raw < (unsigned)cap ? n_raw : (unsigned)cap);
@@ -207,29 +263,7 @@ __global__ __launch_bounds__(64 * kSelectWaves) void topk_select(int T, int k, k
       n_have = M;
       continue;
     }
-    key_t reach = 0;  // grows bit by bit while at least k keys reach it; done when exactly k do
-    for (int b = 63; b >= 0; --b) {
-      const key_t trial = reach | ((key_t)1 << b);
-      int c = 0;
-      for (int e = lane; e < M; e += 64) c += list[e] >= trial ? 1 : 0;
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) c += __shfl_xor(c, o, 64);
-      if (c >= k) {
-        reach = trial;
-        if (c == k) break;
-      }
-    }
-    int w = 0;  // in-place compaction: a step reads 64 entries and writes at or below where it read
-    for (int base = 0; base < M; base += 64) {
-      const int e = base + lane;
-      const key_t x = e < M ? list[e] : 0;
-      const bool keep = e < M && x >= reach;
-      const unsigned long long mask = __ballot(keep);
-      lds_fence();
-      if (keep) list[w + __popcll(mask & (((key_t)1 << lane) - 1))] = x;
-      w += (int)__popcll(mask);
-      lds_fence();
-    }
+    keep_largest(list, M, k, lane);
     n_have = k;
   }
   if (n_have == k) find_worst();
@@ -286,10 +320,154 @@ __global__ __launch_bounds__(64 * kSelectWaves) void topk_select(int T, int k, k
   if (lane == 0) cnt[t] = 0u;
 }
 
-__global__ __launch_bounds__(256) void topk_reset(int T, unsigned* __restrict__ have, float* __restrict__ thr,
-                                                  unsigned* __restrict__ cnt) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t < T) have[t] = 0u, thr[t] = -INFINITY, cnt[t] = 0u;
+// The first chunk's logits [T, pitch] of one token per workgroup -> its k best (unordered) and the first threshold.  A thread
+// keeps 32 logits in registers.
+//   k <= 128: the k-th largest of the threads' maxima is a lower bound of the k-th largest logit that few others reach (about 33
+//     for k = 32, 180 for k = 128); one wave finds it with ballots, the logits that reach it are listed in LDS and keep_largest()
+//     takes the k best of them.
+//   larger k, or so many equal logits that the list overflows: a bisection over the bits of the values (all threads count, one
+//     barrier per bit, fewer when the count comes out exact), and among equal values one over the columns.
+// Bound by the read of the logits.  Filling the lists through the candidate path instead (every logit passes while there is no
+// threshold) took 93 us for 32 tiles of 1024 columns at T=1800; first tiles of 8192 columns and this kernel take 61 + 31 us (the bisection alone: 61 + 45).
+constexpr int kInitLogits = 32;  // per thread
+constexpr int kInitList = 1024;
+constexpr int kInitListK = 128;
+
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void topk_init(int k, const float* __restrict__ dense, int pitch, int columns,
+                                                     key_t* __restrict__ best, unsigned* __restrict__ have,
+                                                     float* __restrict__ thr, unsigned* __restrict__ cnt) {
+  __shared__ int red[2][THREADS / 64];
+  __shared__ unsigned filled;
+  __shared__ uint32_t smallest[THREADS / 64];
+  __shared__ uint32_t maxima[THREADS];
+  __shared__ key_t listed[kInitList];
+  const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const float* row = dense + (size_t)t * (size_t)pitch;
+  uint32_t o[kInitLogits];  // ordered bits; 0 is below every number and stands for "no logit here" (a NaN, or past the columns)
+#pragma unroll
+  for (int u = 0; u < kInitLogits / 4; ++u) {
+    const int c = (u * THREADS + tid) * 4;
+    f32x4 z = {NAN, NAN, NAN, NAN};
+    if (c < columns) z = *(const f32x4*)(row + c);  // the pitch is a multiple of four
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[u * 4 + e] = (c + e < columns && z[e] == z[e]) ? ordered_bits(z[e]) : 0u;
+  }
+  if (tid == 0) filled = 0;
+  if (k <= kInitListK) {
+    uint32_t mx = 0;
+#pragma unroll
+    for (int e = 0; e < kInitLogits; ++e) mx = o[e] > mx ? o[e] : mx;
+    maxima[tid] = mx;
+    __syncthreads();
+    if (wave == 0) {
+      uint32_t m[THREADS / 64], bound = 0;
+#pragma unroll
+      for (int w = 0; w < THREADS / 64; ++w) m[w] = maxima[w * 64 + lane];
+      for (int b = 31; b >= 0; --b) {
+        const uint32_t trial = bound | (1u << b);
+        int c = 0;
+#pragma unroll
+        for (int w = 0; w < THREADS / 64; ++w) c += __popcll(__ballot(m[w] >= trial));
+        if (c >= k) {
+          bound = trial;
+          if (c == k) break;
+        }
+      }
+      if (lane == 0) smallest[0] = bound > 0 ? bound : 1u;  // fewer than k threads hold a logit: everything is listed
+    }
+    __syncthreads();
+    const uint32_t bound = smallest[0];
+#pragma unroll
+    for (int e = 0; e < kInitLogits; ++e) {
+      if (o[e] >= bound) {
+        const unsigned pos = atomicAdd(&filled, 1u);
+        if (pos < (unsigned)kInitList) listed[pos] = ((key_t)o[e] << 32) | (key_t)(uint32_t)(~(((e / 4) * THREADS + tid) * 4 + e % 4));
+      }
+    }
+    __syncthreads();
+    const int M = (int)filled;
+    if (M <= kInitList) {
+      if (wave != 0) return;
+      if (M > k) keep_largest(listed, M, k, lane);
+      const int kept = M < k ? M : k;
+      key_t worst = ~(key_t)0;
+      for (int e = lane; e < kept; e += 64) {
+        const key_t x = listed[e];
+        best[(size_t)t * (size_t)k + e] = x;
+        worst = x < worst ? x : worst;
+      }
+      worst = wave_min_key(worst);
+      if (lane == 0) have[t] = (unsigned)kept, thr[t] = kept == k ? key_value(worst) : -INFINITY, cnt[t] = 0u;
+      return;
+    }
+    __syncthreads();  // everybody has read `filled`
+    if (tid == 0) filled = 0;
+  }
+  int parity = 0;
+  auto total = [&](int mine) {  // sum over the workgroup, in every thread
+#pragma unroll
+    for (int x = 32; x >= 1; x >>= 1) mine += __shfl_xor(mine, x, 64);
+    if (lane == 0) red[parity][wave] = mine;
+    __syncthreads();
+    int sum = 0;
+    for (int w = 0; w < THREADS / 64; ++w) sum += red[parity][w];
+    parity ^= 1;
+    return sum;
+  };
+  auto reaching = [&](uint32_t limit) {
+    int c = 0;
+#pragma unroll
+    for (int e = 0; e < kInitLogits; ++e) c += o[e] >= limit ? 1 : 0;
+    return total(c);
+  };
+  uint32_t reach = 1;
+  int count = reaching(1);
+  const int n = count;
+  if (count > k) {
+    reach = 0;
+    for (int b = 31; b >= 0 && count != k; --b) {
+      const uint32_t trial = reach | (1u << b);
+      const int c = reaching(trial);
+      if (c >= k) reach = trial, count = c;
+    }
+  }
+  int column_limit = 0x7fffffff;
+  if (count > k) {  // several logits equal the k-th largest: the lower columns win
+    const int wanted = k - reaching(reach + 1);
+    int lo = 0, hi = columns;  // smallest limit below which at least `wanted` of them lie
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      int c = 0;
+#pragma unroll
+      for (int e = 0; e < kInitLogits; ++e) c += (o[e] == reach && ((e / 4) * THREADS + tid) * 4 + e % 4 < mid) ? 1 : 0;
+      if (total(c) >= wanted) hi = mid; else lo = mid + 1;
+    }
+    column_limit = lo;
+  }
+  uint32_t low = 0xffffffffu;
+#pragma unroll
+  for (int e = 0; e < kInitLogits; ++e) {
+    const int c = ((e / 4) * THREADS + tid) * 4 + e % 4;
+    if (o[e] > reach || (o[e] == reach && c < column_limit)) {
+      low = o[e] < low ? o[e] : low;
+      const unsigned pos = atomicAdd(&filled, 1u);
+      best[(size_t)t * (size_t)k + pos] = ((key_t)o[e] << 32) | (key_t)(uint32_t)(~c);
+    }
+  }
+#pragma unroll
+  for (int x = 32; x >= 1; x >>= 1) {
+    const uint32_t w = __shfl_xor(low, x, 64);
+    low = w < low ? w : low;
+  }
+  if (lane == 0) smallest[wave] = low;
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w < THREADS / 64; ++w) low = smallest[w] < low ? smallest[w] : low;
+    have[t] = (unsigned)(n < k ? n : k);
+    thr[t] = n >= k ? value_of_bits(low) : -INFINITY;
+    cnt[t] = 0u;
+  }
 }
 
 // fp32 dot product of two bf16 rows, the wave's lanes taking 16-byte pieces; the sum in every lane.

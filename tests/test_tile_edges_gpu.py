@@ -11,7 +11,7 @@ import torch
 
 from oracle import lmhead_oracle as O
 from skyrl_amd import ops
-from skyrl_amd.mtp_soft_ce import soft_ce_from_hidden
+from skyrl_amd.mtp_soft_ce import soft_ce_from_hidden, topk_logits_from_hidden
 
 pytestmark = pytest.mark.gpu
 
@@ -91,3 +91,33 @@ def test_split_hidden_gradient(T, H, V, vc, keep, cuda_device):
     for dw in (dense[1], active[1]):
         _close(dw, ex["d_weight"], f"dW T={T} H={H} V={V} chunk={vc}")
     assert torch.equal(active[0], ops.lmhead_bwd_bf16(h, w, y, lse, pz, gd, qd, 1.0, vc, True)[0])   # a fixed order of addition
+
+
+# The first vocabulary chunk of the top-k search is stored and searched: its width follows the number of tokens, the later ones the
+# room for candidate lists and k.  One chunk only, one column behind the first, many equal logits at the k-th rank, k = V.
+@pytest.mark.parametrize("T,H,V,k", [(3, 64, 8192, 5), (300, 64, 32769, 32), (260, 64, 33025, 1000), (2050, 64, 8449, 64), (5, 64, 40, 40)])
+@pytest.mark.parametrize("ties", [False, True])
+def test_topk_first_chunk(T, H, V, k, ties, cuda_device):
+    gen = torch.Generator().manual_seed(T + V)
+    hidden = torch.randn(T, H, generator=gen).to(torch.bfloat16)
+    weight = torch.randn(V, H, generator=gen).to(torch.bfloat16)
+    if ties:  # small whole numbers: exact in bf16 and fp32, each value many times in a row
+        hidden = torch.zeros(T, H, dtype=torch.bfloat16)
+        hidden[:, 0] = 1.0
+        weight[:, 0] = torch.randint(-3, 4, (V,), generator=gen).to(torch.bfloat16)
+        weight[V // 2, 0] = float("nan")
+    z = hidden.double() @ weight.double().t()
+    if ties:
+        z = weight[:, 0].double().expand(T, V).clone()
+        z[:, V // 2] = -torch.inf
+    values, columns = topk_logits_from_hidden(hidden.to(cuda_device), weight.to(cuda_device), k)
+    values, columns = values.cpu().double(), columns.cpu()
+    if ties:  # value first, then the lower column; the NaN is never taken while numbers are left
+        order = torch.argsort(-z[0] * (V + 1) + torch.arange(V), stable=True)[:k]
+        n = min(k, V - 1)
+        assert torch.equal(columns[:, :n], order[:n].expand(T, n)) and torch.equal(values[:, :n], z[:, order[:n]])
+        return
+    want = z.topk(min(k, V), dim=1)
+    assert float((values - want.values).abs().max()) < 1e-4
+    assert float((values - z.gather(1, columns)).abs().max()) < 1e-4
+    assert all(len(set(r)) == k for r in columns.tolist())
