@@ -359,7 +359,8 @@ int skyrl_packed_gather_grad(const float* d_out, const int64_t* cu_seqlens, int6
  *
  * skyrl_softce_fwd writes loss [T] and the two row log-sum-exps [T] (fp32) that skyrl_softce_bwd takes back.
  * skyrl_softce_bwd writes d_student_hidden [T, H] bf16 = sum_v dloss[t] * (softmax(z_s) - softmax(z_t))_v / temperature *
- * weight[v] (soft_ce.py:146-151 followed by the output layer's input gradient).  The teacher and the weight get no gradient:
+ * weight[v] (soft_ce.py:146-151 followed by the output layer's input gradient).  Tokens with dloss == 0 (masked ones)
+ * take no part and get a zero row (listed on the device, no host synchronisation).  The teacher and the weight get no gradient:
  * the reference detaches both (soft_ce.py:16-19, mtp/adapter.py:51-56).  Workspaces: 256-byte aligned device memory of at
  * least the queried size (0 = bad arguments); vocab_chunk as in skyrl_lmhead_bwd.  Not covered: more than one vocabulary
  * shard.

@@ -599,20 +599,50 @@ __host__ __device__ inline int64_t stacked_row(int64_t t, bool teacher) {
 // One workgroup per stacked row: copies the student's or the teacher's hidden row, zeros for the padding tokens.
 // Teacher row of token t = b * seq_len + s is the teacher's hidden row b * seq_len + (s + shift) mod seq_len: the roll of
 // build_teacher_logits (soft_ce.py:22-34) applied to the hidden states instead of the logits.
+__device__ __forceinline__ const uint16_t* softce_source_row(int t, bool is_teacher, const uint16_t* student, int lds_,
+                                                             const uint16_t* teacher, int ldt, int seq_len, int shift) {
+  if (!is_teacher) return student + (size_t)t * (size_t)lds_;
+  const int b = t / seq_len, sft = (t % seq_len + shift) % seq_len;
+  return teacher + (size_t)(b * seq_len + sft) * (size_t)ldt;
+}
+
 __global__ __launch_bounds__(256) void softce_pack_rows(const uint16_t* __restrict__ student, int lds_,
                                                         const uint16_t* __restrict__ teacher, int ldt, int T, int seq_len,
                                                         int shift, int H, uint16_t* __restrict__ stacked) {
   const int r = blockIdx.x;
   const bool is_teacher = (r / kPairRows) & 1;
   const int t = (r / WN) * kPairRows + r % kPairRows;
+  const uint16_t* src = t < T ? softce_source_row(t, is_teacher, student, lds_, teacher, ldt, seq_len, shift) : nullptr;
+  uint16_t* dst = stacked + (size_t)r * (size_t)H;
+  for (int c = threadIdx.x * 8; c < H; c += 256 * 8)
+    *(uint4*)(dst + c) = src ? *(const uint4*)(src + c) : make_uint4(0, 0, 0, 0);
+}
+
+// The same for the backward, which runs on the tokens with an upstream gradient only (compact_active_rows: idx, counts): stacked
+// rows and per-token inputs of compacted token t are those of token idx[t].  Rows beyond the last tile that holds a token are
+// not written.  As student row, token t also clears d_student[t]; active tokens get their row from the dHidden GEMM.
+__global__ __launch_bounds__(256) void softce_gather_rows(const uint16_t* __restrict__ student, int lds_,
+                                                          const uint16_t* __restrict__ teacher, int ldt, int T, int seq_len,
+                                                          int shift, int H, const int* __restrict__ idx,
+                                                          const int* __restrict__ counts, const float* __restrict__ lse_student,
+                                                          const float* __restrict__ lse_teacher, const float* __restrict__ dloss,
+                                                          uint16_t* __restrict__ stacked, float* __restrict__ lse_student_c,
+                                                          float* __restrict__ lse_teacher_c, float* __restrict__ dloss_c,
+                                                          uint16_t* __restrict__ d_student) {
+  const int r = blockIdx.x;
+  const bool is_teacher = (r / kPairRows) & 1;
+  const int t = (r / WN) * kPairRows + r % kPairRows, n = counts[0];
+  if (!is_teacher && t < T) {
+    uint16_t* zero_row = d_student + (size_t)t * (size_t)H;
+    for (int c = threadIdx.x * 8; c < H; c += 256 * 8) *(uint4*)(zero_row + c) = make_uint4(0, 0, 0, 0);
+  }
+  if (t >= (n + BN / 2 - 1) / (BN / 2) * (BN / 2)) return;
   const uint16_t* src = nullptr;
-  if (t < T) {
-    if (is_teacher) {
-      const int b = t / seq_len, sft = (t % seq_len + shift) % seq_len;
-      src = teacher + (size_t)(b * seq_len + sft) * (size_t)ldt;
-    } else {
-      src = student + (size_t)t * (size_t)lds_;
-    }
+  if (t < n) {
+    const int token = idx[t];
+    src = softce_source_row(token, is_teacher, student, lds_, teacher, ldt, seq_len, shift);
+    if (!is_teacher && threadIdx.x == 0)
+      lse_student_c[t] = lse_student[token], lse_teacher_c[t] = lse_teacher[token], dloss_c[t] = dloss[token];
   }
   uint16_t* dst = stacked + (size_t)r * (size_t)H;
   for (int c = threadIdx.x * 8; c < H; c += 256 * 8)
@@ -645,7 +675,8 @@ struct SoftCeDzArgs {
   const uint16_t* W;
   int ldw;
   const uint16_t* S;  // stacked hidden rows [2 * Tp, H], Tp = T rounded up to whole 128-token tiles
-  int T, Tp, H, V;
+  int Tp, H, V;
+  const int* T_dev;   // the number of tokens, <= Tp, counted on the device; token tiles beyond it return at once
   float rcp_temp;
   const float* lse_student;
   const float* lse_teacher;
@@ -661,10 +692,12 @@ __global__ __launch_bounds__(NTHREADS) void softce_dz_tiles(const SoftCeDzArgs z
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
   const uint16_t* __restrict__ W = z.W;
   const uint16_t* __restrict__ S = z.S;
-  const int T = z.T, H = z.H, V = z.V, vc0 = z.vc0, ldd = z.ldd;
+  const int T = __builtin_amdgcn_readfirstlane(*z.T_dev), H = z.H, V = z.V, vc0 = z.vc0, ldd = z.ldd;
   uint16_t* __restrict__ D = z.D;
+  const int tiles_n = (T + BN / 2 - 1) / (BN / 2);
+  if ((int)blockIdx.x >= z.tiles_m * tiles_n) return;
   int tm, tn;
-  tile_coords(blockIdx.x, z.tiles_m, z.tiles_n, kGroupM, tm, tn);
+  tile_coords(blockIdx.x, z.tiles_m, tiles_n, kGroupM, tm, tn);
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
@@ -681,7 +714,7 @@ __global__ __launch_bounds__(NTHREADS) void softce_dz_tiles(const SoftCeDzArgs z
 #pragma unroll
   for (int j = 0; j < TN / 2; ++j) {
     const int t = tokbase + j * MT + lrow;
-    const int tc = t < T ? t : T - 1;  // T >= 1: the host launches nothing for an empty batch
+    const int tc = t < T ? t : T - 1;  // T >= 1 here: a tile without a token has returned above
     gs_[j] = z.dloss[tc];
     ls2_[j] = z.lse_student[tc];
     lt2_[j] = z.lse_teacher[tc];
@@ -1732,7 +1765,8 @@ SoftCeFwdWorkspace carve_softce_fwd(void* ws, int64_t T, int64_t H, int64_t V) {
 
 struct SoftCeBwdWorkspace {
   uint16_t *S, *Wt, *D;
-  float* dHacc;
+  float *dHacc, *lse_student, *lse_teacher, *dloss;  // the latter three: of the tokens with an upstream gradient
+  int *idx, *counts;
   int64_t slots;
   size_t bytes;
 };
@@ -1743,9 +1777,15 @@ SoftCeBwdWorkspace carve_softce_bwd(void* ws, int64_t T, int64_t H, int64_t V, i
   SoftCeBwdWorkspace w;
   w.S = c.take<uint16_t>((size_t)(2 * Tp) * (size_t)H);
   w.Wt = V % (2 * BK) == 0 ? nullptr : c.take<uint16_t>((size_t)H * (Vpad + kLdPad));  // as in carve_bwd
-  w.slots = slab_slots(T, H, vc);
+  w.slots = slab_slots(T, H, vc);  // at least; a quarter more lets a batch with few active tokens split further
+  w.slots += w.slots / 4;
   w.dHacc = c.take<float>((size_t)(w.slots * kSlabTileFloats));
   w.D = c.take<uint16_t>((size_t)Tp * (vc + kLdPad));
+  w.lse_student = c.take<float>((size_t)T);
+  w.lse_teacher = c.take<float>((size_t)T);
+  w.dloss = c.take<float>((size_t)T);
+  w.idx = c.take<int>((size_t)T);
+  w.counts = c.take<int>(3);
   w.bytes = (size_t)round_up((int64_t)c.off, 256);
   return w;
 }
@@ -2172,11 +2212,23 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
   hipStream_t s = (hipStream_t)stream;
   const SoftCeBwdWorkspace w = carve_softce_bwd(workspace, T, H, V, vc);
   const uint16_t* Wp = (const uint16_t*)weight;
-  hipError_t e = launch_softce_pack(s, student_hidden, ld_student, teacher_hidden, ld_teacher, T, seq_len, shift, H, w.S);
-  if (e != hipSuccess) return (int)e;
+  hipError_t e;
   const bool w_in_place = reads_weight_in_place(V);
   const VocabTail tail = vocab_tail(V);
-  const int splits = w_in_place ? best_splits(split_problem(T, H, vc, false, w.slots, compute_units()), T) : 1;
+  {  // tokens without an upstream gradient (what the supervision mask removes) have a zero row and take no part
+    Timed timed(kCompactRows, s);
+    hipLaunchKernelGGL(compact_active_rows, dim3(1), dim3(kCompactThreads), 0, s, dloss, (const float*)nullptr, (int)T, (int)T, 1,
+                       split_problem(T, H, vc, false, w.slots, compute_units()), w.idx, w.counts);
+  }
+  if ((e = hipGetLastError()) != hipSuccess) return (int)e;
+  {
+    Timed timed(kSoftCePack, s);
+    hipLaunchKernelGGL(softce_gather_rows, dim3((unsigned)(2 * Tp)), dim3(256), 0, s, (const uint16_t*)student_hidden, (int)ld_student,
+                       (const uint16_t*)teacher_hidden, (int)ld_teacher, (int)T, (int)seq_len, (int)(shift % seq_len), (int)H,
+                       (const int*)w.idx, (const int*)w.counts, lse_student, lse_teacher, dloss, w.S, w.lse_student, w.lse_teacher,
+                       w.dloss, (uint16_t*)d_student_hidden);
+  }
+  if ((e = hipGetLastError()) != hipSuccess) return (int)e;
   if (!w_in_place) {
     Timed timed(kTranspose, s);
     hipLaunchKernelGGL(transpose_bf16, dim3((unsigned)(Vpad / 64), (unsigned)(H / 64)), dim3(256), 0, s, Wp, (int)ld_weight,
@@ -2187,8 +2239,8 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
   const GemmArgs none{};
   for (int64_t ci = 0; ci < nchunks; ++ci) {
     const int64_t vc0 = ci * vc, vcw = (Vpad - vc0) < vc ? (Vpad - vc0) : vc;
-    const SoftCeDzArgs z{Wp, (int)ld_weight, w.S, (int)T, (int)Tp, (int)H, (int)V, rcp_temperature, lse_student, lse_teacher,
-                         dloss, (int)vc0, (int)(vcw / 256), (int)(2 * Tp / BN), tail, w.D, (int)(vcw + kLdPad)};
+    const SoftCeDzArgs z{Wp, (int)ld_weight, w.S, (int)Tp, (int)H, (int)V, w.counts + 1, rcp_temperature, w.lse_student,
+                         w.lse_teacher, w.dloss, (int)vc0, (int)(vcw / 256), (int)(2 * Tp / BN), tail, w.D, (int)(vcw + kLdPad)};
     {
       Timed timed(kSoftCeDz, s);
       auto kernel = even_ktiles(H) ? softce_dz_tiles<true> : softce_dz_tiles<false>;
@@ -2199,8 +2251,8 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
     // partial sums carried from chunk to chunk in accumulator order, bf16 rows written by the last chunk.
     const bool first = ci == 0, last = ci == nchunks - 1;
     GemmArgs gh = dhidden_gemm(w.D, vcw + kLdPad, Tp, Wp, ld_weight, w_in_place ? nullptr : w.Wt, Vpad + kLdPad, vc0, vcw, V, T, H,
-                               (uint16_t*)d_student_hidden, w.dHacc, first, last, nullptr);
-    gh.splits = splits;
+                               (uint16_t*)d_student_hidden, w.dHacc, first, last, w.counts + 1);
+    gh.splits_dev = w_in_place ? w.counts + 2 : nullptr, gh.row_map = w.idx;
     e = launch_bwd_gemm(s, gh, none, w.slots);
     if (e == hipSuccess && last) e = launch_dh_reduce(s, gh, w.slots);
     if (e != hipSuccess) return (int)e;

@@ -121,3 +121,25 @@ def test_topk_first_chunk(T, H, V, k, ties, cuda_device):
     assert float((values - want.values).abs().max()) < 1e-4
     assert float((values - z.gather(1, columns)).abs().max()) < 1e-4
     assert all(len(set(r)) == k for r in columns.tolist())
+
+
+# The draft loss's backward runs on the tokens with an upstream gradient only: none, one, one 128-token tile, just over one, all.
+@pytest.mark.parametrize("active", [0, 1, 128, 129, 600])
+@pytest.mark.parametrize("V,vc", [(2304, 0), (5001, 1024)])
+def test_draft_loss_backward_on_active_tokens(active, V, vc, cuda_device):
+    B, S, H = 3, 200, 128
+    hidden, weight, _, g, _ = _operands(B * S, H, V, seed=V + active)
+    teacher = torch.randn(B, S, H, generator=torch.Generator().manual_seed(V)).to(torch.bfloat16)
+    keep = torch.zeros(B * S)
+    keep[torch.randperm(B * S, generator=torch.Generator().manual_seed(active))[:active]] = 1.0
+    g = (g * keep).reshape(B, S)
+    s = hidden.reshape(B, S, H).to(cuda_device).requires_grad_(True)
+    loss = soft_ce_from_hidden(s, teacher.to(cuda_device), weight.to(cuda_device), shift=2, vocab_chunk=vc)
+    (loss * g.to(cuda_device)).sum().backward()
+    grad = s.grad.reshape(B * S, H)
+    assert not grad[(keep == 0).to(cuda_device)].any()
+    if active:
+        zs = hidden.double() @ weight.double().t()
+        zt = teacher.roll(-2, dims=1).reshape(B * S, H).double() @ weight.double().t()
+        want = (g.reshape(-1).double()[:, None] * (zs.softmax(-1) - zt.softmax(-1))) @ weight.double()
+        _close(grad, want, f"{active} active tokens, V={V}")
