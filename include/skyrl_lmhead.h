@@ -281,7 +281,8 @@ int skyrl_approx_kl(const float* logprobs, const float* base_logprobs, const flo
  *     dlogprobs = d out6[0] / d logprobs        dentropy = d out6[0] / d entropy
  * All arrays fp32 [rows, cols]; loss_mask, loss_weight, base_logprobs, entropy, dlogprobs, dentropy may be NULL (dentropy needs
  * entropy).  policy_scale is the factor the worker applies to the pre-scaled policy loss (its data-parallel size), term_scale
- * the micro-batch weight of the two mean-reduced terms.  row_sums: fp32 scratch [rows, 6].
+ * the micro-batch weight of the two mean-reduced terms.  row_sums: fp32 scratch [rows, 6]; row_sums[5] is left holding the
+ * statistic as it is logged, out6[2] / max(out6[3], 1) (importance sampling: without the maximum, as the reference).
  */
 int skyrl_actor_loss(const float* logprobs, const float* old_logprobs, const float* advantages, const float* loss_mask,
                      const float* loss_weight, const float* base_logprobs, const float* entropy, int64_t rows, int64_t cols,

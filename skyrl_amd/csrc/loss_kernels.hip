@@ -423,7 +423,7 @@ struct ActorLossArgs {
   int64_t rows, cols;
   int loss_type, kl_estimator;
   float lo, hi, clip_c, policy_scale, term_scale, kl_coef, entropy_coef;
-  float* row_sums;  // [rows, 6]: policy loss, statistic, mask, kl row mean, entropy * mask, (unused)
+  float* row_sums;  // [rows, 6]: policy loss, statistic, mask, kl row mean, entropy * mask, (row 0: the metric, else unused)
   float* out;       // [6]: loss, policy_loss, statistic, mask count, kl, entropy_mean
   float *dlp, *dent;
 };
@@ -488,6 +488,8 @@ __global__ __launch_bounds__(kRowThreads) void actor_loss_finish_kernel(const Ac
   if (threadIdx.x == 0) {
     a.out[0] = a.policy_scale * t[0] + a.term_scale * (a.kl_coef * kl - a.entropy_coef * ent);
     a.out[1] = t[0], a.out[2] = t[1], a.out[3] = t[2], a.out[4] = kl, a.out[5] = ent;
+    // The statistic as it is logged: over the mask count, which the importance-sampling loss does not clamp.
+    a.row_sums[5] = t[1] / (a.loss_type == SKYRL_POLICY_LOSS_IMPORTANCE_SAMPLING ? t[2] : mask_denom);
   }
 }
 

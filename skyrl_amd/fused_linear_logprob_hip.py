@@ -95,6 +95,17 @@ def _require_single_shard(group: Optional[dist.ProcessGroup], what: str) -> None
         )
 
 
+def shard_labels(target: torch.Tensor, vocab_start_index: int, vocab_end_index: int, local_vocab: int) -> torch.Tensor:
+    """Token ids -> int64 rows of the weight shard; ids outside ``[vocab_start_index, vocab_end_index)`` become a value that
+    matches no row.  The kernels take any value outside ``[0, local_vocab)`` that way, so for the whole vocabulary (the single
+    shard of this backend) the ids already are the labels and nothing is launched."""
+    if vocab_start_index == 0 and vocab_end_index >= local_vocab:
+        return target.to(torch.int64)
+    outside = (target < vocab_start_index) | (target >= vocab_end_index)
+    target = target.to(torch.int64)  # int32 ids: the sentinel does not fit their dtype
+    return torch.where(outside, _OOV_LABEL_SENTINEL, target - vocab_start_index)
+
+
 class LinearCrossEntropy(torch.autograd.Function):
     """verl-style fused linear + log-prob + entropy.  See the module docstring for the reference lines."""
 
@@ -184,9 +195,9 @@ class FusedLinearLogprobHip(torch.autograd.Function):
         local_vocab = int(weight.shape[0])
         # Targets outside [vocab_start_index, vocab_end_index) get a label that matches no column: forward 0, backward keeps
         # -softmax * grad (fused_linear_logprob_triton.py:1876-1878, 1898-1905, 1929-1931).
-        target_mask = (target < vocab_start_index) | (target >= vocab_end_index)
-        target = target.to(torch.int64)  # int32 ids: the sentinel below does not fit their dtype
-        labels = torch.where(target_mask, _OOV_LABEL_SENTINEL, target - vocab_start_index).reshape(-1).contiguous()
+        labels = shard_labels(target, vocab_start_index, vocab_end_index, local_vocab).reshape(-1).contiguous()
+        if not inference_only and labels.data_ptr() == target.data_ptr():
+            labels = labels.clone()  # kept for the backward: the caller may reuse its tensor of ids meanwhile
         # The kernel needs 2-D operands with matching dtypes: hidden follows the weight (model_utils.py:328-333).
         hidden_2d = ops.hidden_for_weight(hidden.reshape(B * S, H), weight).contiguous()
         weight_c = weight.contiguous()

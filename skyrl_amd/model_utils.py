@@ -31,7 +31,8 @@ import torch
 import torch.distributed as dist
 
 from . import ops
-from .fused_linear_logprob_hip import FusedLinearLogprobHip, _group_size, _require_single_shard, linear_cross_entropy
+from .fused_linear_logprob_hip import (FusedLinearLogprobHip, _group_size, _require_single_shard, linear_cross_entropy,
+                                       shard_labels)
 from .packed import packed_next_token_labels, packed_scatter_logprobs
 
 FUSED_LM_HEAD_LOGPROB_BACKENDS = ("hip",)
@@ -70,9 +71,7 @@ def _fused_lm_head_logprob_apply(
                                            inference_only)
     _require_single_shard(tp_group, "_fused_lm_head_logprob_apply")
     B, S, H = hidden.shape
-    target_mask = (target < vocab_start_index) | (target >= vocab_end_index)
-    target = target.to(torch.int64)
-    labels = torch.where(target_mask, torch.iinfo(torch.int64).max, target - vocab_start_index)
+    labels = shard_labels(target, vocab_start_index, vocab_end_index, int(weight.shape[0]))
     hidden_c = ops.hidden_for_weight(hidden, weight)
     # log-probabilities only: no entropy is accumulated in the forward, none differentiated in the backward
     if inference_only:

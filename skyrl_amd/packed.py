@@ -77,7 +77,10 @@ def _scatter_operands(cu_seqlens, seg_row, seg_col, seg_len, attention_mask, row
         if tuple(attention_mask.shape) != (rows, cols + 1) or rows != n:
             raise ValueError(f"attention_mask must be [{n}, {cols + 1}] (one row per packed sequence, unpacked_seqlen "
                              f"columns), got {tuple(attention_mask.shape)} for rows={rows}")
-        attention_mask = (attention_mask.to(device=dev) != 0).to(torch.uint8).contiguous()
+        attention_mask = attention_mask.to(device=dev)
+        if attention_mask.dtype not in (torch.bool, torch.uint8):  # the kernels test single bytes against zero
+            attention_mask = attention_mask != 0
+        attention_mask = attention_mask.contiguous().view(torch.uint8)
     return cu, segs[0], segs[1], segs[2], attention_mask
 
 

@@ -131,6 +131,12 @@ def _(log_probs, old_log_probs, advantages, loss_mask, loss_weight, eps_clip_low
     return log_probs.new_empty(3, dtype=torch.float32), log_probs.new_empty(log_probs.numel(), dtype=torch.float32)
 
 
+def _own_scalar(t: torch.Tensor) -> torch.Tensor:
+    """The first element of ``t`` as a 0-dim tensor of its own over that storage, not a view as autograd counts them: nothing else
+    reads that element, so the caller may scale the loss in place, and no copy is launched."""
+    return torch.empty(0, dtype=t.dtype, device=t.device).set_(t.untyped_storage(), t.storage_offset(), (), ())
+
+
 class _PolicyLoss(torch.autograd.Function):
     @staticmethod
     def forward(ctx, log_probs, old_log_probs, advantages, loss_mask, loss_weight, eps_low, eps_high, clip_c, loss_type):
@@ -142,11 +148,14 @@ class _PolicyLoss(torch.autograd.Function):
         ctx.save_for_backward(grad)
         ctx.shape, ctx.dtype = log_probs.shape, log_probs.dtype
         ctx.mark_non_differentiable(sums)
-        return sums[0].clone(), sums
+        ctx.set_materialize_grads(False)
+        return _own_scalar(sums), sums
 
     @staticmethod
     def backward(ctx, grad_loss, _grad_sums):
         (grad,) = ctx.saved_tensors
+        if grad_loss is None:
+            return (None,) * 9
         return (grad * grad_loss).reshape(ctx.shape).to(ctx.dtype), None, None, None, None, None, None, None, None
 
 
@@ -391,8 +400,8 @@ def gspo_policy_loss(log_probs, old_log_probs, advantages, config, loss_mask=Non
         raise ValueError("gspo_policy_loss needs [B, S] inputs: the importance weight is a row mean")
     loss_weight, extra = _with_off_policy_correction(config, old_log_probs, rollout_logprobs, loss_mask, loss_weight, sync_metrics)
     scalars = (LOSS_GSPO, float(config.eps_clip_low), float(config.eps_clip_high), 0.0, 3, 1.0, 1.0, 0.0, 0.0)
-    loss, out6 = _ActorLoss.apply(log_probs, None, (old_log_probs, advantages, loss_mask, loss_weight, None), scalars)
-    clip_ratio = out6[2] / out6[3].clamp(min=1.0)
+    loss, out = _ActorLoss.apply(log_probs, None, (old_log_probs, advantages, loss_mask, loss_weight, None), scalars)
+    clip_ratio = out[11]
     return loss, {"clip_ratio": clip_ratio.item() if sync_metrics else clip_ratio, **extra}
 
 
@@ -565,15 +574,15 @@ def _actor_loss(log_probs: torch.Tensor, old_log_probs: Optional[torch.Tensor], 
                 entropy: Optional[torch.Tensor], loss_type: int, eps_clip_low: float, eps_clip_high: float, clip_ratio_c: float,
                 kl_estimator: int, policy_scale: float, term_scale: float, kl_coef: float, entropy_coef: float,
                 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    """``(out6, dlogprobs, dentropy)`` for contiguous fp32 ``[rows, cols]`` inputs; ``dentropy`` is empty without ``entropy``."""
+    """``(out, dlogprobs, dentropy)`` for contiguous fp32 ``[rows, cols]`` inputs; ``dentropy`` is empty without ``entropy``.  ``out``
+    holds the six results of ``skyrl_actor_loss`` and behind them its row sums, whose element 5 is the statistic as it is logged."""
     dev = _require_device(log_probs)
     rows, cols = log_probs.shape
     for name, t in (("old_log_probs", old_log_probs), ("advantages", advantages), ("loss_mask", loss_mask),
                     ("loss_weight", loss_weight), ("base_log_probs", base_log_probs), ("entropy", entropy)):
         if t is not None and (t.dtype != torch.float32 or t.shape != log_probs.shape or not t.is_contiguous()):
             raise ValueError(f"{name} must be a contiguous fp32 tensor of shape {tuple(log_probs.shape)}")
-    out6 = torch.empty(6, dtype=torch.float32, device=dev)
-    row_sums = torch.empty((rows, 6), dtype=torch.float32, device=dev)
+    out = torch.empty(6 + 6 * rows, dtype=torch.float32, device=dev)
     dlp = torch.empty_like(log_probs)
     dent = torch.empty_like(log_probs) if entropy is not None else torch.empty(0, dtype=torch.float32, device=dev)
     ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
@@ -581,17 +590,17 @@ def _actor_loss(log_probs: torch.Tensor, old_log_probs: Optional[torch.Tensor], 
         st = _lib.load().skyrl_actor_loss(
             log_probs.data_ptr(), ptr(old_log_probs), ptr(advantages), ptr(loss_mask), ptr(loss_weight), ptr(base_log_probs),
             ptr(entropy), rows, cols, int(loss_type), float(eps_clip_low), float(eps_clip_high), float(clip_ratio_c),
-            int(kl_estimator), float(policy_scale), float(term_scale), float(kl_coef), float(entropy_coef), row_sums.data_ptr(),
-            out6.data_ptr(), dlp.data_ptr(), dent.data_ptr() if entropy is not None else None,
+            int(kl_estimator), float(policy_scale), float(term_scale), float(kl_coef), float(entropy_coef), out.data_ptr() + 24,
+            out.data_ptr(), dlp.data_ptr(), dent.data_ptr() if entropy is not None else None,
             torch.cuda.current_stream(dev).cuda_stream)
     _lib.check(st, "skyrl_actor_loss")
-    return out6, dlp, dent
+    return out, dlp, dent
 
 
 @_actor_loss.register_fake
 def _(log_probs, old_log_probs, advantages, loss_mask, loss_weight, base_log_probs, entropy, loss_type, eps_clip_low,
       eps_clip_high, clip_ratio_c, kl_estimator, policy_scale, term_scale, kl_coef, entropy_coef):
-    return (log_probs.new_empty(6), torch.empty_like(log_probs),
+    return (log_probs.new_empty(6 + 6 * log_probs.shape[0]), torch.empty_like(log_probs),
             torch.empty_like(log_probs) if entropy is not None else log_probs.new_empty(0))
 
 
@@ -605,17 +614,20 @@ class _ActorLoss(torch.autograd.Function):
                         ("base_log_probs", base), ("entropy", entropy)):
             if t is not None and t.shape != log_probs.shape:
                 raise ValueError(f"{name} has shape {tuple(t.shape)}, expected {tuple(log_probs.shape)}")
-        out6, dlp, dent = _actor_loss(flat(log_probs), flat(old), flat(adv), flat(mask), flat(weight), flat(base), flat(entropy),
-                                      *scalars)
+        out, dlp, dent = _actor_loss(flat(log_probs), flat(old), flat(adv), flat(mask), flat(weight), flat(base), flat(entropy),
+                                     *scalars)
+        ctx.set_materialize_grads(False)
         ctx.save_for_backward(dlp, dent)
         ctx.lp_meta = (log_probs.shape, log_probs.dtype)
         ctx.ent_meta = None if entropy is None else (entropy.shape, entropy.dtype)
-        ctx.mark_non_differentiable(out6)
-        return out6[0].clone(), out6
+        ctx.mark_non_differentiable(out)
+        return _own_scalar(out), out
 
     @staticmethod
-    def backward(ctx, grad_loss, _grad_out6):
+    def backward(ctx, grad_loss, _grad_out):
         dlp, dent = ctx.saved_tensors
+        if grad_loss is None:
+            return None, None, None, None
         shape, dtype = ctx.lp_meta
         g_lp = (dlp * grad_loss).reshape(shape).to(dtype)
         g_ent = None
@@ -674,10 +686,9 @@ def actor_loss(
                float(config.kl_loss_coef) if use_kl else 0.0, float(config.entropy_loss_coef) if use_ent else 0.0)
     consts = (behaviour, advantages, loss_mask, loss_weight, base_log_probs if use_kl else None)
     # The entropy is reduced for the metric even when it is not part of the loss, as the worker does.
-    loss, out6 = _ActorLoss.apply(log_probs, entropy, consts, scalars)
-    stat = out6[2] / (out6[3] if loss_type == LOSS_IMPORTANCE_SAMPLING else out6[3].clamp(min=1.0))
-    metrics = {"policy_loss": out6[1], "policy_kl": out6[4], "policy_entropy": out6[5],
-               ("importance_ratio" if loss_type == LOSS_IMPORTANCE_SAMPLING else "clip_ratio"): stat, **extra}
+    loss, out = _ActorLoss.apply(log_probs, entropy, consts, scalars)
+    metrics = {"policy_loss": out[1], "policy_kl": out[4], "policy_entropy": out[5],
+               ("importance_ratio" if loss_type == LOSS_IMPORTANCE_SAMPLING else "clip_ratio"): out[11], **extra}
     return loss, metrics
 
 
