@@ -13,6 +13,8 @@
 //
 //   forward   y = z / temperature;  lse = log sum exp y;  logprob = y[label] - lse;  pz = sum softmax(y) * y;  entropy = lse - pz
 //   backward  dz = ( g * (onehot - p) - q * p * (y - pz) ) / temperature,   p = exp(y - lse)
+// Rows need not be aligned: a row is the logits in front of its first 16-byte boundary, 16-byte pieces, and the logits behind the
+// last one (RowPieces), so that an odd vocabulary, whose rows start anywhere, is read at the same rate.
 // One workgroup per row; a thread keeps a running (max, sum, sum z*e) in base 2 and rescales only when a wave-wide vote says
 // some lane's maximum moved, which after the first few pieces of a row is rare.
 #include <hip/hip_runtime.h>
@@ -33,6 +35,7 @@ constexpr float kLowest = -3.0e38f;  // start of a running maximum: finite, so t
 constexpr float kMostNegativeFactor = -1.0e30f;
 constexpr int kThreads = 512;
 constexpr int kWaves = kThreads / 64;
+constexpr int kBwdThreads = 1024;
 constexpr int kInFlight = 4;  // 16-byte loads a thread has in flight
 
 // Eight bf16 or four fp32 logits of one 16-byte piece, widened to fp32.
@@ -55,6 +58,20 @@ struct Piece {
     }
   }
 };
+
+// Where the 16-byte pieces of a row lie: logits [head, head + pieces * E); the other `single` logits are numbered head first.
+struct RowPieces {
+  int head, pieces, single;
+};
+template <bool F32>
+__device__ __forceinline__ RowPieces row_pieces(const char* row, int V, bool vector_ok) {
+  constexpr int E = Piece<F32>::kElems, ES = F32 ? 4 : 2;
+  int head = (int)((16u - (uint32_t)((uintptr_t)row & 15u)) & 15u) / ES;
+  head = head < V ? head : V;
+  const int pieces = vector_ok ? (V - head) / E : 0;
+  return RowPieces{head, pieces, V - pieces * E};
+}
+__device__ __forceinline__ int single_column(const RowPieces& r, int elems, int i) { return i < r.head ? i : i + r.pieces * elems; }
 
 __device__ __forceinline__ float load_one(const void* base, size_t i, bool f32) {
   return f32 ? ((const float*)base)[i] : __uint_as_float((uint32_t)((const uint16_t*)base)[i] << 16);
@@ -127,20 +144,21 @@ __device__ __forceinline__ Stats block_merge(Stats st, Stats* sm) {
   return all;
 }
 
-// Statistics of row `row`: vector pieces where the row start and pitch allow 16-byte loads, single logits otherwise and
-// for the ragged end.
+// Statistics of row `row`.
 template <bool F32, bool ENT>
-__device__ __forceinline__ Stats row_stats(const void* logits, int64_t ld, int64_t row, int V, float scale2, bool vector_ok) {
+__device__ __forceinline__ Stats row_stats(const void* logits, int64_t ld, int64_t row, int V, float scale2) {
   constexpr int E = Piece<F32>::kElems;
   const char* base = (const char*)logits + (size_t)row * (size_t)ld * (F32 ? 4 : 2);
   Stats st{kLowest, 0.f, 0.f};
-  const int pieces = vector_ok ? V / E : 0;
+  const RowPieces rp = row_pieces<F32>(base, V, true);
+  const char* vec = base + (size_t)rp.head * (F32 ? 4 : 2);
+  const int pieces = rp.pieces;
   for (int p0 = threadIdx.x; p0 < pieces; p0 += kThreads * kInFlight) {
     Piece<F32> pc[kInFlight];
 #pragma unroll
     for (int u = 0; u < kInFlight; ++u) {
       const int p = p0 + u * kThreads;
-      pc[u].load(base + (size_t)(p < pieces ? p : p0) * 16);
+      pc[u].load(vec + (size_t)(p < pieces ? p : p0) * 16);
     }
 #pragma unroll
     for (int u = 0; u < kInFlight; ++u) {
@@ -154,8 +172,8 @@ __device__ __forceinline__ Stats row_stats(const void* logits, int64_t ld, int64
       }
     }
   }
-  for (int i = pieces * E + threadIdx.x; i < V; i += kThreads) {
-    const float z = load_one(base, (size_t)i, F32);
+  for (int i = threadIdx.x; i < rp.single; i += kThreads) {
+    const float z = load_one(base, (size_t)single_column(rp, E, i), F32);
     raise_max(st, z * scale2);
     absorb<ENT>(st, z, scale2);
   }
@@ -165,13 +183,13 @@ __device__ __forceinline__ Stats row_stats(const void* logits, int64_t ld, int64
 // labels may be NULL (no log-probability wanted).  A label outside [0, V) gives log-probability 0 (model_utils.py:89-99).
 template <bool F32, bool ENT>
 __global__ __launch_bounds__(kThreads) void logits_fwd_rows(const void* __restrict__ logits, int64_t ld, const int64_t* __restrict__ labels,
-                                                            int V, float rcp_temp, int vector_ok, float* __restrict__ logprobs,
+                                                            int V, float rcp_temp, float* __restrict__ logprobs,
                                                             float* __restrict__ entropy, float* __restrict__ row_lse,
                                                             float* __restrict__ row_pz) {
   __shared__ Stats sm[kWaves];
   const int64_t row = blockIdx.x;
   const float scale2 = rcp_temp * kLog2e;
-  const Stats st = block_merge(row_stats<F32, ENT>(logits, ld, row, V, scale2, vector_ok != 0), sm);
+  const Stats st = block_merge(row_stats<F32, ENT>(logits, ld, row, V, scale2), sm);
   if (threadIdx.x == 0) {
     const float log_s = logf(st.s);
     const float lse = fmaf(st.m, kLn2, log_s);
@@ -192,8 +210,11 @@ __global__ __launch_bounds__(kThreads) void logits_fwd_rows(const void* __restri
 }
 
 // dlogits may be the logits themselves (every logit is read before its place is written, by the same thread).
+// vector_ok: the rows of dlogits have the same offset from a 16-byte boundary as those of the logits.
+// HBM-bound, a read and a write per logit; 1024 threads a row instead of 512: 198 -> 187 us at 1545 x 151936 (5.0 TB/s), 786 -> 715
+// us at 16384 x 60000 (5.5 TB/s); the forward is better off with 512 (94 against 104 us).
 template <bool F32, bool ENTGRAD>
-__global__ __launch_bounds__(kThreads) void logits_bwd_rows(const void* logits, int64_t ld, const int64_t* __restrict__ labels, int V,
+__global__ __launch_bounds__(kBwdThreads) void logits_bwd_rows(const void* logits, int64_t ld, const int64_t* __restrict__ labels, int V,
                                                             float rcp_temp, int vector_ok, const float* __restrict__ row_lse,
                                                             const float* __restrict__ row_pz, const float* __restrict__ dlogprobs,
                                                             const float* __restrict__ dentropy, void* dlogits, int64_t ldd) {
@@ -218,23 +239,26 @@ __global__ __launch_bounds__(kThreads) void logits_bwd_rows(const void* logits, 
     if (col == y) d += g * rcp_temp;
     return d;
   };
-  const int pieces = vector_ok ? V / E : 0;
-  for (int p0 = threadIdx.x; p0 < pieces; p0 += kThreads * kInFlight) {
+  const RowPieces rp = row_pieces<F32>(src, V, vector_ok != 0);
+  const char* vsrc = src + (size_t)rp.head * ES;
+  char* vdst = dst + (size_t)rp.head * ES;
+  const int pieces = rp.pieces;
+  for (int p0 = threadIdx.x; p0 < pieces; p0 += kBwdThreads * kInFlight) {
     Piece<F32> pc[kInFlight];
     if (!zero_row) {
 #pragma unroll
       for (int u = 0; u < kInFlight; ++u) {
-        const int p = p0 + u * kThreads;
-        pc[u].load(src + (size_t)(p < pieces ? p : p0) * 16);
+        const int p = p0 + u * kBwdThreads;
+        pc[u].load(vsrc + (size_t)(p < pieces ? p : p0) * 16);
       }
     }
 #pragma unroll
     for (int u = 0; u < kInFlight; ++u) {
-      const int p = p0 + u * kThreads;
+      const int p = p0 + u * kBwdThreads;
       if (p >= pieces) continue;
       float d[E];
 #pragma unroll
-      for (int i = 0; i < E; ++i) d[i] = zero_row ? 0.f : dz(pc[u].v[i], (int64_t)p * E + i);
+      for (int i = 0; i < E; ++i) d[i] = zero_row ? 0.f : dz(pc[u].v[i], rp.head + (int64_t)p * E + i);
       uint4 out;
       if (F32) {
         out = make_uint4(__float_as_uint(d[0]), __float_as_uint(d[1]), __float_as_uint(d[2]), __float_as_uint(d[3]));
@@ -246,20 +270,22 @@ __global__ __launch_bounds__(kThreads) void logits_bwd_rows(const void* logits, 
         const uint2 a = *(const uint2*)&lo, b = *(const uint2*)&hi;
         out = make_uint4(a.x, a.y, b.x, b.y);
       }
-      *(uint4*)(dst + (size_t)p * 16) = out;
+      *(uint4*)(vdst + (size_t)p * 16) = out;
     }
   }
-  for (int i = pieces * E + threadIdx.x; i < V; i += kThreads) {
-    const float d = zero_row ? 0.f : dz(load_one(src, (size_t)i, F32), (int64_t)i);
-    if (F32) ((float*)dst)[i] = d;
-    else ((uint16_t*)dst)[i] = bf16_bits(d);
+  for (int i = threadIdx.x; i < rp.single; i += kBwdThreads) {
+    const int c = single_column(rp, E, i);
+    const float d = zero_row ? 0.f : dz(load_one(src, (size_t)c, F32), (int64_t)c);
+    if (F32) ((float*)dst)[c] = d;
+    else ((uint16_t*)dst)[c] = bf16_bits(d);
   }
 }
 
 constexpr int64_t kMaxRows = (int64_t)1 << 31;  // the grid's x extent
 
-bool pieces_aligned(const void* p, int64_t ld, bool f32) {
-  return ((uintptr_t)p & 15u) == 0 && (ld * (f32 ? 4 : 2)) % 16 == 0;
+// Whether every row of b starts as far from a 16-byte boundary as the same row of a.
+bool same_row_offsets(const void* a, int64_t lda, const void* b, int64_t ldb, bool f32) {
+  return (((uintptr_t)a - (uintptr_t)b) & 15u) == 0 && (lda - ldb) * (f32 ? 4 : 2) % 16 == 0;
 }
 
 int check_logits(const void* logits, int dtype, int64_t ld, int64_t T, int64_t V, float rcp_temperature) {
@@ -283,11 +309,10 @@ int skyrl_logits_fwd(const void* logits, int logits_dtype, int64_t ld_logits, co
   if (!logprobs && !entropy && !row_lse && !row_pz) return SKYRL_LMHEAD_ERR_NULL;
   if (labels && ((uintptr_t)labels & 7u)) return SKYRL_LMHEAD_ERR_ALIGN;
   const bool f32 = logits_dtype == SKYRL_LOGITS_F32;
-  const int vec = pieces_aligned(logits, ld_logits, f32) ? 1 : 0;
   hipStream_t s = (hipStream_t)stream;
   const bool ent = entropy || row_pz;
   auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)T), dim3(kThreads), 0, s, logits, ld_logits, labels, (int)V, rcp_temperature, vec,
+    hipLaunchKernelGGL(kernel, dim3((unsigned)T), dim3(kThreads), 0, s, logits, ld_logits, labels, (int)V, rcp_temperature,
                        logprobs, entropy, row_lse, row_pz);
   };
   if (f32 && ent) launch(logits_fwd_rows<true, true>);
@@ -315,11 +340,11 @@ int skyrl_logits_bwd(const void* logits, int logits_dtype, int64_t ld_logits, co
     const char *a1 = a0 + ((size_t)(T - 1) * (size_t)ld_logits + (size_t)V) * es, *b1 = b0 + ((size_t)(T - 1) * (size_t)ld_dlogits + (size_t)V) * es;
     if (a0 < b1 && b0 < a1) return SKYRL_LMHEAD_ERR_ARG;
   }
-  const int vec = (pieces_aligned(logits, ld_logits, f32) && pieces_aligned(dlogits, ld_dlogits, f32)) ? 1 : 0;
+  const int vec = same_row_offsets(logits, ld_logits, dlogits, ld_dlogits, f32) ? 1 : 0;
   hipStream_t s = (hipStream_t)stream;
   const bool entgrad = dentropy != nullptr;
   auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)T), dim3(kThreads), 0, s, logits, ld_logits, labels, (int)V, rcp_temperature, vec,
+    hipLaunchKernelGGL(kernel, dim3((unsigned)T), dim3(kBwdThreads), 0, s, logits, ld_logits, labels, (int)V, rcp_temperature, vec,
                        row_lse, row_pz, dlogprobs, dentropy, dlogits, ld_dlogits);
   };
   if (f32 && entgrad) launch(logits_bwd_rows<true, true>);

@@ -11,6 +11,7 @@ import torch
 
 from oracle import lmhead_oracle as O
 from skyrl_amd import ops
+from skyrl_amd import torch_utils as TU
 from skyrl_amd.mtp_soft_ce import soft_ce_from_hidden, topk_logits_from_hidden
 
 pytestmark = pytest.mark.gpu
@@ -143,3 +144,35 @@ def test_draft_loss_backward_on_active_tokens(active, V, vc, cuda_device):
         zt = teacher.roll(-2, dims=1).reshape(B * S, H).double() @ weight.double().t()
         want = (g.reshape(-1).double()[:, None] * (zs.softmax(-1) - zt.softmax(-1))) @ weight.double()
         _close(grad, want, f"{active} active tokens, V={V}")
+
+
+# Logits rows that start anywhere: every offset of a row from a 16-byte boundary, rows shorter than the way to it, odd pitches, a
+# gradient buffer whose rows start elsewhere than the logits' (single accesses) and one written in place.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("V,pitch", [(1, 1), (5, 7), (7, 9), (63, 65), (4099, 4099), (9001, 9008)])
+def test_logits_rows_at_any_offset(dtype, V, pitch, cuda_device):
+    T, t = 9, 0.7
+    gen = torch.Generator().manual_seed(V)
+    for offset in range(8):
+        buf = torch.randn(offset + T * pitch, generator=gen).mul(3).to(dtype).to(cuda_device)
+        z = buf[offset:].as_strided((T, V), (pitch, 1))
+        labels = torch.randint(0, V, (T,), generator=gen)
+        g, q = torch.randn(T, generator=gen), torch.randn(T, generator=gen) * 0.1
+        zd = z.detach().cpu().double().requires_grad_(True)
+        ls = torch.log_softmax(zd / t, dim=1)
+        want_lp, want_ent = ls.gather(1, labels[:, None])[:, 0], -(ls.exp() * ls).sum(1)
+        (want_lp * g + want_ent * q).sum().backward()
+        lp, ent, lse, pz = TU.logits_fwd(z, labels.to(cuda_device), 1.0 / t, True)
+        assert float((lp.cpu().double() - want_lp.detach()).abs().max()) < 1e-5 * (1 + float(want_lp.detach().abs().max()))
+        assert float((ent.cpu().double() - want_ent.detach()).abs().max()) < 1e-5 * (1 + float(want_ent.detach().abs().max()))
+        args = (labels.to(cuda_device), lse, pz, g.to(cuda_device), q.to(cuda_device), 1.0 / t)
+        apart = TU.logits_bwd(z, *args).cpu().double()
+        # one rounding to the result's type, on top of fp32 arithmetic on terms of the order of the upstream gradients
+        bound = zd.grad.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 0.0) + 4e-6
+        assert bool(((apart - zd.grad).abs() <= bound).all())
+        rest = buf.clone()
+        TU.logits_bwd_(z, *args)
+        assert torch.equal(z.cpu().double(), apart)
+        untouched = torch.ones(buf.numel(), dtype=torch.bool)
+        untouched[offset:].as_strided((T, V), (pitch, 1)).fill_(False)
+        assert torch.equal(buf.cpu()[untouched], rest.cpu()[untouched])
