@@ -22,6 +22,7 @@ import torch
 import torch.distributed as dist
 
 from . import ops
+from ._launch import call
 
 _OOV_LABEL_SENTINEL = torch.iinfo(torch.int64).max
 
@@ -137,7 +138,7 @@ class LinearCrossEntropy(torch.autograd.Function):
         labels1 = labels1.to(torch.int64).contiguous()  # what the kernel reads is what the backward gets back
         rcp_t = 1.0 / temperature
         with torch.no_grad():
-            logprobs, entropy, row_lse, row_pz = ops.lmhead_fwd(hidden2, weight, labels1, rcp_t, bool(want_entropy))
+            logprobs, entropy, row_lse, row_pz = call(ops.lmhead_fwd, hidden2, weight, labels1, rcp_t, bool(want_entropy))
         ctx.save_for_backward(hidden2, weight, labels1, row_lse, row_pz)
         # An output nobody uses arrives in backward as None, not as a tensor of zeros: an unused entropy then costs nothing.
         ctx.set_materialize_grads(False)
@@ -204,7 +205,7 @@ class FusedLinearLogprobHip(torch.autograd.Function):
         assert local_vocab == weight_c.shape[0]
 
         with torch.no_grad():
-            logprobs, _, row_lse, _ = ops.lmhead_fwd(hidden_2d, weight_c, labels, 1.0, False)
+            logprobs, _, row_lse, _ = call(ops.lmhead_fwd, hidden_2d, weight_c, labels, 1.0, False)
         ctx.set_materialize_grads(False)
         if not inference_only:
             ctx.save_for_backward(hidden_2d, weight_c, labels, row_lse)

@@ -31,6 +31,7 @@ import torch
 import torch.distributed as dist
 
 from . import ops
+from ._launch import call
 from .fused_linear_logprob_hip import (FusedLinearLogprobHip, _group_size, _require_single_shard, linear_cross_entropy,
                                        shard_labels)
 from .packed import packed_next_token_labels, packed_scatter_logprobs
@@ -185,7 +186,7 @@ def from_parallel_hidden_to_logprobs_packed_sequences(
 
     # Labels: every token's successor inside its own sequence, one kernel (reference: index arithmetic, :810-815).
     cu = cu_seqlens_padded.to(device=target.device, dtype=torch.long)
-    rolled_targets = packed_next_token_labels(target.to(torch.long).contiguous(), cu).unsqueeze(0)
+    rolled_targets = call(packed_next_token_labels, target.to(torch.long).contiguous(), cu).unsqueeze(0)
     hidden = hidden.unsqueeze(0)
     cols = unpacked_seqlen - 1
     if sub_seq_lengths is not None:
@@ -239,8 +240,8 @@ def _fused_vocab_parallel_entropy_from_hidden(
     B, S, H = hidden.shape
     with torch.no_grad():
         labels = torch.full((B * S,), torch.iinfo(torch.int64).max, dtype=torch.int64, device=hidden.device)
-        _, entropy, _, _ = ops.lmhead_fwd(ops.hidden_for_weight(hidden.reshape(B * S, H), lm_head_weight).contiguous(),
-                                          lm_head_weight.contiguous(), labels, 1.0 / float(temperature), True)
+        _, entropy, _, _ = call(ops.lmhead_fwd, ops.hidden_for_weight(hidden.reshape(B * S, H), lm_head_weight).contiguous(),
+                                lm_head_weight.contiguous(), labels, 1.0 / float(temperature), True)
     return entropy.reshape(B, S)
 
 

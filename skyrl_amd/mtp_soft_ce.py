@@ -30,6 +30,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
+from ._launch import call, device_guard, raw_stream, registered_op
 from .ops import _require_device
 
 __all__ = ["soft_ce_from_hidden", "draft_soft_ce_from_hidden", "shift_mask_for_mtp", "softce_fwd", "softce_bwd",
@@ -55,7 +56,7 @@ def _check(student: torch.Tensor, teacher: torch.Tensor, weight: torch.Tensor, s
     return int(T), int(H), int(weight.shape[0])
 
 
-@torch.library.custom_op("skyrl_amd::softce_fwd", mutates_args=())
+@registered_op("skyrl_amd::softce_fwd", mutates_args=())
 def softce_fwd(student_hidden: torch.Tensor, teacher_hidden: torch.Tensor, weight: torch.Tensor, seq_len: int, shift: int,
                rcp_temperature: float) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """``(loss, lse_student, lse_teacher)``, each fp32 ``[T]``, for bf16 ``[T, H]`` hidden states and a bf16 ``[V, H]`` weight;
@@ -65,11 +66,11 @@ def softce_fwd(student_hidden: torch.Tensor, teacher_hidden: torch.Tensor, weigh
     lib = _lib.load()
     ws = torch.empty(int(lib.skyrl_softce_fwd_workspace_bytes(T, H, V)), dtype=torch.uint8, device=dev)
     loss, lse_s, lse_t = (torch.empty(T, dtype=torch.float32, device=dev) for _ in range(3))
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         st = lib.skyrl_softce_fwd(student_hidden.data_ptr(), student_hidden.stride(0), teacher_hidden.data_ptr(),
                                   teacher_hidden.stride(0), weight.data_ptr(), weight.stride(0), T, int(seq_len), int(shift), H, V,
                                   float(rcp_temperature), loss.data_ptr(), lse_s.data_ptr(), lse_t.data_ptr(), ws.data_ptr(),
-                                  ws.numel(), torch.cuda.current_stream(dev).cuda_stream)
+                                  ws.numel(), raw_stream(dev))
     _lib.check(st, "skyrl_softce_fwd")
     return loss, lse_s, lse_t
 
@@ -80,7 +81,7 @@ def _(student_hidden, teacher_hidden, weight, seq_len, shift, rcp_temperature):
     return tuple(student_hidden.new_empty(T, dtype=torch.float32) for _ in range(3))
 
 
-@torch.library.custom_op("skyrl_amd::softce_bwd", mutates_args=())
+@registered_op("skyrl_amd::softce_bwd", mutates_args=())
 def softce_bwd(student_hidden: torch.Tensor, teacher_hidden: torch.Tensor, weight: torch.Tensor, lse_student: torch.Tensor,
                lse_teacher: torch.Tensor, dloss: torch.Tensor, seq_len: int, shift: int, rcp_temperature: float,
                vocab_chunk: int) -> torch.Tensor:
@@ -96,12 +97,12 @@ def softce_bwd(student_hidden: torch.Tensor, teacher_hidden: torch.Tensor, weigh
         raise ValueError(f"bad vocab_chunk {vocab_chunk}: must be 0 (library default) or a multiple of 256")
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     d_student = torch.empty((T, H), dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         st = lib.skyrl_softce_bwd(student_hidden.data_ptr(), student_hidden.stride(0), teacher_hidden.data_ptr(),
                                   teacher_hidden.stride(0), weight.data_ptr(), weight.stride(0), lse_student.data_ptr(),
                                   lse_teacher.data_ptr(), dloss.data_ptr(), T, int(seq_len), int(shift), H, V,
                                   float(rcp_temperature), d_student.data_ptr(), int(vocab_chunk), ws.data_ptr(), ws.numel(),
-                                  torch.cuda.current_stream(dev).cuda_stream)
+                                  raw_stream(dev))
     _lib.check(st, "skyrl_softce_bwd")
     return d_student
 
@@ -114,7 +115,7 @@ def _(student_hidden, teacher_hidden, weight, lse_student, lse_teacher, dloss, s
 class _SoftCE(torch.autograd.Function):
     @staticmethod
     def forward(ctx, student_hidden, teacher_hidden, weight, seq_len, shift, rcp_temperature, vocab_chunk):
-        loss, lse_s, lse_t = softce_fwd(student_hidden, teacher_hidden, weight, seq_len, shift, rcp_temperature)
+        loss, lse_s, lse_t = call(softce_fwd, student_hidden, teacher_hidden, weight, seq_len, shift, rcp_temperature)
         ctx.save_for_backward(student_hidden, teacher_hidden, weight, lse_s, lse_t)
         ctx.args = (seq_len, shift, rcp_temperature, vocab_chunk)
         return loss
@@ -123,8 +124,8 @@ class _SoftCE(torch.autograd.Function):
     def backward(ctx, dloss):
         student_hidden, teacher_hidden, weight, lse_s, lse_t = ctx.saved_tensors
         seq_len, shift, rcp_temperature, vocab_chunk = ctx.args
-        d_student = softce_bwd(student_hidden, teacher_hidden, weight, lse_s, lse_t, dloss.to(torch.float32).contiguous(), seq_len,
-                               shift, rcp_temperature, vocab_chunk)
+        d_student = call(softce_bwd, student_hidden, teacher_hidden, weight, lse_s, lse_t, dloss.to(torch.float32).contiguous(),
+                         seq_len, shift, rcp_temperature, vocab_chunk)
         return d_student, None, None, None, None, None, None
 
 
@@ -183,7 +184,7 @@ def draft_soft_ce_from_hidden(
     return (per_token * mask).sum() / mask.sum().clamp(min=1.0)
 
 
-@torch.library.custom_op("skyrl_amd::topk_logits", mutates_args=())
+@registered_op("skyrl_amd::topk_logits", mutates_args=())
 def topk_logits(hidden: torch.Tensor, weight: torch.Tensor, k: int, rcp_temperature: float) -> Tuple[torch.Tensor, torch.Tensor]:
     """``(values [T, k] fp32, columns [T, k] int32)``: the k largest entries of every row of ``hidden @ weight.T *
     rcp_temperature``, best first, the lower column first among equal values.  bf16 operands, ``1 <= k <= min(V, 1024)``."""
@@ -200,10 +201,10 @@ def topk_logits(hidden: torch.Tensor, weight: torch.Tensor, k: int, rcp_temperat
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     values = torch.empty((T, k), dtype=torch.float32, device=dev)
     columns = torch.empty((T, k), dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         st = lib.skyrl_lmhead_topk_logits(hidden.data_ptr(), hidden.stride(0), weight.data_ptr(), weight.stride(0), T, H, V, int(k),
                                           float(rcp_temperature), values.data_ptr(), columns.data_ptr(), ws.data_ptr(), ws.numel(),
-                                          torch.cuda.current_stream(dev).cuda_stream)
+                                          raw_stream(dev))
     _lib.check(st, "skyrl_lmhead_topk_logits")
     return values, columns
 
@@ -214,7 +215,7 @@ def _(hidden, weight, k, rcp_temperature):
     return hidden.new_empty((T, k), dtype=torch.float32), hidden.new_empty((T, k), dtype=torch.int32)
 
 
-@torch.library.custom_op("skyrl_amd::softce_topk_fwd", mutates_args=())
+@registered_op("skyrl_amd::softce_topk_fwd", mutates_args=())
 def softce_topk_fwd(student_hidden: torch.Tensor, weight: torch.Tensor, teacher_values: torch.Tensor, teacher_columns: torch.Tensor,
                     seq_len: int, shift: int, rcp_temperature: float) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """``(loss [T] fp32, coef [T, k] fp32, columns [T, k] int32)`` for bf16 ``student_hidden [T, H]``, ``weight [V, H]`` and the
@@ -229,11 +230,11 @@ def softce_topk_fwd(student_hidden: torch.Tensor, weight: torch.Tensor, teacher_
     loss = torch.empty(T, dtype=torch.float32, device=dev)
     coef = torch.empty((T, k), dtype=torch.float32, device=dev)
     columns = torch.empty((T, k), dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         st = lib.skyrl_softce_topk_fwd(student_hidden.data_ptr(), student_hidden.stride(0), weight.data_ptr(), weight.stride(0),
                                        teacher_values.data_ptr(), teacher_columns.data_ptr(), T, int(seq_len), int(shift), H, V, k,
                                        float(rcp_temperature), loss.data_ptr(), coef.data_ptr(), columns.data_ptr(),
-                                       torch.cuda.current_stream(dev).cuda_stream)
+                                       raw_stream(dev))
     _lib.check(st, "skyrl_softce_topk_fwd")
     return loss, coef, columns
 
@@ -244,7 +245,7 @@ def _(student_hidden, weight, teacher_values, teacher_columns, seq_len, shift, r
     return (student_hidden.new_empty(T, dtype=torch.float32), torch.empty_like(teacher_values), torch.empty_like(teacher_columns))
 
 
-@torch.library.custom_op("skyrl_amd::softce_topk_bwd", mutates_args=())
+@registered_op("skyrl_amd::softce_topk_bwd", mutates_args=())
 def softce_topk_bwd(weight: torch.Tensor, coef: torch.Tensor, columns: torch.Tensor, dloss: torch.Tensor,
                     rcp_temperature: float) -> torch.Tensor:
     """d loss / d student_hidden, bf16 ``[T, H]``, from what ``softce_topk_fwd`` kept and the upstream gradient ``dloss [T]``."""
@@ -258,9 +259,9 @@ def softce_topk_bwd(weight: torch.Tensor, coef: torch.Tensor, columns: torch.Ten
         raise ValueError("coef fp32 [T, k], columns int32 [T, k] and dloss fp32 [T] must be contiguous")
     lib = _lib.load()
     d_student = torch.empty((T, H), dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         st = lib.skyrl_softce_topk_bwd(weight.data_ptr(), weight.stride(0), coef.data_ptr(), columns.data_ptr(), dloss.data_ptr(), T, H,
-                                       V, k, float(rcp_temperature), d_student.data_ptr(), H, torch.cuda.current_stream(dev).cuda_stream)
+                                       V, k, float(rcp_temperature), d_student.data_ptr(), H, raw_stream(dev))
     _lib.check(st, "skyrl_softce_topk_bwd")
     return d_student
 
@@ -273,8 +274,8 @@ def _(weight, coef, columns, dloss, rcp_temperature):
 class _SoftCETopk(torch.autograd.Function):
     @staticmethod
     def forward(ctx, student_hidden, teacher_hidden, weight, k, seq_len, shift, rcp_temperature):
-        values, columns = topk_logits(teacher_hidden, weight, k, rcp_temperature)
-        loss, coef, used = softce_topk_fwd(student_hidden, weight, values, columns, seq_len, shift, rcp_temperature)
+        values, columns = call(topk_logits, teacher_hidden, weight, k, rcp_temperature)
+        loss, coef, used = call(softce_topk_fwd, student_hidden, weight, values, columns, seq_len, shift, rcp_temperature)
         ctx.save_for_backward(weight, coef, used)
         ctx.rcp_temperature = rcp_temperature
         return loss
@@ -282,8 +283,8 @@ class _SoftCETopk(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dloss):
         weight, coef, used = ctx.saved_tensors
-        return (softce_topk_bwd(weight, coef, used, dloss.to(torch.float32).contiguous(), ctx.rcp_temperature), None, None, None,
-                None, None, None)
+        d_student = call(softce_topk_bwd, weight, coef, used, dloss.to(torch.float32).contiguous(), ctx.rcp_temperature)
+        return d_student, None, None, None, None, None, None
 
 
 def topk_logits_from_hidden(hidden: torch.Tensor, weight: torch.Tensor, k: int, *, temperature: float = 1.0
@@ -293,8 +294,8 @@ def topk_logits_from_hidden(hidden: torch.Tensor, weight: torch.Tensor, k: int, 
     H = hidden.shape[-1]
     k_eff = min(int(k), int(weight.shape[0]))
     with torch.no_grad():
-        values, columns = topk_logits(hidden.detach().reshape(-1, H).to(torch.bfloat16).contiguous(), weight.detach().to(torch.bfloat16),
-                                      k_eff, 1.0 / float(temperature))
+        values, columns = call(topk_logits, hidden.detach().reshape(-1, H).to(torch.bfloat16).contiguous(),
+                               weight.detach().to(torch.bfloat16), k_eff, 1.0 / float(temperature))
     shape = tuple(hidden.shape[:-1]) + (k_eff,)
     return values.reshape(shape), columns.reshape(shape).to(torch.int64)
 

@@ -24,6 +24,7 @@ from typing import Any, Dict, Optional, Tuple
 import torch
 
 from . import _lib
+from ._launch import call, device_guard, raw_stream, registered_op
 from .ops import _require_device
 
 __all__ = ["off_policy_correction_enabled", "compute_off_policy_correction", "apply_off_policy_correction", "correction_weight",
@@ -50,7 +51,7 @@ def off_policy_correction_enabled(off_policy_correction: Any) -> bool:
             or (_get(c, "token_mask_is_threshold_low") is not None and _get(c, "token_mask_is_threshold_high") is not None))
 
 
-@torch.library.custom_op("skyrl_amd::off_policy_correction", mutates_args=())
+@registered_op("skyrl_amd::off_policy_correction", mutates_args=())
 def off_policy_correction_terms(old_log_probs: torch.Tensor, rollout_logprobs: torch.Tensor, loss_mask: Optional[torch.Tensor],
                                 tis_type: int, tis_cap: float, seq_metric: int, seq_low: float, seq_high: float,
                                 outlier_low: Optional[float], outlier_high: Optional[float], token_low: Optional[float],
@@ -71,12 +72,12 @@ def off_policy_correction_terms(old_log_probs: torch.Tensor, rollout_logprobs: t
         return keep, tis, weight, metrics
     row_stats = torch.empty(rows * _ROW_STATS, dtype=torch.float32, device=dev)
     ref = lambda v: None if v is None else ctypes.byref(ctypes.c_float(float(v)))  # noqa: E731
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         st = _lib.load().skyrl_off_policy_correction(
             old_log_probs.data_ptr(), rollout_logprobs.data_ptr(), None if loss_mask is None else loss_mask.data_ptr(), rows, cols,
             int(tis_type), float(tis_cap), int(seq_metric), float(seq_low), float(seq_high), ref(outlier_low), ref(outlier_high),
             ref(token_low), ref(token_high), keep.data_ptr(), tis.data_ptr(), weight.data_ptr(), metrics.data_ptr(),
-            row_stats.data_ptr(), torch.cuda.current_stream(dev).cuda_stream)
+            row_stats.data_ptr(), raw_stream(dev))
     _lib.check(st, "skyrl_off_policy_correction")
     return keep, tis, weight, metrics
 
@@ -112,8 +113,8 @@ def _run(old_log_probs, rollout_logprobs, loss_mask, cfg, sync_metrics: bool):
     for extent in shape[:-1]:
         rows *= int(extent)
     flat = lambda t: None if t is None else t.detach().reshape(rows, cols).to(torch.float32).contiguous()  # noqa: E731
-    keep, tis, weight, m = off_policy_correction_terms(
-        flat(old_log_probs), flat(rollout_logprobs), flat(loss_mask), _TIS[tis_type], float(tis_cap), _SEQ[seq_metric],
+    keep, tis, weight, m = call(
+        off_policy_correction_terms, flat(old_log_probs), flat(rollout_logprobs), flat(loss_mask), _TIS[tis_type], float(tis_cap), _SEQ[seq_metric],
         float(seq_low), float(seq_high), out_low, out_high, tok_low if tok_high is not None else None,
         tok_high if tok_low is not None else None)
     host = m.tolist() if sync_metrics else None                  # one read-back for all metrics

@@ -16,6 +16,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
+from ._launch import call, device_guard, raw_stream, registered_op
 
 __all__ = ["hidden_for_weight", "lmhead_fwd", "lmhead_bwd", "lmhead_bwd_bf16", "lmhead_bwd_hidden", "lmhead_bwd_active_rows", "fwd_workspace_bytes",
            "bwd_workspace_bytes"]
@@ -72,8 +73,8 @@ def _bf16_terms(hidden: torch.Tensor, weight: torch.Tensor) -> Tuple[torch.Tenso
     h2 = torch.empty((T, terms * H), dtype=torch.bfloat16, device=dev)
     w2 = torch.empty((V, terms * H), dtype=torch.bfloat16, device=dev)
     h_layout, w_layout = (_SPLIT_HI_HI, _SPLIT_HI_LO) if terms == 2 else (_SPLIT_HI_HI_LO, _SPLIT_HI_LO_HI)
-    with torch.cuda.device(dev):
-        stream = torch.cuda.current_stream(dev).cuda_stream
+    with device_guard(dev):
+        stream = raw_stream(dev)
         if T > 0:
             _lib.check(lib.skyrl_lmhead_split_operand(hidden.data_ptr(), int(hidden.dtype == torch.float32), hidden.stride(0), T, H,
                                                       h_layout, h2.data_ptr(), terms * H, stream), "skyrl_lmhead_split_operand")
@@ -103,7 +104,7 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
-@torch.library.custom_op("skyrl_amd::lmhead_fwd", mutates_args=())
+@registered_op("skyrl_amd::lmhead_fwd", mutates_args=())
 def lmhead_fwd(
     hidden: torch.Tensor,
     weight: torch.Tensor,
@@ -128,8 +129,8 @@ def lmhead_fwd(
     ws_bytes = int(lib.skyrl_lmhead_fwd_workspace_bytes(T, H, V))
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     hidden, weight, terms = _bf16_terms(hidden, weight)
-    with torch.cuda.device(dev):
-        stream = torch.cuda.current_stream(dev).cuda_stream
+    with device_guard(dev):
+        stream = raw_stream(dev)
         st = lib.skyrl_lmhead_fwd(
             hidden.data_ptr(), hidden.stride(0), weight.data_ptr(), weight.stride(0), labels.data_ptr(), T, terms * H, V,
             float(rcp_temperature), logprobs.data_ptr(), _ptr(entropy if want_entropy else None), row_lse.data_ptr(),
@@ -147,7 +148,7 @@ def _(hidden, weight, labels, rcp_temperature, want_entropy):
     return torch.empty(T, **f32), torch.empty(n, **f32), torch.empty(T, **f32), torch.empty(n, **f32)
 
 
-@torch.library.custom_op("skyrl_amd::lmhead_bwd", mutates_args=())
+@registered_op("skyrl_amd::lmhead_bwd", mutates_args=())
 def lmhead_bwd(
     hidden: torch.Tensor,
     weight: torch.Tensor,
@@ -174,7 +175,7 @@ def lmhead_bwd(
     return d_hidden, d_weight
 
 
-@torch.library.custom_op("skyrl_amd::lmhead_bwd_bf16", mutates_args=())
+@registered_op("skyrl_amd::lmhead_bwd_bf16", mutates_args=())
 def lmhead_bwd_bf16(
     hidden: torch.Tensor,
     weight: torch.Tensor,
@@ -206,7 +207,7 @@ def _(hidden, weight, labels, row_lse, row_pz, dlogprobs, dentropy, rcp_temperat
             torch.empty(weight.shape, dtype=torch.bfloat16, device=weight.device))
 
 
-@torch.library.custom_op("skyrl_amd::lmhead_bwd_hidden", mutates_args=())
+@registered_op("skyrl_amd::lmhead_bwd_hidden", mutates_args=())
 def lmhead_bwd_hidden(
     hidden: torch.Tensor,
     weight: torch.Tensor,
@@ -267,8 +268,8 @@ def lmhead_bwd_active_rows(
         raise TypeError(f"d_weight is fp32 or bf16, not {dweight_dtype}")
     args = (hidden, weight, labels, row_lse, row_pz, dlogprobs, dentropy, rcp_temperature, vocab_chunk, True)
     if want_dweight:
-        return lmhead_bwd(*args) if dweight_dtype == torch.float32 else lmhead_bwd_bf16(*args)
-    return lmhead_bwd_hidden(*args), None
+        return call(lmhead_bwd if dweight_dtype == torch.float32 else lmhead_bwd_bf16, *args)
+    return call(lmhead_bwd_hidden, *args), None
 
 
 # SKYRL_BWD_FLUSH_TINY_DZ of include/skyrl_lmhead.h: an option of every backward call made through this module, off by default.
@@ -308,8 +309,8 @@ def _bwd_into(lib, hidden, weight, labels, row_lse, row_pz, dlogprobs, dentropy,
         raise ValueError(f"no backward workspace for T={T}, H={H}, V={V}: every extent must be at least 1")
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     hidden, weight, terms = _bf16_terms(hidden, weight)  # recomputed rather than kept from the forward: a pass over W, no 2x copy held
-    with torch.cuda.device(dev):
-        stream = torch.cuda.current_stream(dev).cuda_stream
+    with device_guard(dev):
+        stream = raw_stream(dev)
         st = lib.skyrl_lmhead_bwd_split(
             hidden.data_ptr(), hidden.stride(0), weight.data_ptr(), weight.stride(0), labels.data_ptr(),
             row_lse.data_ptr(), _ptr(row_pz if dentropy is not None else None), dlogprobs.data_ptr(), _ptr(dentropy),

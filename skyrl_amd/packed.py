@@ -16,6 +16,7 @@ from typing import Optional
 import torch
 
 from . import _lib
+from ._launch import call, device_guard, raw_stream, registered_op
 from .ops import _require_device
 
 __all__ = ["packed_next_token_labels", "packed_scatter_logprobs"]
@@ -28,7 +29,7 @@ def _i64_vector(name: str, t: torch.Tensor, dev: torch.device, numel: Optional[i
     return t.to(device=dev, dtype=torch.int64).contiguous()
 
 
-@torch.library.custom_op("skyrl_amd::packed_next_token_labels", mutates_args=())
+@registered_op("skyrl_amd::packed_next_token_labels", mutates_args=())
 def packed_next_token_labels(tokens: torch.Tensor, cu_seqlens: torch.Tensor) -> torch.Tensor:
     """``tokens`` int64 [T] (packed), ``cu_seqlens`` [n+1] -> labels int64 [T]: ``tokens[cu[s] + (off + 1) mod len_s]``."""
     dev = _require_device(tokens)
@@ -39,9 +40,9 @@ def packed_next_token_labels(tokens: torch.Tensor, cu_seqlens: torch.Tensor) -> 
     if cu.numel() < 1:
         raise ValueError("cu_seqlens needs at least one element")
     labels = torch.empty_like(tokens)
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         st = _lib.load().skyrl_packed_next_token_labels(tokens.data_ptr(), cu.data_ptr(), cu.numel() - 1, tokens.numel(),
-                                                        labels.data_ptr(), torch.cuda.current_stream(dev).cuda_stream)
+                                                        labels.data_ptr(), raw_stream(dev))
     _lib.check(st, "skyrl_packed_next_token_labels")
     return labels
 
@@ -54,10 +55,10 @@ def _(tokens, cu_seqlens):
 def _scatter_call(fn_name: str, src: torch.Tensor, dst: torch.Tensor, cu, seg_row, seg_col, seg_len, attention_mask, T: int,
                   rows: int, cols: int, dev: torch.device) -> None:
     ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         st = getattr(_lib.load(), fn_name)(src.data_ptr(), cu.data_ptr(), cu.numel() - 1, T, ptr(seg_row), ptr(seg_col),
                                            ptr(seg_len), ptr(attention_mask), rows, cols, dst.data_ptr(),
-                                           torch.cuda.current_stream(dev).cuda_stream)
+                                           raw_stream(dev))
     _lib.check(st, fn_name)
 
 
@@ -84,7 +85,7 @@ def _scatter_operands(cu_seqlens, seg_row, seg_col, seg_len, attention_mask, row
     return cu, segs[0], segs[1], segs[2], attention_mask
 
 
-@torch.library.custom_op("skyrl_amd::packed_scatter_logprobs", mutates_args=())
+@registered_op("skyrl_amd::packed_scatter_logprobs", mutates_args=())
 def _packed_scatter(packed: torch.Tensor, cu_seqlens: torch.Tensor, seg_row: Optional[torch.Tensor],
                     seg_col: Optional[torch.Tensor], seg_len: Optional[torch.Tensor],
                     attention_mask: Optional[torch.Tensor], rows: int, cols: int) -> torch.Tensor:
@@ -104,7 +105,7 @@ def _(packed, cu_seqlens, seg_row, seg_col, seg_len, attention_mask, rows, cols)
     return packed.new_empty((rows, cols))
 
 
-@torch.library.custom_op("skyrl_amd::packed_gather_grad", mutates_args=())
+@registered_op("skyrl_amd::packed_gather_grad", mutates_args=())
 def _packed_gather(d_out: torch.Tensor, cu_seqlens: torch.Tensor, seg_row: Optional[torch.Tensor],
                    seg_col: Optional[torch.Tensor], seg_len: Optional[torch.Tensor],
                    attention_mask: Optional[torch.Tensor], T: int) -> torch.Tensor:
@@ -136,7 +137,7 @@ def _scatter_backward(ctx, d_out):
     cu = saved.pop(0)
     seg_row, seg_col, seg_len = (saved.pop(0), saved.pop(0), saved.pop(0)) if ctx.has_segs else (None, None, None)
     mask = saved.pop(0) if ctx.has_mask else None
-    d_packed = _packed_gather(d_out.to(torch.float32).contiguous(), cu, seg_row, seg_col, seg_len, mask, ctx.T)
+    d_packed = call(_packed_gather, d_out.to(torch.float32).contiguous(), cu, seg_row, seg_col, seg_len, mask, ctx.T)
     return d_packed, None, None, None, None, None, None, None
 
 
@@ -154,4 +155,5 @@ def packed_scatter_logprobs(packed: torch.Tensor, cu_seqlens: torch.Tensor, rows
     ``o < seg_len[s] - 1``.  With ``attention_mask`` ``[rows, cols + 1]`` the j-th real token of row ``s`` takes packed
     token ``cu[s] + j`` (all real tokens but the last).  Differentiable with respect to ``packed``.
     """
-    return _packed_scatter(packed, cu_seqlens, seg_row, seg_col, seg_len, attention_mask, int(rows), int(cols))
+    args = (packed, cu_seqlens, seg_row, seg_col, seg_len, attention_mask, int(rows), int(cols))
+    return _packed_scatter(*args) if packed.requires_grad and torch.is_grad_enabled() else call(_packed_scatter, *args)

@@ -38,6 +38,7 @@ from typing import Any, Dict, Optional, Tuple
 import torch
 
 from . import _lib
+from ._launch import call, device_guard, raw_stream, registered_op
 from .ops import _require_device
 
 __all__ = ["ppo_policy_loss", "cross_entropy_loss", "importance_sampling_loss", "sapo_policy_loss", "gspo_policy_loss",
@@ -85,7 +86,7 @@ def _flat_f32(name: str, t: Optional[torch.Tensor], numel: int) -> Optional[torc
     return t.detach().reshape(-1).to(torch.float32).contiguous()
 
 
-@torch.library.custom_op("skyrl_amd::ppo_policy_loss", mutates_args=())
+@registered_op("skyrl_amd::ppo_policy_loss", mutates_args=())
 def ppo_policy_loss_terms(
     log_probs: torch.Tensor,
     old_log_probs: Optional[torch.Tensor],
@@ -117,11 +118,11 @@ def ppo_policy_loss_terms(
     grad = torch.empty(n, dtype=torch.float32, device=dev)
     partials = torch.empty(3 * _LOSS_PARTIALS, dtype=torch.float32, device=dev)   # per-workgroup sums of the kernel
     ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         st = _lib.load().skyrl_ppo_policy_loss(
             log_probs.data_ptr(), ptr(old_log_probs), ptr(advantages), ptr(loss_mask), ptr(loss_weight), n,
             float(eps_clip_low), float(eps_clip_high), float(clip_ratio_c), int(loss_type), sums.data_ptr(),
-            grad.data_ptr(), partials.data_ptr(), torch.cuda.current_stream(dev).cuda_stream)
+            grad.data_ptr(), partials.data_ptr(), raw_stream(dev))
     _lib.check(st, "skyrl_ppo_policy_loss")
     return sums, grad
 
@@ -141,8 +142,8 @@ class _PolicyLoss(torch.autograd.Function):
     @staticmethod
     def forward(ctx, log_probs, old_log_probs, advantages, loss_mask, loss_weight, eps_low, eps_high, clip_c, loss_type):
         n = log_probs.numel()
-        sums, grad = ppo_policy_loss_terms(
-            _flat_f32("log_probs", log_probs, n), _flat_f32("old_log_probs", old_log_probs, n),
+        sums, grad = call(
+            ppo_policy_loss_terms, _flat_f32("log_probs", log_probs, n), _flat_f32("old_log_probs", old_log_probs, n),
             _flat_f32("advantages", advantages, n), _flat_f32("loss_mask", loss_mask, n),
             _flat_f32("loss_weight", loss_weight, n), eps_low, eps_high, clip_c, loss_type)
         ctx.save_for_backward(grad)
@@ -423,7 +424,7 @@ def _same_f32(name: str, t: Optional[torch.Tensor], like: torch.Tensor) -> Optio
     return t.detach().to(torch.float32).contiguous()
 
 
-@torch.library.custom_op("skyrl_amd::approx_kl", mutates_args=())
+@registered_op("skyrl_amd::approx_kl", mutates_args=())
 def _approx_kl(log_probs: torch.Tensor, log_probs_base: torch.Tensor, loss_mask: Optional[torch.Tensor], estimator: int,
                grad_mode: int) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """``(kld, row_mean, mean, grad)`` for contiguous fp32 ``[rows, cols]`` inputs; grad_mode 1: elementwise derivative of
@@ -434,11 +435,11 @@ def _approx_kl(log_probs: torch.Tensor, log_probs_base: torch.Tensor, loss_mask:
     row_mean = torch.empty(rows, dtype=torch.float32, device=dev)
     mean = torch.empty((), dtype=torch.float32, device=dev)
     grad = torch.empty_like(log_probs) if grad_mode else torch.empty(0, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         st = _lib.load().skyrl_approx_kl(
             log_probs.data_ptr(), log_probs_base.data_ptr(), None if loss_mask is None else loss_mask.data_ptr(), rows, cols,
             int(estimator), kld.data_ptr(), row_mean.data_ptr(), mean.data_ptr(), int(grad_mode),
-            grad.data_ptr() if grad_mode else None, torch.cuda.current_stream(dev).cuda_stream)
+            grad.data_ptr() if grad_mode else None, raw_stream(dev))
     _lib.check(st, "skyrl_approx_kl")
     return kld, row_mean, mean, grad
 
@@ -466,7 +467,7 @@ class _ApproxKL(torch.autograd.Function):
     @staticmethod
     def forward(ctx, log_probs, log_probs_base, loss_mask, kl_estimator_type, grad_mode):
         lp, base, mask, est = _kl_operands(log_probs, log_probs_base, loss_mask, kl_estimator_type)
-        kld, _, mean, grad = _approx_kl(lp, base, mask, est, grad_mode)
+        kld, _, mean, grad = call(_approx_kl, lp, base, mask, est, grad_mode)
         ctx.save_for_backward(grad)
         ctx.shape, ctx.dtype = log_probs.shape, log_probs.dtype
         return kld.reshape(log_probs.shape) if grad_mode == 1 else mean
@@ -508,17 +509,17 @@ def approx_kl_loss(
     return _ApproxKL.apply(log_probs, log_probs_base, loss_mask, kl_estimator_type, 2)
 
 
-@torch.library.custom_op("skyrl_amd::masked_mean", mutates_args=())
+@registered_op("skyrl_amd::masked_mean", mutates_args=())
 def _masked_mean(values: torch.Tensor, mask: Optional[torch.Tensor], want_grad: bool) -> Tuple[torch.Tensor, torch.Tensor]:
     """``(means [rows], dvalues [rows, cols] or empty)`` for contiguous fp32 ``[rows, cols]`` inputs."""
     dev = _require_device(values)
     rows, cols = values.shape
     means = torch.empty(rows, dtype=torch.float32, device=dev)
     dv = torch.empty_like(values) if want_grad else torch.empty(0, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         st = _lib.load().skyrl_masked_mean(values.data_ptr(), None if mask is None else mask.data_ptr(), rows, cols,
                                            means.data_ptr(), dv.data_ptr() if want_grad else None,
-                                           torch.cuda.current_stream(dev).cuda_stream)
+                                           raw_stream(dev))
     _lib.check(st, "skyrl_masked_mean")
     return means, dv
 
@@ -533,7 +534,7 @@ class _MaskedMean(torch.autograd.Function):
     def forward(ctx, tensor, mask, rows, cols, out_shape):
         v = tensor.detach().to(torch.float32).contiguous().reshape(rows, cols)
         m = None if mask is None else mask.detach().to(torch.float32).expand_as(tensor).contiguous().reshape(rows, cols)
-        means, dv = _masked_mean(v, m, bool(ctx.needs_input_grad[0]))
+        means, dv = call(_masked_mean, v, m, bool(ctx.needs_input_grad[0]))
         ctx.save_for_backward(dv)
         ctx.shape, ctx.dtype, ctx.rows = tensor.shape, tensor.dtype, rows
         return means.reshape(out_shape)
@@ -568,7 +569,7 @@ def masked_mean(tensor: torch.Tensor, mask: Optional[torch.Tensor], dim: Optiona
 # ----------------------------------------------------------------------------------------------------------------------
 # the assembled actor loss
 # ----------------------------------------------------------------------------------------------------------------------
-@torch.library.custom_op("skyrl_amd::actor_loss", mutates_args=())
+@registered_op("skyrl_amd::actor_loss", mutates_args=())
 def _actor_loss(log_probs: torch.Tensor, old_log_probs: Optional[torch.Tensor], advantages: Optional[torch.Tensor],
                 loss_mask: Optional[torch.Tensor], loss_weight: Optional[torch.Tensor], base_log_probs: Optional[torch.Tensor],
                 entropy: Optional[torch.Tensor], loss_type: int, eps_clip_low: float, eps_clip_high: float, clip_ratio_c: float,
@@ -586,13 +587,13 @@ def _actor_loss(log_probs: torch.Tensor, old_log_probs: Optional[torch.Tensor], 
     dlp = torch.empty_like(log_probs)
     dent = torch.empty_like(log_probs) if entropy is not None else torch.empty(0, dtype=torch.float32, device=dev)
     ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         st = _lib.load().skyrl_actor_loss(
             log_probs.data_ptr(), ptr(old_log_probs), ptr(advantages), ptr(loss_mask), ptr(loss_weight), ptr(base_log_probs),
             ptr(entropy), rows, cols, int(loss_type), float(eps_clip_low), float(eps_clip_high), float(clip_ratio_c),
             int(kl_estimator), float(policy_scale), float(term_scale), float(kl_coef), float(entropy_coef), out.data_ptr() + 24,
             out.data_ptr(), dlp.data_ptr(), dent.data_ptr() if entropy is not None else None,
-            torch.cuda.current_stream(dev).cuda_stream)
+            raw_stream(dev))
     _lib.check(st, "skyrl_actor_loss")
     return out, dlp, dent
 
@@ -614,8 +615,8 @@ class _ActorLoss(torch.autograd.Function):
                         ("base_log_probs", base), ("entropy", entropy)):
             if t is not None and t.shape != log_probs.shape:
                 raise ValueError(f"{name} has shape {tuple(t.shape)}, expected {tuple(log_probs.shape)}")
-        out, dlp, dent = _actor_loss(flat(log_probs), flat(old), flat(adv), flat(mask), flat(weight), flat(base), flat(entropy),
-                                     *scalars)
+        out, dlp, dent = call(_actor_loss, flat(log_probs), flat(old), flat(adv), flat(mask), flat(weight), flat(base),
+                              flat(entropy), *scalars)
         ctx.set_materialize_grads(False)
         ctx.save_for_backward(dlp, dent)
         ctx.lp_meta = (log_probs.shape, log_probs.dtype)

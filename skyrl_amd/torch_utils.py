@@ -23,6 +23,7 @@ from typing import Any, Optional, Tuple
 import torch
 
 from . import _lib
+from ._launch import call, device_guard, raw_stream, registered_op
 from .ops import _require_device as _require_device_all
 
 __all__ = ["logprobs_from_logits", "logprobs_from_logits_v2", "logprobs_from_logits_flash_attn", "chunked_entropy_from_logits",
@@ -85,7 +86,7 @@ def _check_rows(name: str, t: Optional[torch.Tensor], T: int, dtype: torch.dtype
         raise ValueError(f"{name} must be a contiguous {dtype} tensor of shape [{T}], got {t.dtype} {tuple(t.shape)}")
 
 
-@torch.library.custom_op("skyrl_amd::logits_fwd", mutates_args=())
+@registered_op("skyrl_amd::logits_fwd", mutates_args=())
 def logits_fwd(logits: torch.Tensor, labels: Optional[torch.Tensor], rcp_temperature: float, want_entropy: bool
                ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """``(logprobs, entropy, row_lse, row_pz)``, fp32 ``[T]``, of ``logits [T, V] * rcp_temperature``.  Without ``labels`` the
@@ -99,8 +100,8 @@ def logits_fwd(logits: torch.Tensor, labels: Optional[torch.Tensor], rcp_tempera
     if T == 0:
         return lp, ent, lse, pz
     lib = _lib.load()
-    with torch.cuda.device(dev):
-        stream = torch.cuda.current_stream(dev).cuda_stream
+    with device_guard(dev):
+        stream = raw_stream(dev)
         for view, r0 in pieces:
             rows, _, ld = _rows(view)
             st = lib.skyrl_logits_fwd(view.data_ptr(), _DTYPES[logits.dtype], ld, None if labels is None else labels.data_ptr() + 8 * r0,
@@ -141,8 +142,8 @@ def _bwd_into(out: torch.Tensor, logits, labels, row_lse, row_pz, dlogprobs, den
     runs = pieces if len(pieces) >= len(out_pieces) else out_pieces        # the finer of the two partitions
     ptr = lambda t, r0, size: None if t is None else t.data_ptr() + size * r0  # noqa: E731
     lib = _lib.load()
-    with torch.cuda.device(dev):
-        stream = torch.cuda.current_stream(dev).cuda_stream
+    with device_guard(dev):
+        stream = raw_stream(dev)
         for run, r0 in runs:
             n = int(run.shape[0])
             src, dst = _row_run(pieces, r0, n), _row_run(out_pieces, r0, n)
@@ -153,7 +154,7 @@ def _bwd_into(out: torch.Tensor, logits, labels, row_lse, row_pz, dlogprobs, den
             _lib.check(st, "skyrl_logits_bwd")
 
 
-@torch.library.custom_op("skyrl_amd::logits_bwd", mutates_args=())
+@registered_op("skyrl_amd::logits_bwd", mutates_args=())
 def logits_bwd(logits: torch.Tensor, labels: Optional[torch.Tensor], row_lse: torch.Tensor, row_pz: Optional[torch.Tensor],
                dlogprobs: Optional[torch.Tensor], dentropy: Optional[torch.Tensor], rcp_temperature: float) -> torch.Tensor:
     """d loss / d logits, a new ``[T, V]`` tensor in the logits' dtype."""
@@ -167,7 +168,7 @@ def _(logits, labels, row_lse, row_pz, dlogprobs, dentropy, rcp_temperature):
     return logits.new_empty(logits.shape)
 
 
-@torch.library.custom_op("skyrl_amd::logits_bwd_", mutates_args=("logits",))
+@registered_op("skyrl_amd::logits_bwd_", mutates_args=("logits",))
 def logits_bwd_(logits: torch.Tensor, labels: Optional[torch.Tensor], row_lse: torch.Tensor, row_pz: Optional[torch.Tensor],
                 dlogprobs: Optional[torch.Tensor], dentropy: Optional[torch.Tensor], rcp_temperature: float) -> None:
     """The same gradient written over the logits (what the flash-attn cross-entropy does with ``inplace_backward=True``)."""
@@ -179,7 +180,7 @@ class _FromLogits(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, logits, labels, rcp_temperature, want_entropy, inplace_backward):
-        lp, ent, lse, pz = logits_fwd(logits, labels, rcp_temperature, want_entropy)
+        lp, ent, lse, pz = call(logits_fwd, logits, labels, rcp_temperature, want_entropy)
         ctx.save_for_backward(logits, labels, lse, pz if want_entropy else None)
         ctx.args = (rcp_temperature, want_entropy, inplace_backward)
         ctx.set_materialize_grads(False)
@@ -199,7 +200,7 @@ class _FromLogits(torch.autograd.Function):
         if inplace:
             logits_bwd_(logits, labels, lse, pz, f(dlp), f(dent), rcp_temperature)
             return logits, None, None, None, None
-        return logits_bwd(logits, labels, lse, pz, f(dlp), f(dent), rcp_temperature), None, None, None, None
+        return call(logits_bwd, logits, labels, lse, pz, f(dlp), f(dent), rcp_temperature), None, None, None, None
 
 
 def _flat(logits: torch.Tensor) -> torch.Tensor:
@@ -289,7 +290,7 @@ class DistributedLogprob(torch.autograd.Function):
         t64 = target.reshape(-1).to(torch.int64)
         outside = (t64 < vocab_start_index) | (t64 >= vocab_end_index)
         labels = torch.where(outside, torch.full_like(t64, -1), t64 - vocab_start_index).contiguous()
-        lp, _, lse, _ = logits_fwd(flat, labels, 1.0, False)
+        lp, _, lse, _ = call(logits_fwd, flat, labels, 1.0, False)
         if not inference_only:
             ctx.save_for_backward(flat, labels, lse)
         ctx.in_dtype, ctx.in_shape = vocab_parallel_logits.dtype, vocab_parallel_logits.shape
@@ -299,7 +300,7 @@ class DistributedLogprob(torch.autograd.Function):
     def backward(ctx, *grad_outputs):
         flat, labels, lse = ctx.saved_tensors
         g = grad_outputs[0].reshape(-1).to(torch.float32).contiguous()
-        grad = logits_bwd(flat, labels, lse, None, g, None, 1.0)
+        grad = call(logits_bwd, flat, labels, lse, None, g, None, 1.0)
         return grad.reshape(ctx.in_shape).to(ctx.in_dtype), None, None, None, None, None
 
 
@@ -345,7 +346,7 @@ def from_parallel_logits_to_logprobs_packed_sequences(vocab_parallel_logits: tor
     device = target.device
     batch_size = len(sub_seq_lengths) if sub_seq_lengths is not None else cu_seqlens_padded.shape[0] - 1
     cu = cu_seqlens_padded.to(device=device, dtype=torch.long)
-    rolled = packed_next_token_labels(target.to(torch.long).contiguous(), cu).unsqueeze(0)
+    rolled = call(packed_next_token_labels, target.to(torch.long).contiguous(), cu).unsqueeze(0)
     if sub_seq_lengths is not None:
         rows, row_offs, seq_lens = _packed_subseq_row_indices_offsets_and_lens(cu, sub_seq_lengths, device)
         layout = dict(seg_row=rows, seg_col=row_offs, seg_len=seq_lens)

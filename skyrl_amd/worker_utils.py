@@ -14,6 +14,7 @@ from typing import Any, Dict, Optional
 import torch
 
 from . import _lib
+from ._launch import call, device_guard, raw_stream, registered_op
 from .ops import _require_device
 
 __all__ = ["compute_minibatch_rollout_logprob_diff_metrics", "logprob_diff_terms", "MINIBATCH_ROLLOUT_LOGPROB_DIFF_PREFIX",
@@ -29,7 +30,7 @@ MINIBATCH_ROLLOUT_LOGPROB_DIFF_MIN_KEY = f"{MINIBATCH_ROLLOUT_LOGPROB_DIFF_PREFI
 _PARTIALS = 5 * 256   # 5 * SKYRL_POLICY_LOSS_PARTIALS of the header
 
 
-@torch.library.custom_op("skyrl_amd::logprob_diff_metrics", mutates_args=())
+@registered_op("skyrl_amd::logprob_diff_metrics", mutates_args=())
 def logprob_diff_terms(log_probs: torch.Tensor, rollout_logprobs: torch.Tensor, loss_mask: Optional[torch.Tensor]) -> torch.Tensor:
     """``[mean, mean of squares, max, min]`` of ``|log_probs - rollout_logprobs|`` over the masked tokens, fp32 ``[4]``, for
     contiguous fp32 inputs of one shape."""
@@ -41,10 +42,10 @@ def logprob_diff_terms(log_probs: torch.Tensor, rollout_logprobs: torch.Tensor, 
         raise ValueError("the statistics of an empty micro-batch are undefined (Tensor.max() raises as well)")
     out = torch.empty(4, dtype=torch.float32, device=dev)
     partials = torch.empty(_PARTIALS, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         st = _lib.load().skyrl_logprob_diff_metrics(
             log_probs.data_ptr(), rollout_logprobs.data_ptr(), None if loss_mask is None else loss_mask.data_ptr(), log_probs.numel(),
-            out.data_ptr(), partials.data_ptr(), torch.cuda.current_stream(dev).cuda_stream)
+            out.data_ptr(), partials.data_ptr(), raw_stream(dev))
     _lib.check(st, "skyrl_logprob_diff_metrics")
     return out
 
@@ -62,7 +63,7 @@ def compute_minibatch_rollout_logprob_diff_metrics(action_log_probs: torch.Tenso
     if rollout_logprobs is None:
         return {}
     flat = lambda t: None if t is None else t.detach().to(torch.float32).expand(action_log_probs.shape).contiguous()  # noqa: E731
-    out = logprob_diff_terms(flat(action_log_probs), flat(rollout_logprobs), flat(loss_mask))
+    out = call(logprob_diff_terms, flat(action_log_probs), flat(rollout_logprobs), flat(loss_mask))
     values = out.tolist() if sync_metrics else out.unbind(0)   # one read-back for the four
     return dict(zip((MINIBATCH_ROLLOUT_LOGPROB_DIFF_MEAN_KEY, MINIBATCH_ROLLOUT_LOGPROB_DIFF_SQ_MEAN_KEY,
                      MINIBATCH_ROLLOUT_LOGPROB_DIFF_MAX_KEY, MINIBATCH_ROLLOUT_LOGPROB_DIFF_MIN_KEY), values))
