@@ -11,7 +11,7 @@ import contextlib
 
 import torch
 
-__all__ = ["registered_op", "call", "device_guard", "raw_stream"]
+__all__ = ["registered_op", "plain_eager", "call", "device_guard", "raw_stream"]
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 _NO_GUARD = contextlib.nullcontext()
@@ -26,11 +26,18 @@ def registered_op(name: str, mutates_args=()):
     return register
 
 
+def plain_eager() -> bool:
+    """Whether nothing follows the ops of this call: no compiler or tracer, no dispatch or function mode, no functorch transform, no
+    profiler (whose record names them)."""
+    return not (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
+                or torch._C._len_torch_function_stack() > 0 or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch._C._is_tracing() or torch._C._autograd._profiler_enabled())
+
+
 def call(op, *args):
-    """``op(*args)`` for a caller that needs no gradient from it: the registered function itself unless a compiler, a dispatch mode,
-    a functorch transform or a tensor subclass takes part."""
-    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
-            or torch._C._functorch.peek_interpreter_stack() is not None):
+    """``op(*args)`` for a caller that needs no gradient from it: the registered function itself in a plain eager call without tensor
+    subclasses."""
+    if not plain_eager():
         return op(*args)
     for a in args:
         if isinstance(a, torch.Tensor) and type(a) not in _PLAIN:

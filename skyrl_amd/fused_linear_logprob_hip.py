@@ -96,12 +96,14 @@ def _require_single_shard(group: Optional[dist.ProcessGroup], what: str) -> None
         )
 
 
-def shard_labels(target: torch.Tensor, vocab_start_index: int, vocab_end_index: int, local_vocab: int) -> torch.Tensor:
+def shard_labels(target: torch.Tensor, vocab_start_index: int, vocab_end_index: int, local_vocab: int,
+                 own: bool = False) -> torch.Tensor:
     """Token ids -> int64 rows of the weight shard; ids outside ``[vocab_start_index, vocab_end_index)`` become a value that
     matches no row.  The kernels take any value outside ``[0, local_vocab)`` that way, so for the whole vocabulary (the single
-    shard of this backend) the ids already are the labels and nothing is launched."""
+    shard of this backend) the ids already are the labels and nothing is launched.  ``own``: never the caller's tensor, which it
+    may reuse before the backward."""
     if vocab_start_index == 0 and vocab_end_index >= local_vocab:
-        return target.to(torch.int64)
+        return target.to(torch.int64, copy=own)
     outside = (target < vocab_start_index) | (target >= vocab_end_index)
     target = target.to(torch.int64)  # int32 ids: the sentinel does not fit their dtype
     return torch.where(outside, _OOV_LABEL_SENTINEL, target - vocab_start_index)
@@ -196,9 +198,8 @@ class FusedLinearLogprobHip(torch.autograd.Function):
         local_vocab = int(weight.shape[0])
         # Targets outside [vocab_start_index, vocab_end_index) get a label that matches no column: forward 0, backward keeps
         # -softmax * grad (fused_linear_logprob_triton.py:1876-1878, 1898-1905, 1929-1931).
-        labels = shard_labels(target, vocab_start_index, vocab_end_index, local_vocab).reshape(-1).contiguous()
-        if not inference_only and labels.data_ptr() == target.data_ptr():
-            labels = labels.clone()  # kept for the backward: the caller may reuse its tensor of ids meanwhile
+        labels = shard_labels(target, vocab_start_index, vocab_end_index, local_vocab, own=not inference_only)
+        labels = labels.reshape(-1).contiguous()
         # The kernel needs 2-D operands with matching dtypes: hidden follows the weight (model_utils.py:328-333).
         hidden_2d = ops.hidden_for_weight(hidden.reshape(B * S, H), weight).contiguous()
         weight_c = weight.contiguous()

@@ -72,7 +72,7 @@ def _fused_lm_head_logprob_apply(
                                            inference_only)
     _require_single_shard(tp_group, "_fused_lm_head_logprob_apply")
     B, S, H = hidden.shape
-    labels = shard_labels(target, vocab_start_index, vocab_end_index, int(weight.shape[0]))
+    labels = shard_labels(target, vocab_start_index, vocab_end_index, int(weight.shape[0]), own=not inference_only)
     hidden_c = ops.hidden_for_weight(hidden, weight)
     # log-probabilities only: no entropy is accumulated in the forward, none differentiated in the backward
     if inference_only:

@@ -38,7 +38,7 @@ from typing import Any, Dict, Optional, Tuple
 import torch
 
 from . import _lib
-from ._launch import call, device_guard, raw_stream, registered_op
+from ._launch import call, device_guard, plain_eager, raw_stream, registered_op
 from .ops import _require_device
 
 __all__ = ["ppo_policy_loss", "cross_entropy_loss", "importance_sampling_loss", "sapo_policy_loss", "gspo_policy_loss",
@@ -134,7 +134,9 @@ def _(log_probs, old_log_probs, advantages, loss_mask, loss_weight, eps_clip_low
 
 def _own_scalar(t: torch.Tensor) -> torch.Tensor:
     """The first element of ``t`` as a 0-dim tensor of its own over that storage, not a view as autograd counts them: nothing else
-    reads that element, so the caller may scale the loss in place, and no copy is launched."""
+    reads that element, so the caller may scale the loss in place, and no copy is launched.  A copy where something traces the call."""
+    if not plain_eager():
+        return t[0].clone()
     return torch.empty(0, dtype=t.dtype, device=t.device).set_(t.untyped_storage(), t.storage_offset(), (), ())
 
 

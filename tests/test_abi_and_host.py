@@ -505,3 +505,34 @@ def test_bench_refuses_more_than_one_gpu():
     proc = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True, text=True, timeout=300)
     assert proc.returncode != 0
     assert "ONE GPU" in (proc.stdout + proc.stderr)
+
+
+def test_training_calls_are_captured_as_one_graph():
+    """The compiler sees a training call as registered ops without a break: nothing on the host looks at addresses or storages."""
+    from types import SimpleNamespace
+
+    from skyrl_amd.policy_loss import actor_loss
+
+    B, S, H, V = 2, 16, 64, 256
+    hidden = torch.zeros(B, S, H, dtype=torch.bfloat16, requires_grad=True)
+    weight = torch.zeros(V, H, dtype=torch.bfloat16, requires_grad=True)
+    ids, per_token = torch.zeros(B, S, dtype=torch.int64), torch.ones(B, S - 1)
+    algorithm = SimpleNamespace(policy_loss_type="regular", eps_clip_low=0.2, eps_clip_high=0.28, clip_ratio_c=3.0,
+                                use_kl_loss=False, use_entropy_loss=False, off_policy_correction=None)
+    calls = {
+        "lmhead_fwd": (lambda h, w, t: FusedLinearLogprobHip.apply(h, w, t, 0, V, 1024, None, False), (hidden, weight, ids)),
+        "actor_loss": (lambda lp, old, adv, mask: actor_loss(lp, old, adv, algorithm, mask)[0],
+                       (per_token.clone().requires_grad_(True), per_token, per_token, per_token)),
+    }
+    for op, (call, args) in calls.items():
+        graphs = []
+
+        def backend(graph, _inputs):
+            graphs.append(str(graph.graph))
+            raise RuntimeError("captured")
+
+        torch._dynamo.reset()
+        with pytest.raises(Exception, match="captured"):
+            torch.compile(call, backend=backend, fullgraph=True)(*args)
+        assert len(graphs) == 1, op
+    torch._dynamo.reset()
