@@ -176,3 +176,25 @@ def test_logits_rows_at_any_offset(dtype, V, pitch, cuda_device):
         untouched = torch.ones(buf.numel(), dtype=torch.bool)
         untouched[offset:].as_strided((T, V), (pitch, 1)).fill_(False)
         assert torch.equal(buf.cpu()[untouched], rest.cpu()[untouched])
+
+
+# Logits that overflow to -inf have no probability.  A whole half tile of them (128 vocabulary rows) has a maximum of -inf and
+# sums that are NaN: it takes no part in the merge, wherever it lies among the parts.  Bounds: fp32 sums, as elsewhere.
+@pytest.mark.parametrize("first_row", [0, 128, 256 * 31])
+@pytest.mark.parametrize("want_entropy", [False, True])
+def test_half_tile_of_minus_infinity(first_row, want_entropy, cuda_device):
+    T, H, V = 70, 128, 256 * 34
+    hidden, weight, _, _, _ = _operands(T, H, V, seed=first_row)
+    hidden = hidden.abs()
+    weight[first_row:first_row + 128] = -3.0e38
+    kept = torch.cat([torch.arange(first_row), torch.arange(first_row + 128, V)])
+    labels = kept[torch.randint(0, kept.numel(), (T,), generator=torch.Generator().manual_seed(1))]
+    lp, ent, lse, _ = ops.lmhead_fwd(hidden.to(cuda_device), weight.to(cuda_device), labels.to(cuda_device), 1.0, want_entropy)
+    z = hidden.double() @ weight[kept].double().t()
+    want_lse = torch.logsumexp(z, dim=1)
+    label_z = (hidden.double() * weight[labels].double()).sum(dim=1)
+    assert torch.allclose(lse.cpu().double(), want_lse, rtol=0, atol=1e-4)
+    assert torch.allclose(lp.cpu().double(), label_z - want_lse, rtol=0, atol=1e-4)
+    if want_entropy:
+        p = torch.softmax(z, dim=1)
+        assert torch.allclose(ent.cpu().double(), want_lse - (p * z).sum(dim=1), rtol=1e-4, atol=1e-4)
