@@ -28,6 +28,7 @@
 
 #include "../../include/skyrl_lmhead.h"
 #include "../../include/skyrl_lmhead_bench.h"
+#include "few_tokens.hpp"
 #include "gemm_core.hpp"
 #include "topk_kernels.hpp"
 
@@ -1346,7 +1347,7 @@ __global__ __launch_bounds__(256) void zero_f32(float* __restrict__ p, int n) {
 // HIP events on the launch stream.  Closed profiles cost one thread-local load per launch.
 enum KernelKind {
   kFwdTiles = 0, kFwdMerge, kTranspose, kBwdChunkDz, kBwdChunkGemm, kSoftCePack, kSoftCeFwdTiles, kSoftCeFinish, kSoftCeDz,
-  kCompactRows, kSplitOperand, kTopkFilter, kTopkSelect, kTopkRows, kTopkBwdRows, kDhReduce,
+  kCompactRows, kSplitOperand, kTopkFilter, kTopkSelect, kTopkRows, kTopkBwdRows, kDhReduce, kBwdDwFew,
   kNumKernelKinds
 };
 const char* const kKernelNames[kNumKernelKinds] = {"lmhead_fwd_tiles", "lmhead_fwd_merge", "transpose_bf16",
@@ -1354,7 +1355,7 @@ const char* const kKernelNames[kNumKernelKinds] = {"lmhead_fwd_tiles", "lmhead_f
                                                    "softce_fwd_tiles", "softce_finish", "softce_dz_tiles",
                                                    "active_rows[compact+gather]", "split_operand_rows",
                                                    "topk_filter_tiles", "topk_select", "topk_softce_rows",
-                                                   "topk_softce_bwd_rows", "lmhead_dh_reduce"};
+                                                   "topk_softce_bwd_rows", "lmhead_dh_reduce", "lmhead_bwd_dw_few"};
 struct Profile {
   struct Rec {
     int kind;
@@ -1728,6 +1729,16 @@ hipError_t launch_bwd_gemm(hipStream_t s, const GemmArgs& p0, const GemmArgs& p1
   return hipGetLastError();
 }
 
+// Whether dW of a call has a launch of its own, lmhead_bwd_dw_few, rather than 256 x 256 tiles next to the dHidden tiles.  Both sides of
+// the line, all launches behind the dz tiles, tiles in one launch -> own launch: T=137 248 -> 177 us at H=896, 375 -> 276 at H=1536
+// (V=151936), 860 -> 604 at H=4096, V=128261; T=400 554 -> 451 and 1315 -> 1080; T=768, H=3584, V=152064 1760 -> 1630; T=1024 947 -> 883
+// and 2017 -> 2037; T=1400, H=4096 2776 -> 3074.  Below three rounds of two tiles per CU the second launch costs what it gains: 1000
+// tiles (V=32000, H=1024) 75 -> 85 us at T=256, 2000 tiles (V=32000, H=2048) 114 -> 108.
+constexpr int64_t kDwFewTokens = 768, kDwFewTiles = 1536;
+inline bool few_token_dw(bool want_dw, bool adds, int64_t T, int64_t H, int64_t V) {
+  return want_dw && !adds && T <= kDwFewTokens && dw_few_tiles(H, V) >= kDwFewTiles;
+}
+
 // The sum over the slabs of a split dHidden contraction; g is the GEMM of the last chunk.
 hipError_t launch_dh_reduce(hipStream_t s, const GemmArgs& g, int64_t slots) {
   if (!g.splits_dev && g.splits < 2) return hipSuccess;
@@ -1866,7 +1877,8 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
   const int64_t Tpad = round_up(Tb, 256), Vpad = round_up(V, 256);
   const bool w_in_place = reads_weight_in_place(V);
   hipError_t e;
-  if (want_dw) {  // only the dW product reads hidden^T [H, Tpad]; zero in the padding columns
+  const bool few = few_token_dw(want_dw, dw_in != nullptr, Tb, H, V);
+  if (want_dw && !few) {  // only the dW product reads hidden^T [H, Tpad]; zero in the padding columns
     Timed timed(kTranspose, s);
     hipLaunchKernelGGL(transpose_bf16, dim3((unsigned)(Tpad / 64), (unsigned)(H / 64)), dim3(256), 0, s, Hp, (int)ld_hidden,
                        (int)Tb, (int)H, w.Ht, (int)(Tpad + kLdPad), (int)Tpad, T_dev);
@@ -1882,7 +1894,7 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
   const VocabTail tail = vocab_tail(V);
   // The splits are those of a full chunk: the slabs are carried from chunk to chunk.
   const int splits =
-      !T_dev && w_in_place ? best_splits(split_problem(Tb, H, vc < Vpad ? vc : Vpad, want_dw, w.slots, compute_units()), Tb) : 1;
+      !T_dev && w_in_place ? best_splits(split_problem(Tb, H, vc < Vpad ? vc : Vpad, want_dw && !few, w.slots, compute_units()), Tb) : 1;
   const int64_t nchunks = (Vpad + vc - 1) / vc;
   auto chunk_width = [&](int64_t ci) { return (Vpad - ci * vc) < vc ? (Vpad - ci * vc) : vc; };  // multiple of 256
   const GemmArgs none{};
@@ -1906,13 +1918,20 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
     gh.splits = splits, gh.splits_dev = w_in_place ? splits_dev : nullptr, gh.row_map = row_map;
     // A frozen LM head needs no dW: the launch then carries the dHidden tiles alone.
     const bool moved = last && tail.back > 0;  // the chunk ends with a moved group
-    GemmArgs gw = want_dw ? make_gemm(w.Ht, Tpad + kLdPad, H, w.D, vcw + kLdPad, vcw, true, false, Tpad / BK, H,
-                                            moved ? round_up(rows, 2 * BK) : rows,
-                                            dw_in ? dw_in + dw_off : (const float*)nullptr,
-                                            dw_f32 ? dw_f32 + dw_off : (float*)nullptr,
-                                            dw_bf16 ? dw_bf16 + dw_off : (uint16_t*)nullptr, H, T_dev, kTokensOnK)
-                                : none;
-    if (moved && want_dw) gw.n_tail = (int)(tail.from - vc0), gw.n_back = tail.back;
+    const int64_t n_rows = moved ? round_up(rows, 2 * BK) : rows;
+    const float* const cin = dw_in ? dw_in + dw_off : nullptr;
+    float* const cf = dw_f32 ? dw_f32 + dw_off : nullptr;
+    uint16_t* const cb = dw_bf16 ? dw_bf16 + dw_off : nullptr;
+    GemmArgs gw = want_dw && !few ? make_gemm(w.Ht, Tpad + kLdPad, H, w.D, vcw + kLdPad, vcw, true, false, Tpad / BK, H, n_rows, cin,
+                                              cf, cb, H, T_dev, kTokensOnK)
+                                  : none;
+    if (moved) gw.n_tail = (int)(tail.from - vc0), gw.n_back = tail.back;
+    if (few) {
+      Timed timed(kBwdDwFew, s);
+      e = launch_bwd_dw_few(s, DwFewArgs{Hp, (int)ld_hidden, w.D, (int)(vcw + kLdPad), (int)Tb, T_dev, (int)H, (int)n_rows,
+                                         moved ? gw.n_tail : 0x7fffffff, gw.n_back, cf, cb});
+      if (e != hipSuccess) return (int)e;
+    }
     e = launch_bwd_gemm(s, gh, gw, w.slots);
     if (e == hipSuccess && last) e = launch_dh_reduce(s, gh, w.slots);
     if (e != hipSuccess) return (int)e;
@@ -1958,10 +1977,12 @@ int bwd_entry(const void* hidden, int64_t ld_hidden, const void* weight, int64_t
   const int64_t nblocks = bwd_num_blocks(T);
   hipError_t e;
 
+  // dW in the launch of the dHidden tiles (bwd_token_block decides the same way)
+  const bool dw_in_gemm = d_weight && !few_token_dw(true, dw_mode == SKYRL_DW_FP32_ACCUMULATE || nblocks > 1, Tb, H, V);
   if (compact) {
     Timed timed(kCompactRows, s);
     hipLaunchKernelGGL(compact_active_rows, dim3(1), dim3(kCompactThreads), 0, s, dlogprobs, dentropy, (int)T, (int)Tb,
-                       (int)nblocks, split_problem(Tb, H, vc, d_weight != nullptr, w.slots, compute_units()), w.idx, w.counts);
+                       (int)nblocks, split_problem(Tb, H, vc, dw_in_gemm, w.slots, compute_units()), w.idx, w.counts);
     hipLaunchKernelGGL(gather_active_rows, dim3((unsigned)T), dim3(256), 0, s, (const int*)w.idx, (const int*)w.counts, Hp,
                        (int)ld_hidden, (int)Hk, (int)H, labels, row_lse, row_pz, dlogprobs, dentropy, w.hidden_c, w.labels_c,
                        w.lse_c, w.pz_c, w.g_c, w.q_c, (uint16_t*)d_hidden);

@@ -198,3 +198,30 @@ def test_half_tile_of_minus_infinity(first_row, want_entropy, cuda_device):
     if want_entropy:
         p = torch.softmax(z, dim=1)
         assert torch.allclose(ent.cpu().double(), want_lse - (p * z).sum(dim=1), rtol=1e-4, atol=1e-4)
+
+
+# dW of few tokens has a kernel of its own (256 x 128 tiles, steps of 32 tokens): one token, a step that is full, one short and one
+# over, the last size of the rule and the first behind it; a hidden size that overhangs a tile, a last vocabulary group moved back,
+# several chunks.  The accumulating call keeps the 256 x 256 tiles: the same dz panel, so both differ by fp32 sums of T products in
+# another order, sqrt(T) 2^-24 = 2e-6.
+@pytest.mark.parametrize("T,vc", [(1, 0), (31, 0), (32, 4096), (33, 0), (257, 4096), (768, 0), (769, 0)])
+def test_weight_gradient_of_few_tokens(T, vc, cuda_device):
+    H, V = 4160, 12100
+    hidden, weight, labels, g, q = _operands(T, H, V, seed=T)
+    labels[0] = V - 1
+    if T > 2:
+        g[1::3], q[1::3] = 0.0, 0.0
+    h, w, y, gd, qd = (x.to(cuda_device) for x in (hidden, weight, labels, g, q))
+    _, _, lse, pz = ops.lmhead_fwd(h, w, y, 1.0, True)
+    want = torch.zeros(V, H, device=cuda_device)
+    dh = ops.lmhead_bwd_accumulate(h, w, y, lse, pz, gd, qd, 1.0, want, vc)
+    for active in (False, True):
+        dh32, dw32 = ops.lmhead_bwd(h, w, y, lse, pz, gd, qd, 1.0, vc, active)
+        dh16, dw16 = ops.lmhead_bwd_bf16(h, w, y, lse, pz, gd, qd, 1.0, vc, active)
+        assert float((dw32 - want).norm() / want.norm()) < 1e-5
+        assert torch.equal(dw16, dw32.to(torch.bfloat16)) and torch.equal(dh16, dh32)
+        _close(dh16, dh.cpu(), f"dHidden T={T}")
+    if T <= 33:
+        _close(dw16, O.exact_fwd_bwd(hidden, weight, labels, 1.0, g, q)["d_weight"], f"dW T={T}")
+    zero = torch.zeros_like(gd)
+    assert not any(t.any() for t in ops.lmhead_bwd_bf16(h, w, y, lse, pz, zero, zero, 1.0, vc, True))
