@@ -4,11 +4,10 @@
 #include "few_tokens.hpp"
 
 #include "gemm_core.hpp"
+#include "half_tile.hpp"
 
 namespace lmhead {
 namespace {
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // ------------------------------------------------------------------------------------------------------------
 // Weight gradient of a chunk for few tokens: dW[v, h] = sum_t D[t, v] . hidden[t, h], a contraction of a few 32-token steps that
@@ -164,11 +163,56 @@ __global__ __launch_bounds__(kDwThreads, 4) void lmhead_bwd_dw_few(const DwFewAr
   }
 }
 
+// ------------------------------------------------------------------------------------------------------------
+// Logits of few tokens on half tiles (half_tile.hpp): the forward's statistics and the backward's dz values.  Same bits as on
+// the square tiles.
+// ------------------------------------------------------------------------------------------------------------
+template <bool ENTROPY>
+__global__ __launch_bounds__(NTHREADS, 2) void lmhead_fwd_half_tiles(const uint16_t* __restrict__ W, int ldw,
+                                                                     const uint16_t* __restrict__ Hd, int ldh, int T, int H, int V,
+                                                                     float rcp_temp, float* __restrict__ part_max,
+                                                                     float* __restrict__ part_sum, float* __restrict__ part_pz) {
+  __shared__ __attribute__((aligned(1024))) char lds[kHalfLdsBytes];
+  const int tiles_m = (V + BM - 1) / BM, tiles_n = (T + kHalfBN - 1) / kHalfBN;
+  int tm, tn;
+  tile_coords(blockIdx.x, tiles_m, tiles_n, kGroupM, tm, tn);
+  half_acc_t acc;
+  half_tile_product(Operand{W, ldw, tm * BM, V}, Operand{Hd, ldh, tn * kHalfBN, T}, H / kHalfBK, lds, acc);
+  fwd_epilogue<ENTROPY, false>(acc, tm, tn, tiles_m, T, V, rcp_temp, part_max, part_sum, part_pz);
+}
+
+constexpr int kHalfDzLdsBytes = NWAVES * kHalfWN * (kDzTokRow + kDzTokBytes);  // 74 KiB: the epilogue's staging, before it the ring
+static_assert(kHalfDzLdsBytes >= kHalfLdsBytes && 2 * kHalfDzLdsBytes <= LDS_BYTES, "two workgroups per CU");
+template <bool ENTGRAD>
+__global__ __launch_bounds__(NTHREADS, 2) void lmhead_bwd_half_dz(const DzArgs z) {
+  __shared__ __attribute__((aligned(1024))) char lds[kHalfDzLdsBytes];
+  dz_tile<ENTGRAD, kHalfTN>(
+      z, blockIdx.x, lds,
+      [&](const Operand& a, const Operand& b, int, int, half_acc_t& acc) {
+        half_tile_product(a, b, z.H / kHalfBK, lds, acc);
+        return true;
+      },
+      [](u32x4 v, u32x4* p) { __builtin_nontemporal_store(v, p); });
+}
+
 }  // namespace
 
 hipError_t launch_bwd_dw_few(hipStream_t s, const DwFewArgs& a) {
   hipLaunchKernelGGL(a.Cf ? lmhead_bwd_dw_few<true> : lmhead_bwd_dw_few<false>, dim3((unsigned)dw_few_tiles(a.H, a.N)),
                      dim3(kDwThreads), 0, s, a);
+  return hipGetLastError();
+}
+
+void launch_fwd_half_tiles(hipStream_t s, bool entropy, const uint16_t* W, int ldw, const uint16_t* Hd, int ldh, int T, int H, int V,
+                           float rcp_temp, float* part_max, float* part_sum, float* part_pz) {
+  const int tiles = (V + BM - 1) / BM * ((T + kHalfBN - 1) / kHalfBN);
+  hipLaunchKernelGGL(entropy ? lmhead_fwd_half_tiles<true> : lmhead_fwd_half_tiles<false>, dim3((unsigned)tiles), dim3(NTHREADS), 0, s, W,
+                     ldw, Hd, ldh, T, H, V, rcp_temp, part_max, part_sum, part_pz);
+}
+
+hipError_t launch_bwd_half_dz(hipStream_t s, bool entgrad, const DzArgs& z) {
+  hipLaunchKernelGGL(entgrad ? lmhead_bwd_half_dz<true> : lmhead_bwd_half_dz<false>, dim3((unsigned)(z.tiles_m * z.tiles_n)),
+                     dim3(NTHREADS), 0, s, z);
   return hipGetLastError();
 }
 

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "logits_tile.hpp"
+
 namespace lmhead {
 
 constexpr int kDwH = 128, kDwV = 256;  // tile of the weight gradient: hidden columns, vocabulary rows
@@ -25,5 +27,17 @@ struct DwFewArgs {
 inline int64_t dw_few_tiles(int64_t H, int64_t N) { return (N + kDwV - 1) / kDwV * ((H + kDwH - 1) / kDwH); }
 
 hipError_t launch_bwd_dw_few(hipStream_t s, const DwFewArgs& a);
+
+// Whether the logits of a call, forward or backward, are made on half tiles (half_tile.hpp): where one of them holds all tokens.
+// Forward / whole backward with dW, square -> half tiles, V=151936: H=512 57 -> 39 / 183 -> 157 us at T=16, 58 -> 42 / 207 -> 186 at
+// T=128; H=896 84 -> 62 / 285 -> 258, 86 -> 67 / 327 -> 308; H=1536 144 -> 121 / 425 -> 407, 150 -> 133 / 488 -> 479; H=4096, V=128261
+// 259 -> 219, 270 -> 238; H=1024, V=32000 29 -> 25 at both.  Two half tiles along the tokens instead of one square tile:
+// 88 -> 98 us at T=137, H=896, 145 -> 177 at H=1536, 269 -> 374 at H=4096; 58 -> 57 at H=512.
+constexpr int64_t kHalfTileTokens = 128;
+inline bool half_tile_logits(int64_t T) { return T <= kHalfTileTokens; }
+
+void launch_fwd_half_tiles(hipStream_t s, bool entropy, const uint16_t* W, int ldw, const uint16_t* Hd, int ldh, int T, int H, int V,
+                           float rcp_temp, float* part_max, float* part_sum, float* part_pz);
+hipError_t launch_bwd_half_dz(hipStream_t s, bool entgrad, const DzArgs& z);
 
 }  // namespace lmhead

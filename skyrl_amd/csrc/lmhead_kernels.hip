@@ -5,6 +5,7 @@
 //                      scale by 1/temperature, per-token max / sum-exp / sum (z-max)*exp over the tile's vocab rows;
 //                      writes one (max, sum, pz) partial per token per 128-row half tile, in blocks of 64 tokens.  Logits
 //                      never leave VGPRs.
+//                      (Up to 128 tokens, here and for the dz tiles: half tiles, few_tokens.hip.)
 //   lmhead_fwd_merge   per 16 tokens: merges the partials (online log-sum-exp), gathers the label logit with an
 //                      fp32 dot product hidden[t] . weight[label], writes logprob / entropy / lse / pz.
 // Backward (6*T*V*H flop), looped over vocab chunks of `vocab_chunk` columns:
@@ -30,20 +31,13 @@
 #include "../../include/skyrl_lmhead_bench.h"
 #include "few_tokens.hpp"
 #include "gemm_core.hpp"
+#include "logits_tile.hpp"
 #include "topk_kernels.hpp"
 
 using namespace lmhead;
 
 namespace {
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kLn2 = 0.6931471805599453f;
-#ifndef LMHEAD_GROUP_M
-#define LMHEAD_GROUP_M 4  // measured best of 2, 4, 6, 8, 16, 32 on both passes
-#endif
-constexpr int kGroupM = LMHEAD_GROUP_M;
 // Timing-only ablations for skyrl_amd/bench_ablations.py (results are wrong with any of them; 0 in the product build):
 //   1  forward tiles skip their statistics epilogue        2  dz tiles skip their epilogue (arithmetic, staging, stores)
 //   4  dz tiles do everything but the global stores        8  forward and dz tiles read the operand panels of one 4 x 8 patch
@@ -66,70 +60,12 @@ inline bool even_ktiles(int64_t contraction) { return (contraction / BK) % 2 == 
 constexpr size_t kStaticScratchBytes = SKYRL_LMHEAD_STATIC_SCRATCH_BYTES;
 static __device__ __align__(256) unsigned char static_scratch[kStaticScratchBytes];
 
-// Partial statistics live in blocks of 64 tokens: [token block][part][64 tokens].  A wave of the tile kernel writes 64
-// contiguous bytes (16 tokens) of one part; the merge kernel reads a token block's parts as one contiguous stream, 256 bytes
-// per wave instruction.  The arrays hold nparts * round_up(T, 64) floats.
-constexpr int kPartTokens = 64;
-__host__ __device__ inline size_t part_index(int part, int t, int nparts) {
-  return ((size_t)(t / kPartTokens) * (size_t)nparts + (size_t)part) * kPartTokens + (size_t)(t % kPartTokens);
-}
-__host__ __device__ inline size_t part_elems(size_t nparts, int64_t T) {
-  return nparts * (size_t)((T + kPartTokens - 1) / kPartTokens * kPartTokens);
-}
-
 // ------------------------------------------------------------------------------------------------------------
 // Forward tile kernel.  M axis = vocab (A = weight), N axis = tokens (B = hidden).
 // Online softmax statistics follow efficient_entropy_kernel_general_mainloop
 // (fused_linear_logprob_triton.py:296-385): scale, running max, sum exp, sum z*exp (kept relative to the maximum here); vocab rows past V take no part.
 // The label-logit gather of that kernel (:364-385) is done in lmhead_fwd_merge instead.
 // ------------------------------------------------------------------------------------------------------------
-// PAIRED (the soft cross-entropy, below): token blocks j >= TN / 2 hold teacher rows, and their third statistic weighs the
-// *student's* logit -- the same lane's accumulator TN / 2 blocks earlier -- with the teacher's exp: sum z_student e^(z_teacher - m).
-template <bool ENTROPY, bool MASKED, bool PAIRED>
-__device__ __forceinline__ void fwd_tile_stats(const acc_t& acc, int j, int vbase, int V, float scale2, int kq, float& m_out,
-                                               float& s_out, float& e_out) {
-  const int jy = (PAIRED && j >= TN / 2) ? j - TN / 2 : j;  // j is a constant of the caller's unrolled loop
-  // Two read-only passes over the accumulators (they live in AGPRs; writing scaled values back would cost a move each
-  // way).  scale2 > 0, so the maximum commutes with the scaling.  The third statistic of an ordinary row is taken relative
-  // to the tile's maximum, sum (z - m) e^(z - m): the exponent is at hand, and the entropy ln s - e / s then comes out of two
-  // small numbers when the row is nearly deterministic, where lse - sum p z would cancel two large ones.  (The paired
-  // statistic of the soft cross-entropy stays sum z_student e^(z_teacher - m): it is an expectation of another row's logit.)
-  float mx = -INFINITY;
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float x = acc[i][j][r];
-      if (MASKED) {
-        const int v = vbase + i * MT + kq * 4 + r;
-        if (v >= V) x = -INFINITY;
-      }
-      mx = fmaxf(mx, x);
-    }
-  mx = col_max(mx);  // finite: the wave has at least one row below V
-  const float m2 = mx * scale2;
-  float s = 0.f, e = 0.f;
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float x = acc[i][j][r];
-      const float t2 = fmaf(x, scale2, -m2);
-      float p = __builtin_amdgcn_exp2f(t2);
-      if (MASKED) {
-        const int v = vbase + i * MT + kq * 4 + r;
-        if (v >= V) p = 0.f;
-      }
-      s += p;
-      if (ENTROPY) e = fmaf(PAIRED ? acc[i][jy][r] : t2, p, e);
-    }
-  s = col_sum(s);
-  if (ENTROPY) e = col_sum(e);
-  m_out = m2 * kLn2;
-  s_out = s;
-  e_out = PAIRED ? e * scale2 * kLn2 : e * kLn2;
-}
-
 // EVEN: H / 64 is even, which selects the accumulator-stationary mainloop (gemm_core.hpp).
 template <bool ENTROPY, bool PAIRED, bool EVEN>
 __device__ __forceinline__ void fwd_tile(const uint16_t* __restrict__ W, int ldw, const uint16_t* __restrict__ Hd, int ldh, int T,
@@ -155,33 +91,7 @@ __device__ __forceinline__ void fwd_tile(const uint16_t* __restrict__ W, int ldw
   return;
 #endif
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-  const int lrow = lane & 15, kq = lane >> 4;
-  const int vbase = tm * BM + wm * WM;
-  const int part = tm * WAVES_M + wm, nparts = tiles_m * WAVES_M;
-  const float scale2 = rcp_temp * kLog2e;
-  // Whether the wave's 128 vocab rows all exist (0), partly (1: the last vocab tile) or not at all (2) is the same for the
-  // whole wave: decided once, outside the unrolled loop over the token blocks.
-  const int rows_kind = __builtin_amdgcn_readfirstlane(vbase + WM <= V ? 0 : (vbase < V ? 1 : 2));
-  auto token_blocks = [&](auto kind) {
-    constexpr int KIND = decltype(kind)::value;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int t = tn * BN + wn * WN + j * MT + lrow;
-      float m = -INFINITY, s = 0.f, e = 0.f;
-      if (KIND < 2) fwd_tile_stats<ENTROPY, KIND == 1, PAIRED>(acc, j, vbase, V, scale2, kq, m, s, e);
-      if (kq == 0 && t < T) {
-        const size_t idx = part_index(part, t, nparts);
-        part_max[idx] = m;
-        part_sum[idx] = s;
-        if (ENTROPY) part_pz[idx] = e;
-      }
-    }
-  };
-  if (rows_kind == 0) token_blocks(std::integral_constant<int, 0>{});
-  else if (rows_kind == 1) token_blocks(std::integral_constant<int, 1>{});
-  else token_blocks(std::integral_constant<int, 2>{});
+  fwd_epilogue<ENTROPY, PAIRED>(acc, tm, tn, tiles_m, T, V, rcp_temp, part_max, part_sum, part_pz);
 }
 
 template <bool ENTROPY, bool EVEN>
@@ -334,250 +244,33 @@ __global__ __launch_bounds__(kMergeThreads) void lmhead_fwd_merge(const float* _
   if (row_pz) row_pz[t] = RELATIVE ? lse - third : third;
 }
 
-// ------------------------------------------------------------------------------------------------------------
-// Backward dz producer.  Same tile as the forward; the epilogue is purely element-wise because the row
-// statistics come from the forward pass.  Formula of efficient_entropy_backward_kernel_general_d_logits_split_N
-// (fused_linear_logprob_triton.py:1402-1538, the arithmetic is at :947-957 of the fused variant):
-//     p  = exp(z - lse);   dz = ( g*(onehot - p) - q*p*(z - pz) ) / temperature
-// written as  p * (c0 + c1*x) + onehot*g/temperature  with x the raw dot product.
-// Out-of-range labels get no one-hot term but keep -p*g (model_utils.py:405-411).
-// ------------------------------------------------------------------------------------------------------------
-struct DzArgs {
-  const uint16_t* W;
-  int ldw;
-  const uint16_t* Hd;
-  int ldh;
-  int T, H, V;
-  float rcp_temp;
-  const int64_t* labels;
-  const float* row_lse;
-  const float* row_pz;
-  const float* dlogprobs;
-  const float* dentropy;
-  int vc0, tiles_m, tiles_n;  // first vocab row of the chunk; tiles of the chunk panel along vocab and tokens
-  VocabTail tail;
-  uint16_t* D;                // [tiles_n * 256, ldd]  dz, token-major
-  int ldd;
-  // When not NULL: the number of tokens, <= T, as a value in device memory (what a compaction kernel counted).  T then
-  // only sizes the grid: token tiles at or beyond the device-side count return at once.
-  const int* T_dev;
-  // When not NULL (fp32 weights): for every token whose label lies in the vocabulary, its label's dz value before the
-  // rounding to bf16, fp32 [T].  That one value per token, g (1 - p) / temperature, is of order 1 where every other dz value
-  // of the row is of order p; the caller adds what the bf16 product dropped of it (label_residual_update) so that the label
-  // rows of dW keep fp32 accuracy.
-  float* label_resid;
-  // 0, or 126 - n: softmax probabilities below 2^-n are treated as zero (SKYRL_BWD_FLUSH_TINY_DZ).
-  float p_shift;
-};
-
-// Which vocabulary rows the 128 panel columns of a wave (columns panel0 .. panel0 + 127 in the full numbering) stand for:
-// column vl is vocabulary row v0 + vl for lo <= vl < hi and carries zeros elsewhere.
-struct WaveRows {
-  int v0, lo, hi;
-};
-__device__ __forceinline__ WaveRows wave_vocab_rows(int panel0, int V, const VocabTail& tail) {
-  const bool moved = tail.back > 0 && panel0 == tail.from;
-  const int v0 = panel0 - (moved ? tail.back : 0);
-  const int left = (tail.back > 0 && panel0 > tail.from) ? 0 : V - v0;  // no rows at all behind the moved group
-  return WaveRows{v0, moved ? tail.back : 0, left < 0 ? 0 : (left < WM ? left : WM)};
-}
-
-// The A operand of a dz tile: weight rows of panel columns panel0 .. panel0 + 255, the moved group included.
-__device__ __forceinline__ Operand dz_weight_rows(const uint16_t* W, int ldw, int panel0, int V, const VocabTail& tail) {
-  Operand a{W, ldw, panel0, V};
-  if (tail.back > 0 && panel0 == tail.from) a.row0 -= tail.back;
-  if (tail.back > 0 && panel0 + WM == tail.from) a.upper_back = tail.back;
-  return a;
-}
-
+// The dz tiles (logits_tile.hpp) on square products.
 template <bool ENTGRAD, bool EVEN>
-__device__ __forceinline__ void dz_tile(const DzArgs& z, int id, char* lds) {
-  const uint16_t* __restrict__ W = z.W;
-  const uint16_t* __restrict__ Hd = z.Hd;
-  const int ldw = z.ldw, ldh = z.ldh, H = z.H, V = z.V, vc0 = z.vc0, ldd = z.ldd;
-  const int T = z.T_dev ? __builtin_amdgcn_readfirstlane(*z.T_dev) : z.T;
-  const float rcp_temp = z.rcp_temp;
-  const int64_t* __restrict__ labels = z.labels;
-  const float* __restrict__ row_lse = z.row_lse;
-  const float* __restrict__ row_pz = z.row_pz;
-  const float* __restrict__ dlogprobs = z.dlogprobs;
-  const float* __restrict__ dentropy = z.dentropy;
-  uint16_t* __restrict__ D = z.D;
-  // With a device-side count the tiles that hold tokens are numbered 0 .. tiles_m * ceil(T / 256) - 1, so that the hardware's
-  // round-robin of workgroup ids over the XCDs spreads exactly those; the other workgroups of the (static) grid return at once.
-  const int tiles_n = z.T_dev ? (T + BN - 1) / BN : z.tiles_n;
-  if (id >= z.tiles_m * tiles_n) return;
-  int tm, tn;
-  tile_coords(id, z.tiles_m, tiles_n, kGroupM, tm, tn);
-
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-  const int lrow = lane & 15, kq = lane >> 4;
-  const int vloc_base = tm * BM + wm * WM;    // first column of this wave inside the chunk panel
-  const WaveRows rows = wave_vocab_rows(vc0 + vloc_base, V, z.tail);
-  const int vbase = rows.v0;                  // the vocabulary row of its first column
-  const int tbase = tn * BN + wn * WN;        // first token of this wave (always inside the padded panels)
-  const bool full = rows.lo == 0 && rows.hi == WM;
-  const float scale2 = rcp_temp * kLog2e;
-
-  // Per-token inputs of the epilogue.  The loads are issued here, before the mainloop, and their values are first touched
-  // behind it, so the mainloop hides their latency; they are unconditional loads from a clamped token index (a load under
-  // `t < T` becomes a branch with its own wait: one memory round trip per token block before the first copy is issued).  Lane
-  // l loads tokens l and 64 + l of the wave's 128 -- twelve registers to carry through the mainloop -- and the values reach
-  // the lanes that need them (token j * 16 + lrow for every token block j) through LDS afterwards.
-  float g_[2], q_[2], lse_[2], pz_[2];
-  int64_t y_[2];
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int t = tbase + u * 64 + lane;
-    const int tc = t < T ? t : T - 1;  // T >= 1 here: a tile without a token has returned above
-    g_[u] = dlogprobs[tc];
-    q_[u] = ENTGRAD ? dentropy[tc] : 0.f;
-    lse_[u] = row_lse[tc];
-    pz_[u] = ENTGRAD ? row_pz[tc] : 0.f;
-    y_[u] = labels[tc];
-  }
-
+__device__ __forceinline__ void dz_square_tile(const DzArgs& z, int id, char* lds) {
+  static_assert(NWAVES * WN * (kDzTokRow + kDzTokBytes) <= LDS_BYTES, "dz staging and per-token values do not fit LDS");
+  dz_tile<ENTGRAD, TN>(
+      z, id, lds,
+      [&](Operand a, Operand b, int tm, int tn, acc_t& acc) {
 #if LMHEAD_ABLATE & 8
-  Operand a{W, ldw, vc0 + (tm % 4) * BM, V};
-  Operand b{Hd, ldh, (tn % 8) * BN, T};
-#else
-  const Operand a = dz_weight_rows(W, ldw, vc0 + tm * BM, V, z.tail);
-  Operand b{Hd, ldh, tn * BN, T};
+        a.row0 = z.vc0 + (tm % 4) * BM, b.row0 = (tn % 8) * BN;
 #endif
-  acc_t acc;
-  prefetch_first_tiles(a, b, 0, H / BK, lds);  // the first copies travel while the accumulators are cleared
-  zero_acc(acc);
-  mainloop<false, EVEN>(a, b, 0, H / BK, lds, acc);
+        prefetch_first_tiles(a, b, 0, z.H / BK, lds);  // the first copies travel while the accumulators are cleared
+        zero_acc(acc);
+        mainloop<false, EVEN>(a, b, 0, z.H / BK, lds, acc);
 #if LMHEAD_ABLATE & 2
-  return;
-#endif
-
-  constexpr int kTokRow = WM * 2 + 16;  // dz staging (below): 128 token rows x (128 vocab x 2 B + pad) per wave
-  constexpr int kStage = WN * kTokRow;
-  // The wave's per-token values, through a private 3 KiB of LDS behind the four staging regions (LDS operations of one wave
-  // execute in order, so no barrier).
-  constexpr int kTokBytes = WN * 24;
-  static_assert(NWAVES * (kStage + kTokBytes) <= LDS_BYTES, "dz staging and per-token values do not fit LDS");
-  char* tokv = lds + NWAVES * kStage + wave * kTokBytes;  // float4 {g, q, lse, pz} [128], then int64 label [128]
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const f32x4 v = {g_[u], q_[u], lse_[u], pz_[u]};
-    *(f32x4*)(tokv + (u * 64 + lane) * 16) = v;
-    *(int64_t*)(tokv + WN * 16 + (u * 64 + lane) * 8) = y_[u];
-  }
-  float gs_[TN], c0_[TN], c1_[TN], lse2_[TN];
-  int yrel_[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const bool valid = tbase + j * MT + lrow < T;
-    const f32x4 v = *(const f32x4*)(tokv + (j * MT + lrow) * 16);
-    const float g = valid ? v[0] : 0.f;
-    const float q = (ENTGRAD && valid) ? v[1] : 0.f;
-    lse2_[j] = valid ? v[2] * kLog2e : INFINITY;
-    const float pz = (ENTGRAD && valid) ? v[3] : 0.f;
-    const int64_t y = valid ? *(const int64_t*)(tokv + WN * 16 + (j * MT + lrow) * 8) : (int64_t)-1;
-    const int64_t yrel64 = y - (int64_t)vbase;
-    yrel_[j] = (y >= 0 && y < (int64_t)V && yrel64 >= rows.lo && yrel64 < rows.hi) ? (int)yrel64 : -1;
-    gs_[j] = g * rcp_temp;
-    c0_[j] = -(g - q * pz) * rcp_temp;
-    c1_[j] = -q * rcp_temp * rcp_temp;
-    // Optional (DzArgs::p_shift > 0): probabilities below 2^(p_shift - 126) count as zero.  The exponent is moved down by
-    // p_shift so that v_exp_f32 -- which returns 0 where the result would be a denormal, below 2^-126 -- does the flush,
-    // and the two coefficients carry the power of two back (exact).  Not for coefficients so large that the scaled ones
-    // could overflow.
-    if (z.p_shift > 0.f && fabsf(c0_[j]) < 0x1p30f && fabsf(c1_[j]) < 0x1p20f) {
-      const float up = __builtin_amdgcn_exp2f(z.p_shift);
-      lse2_[j] += z.p_shift;
-      c0_[j] *= up;
-      c1_[j] *= up;
-    }
-  }
-
-  // The wave's 128 x 128 dz block leaves through LDS so that the panel is written with 16-byte stores: a lane holds four
-  // consecutive vocab rows of one token, an 8-byte piece of a D row.  mainloop() left LDS free and every wave uses a
-  // private region, so no barrier is needed (LDS operations of one wave execute in order).  The stores are marked
-  // non-temporal: the panel is a gigabyte that is read back only by the next launch, and letting it displace the operand
-  // panels from L2 costs the mainloops of the neighbouring tiles more than the stores themselves.
-  char* stage = lds + wave * kStage;
-  // Every staging address is one per-lane base plus a compile-time constant (an immediate of the LDS instruction), and the
-  // panel rows are walked with one running pointer: written as (j * 16 + row) * pitch the compiler keeps eight row indices
-  // alive across the whole epilogue and spills them, and a spill reload waits for vmcnt(0) -- i.e. for every panel store in flight.
-  char* const st_w = stage + lrow * kTokRow + kq * 8;                      // + (j * MT) * kTokRow + i * MT * 2
-  const char* const st_r = stage + (lane >> 4) * kTokRow + (lane & 15) * 16;  // + (j * MT + it * 4) * kTokRow
-  uint16_t* d_row = D + (size_t)(tbase + (lane >> 4)) * (size_t)ldd + vloc_base + (lane & 15) * 8;  // four rows further per store
-  const size_t d_step = (size_t)4 * (size_t)ldd;
-
-  // A token block j (16 token rows x 128 vocab, 4 KiB of the staging region) is complete after its eight i-steps; its 256
-  // 16-byte pieces (4 per lane; 16 lanes cover one token row of 256 bytes) go out in the middle of block j + 1, so that the
-  // read-back and the store issue hide behind that block's arithmetic instead of forming a tail of their own.  Blocks are
-  // flushed in order, j = 0 .. TN - 1.
-  auto flush_block = [&](int j) {
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const u32x4 v = *(const u32x4*)(st_r + (j * MT + it * 4) * kTokRow);
-#if LMHEAD_ABLATE & 4
-      asm volatile("" ::"v"(v));  // staged and read back, not stored
+        return false;
 #else
-      __builtin_nontemporal_store(v, (u32x4*)d_row);
+        return true;
 #endif
-      d_row += d_step;
-    }
-  };
-  // One token block: eight i-steps of four values per lane.  What is the same for the whole wave -- rows past the
-  // vocabulary's end (RAGGED: only the last vocab tile), a label of some token inside the wave's rows (LABEL, decided per
-  // token block by a ballot), the fp32 residual of the label's value (fp32 operands only) -- is decided once outside the
-  // unrolled loops: as tests inside them they cost three branches per i-step, a third of the epilogue's time.
-  auto token_block = [&](int j, auto ragged, auto label) {
-    constexpr bool RAGGED = decltype(ragged)::value, LABEL = decltype(label)::value;
-    const float gs = gs_[j], c0 = c0_[j], c1 = c1_[j], lse2 = lse2_[j];
-    const int yrel = yrel_[j];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      float d[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float x = acc[i][j][r];
-        const float p = __builtin_amdgcn_exp2f(fmaf(x, scale2, -lse2));
-        d[r] = ENTGRAD ? p * fmaf(c1, x, c0) : p * c0;
-      }
-      const int vl = i * MT + kq * 4;  // vocab row inside the wave block; this lane holds vl .. vl+3
-      if (LABEL) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (yrel == vl + r) d[r] += gs;
-      }
-      if (RAGGED) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (vl + r < rows.lo || vl + r >= rows.hi) d[r] = 0.f;
-      }
-      f32x4 v4 = {d[0], d[1], d[2], d[3]};
-      const bf16x4 b4 = __builtin_convertvector(v4, bf16x4);
-      *(uint2*)(st_w + (j * MT) * kTokRow + i * (MT * 2)) = *(const uint2*)&b4;
-      if (LABEL && z.label_resid) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (yrel == vl + r) z.label_resid[tbase + j * MT + lrow] = d[r];
-      }
-      if (i == TM / 2 - 1 && j > 0) flush_block(j - 1);
-    }
-  };
-  std::true_type yes;
-  std::false_type no;
-  if (__builtin_amdgcn_readfirstlane((int)full)) {
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      if (__any(yrel_[j] >= 0)) token_block(j, no, yes);  // some token of this block has its label inside the wave's rows
-      else token_block(j, no, no);
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < TN; ++j) token_block(j, yes, yes);
-  }
-  flush_block(TN - 1);
+      },
+      [](u32x4 v, u32x4* p) {
+#if LMHEAD_ABLATE & 4
+        asm volatile("" ::"v"(v), "v"(p));  // staged and read back, not stored
+#else
+        __builtin_nontemporal_store(v, p);
+#endif
+      });
 }
-
 
 // ------------------------------------------------------------------------------------------------------------
 // Soft cross-entropy from hidden states (the draft-head loss of multi-token prediction, skyrl/backends/skyrl_train/mtp/
@@ -1005,7 +698,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bid, char* lds)
 template <bool ENTGRAD, bool EVEN>
 __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_dz(const DzArgs z) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  dz_tile<ENTGRAD, EVEN>(z, blockIdx.x, lds);
+  dz_square_tile<ENTGRAD, EVEN>(z, blockIdx.x, lds);
 }
 
 __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_gemm(const GemmArgs p0, const GemmArgs p1, int tiles0) {
@@ -1541,6 +1234,7 @@ size_t fwd_partials_bytes(int64_t tokens, int64_t V) {
 // for any block size.
 constexpr int64_t kFwdTokenBlock = 32768;
 
+
 // Tokens per block: what the caller's scratch allows, at least one 256-token tile.
 int64_t fwd_block_tokens(int64_t wanted, int64_t ld_hidden) {
   (void)ld_hidden;
@@ -1556,6 +1250,7 @@ int fwd_token_blocks(const void* hidden, int64_t ld_hidden, const void* weight, 
   const uint16_t* Wp = (const uint16_t*)weight;
   for (int64_t t0 = 0; t0 < T; t0 += block_tokens) {
     const int64_t Tb = (T - t0) < block_tokens ? (T - t0) : block_tokens;
+    const bool half = half_tile_logits(Tb);
     const int tiles_n = (int)((Tb + BN - 1) / BN);
     Carver c(scratch);
     float* pmax = c.take<float>(part_elems(nparts, Tb));
@@ -1567,7 +1262,10 @@ int fwd_token_blocks(const void* hidden, int64_t ld_hidden, const void* weight, 
       Timed timed(kFwdTiles, s);
       auto kernel = want_pz ? (even_ktiles(H) ? lmhead_fwd_tiles<true, true> : lmhead_fwd_tiles<true, false>)
                             : (even_ktiles(H) ? lmhead_fwd_tiles<false, true> : lmhead_fwd_tiles<false, false>);
-      hipLaunchKernelGGL(kernel, grid, block, 0, s, Wp, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)H, (int)V,
+      if (half)
+        launch_fwd_half_tiles(s, want_pz, Wp, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)H, (int)V, rcp_temperature, pmax, psum, ppz);
+      else
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, Wp, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)H, (int)V,
                          rcp_temperature, pmax, psum, ppz);
     }
     hipError_t e = hipGetLastError();
@@ -1702,10 +1400,15 @@ GemmArgs dhidden_gemm(const uint16_t* D, int64_t ldd, int64_t d_rows, const uint
   return g;
 }
 
-hipError_t launch_bwd_dz(hipStream_t s, bool entgrad, const DzArgs& z, unsigned dz_tiles) {
+hipError_t launch_bwd_dz(hipStream_t s, bool entgrad, DzArgs z) {
   Timed timed(kBwdChunkDz, s);
+  if (half_tile_logits(z.T)) {
+    z.tiles_n = 1;
+    return launch_bwd_half_dz(s, entgrad, z);
+  }
   const bool even = even_ktiles(z.H);
-  const dim3 grid(dz_tiles), block(NTHREADS);
+  z.tiles_n = (z.T + BN - 1) / BN;
+  const dim3 grid((unsigned)(z.tiles_m * z.tiles_n)), block(NTHREADS);
   if (entgrad) {
     if (even) hipLaunchKernelGGL((lmhead_bwd_dz<true, true>), grid, block, 0, s, z);
     else hipLaunchKernelGGL((lmhead_bwd_dz<true, false>), grid, block, 0, s, z);
@@ -1890,7 +1593,6 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
     hipLaunchKernelGGL(zero_f32, dim3((unsigned)(Tpad / 256)), dim3(256), 0, s, resid, (int)Tpad);
     if ((e = hipGetLastError()) != hipSuccess) return (int)e;
   }
-  const int tiles_t = (int)(Tpad / 256);
   const VocabTail tail = vocab_tail(V);
   // The splits are those of a full chunk: the slabs are carried from chunk to chunk.
   const int splits =
@@ -1904,8 +1606,8 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
     // width, and it needs a second panel.
     const int64_t vc0 = ci * vc, vcw = chunk_width(ci);
     const DzArgs z{Wp, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)Hk, (int)V, rcp_temperature, labels, row_lse, row_pz,
-                   dlogprobs, dentropy, (int)vc0, (int)(vcw / 256), tiles_t, tail, w.D, (int)(vcw + kLdPad), T_dev, resid, p_shift};
-    e = launch_bwd_dz(s, dentropy != nullptr, z, (unsigned)(vcw / 256 * tiles_t));
+                   dlogprobs, dentropy, (int)vc0, (int)(vcw / 256), 0, tail, w.D, (int)(vcw + kLdPad), T_dev, resid, p_shift};
+    e = launch_bwd_dz(s, dentropy != nullptr, z);
     if (e != hipSuccess) return (int)e;
     // dHidden[t, h] (+)= sum_v D[t, v] . weight^T[h, vc0 + v]        (A = weight^T rows at k offset vc0, B = D rows)
     // dW[vc0 + v, h]  (+)= sum_t D[t, v] . hidden^T[h, t]             (A = hidden^T rows, B = D read K-major)
@@ -1922,7 +1624,7 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
     const float* const cin = dw_in ? dw_in + dw_off : nullptr;
     float* const cf = dw_f32 ? dw_f32 + dw_off : nullptr;
     uint16_t* const cb = dw_bf16 ? dw_bf16 + dw_off : nullptr;
-    GemmArgs gw = want_dw && !few ? make_gemm(w.Ht, Tpad + kLdPad, H, w.D, vcw + kLdPad, vcw, true, false, Tpad / BK, H, n_rows, cin,
+    GemmArgs gw = want_dw && !few ? make_gemm(w.Ht, Tpad + kLdPad, H, w.D, vcw + kLdPad, vcw, true, false, round_up(Tb, 2 * BK) / BK, H, n_rows, cin,
                                               cf, cb, H, T_dev, kTokensOnK)
                                   : none;
     if (moved) gw.n_tail = (int)(tail.from - vc0), gw.n_back = tail.back;

@@ -225,3 +225,31 @@ def test_weight_gradient_of_few_tokens(T, vc, cuda_device):
         _close(dw16, O.exact_fwd_bwd(hidden, weight, labels, 1.0, g, q)["d_weight"], f"dW T={T}")
     zero = torch.zeros_like(gd)
     assert not any(t.any() for t in ops.lmhead_bwd_bf16(h, w, y, lse, pz, zero, zero, 1.0, vc, True))
+
+
+# Logits of at most 128 tokens come from 256 x 128 tiles (two steps of 32 k at H=64, the shortest): one token, a wave's 64 and one
+# more, the last size of the rule and the first behind it; a vocabulary that ends inside a tile, its last group moved back (V >= 1024) or
+# not, chunks of one tile, a fp32 weight with its label residual.  The forward accumulates every logit in the same order as the square
+# tiles: the statistics are the bits that the same tokens get in a longer call.
+@pytest.mark.parametrize("T", [1, 63, 64, 65, 127, 128, 129])
+@pytest.mark.parametrize("H,V,vc,dtype", [(64, 1153, 256, torch.bfloat16), (192, 777, 0, torch.bfloat16), (320, 5001, 0, torch.bfloat16),
+                                          (64, 1300, 512, torch.float32)])
+def test_logits_of_few_tokens(T, H, V, vc, dtype, cuda_device):
+    t = 0.7
+    hidden, weight, labels, g, q = _operands(300, H, V, seed=T + V, dtype=dtype)
+    labels[0], labels[T - 1] = V - 1, -1  # the vocabulary's last row; no target
+    h, w, y, gd, qd = (x.to(cuda_device) for x in (hidden, weight, labels, g, q))
+    longer = ops.lmhead_fwd(h, w, y, 1.0 / t, True)
+    h, y, gd, qd = h[:T], y[:T], gd[:T].clone(), qd[:T]
+    few = ops.lmhead_fwd(h, w, y, 1.0 / t, True)
+    assert all(torch.equal(a, b[:T]) for a, b in zip(few, longer))
+    if T > 2:
+        gd[1::3], qd[1::3] = 0.0, 0.0
+    ex = O.exact_fwd_bwd(hidden[:T], weight, labels[:T], t, gd.cpu(), qd.cpu())
+    for entropy_grad in (True, False):
+        if not entropy_grad:
+            ex = O.exact_fwd_bwd(hidden[:T], weight, labels[:T], t, gd.cpu(), torch.zeros(T))
+        for active in (False, True):
+            dh, dw = ops.lmhead_bwd(h, w, y, few[2], few[3], gd, qd if entropy_grad else None, 1.0 / t, vc, active)
+            _close(dh, ex["d_hidden"], f"dHidden T={T}")
+            _close(dw, ex["d_weight"], f"dW T={T}")
