@@ -551,3 +551,19 @@ def test_sliced_logits_are_walked_where_they_lie(view, dtype, cuda_device):
     assert torch.equal(TU.chunked_entropy_from_logits(sub), TU.chunked_entropy_from_logits(sub.clone()))
     assert torch.equal(TU.logprobs_from_logits_v2(sub, labels), TU.logprobs_from_logits_v2(sub.clone(), labels))
     assert torch.equal(TU.DistributedLogprob.apply(sub, labels, 0, v, None, True), TU.DistributedLogprob.apply(sub.clone(), labels, 0, v, None, True))
+
+
+# Gradients of more than 256 MiB are stored past the cache: the rows on both sides of the line are the same bits, from aligned
+# and unaligned rows, out of place and over the logits.
+@pytest.mark.parametrize("V,dtype", [(65536, torch.bfloat16), (65537, torch.bfloat16), (33001, torch.float32)])
+def test_gradients_beyond_the_cache(V, dtype, cuda_device):
+    es = 2 if dtype == torch.bfloat16 else 4
+    fits = (256 << 20) // (V * es)
+    gen = torch.Generator(device=cuda_device).manual_seed(V)
+    z = torch.randn(fits + 1, V, generator=gen, device=cuda_device).to(dtype)
+    y = torch.randint(0, V, (fits + 1,), generator=gen, device=cuda_device)
+    g, q = (torch.randn(fits + 1, generator=gen, device=cuda_device) for _ in range(2))
+    _, _, lse, pz = TU.logits_fwd(z, y, 1.0, True)
+    cached = TU.logits_bwd(z[:fits], y[:fits], lse[:fits], pz[:fits], g[:fits], q[:fits], 1.0)
+    beyond = TU.logits_bwd(z, y, lse, pz, g, q, 1.0)
+    assert torch.equal(beyond[:fits], cached)
