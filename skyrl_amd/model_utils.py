@@ -104,6 +104,13 @@ def from_parallel_hidden_to_logprobs(
     ``S - 1 - n .. S - 2`` -- the slice the worker takes next -- instead of on all ``S`` positions."""
     if _group_size(cp_group) > 1:
         raise NotImplementedError("context parallelism is outside the one-GPU scope of the HIP fused LM-head path")
+    if action_window is None and inference_only and target.shape == hidden.shape[:2] and target.shape[0] == 1 and target.shape[1] > 1:
+        # One sequence without a gradient: its successors are the ids behind the first, in place, and the last position, whose
+        # result nobody gets, is not computed.  The roll is a launch of its own: 91.8 -> 89.3 us at 137 tokens, H=896.
+        n = hidden.shape[1] - 1
+        return _fused_lm_head_logprob_apply(
+            fused_backend, hidden[:, :n], lm_head_weight, target[:, 1:], vocab_start_index, vocab_end_index,
+            n if chunk_size is None else min(chunk_size, n), tp_group, inference_only, temperature).contiguous()
     target = target.roll(shifts=-1, dims=-1)
     if action_window is not None:
         n_act, S = int(action_window), hidden.shape[1]

@@ -12,6 +12,7 @@ import torch
 from oracle import lmhead_oracle as O
 from skyrl_amd import ops
 from skyrl_amd import torch_utils as TU
+from skyrl_amd.model_utils import from_parallel_hidden_to_logprobs
 from skyrl_amd.mtp_soft_ce import soft_ce_from_hidden, topk_logits_from_hidden
 
 pytestmark = pytest.mark.gpu
@@ -253,3 +254,17 @@ def test_logits_of_few_tokens(T, H, V, vc, dtype, cuda_device):
             dh, dw = ops.lmhead_bwd(h, w, y, few[2], few[3], gd, qd if entropy_grad else None, 1.0 / t, vc, active)
             _close(dh, ex["d_hidden"], f"dHidden T={T}")
             _close(dw, ex["d_weight"], f"dW T={T}")
+
+
+# One sequence scored without a gradient runs on its first S - 1 positions with the ids behind the first in place of a roll: the bits of
+# the differentiable call, at the shortest sequences and on both sides of the few-token rule, ids outside the vocabulary included.
+@pytest.mark.parametrize("S", [1, 2, 129, 130, 300])
+@pytest.mark.parametrize("temperature,ids", [(1.0, torch.int64), (0.7, torch.int32)])
+def test_scoring_one_sequence(S, temperature, ids, cuda_device):
+    H, V = 128, 3001
+    hidden, weight, _, _, _ = _operands(S, H, V, seed=S)
+    h, w = hidden.reshape(1, S, H).to(cuda_device), weight.to(cuda_device)
+    tokens = torch.randint(0, V + 2, (1, S), generator=torch.Generator().manual_seed(S)).to(ids).to(cuda_device)
+    scored = from_parallel_hidden_to_logprobs(h, w, tokens, 0, V, None, inference_only=True, temperature=temperature)
+    assert scored.shape == (1, S - 1)
+    assert torch.equal(scored, from_parallel_hidden_to_logprobs(h, w, tokens, 0, V, None, temperature=temperature).detach())
