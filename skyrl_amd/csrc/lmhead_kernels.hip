@@ -122,8 +122,8 @@ static_assert(kMergeWaves == kMergeTokens && kPartTokens % kMergeTokens == 0, "o
 
 // Partial triples (maximum, sum e^(z - max), third statistic) of one token become one.  RELATIVE: the third statistic is
 // sum (z - max) e^(z - max) and moves with the maximum, e' = c (e + (max - max') s); otherwise it is sum y e^(z - max) of some y that
-// does not depend on the maximum and only scales.  A part whose maximum is -inf (no vocabulary row, or logits that are all -inf)
-// must come in with zero sums: the tile's own are NaN there, from -inf - -inf.
+// does not depend on the maximum and only scales.  A part without a sum (no vocabulary row, or logits that are all -inf) must come
+// in with a maximum of -inf and zeros, so that it raises no maximum; a NaN in a sum stays.
 // One exponential per part, taken relative to the largest maximum of the batch: the parts of a batch do not wait for each
 // other.  (2^(d log2 e) through v_exp_f32: its relative error grows with |d|, the part's weight falls faster; |d| e^d < 0.4.)
 template <bool RELATIVE, int N>
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(kMergeThreads) void lmhead_fwd_merge(const float* _
         }
 #pragma unroll
         for (int u = 0; u < kBatch; ++u)
-          if (p0 + u * kStreams >= nparts || !(m[u] > -INFINITY)) m[u] = -INFINITY, sv[u] = 0.f, ev[u] = 0.f;
+          if (p0 + u * kStreams >= nparts || sv[u] == 0.f) m[u] = -INFINITY, sv[u] = 0.f, ev[u] = 0.f;
         merge_partials<RELATIVE>(M, S, E, m, sv, ev);
       }
     }

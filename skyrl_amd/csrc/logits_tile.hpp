@@ -11,6 +11,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
+constexpr float kLowestMax = -3.0e38f;
 #ifndef LMHEAD_GROUP_M
 #define LMHEAD_GROUP_M 4  // measured best of 2, 4, 6, 8, 16, 32 on both passes
 #endif
@@ -51,8 +52,9 @@ __device__ __forceinline__ void fwd_tile_stats(const f32x4 (&acc)[TM][N], int j,
       }
       mx = fmaxf(mx, x);
     }
-  mx = col_max(mx);  // finite: the wave has at least one row below V
-  const float m2 = mx * scale2;
+  // Logits that are all -inf or NaN have a maximum of -inf (fmaxf passes NaN over).  Relative to a finite floor instead, the former
+  // sum to 0, which the merge passes over, and a NaN among them to NaN, which it keeps.
+  const float m2 = fmaxf(col_max(mx) * scale2, kLowestMax);
   float s = 0.f, e = 0.f;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -70,6 +72,7 @@ __device__ __forceinline__ void fwd_tile_stats(const f32x4 (&acc)[TM][N], int j,
     }
   s = col_sum(s);
   if (ENTROPY) e = col_sum(e);
+  if (ENTROPY && s == 0.f) e = 0.f;  // the logits are all -inf: e holds 0 * -inf
   m_out = m2 * kLn2;
   s_out = s;
   e_out = PAIRED ? e * scale2 * kLn2 : e * kLn2;

@@ -201,6 +201,34 @@ def test_half_tile_of_minus_infinity(first_row, want_entropy, cuda_device):
         assert torch.allclose(ent.cpu().double(), want_lse - (p * z).sum(dim=1), rtol=1e-4, atol=1e-4)
 
 
+# A NaN among the logits of a token makes its log-probability, entropy and log-sum-exp NaN, also where all rows of a half tile are NaN
+# and their maximum says nothing: a whole half tile, the single row of a last one, one row next to others, one next to logits that are
+# -inf, every row, and a token whose hidden state is NaN.  On both kinds of tiles; tokens and calls without a NaN keep their numbers.
+@pytest.mark.parametrize("T", [70, 200])
+@pytest.mark.parametrize("V,first,count", [(256 * 34, 128, 128), (256 * 8 + 1, 256 * 8, 1), (256 * 8 + 133, 256 * 8 + 128, 5), (1000, 17, 1),
+                                           (1000, 0, 1000)])
+@pytest.mark.parametrize("want_entropy", [False, True])
+def test_not_a_number_stays(T, V, first, count, want_entropy, cuda_device):
+    H = 128
+    hidden, weight, labels, _, _ = _operands(T, H, V, seed=V + first)
+    hidden = hidden.abs()
+    hidden[3] = float("nan")
+    h, y = hidden.to(cuda_device), labels.to(cuda_device)
+
+    def forward(w):
+        lp, ent, lse, pz = ops.lmhead_fwd(h, w.to(cuda_device), y, 1.0, want_entropy)
+        return (lp, ent, lse, pz) if want_entropy else (lp, lse)
+
+    others = torch.arange(T, device=cuda_device) != 3
+    for out in forward(weight):
+        assert bool(out[~others].isnan().all()) and bool(out[others].isfinite().all())
+    weight[first:first + count] = float("nan")
+    assert all(bool(out.isnan().all()) for out in forward(weight))
+    if first >= 128:  # and with a half tile of logits that are -inf in front of it
+        weight[:128] = -3.0e38
+        assert all(bool(out.isnan().all()) for out in forward(weight))
+
+
 # dW of few tokens has a kernel of its own (256 x 128 tiles, steps of 32 tokens): one token, a step that is full, one short and one
 # over, the last size of the rule and the first behind it; a hidden size that overhangs a tile, a last vocabulary group moved back,
 # several chunks.  The accumulating call keeps the 256 x 256 tiles: the same dz panel, so both differ by fp32 sums of T products in
