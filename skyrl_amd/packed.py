@@ -155,5 +155,4 @@ def packed_scatter_logprobs(packed: torch.Tensor, cu_seqlens: torch.Tensor, rows
     ``o < seg_len[s] - 1``.  With ``attention_mask`` ``[rows, cols + 1]`` the j-th real token of row ``s`` takes packed
     token ``cu[s] + j`` (all real tokens but the last).  Differentiable with respect to ``packed``.
     """
-    args = (packed, cu_seqlens, seg_row, seg_col, seg_len, attention_mask, int(rows), int(cols))
-    return _packed_scatter(*args) if packed.requires_grad and torch.is_grad_enabled() else call(_packed_scatter, *args)
+    return call(_packed_scatter, packed, cu_seqlens, seg_row, seg_col, seg_len, attention_mask, int(rows), int(cols))
