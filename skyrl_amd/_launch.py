@@ -35,14 +35,15 @@ def plain_eager() -> bool:
 
 
 def call(op, *args):
-    """``op(*args)``: the registered function itself in a plain eager call without tensor subclasses and without a gradient to record.
-    What autograd would record goes through the op, also in a backward that is recorded itself (``create_graph=True``): the op
-    knows its formula, or that it has none and a second derivative must raise."""
+    """``op(*args)``: the registered function itself in a plain eager call on real tensors, without a gradient to record.  Tensor
+    subclasses and tensors on the meta device go through the op, and so does what autograd would record, also in a
+    backward that is recorded itself (``create_graph=True``): the op knows its formula, or that it has none and a second derivative
+    must raise."""
     if not plain_eager():
         return op(*args)
     grad = torch.is_grad_enabled()
     for a in args:
-        if isinstance(a, torch.Tensor) and (type(a) not in _PLAIN or (grad and a.requires_grad)):
+        if isinstance(a, torch.Tensor) and (type(a) not in _PLAIN or a.is_meta or (grad and a.requires_grad)):
             return op(*args)
     return op.eager(*args)
 

@@ -250,6 +250,53 @@ def test_fake_kernels_give_shapes_without_a_device():
         assert dh.shape == (12, 128) and dh.dtype == torch.bfloat16 and dw.shape == (40, 128) and dw.dtype == torch.float32
 
 
+def test_public_entry_points_give_shapes_on_the_meta_device():
+    from types import SimpleNamespace
+
+    from skyrl_amd import mtp_soft_ce as M
+    from skyrl_amd import policy_loss as PL
+    from skyrl_amd import torch_utils as TU
+    from skyrl_amd.worker_utils import compute_minibatch_rollout_logprob_diff_metrics
+
+    B, S, H, V = 2, 16, 64, 256
+    meta = torch.device("meta")
+    hidden = torch.empty(B, S, H, dtype=torch.bfloat16, device=meta, requires_grad=True)
+    weight = torch.empty(V, H, dtype=torch.bfloat16, device=meta, requires_grad=True)
+    ids = torch.empty(B, S, dtype=torch.int64, device=meta)
+    logits = torch.empty(B, S, V, device=meta, requires_grad=True)
+    per_token = torch.empty(B, S - 1, device=meta)
+    algorithm = SimpleNamespace(policy_loss_type="regular", eps_clip_low=0.2, eps_clip_high=0.28, clip_ratio_c=3.0,
+                                use_kl_loss=False, use_entropy_loss=False, off_policy_correction=None)
+
+    def grads(out, *leaves):
+        assert out.device == meta
+        got = torch.autograd.grad(out.sum(), leaves)
+        assert all(g.device == meta and g.shape == x.shape for g, x in zip(got, leaves))
+
+    grads(FusedLinearLogprobHip.apply(hidden, weight, ids, 0, V, 1024, None, False), hidden, weight)
+    cu = torch.empty(B + 1, dtype=torch.int32, device=meta)
+    mask = torch.empty(B, S, dtype=torch.bool, device=meta)
+    grads(model_utils.from_parallel_hidden_to_logprobs_packed_sequences(
+        hidden.reshape(1, B * S, H), weight, ids.reshape(1, B * S), cu, S, 0, V, None, attention_mask=mask), hidden, weight)
+    grads(M.soft_ce_from_hidden(hidden, hidden.detach(), weight.detach()), hidden)
+    grads(M.draft_soft_ce_topk_from_hidden(hidden, hidden.detach(), weight.detach(), mask.float(), 8, roll_shift=1), hidden)
+    grads(TU.logprobs_from_logits(logits, ids), logits)
+    leaf = per_token.clone().requires_grad_(True)
+    for loss in (PL.actor_loss(leaf, per_token, per_token, algorithm, per_token)[0],
+                 PL.ppo_policy_loss(leaf, per_token, per_token, algorithm, per_token, sync_metrics=False)[0],
+                 PL.approx_kl_loss(leaf, per_token, per_token), PL.masked_mean(leaf, per_token, dim=-1)):
+        grads(loss, leaf)
+    with torch.no_grad():
+        scored = model_utils.from_parallel_hidden_to_logprobs(hidden[:1], weight, ids[:1], 0, V, None, inference_only=True)
+        assert scored.shape == (1, S - 1) and scored.device == meta
+        values, columns = M.topk_logits_from_hidden(hidden, weight, 8)
+        assert values.shape == columns.shape == (B, S, 8) and values.device == meta
+        diff = compute_minibatch_rollout_logprob_diff_metrics(per_token, per_token, None, sync_metrics=False)
+        assert len(diff) == 4 and all(v.device == meta for v in diff.values())
+        dh, dw = ops.lmhead_bwd_active_rows(hidden[0], weight, ids[0], per_token.new_empty(S), None, per_token.new_empty(S), None, 1.0)
+        assert dh.shape == (S, H) and dw.shape == (V, H) and dh.device == meta
+
+
 def test_signatures_mirror_the_reference():
     # FusedLinearChunkedDistributedLogprob.forward / FusedLinearLogprobTriton.forward (model_utils.py:302-313)
     assert list(inspect.signature(FusedLinearLogprobHip.forward).parameters) == [
