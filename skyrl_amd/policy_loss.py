@@ -134,9 +134,9 @@ def _(log_probs, old_log_probs, advantages, loss_mask, loss_weight, eps_clip_low
 
 def _own_scalar(t: torch.Tensor) -> torch.Tensor:
     """The first element of ``t`` as a 0-dim tensor of its own over that storage, not a view as autograd counts them: nothing else
-    reads that element, so the caller may scale the loss in place, and no copy is launched.  A copy where something traces the call
-    and on the meta device."""
-    if not plain_eager() or t.is_meta:
+    reads that element, so the caller may scale the loss in place, and no copy is launched.  A copy where something traces the call,
+    for tensor subclasses (a fake tensor outside its mode) and on the meta device."""
+    if not plain_eager() or type(t) is not torch.Tensor or t.is_meta:
         return t[0].clone()
     return torch.empty(0, dtype=t.dtype, device=t.device).set_(t.untyped_storage(), t.storage_offset(), (), ())
 

@@ -297,6 +297,23 @@ def test_public_entry_points_give_shapes_on_the_meta_device():
         assert dh.shape == (S, H) and dw.shape == (V, H) and dh.device == meta
 
 
+def test_losses_of_fake_tensors_outside_their_mode():
+    from types import SimpleNamespace
+
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from skyrl_amd import policy_loss as PL
+
+    with FakeTensorMode():
+        x = torch.empty(2, 15)
+    algorithm = SimpleNamespace(policy_loss_type="regular", eps_clip_low=0.2, eps_clip_high=0.28, clip_ratio_c=3.0,
+                                use_kl_loss=False, use_entropy_loss=False, off_policy_correction=None)
+    leaf = x.clone().requires_grad_(True)
+    for loss in (PL.actor_loss(leaf, x, x, algorithm, x)[0], PL.ppo_policy_loss(leaf, x, x, algorithm, x, sync_metrics=False)[0]):
+        (g,) = torch.autograd.grad(loss, [leaf])
+        assert loss.shape == () and type(loss) is type(x) and g.shape == x.shape
+
+
 def test_signatures_mirror_the_reference():
     # FusedLinearChunkedDistributedLogprob.forward / FusedLinearLogprobTriton.forward (model_utils.py:302-313)
     assert list(inspect.signature(FusedLinearLogprobHip.forward).parameters) == [
