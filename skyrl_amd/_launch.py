@@ -36,14 +36,16 @@ def plain_eager() -> bool:
 
 def call(op, *args):
     """``op(*args)``: the registered function itself in a plain eager call on real tensors, without a gradient to record.  Tensor
-    subclasses and tensors on the meta device go through the op, and so does what autograd would record, also in a
-    backward that is recorded itself (``create_graph=True``): the op knows its formula, or that it has none and a second derivative
-    must raise."""
+    subclasses, tensors on the meta device and those whose memory is not their value (negative views, such as the imaginary part of a
+    conjugate, and autograd's zero tensors, which have none) go through the op, whose dispatcher layers know what to do with them.  So
+    does what autograd would record, also in a backward that is recorded itself (``create_graph=True``): the op knows its formula, or
+    that it has none and a second derivative must raise."""
     if not plain_eager():
         return op(*args)
     grad = torch.is_grad_enabled()
     for a in args:
-        if isinstance(a, torch.Tensor) and (type(a) not in _PLAIN or a.is_meta or (grad and a.requires_grad)):
+        if isinstance(a, torch.Tensor) and (type(a) not in _PLAIN or a.is_meta or (grad and a.requires_grad) or a.is_neg()
+                                            or a._is_zerotensor()):
             return op(*args)
     return op.eager(*args)
 

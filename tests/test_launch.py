@@ -2,6 +2,8 @@
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -58,3 +60,16 @@ def test_a_gradient_without_a_formula_raises():
     (g,) = torch.autograd.grad(_Doubled.apply(x).sum(), x, create_graph=True)
     with pytest.raises(RuntimeError, match="no autograd formula"):  # the second derivative is not silently zero
         (x.sum() + g.square().sum()).backward()
+
+
+@registered_op("skyrl_amd_tests::memory_of", mutates_args=())
+def memory_of(x: torch.Tensor) -> torch.Tensor:
+    """What a kernel that is given ``x.data_ptr()`` reads."""
+    if x.data_ptr() == 0:
+        raise RuntimeError("a kernel would read from address 0")
+    return torch.frombuffer((ctypes.c_float * x.numel()).from_address(x.data_ptr()), dtype=torch.float32).clone()
+
+
+def test_tensors_whose_memory_is_not_their_value():
+    assert torch.equal(call(memory_of, torch._neg_view(torch.full((3,), 2.0))), torch.full((3,), -2.0))
+    assert torch.equal(call(memory_of, torch._efficientzerotensor(3)), torch.zeros(3))
