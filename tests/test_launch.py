@@ -65,6 +65,7 @@ def test_a_gradient_without_a_formula_raises():
 @registered_op("skyrl_amd_tests::memory_of", mutates_args=())
 def memory_of(x: torch.Tensor) -> torch.Tensor:
     """What a kernel that is given ``x.data_ptr()`` reads."""
+    x = x.contiguous()  # the dispatcher expands a zero tensor from one element
     if x.data_ptr() == 0:
         raise RuntimeError("a kernel would read from address 0")
     return torch.frombuffer((ctypes.c_float * x.numel()).from_address(x.data_ptr()), dtype=torch.float32).clone()
