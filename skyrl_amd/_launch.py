@@ -17,6 +17,19 @@ _PLAIN = (torch.Tensor, torch.nn.Parameter)
 _NO_GUARD = contextlib.nullcontext()
 
 
+def _followers():
+    """torch's private counters of who follows a call, or None where this torch has them under other names."""
+    try:
+        return (torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack, torch._C._functorch.peek_interpreter_stack,
+                torch._C._is_tracing, torch._C._autograd._profiler_enabled, torch.Tensor._is_zerotensor)
+    except AttributeError:
+        return None
+
+
+_FOLLOWERS = _followers()
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def registered_op(name: str, mutates_args=()):
     """``torch.library.custom_op`` that keeps the function it registers as ``op.eager``."""
     def register(fn):
@@ -28,10 +41,11 @@ def registered_op(name: str, mutates_args=()):
 
 def plain_eager() -> bool:
     """Whether nothing follows the ops of this call: no compiler or tracer, no dispatch or function mode, no functorch transform, no
-    profiler (whose record names them)."""
-    return not (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0
-                or torch._C._len_torch_function_stack() > 0 or torch._C._functorch.peek_interpreter_stack() is not None
-                or torch._C._is_tracing() or torch._C._autograd._profiler_enabled())
+    profiler (whose record names them).  Never where that cannot be told."""
+    if torch.compiler.is_compiling() or _FOLLOWERS is None:
+        return False
+    dispatch_modes, function_modes, transform, tracing, profiling, _ = _FOLLOWERS
+    return not (dispatch_modes() > 0 or function_modes() > 0 or transform() is not None or tracing() or profiling())
 
 
 def call(op, *args):
@@ -57,4 +71,6 @@ def device_guard(dev: torch.device):
 
 def raw_stream(dev: torch.device) -> int:
     """The current stream of ``dev`` as the integer the C ABI takes."""
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if dev.index is None else dev.index)
+    if _raw_stream is None:
+        return torch.cuda.current_stream(dev).cuda_stream
+    return _raw_stream(torch.cuda.current_device() if dev.index is None else dev.index)

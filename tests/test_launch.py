@@ -7,7 +7,11 @@ import ctypes
 import pytest
 import torch
 
-from skyrl_amd._launch import call, registered_op
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from skyrl_amd import _launch
+from skyrl_amd._launch import call, raw_stream, registered_op
 
 
 @registered_op("skyrl_amd_tests::double_it", mutates_args=())
@@ -74,3 +78,50 @@ def memory_of(x: torch.Tensor) -> torch.Tensor:
 def test_tensors_whose_memory_is_not_their_value():
     assert torch.equal(call(memory_of, torch._neg_view(torch.full((3,), 2.0))), torch.full((3,), -2.0))
     assert torch.equal(call(memory_of, torch._efficientzerotensor(3)), torch.zeros(3))
+
+
+class _WatchDispatch(TorchDispatchMode):
+    seen = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.seen.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+class _WatchFunctions(TorchFunctionMode):
+    seen = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.seen.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+def test_whoever_follows_the_call_sees_the_op():
+    """Tracing, profiling, modes and functorch transforms find the registered op by its name; none of them meets the bare function."""
+    x = torch.ones(3)
+    double = lambda t: call(double_it, t)  # noqa: E731
+    assert "skyrl_amd_tests::double_it" in str(torch.jit.trace(double, x, check_trace=False).inlined_graph)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        double(x)
+    assert any("double_it" in e.key for e in prof.key_averages())
+    for mode in (_WatchDispatch, _WatchFunctions):
+        with mode():
+            double(x)
+        assert any("double_it" in name for name in mode.seen)
+    assert torch.equal(torch.func.vmap(double)(x.reshape(3, 1)), torch.full((3, 1), 2.0))  # by the op's batching fallback
+
+
+def test_a_torch_without_the_private_counters_takes_the_op(monkeypatch, route):
+    monkeypatch.setattr(_launch, "_FOLLOWERS", None)
+    assert torch.equal(call(double_it, torch.ones(3)), torch.full((3,), 2.0)) and not route
+    monkeypatch.delattr(torch._C, "_is_tracing")
+    assert _launch._followers() is None
+
+
+def test_raw_stream_without_the_private_accessor(monkeypatch):
+    class Stream:
+        cuda_stream = 77
+
+    monkeypatch.setattr(_launch, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda dev: Stream())
+    assert raw_stream(torch.device("cuda", 0)) == 77
