@@ -63,7 +63,8 @@ size_t skyrl_lmhead_fwd_workspace_bytes(int64_t T, int64_t H, int64_t V);
 /* Scratch needed by skyrl_lmhead_bwd for a given vocab chunk width (0 = library default).  The backward walks the tokens in
  * blocks of T_b = min(T, 32768) and every scratch matrix is sized by the block:
  * hidden^T bf16 [H, T_b'+64], fp32 dHidden partial sums (T_b' x H' values, kept in the kernel's accumulator order between
- * chunks), one bf16 dz panel [T_b', chunk+64] and, only when V is not a multiple of 64, weight^T bf16 [H, V'+64] (otherwise
+ * chunks; below 192 tiles of 256 x 256 values at most 96 MiB of them, because the contraction is then split), one bf16 dz panel
+ * [T_b', chunk+64] and, only when V is below 1024 and not a multiple of 128, weight^T bf16 [H, V'+64] (otherwise
  * the weight is read where it is); for T > 32768 also one fp32 [V, H] matrix in which SKYRL_DW_BF16 sums dW over the blocks
  * (T_b', V', H' = T_b, V, H rounded up to 256; the 64 extra elements keep row pitches off powers of two).
  * The default chunk keeps the panel at or below 1.5 GiB, so nothing here grows with T * V.

@@ -1343,9 +1343,7 @@ BwdWorkspace carve_bwd(void* ws, int64_t T, int64_t H, int64_t Hk, int64_t V, in
   const int64_t Tb = bwd_block_tokens(T), Tpad = round_up(Tb, 256), Vpad = round_up(V, 256);
   Carver c(ws);
   BwdWorkspace w{};
-  // The size a transposed weight would take stays part of the query for every vocabulary that is not a multiple of 128:
-  // callers may have sized their scratch by the documented formula.  It is only written below kInPlaceMinVocab.
-  w.Wt = V % (2 * BK) == 0 ? nullptr : c.take<uint16_t>((size_t)H * (Vpad + kLdPad));
+  w.Wt = reads_weight_in_place(V) ? nullptr : c.take<uint16_t>((size_t)H * (Vpad + kLdPad));
   w.Ht = c.take<uint16_t>((size_t)H * (Tpad + kLdPad));
   // dHidden partial sums in accumulator order, whole tiles.  The row-compacting entry point has more room for them: its token
   // count, and with it the number of tiles, may be far below T.
@@ -1491,7 +1489,7 @@ SoftCeBwdWorkspace carve_softce_bwd(void* ws, int64_t T, int64_t H, int64_t V, i
   Carver c(ws);
   SoftCeBwdWorkspace w;
   w.S = c.take<uint16_t>((size_t)(2 * Tp) * (size_t)H);
-  w.Wt = V % (2 * BK) == 0 ? nullptr : c.take<uint16_t>((size_t)H * (Vpad + kLdPad));  // as in carve_bwd
+  w.Wt = reads_weight_in_place(V) ? nullptr : c.take<uint16_t>((size_t)H * (Vpad + kLdPad));
   w.slots = slab_slots(T, H, vc);  // at least; a quarter more lets a batch with few active tokens split further
   w.slots += w.slots / 4;
   w.dHacc = c.take<float>((size_t)(w.slots * kSlabTileFloats));

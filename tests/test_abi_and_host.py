@@ -59,9 +59,13 @@ def test_workspace_queries():
     # hidden^T + fp32 dHidden + one dz panel; nothing of size T*V, and no copy of the weight (V is a multiple of 64)
     expect = 2 * H * T + 4 * T * H + 2 * T * 4096
     assert expect <= bwd <= expect + (8 << 20)  # + 128 B of row padding per scratch row
-    # a vocabulary that is not a multiple of the k-tile needs the transposed, zero-padded weight as well
+    # nor for one that is not a multiple of the k-tile: its last group of rows is read further back
     odd = lib.skyrl_lmhead_bwd_workspace_bytes(T, H, V - 8, 4096)
-    assert expect + 2 * H * (V - 8) <= odd <= expect + 2 * H * V + (8 << 20)
+    assert expect <= odd <= expect + (8 << 20)
+    # below 1024 rows the transposed, zero-padded weight is needed as well
+    expect = 2 * H * T + 4 * T * H + 2 * T * 1024 + 2 * H * 1000
+    assert expect <= lib.skyrl_lmhead_bwd_workspace_bytes(T, H, 1000, 4096) <= expect + (8 << 20)
+    assert lib.skyrl_softce_bwd_workspace_bytes(T, H, V - 8, 4096) == lib.skyrl_softce_bwd_workspace_bytes(T, H, V, 4096)
     assert bwd < 2 * T * V
     assert lib.skyrl_lmhead_bwd_workspace_bytes(T, H, V, 100) == 0  # not a multiple of 256
     assert lib.skyrl_lmhead_fwd_workspace_bytes(0, H, V) == 0
@@ -480,7 +484,7 @@ def test_default_vocab_chunk_respects_the_panel_cap():
         Tp, Vp, Hp = -(-Tb // 256) * 256, -(-V // 256) * 256, -(-H // 256) * 256
         total = lib.skyrl_lmhead_bwd_workspace_bytes(T, H, V, 0)
         assert total == lib.skyrl_lmhead_bwd_workspace_bytes(T, H, V, 0)
-        fixed = (0 if V % 64 == 0 else 2 * H * (Vp + 64)) + 2 * H * (Tp + 64) + 4 * Tp * Hp
+        fixed = (0 if V % 64 == 0 or V >= 1024 else 2 * H * (Vp + 64)) + 2 * H * (Tp + 64) + 4 * Tp * Hp
         if T > Tb:  # several blocks: the fp32 matrix in which a bf16 dW is summed over the blocks
             fixed += -(-4 * V * H // 256) * 256
         # the row-compacting variant adds the gathered copies: two [T, H] bf16 matrices and 28 bytes per token (+ counters)
