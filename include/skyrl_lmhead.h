@@ -385,8 +385,11 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
  *
  * skyrl_lmhead_topk_logits stands in for `teacher_logits.topk(k, dim=-1)` (:273) on logits = hidden . weight^T *
  * rcp_temperature that are never stored: values [T, k] fp32 and columns [T, k] int32, best first; among equal values the
- * lower column comes first.  1 <= k <= min(V, 1024).  The workspace (256-byte aligned, at least the queried size, 0 = bad
- * arguments) does not grow with T * V: at most 16384 tokens x 8192 candidate slots of 8 bytes.
+ * lower column comes first.  1 <= k <= min(V, 1024).  The workspace (256-byte aligned; query: 0 = bad arguments) does not grow
+ * with T * V: a candidate list of 8-byte slots per token of a block of at most 16384, 1 GiB of lists together and no more than V
+ * slots each, so that few tokens get long lists and few launches (1.07 GB at T=1800, V=151936).  Anything down to lists of 8192
+ * slots, 8 * T_b * (8192 + k) + 12 * T_b bytes plus alignment (118 MB there), is accepted as well and gives the same results in more
+ * launches.
  *
  * skyrl_softce_topk_fwd: token b * seq_len + s takes the teacher's list of token b * seq_len + (s + shift) % seq_len (the roll
  * of the [B, S, k] result, :276-279), gathers the student's logits at those columns (k dot products of student_hidden[t] with

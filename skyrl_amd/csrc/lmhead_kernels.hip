@@ -1542,16 +1542,22 @@ struct TopkWorkspace {
   size_t bytes;
 };
 
-TopkWorkspace carve_topk(void* ws, int64_t T, int64_t V, int64_t k) {
+// The columns of a list: as many as the scratch holds, at most what the 1 GiB allows and at least kTopkListColumns, which any block can
+// have.  A narrower list means more chunks and launches, and the same results.
+TopkWorkspace carve_topk(void* ws, int64_t T, int64_t V, int64_t k, size_t ws_bytes) {
   TopkWorkspace w;
   w.block_tokens = T < kTopkTokenBlock ? T : kTopkTokenBlock;
   const int64_t vpad = round_up(V, 256), room = kTopkTokenBlock * kTopkListColumns / w.block_tokens / 256 * 256;
-  w.cap = vpad < room ? vpad : room;
+  const int64_t widest = vpad < room ? vpad : room, narrowest = vpad < kTopkListColumns ? vpad : kTopkListColumns;
   Carver c(ws);
   w.cnt = c.take<unsigned>((size_t)w.block_tokens);
   w.have = c.take<unsigned>((size_t)w.block_tokens);
   w.thr = c.take<float>((size_t)w.block_tokens);
   w.best = c.take<topk::key_t>((size_t)w.block_tokens * (size_t)k);
+  const size_t column = (size_t)w.block_tokens * sizeof(topk::key_t), fixed = (size_t)round_up((int64_t)c.off, 256);
+  const size_t fits = ws_bytes > fixed ? (ws_bytes - fixed) / column : 0;
+  w.cap = fits < (size_t)widest ? (int64_t)fits / 256 * 256 : widest;
+  if (w.cap < narrowest) w.cap = narrowest;
   w.cand = c.take<topk::key_t>((size_t)w.block_tokens * (size_t)w.cap);
   w.bytes = (size_t)round_up((int64_t)c.off, 256);
   return w;
@@ -1986,7 +1992,7 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
 size_t skyrl_lmhead_topk_workspace_bytes(int64_t T, int64_t H, int64_t V, int64_t k) {
   if (T < 1 || V < 1 || H < 1 || k < 1 || k > V || k > topk::kMaxK) return 0;
   if (T > kMaxExtent || V > kMaxExtent || H > kMaxExtent) return 0;
-  return carve_topk(nullptr, T, V, k).bytes;
+  return carve_topk(nullptr, T, V, k, SIZE_MAX).bytes;
 }
 
 int skyrl_lmhead_topk_logits(const void* hidden, int64_t ld_hidden, const void* weight, int64_t ld_weight, int64_t T, int64_t H,
@@ -1996,11 +2002,11 @@ int skyrl_lmhead_topk_logits(const void* hidden, int64_t ld_hidden, const void* 
   if (st) return st;
   if (!values || !columns) return SKYRL_LMHEAD_ERR_NULL;
   if (k < 1 || k > V || k > topk::kMaxK) return SKYRL_LMHEAD_ERR_ARG;
-  if (!workspace || workspace_bytes < skyrl_lmhead_topk_workspace_bytes(T, H, V, k)) return SKYRL_LMHEAD_ERR_WORKSPACE;
+  const TopkWorkspace w = carve_topk(workspace, T, V, k, workspace_bytes);
+  if (!workspace || workspace_bytes < w.bytes) return SKYRL_LMHEAD_ERR_WORKSPACE;
   if ((uintptr_t)workspace & 255u) return SKYRL_LMHEAD_ERR_ALIGN;
 
   hipStream_t s = (hipStream_t)stream;
-  const TopkWorkspace w = carve_topk(workspace, T, V, k);
   const int64_t block_tokens = fwd_block_tokens(w.block_tokens, ld_hidden);
   const uint16_t* Wp = (const uint16_t*)weight;
   const size_t select_lds = (size_t)topk::kSelectWaves * (size_t)(k + topk::kSelectStage) * sizeof(topk::key_t);

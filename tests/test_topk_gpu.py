@@ -260,6 +260,32 @@ def test_topk_c_abi_argument_errors(cuda_device):
     torch.cuda.synchronize()
 
 
+# Scratch for shorter candidate lists than the query's: down to 8192 columns per token every size is taken and only moves the boundaries
+# of the chunks; one byte less is refused.
+@pytest.mark.parametrize("T,H,V,k", [(7, 64, 30001, 5), (300, 128, 20000, 300)])
+def test_topk_with_less_scratch(T, H, V, k, cuda_device):
+    lib = _lib.load()
+    hidden, weight = _operands(T, H, V, seed=3)
+    h, w = hidden.to(cuda_device), weight.to(cuda_device)
+    full = lib.skyrl_lmhead_topk_workspace_bytes(T, H, V, k)
+    least = sum(-(-n // 256) * 256 for n in (4 * T, 4 * T, 4 * T, 8 * T * k, 8 * T * 8192))
+    assert least < full
+    want = None
+    for size in (full, full - 1, (full + least) // 2, least, least - 1):
+        ws = torch.empty(size, dtype=torch.uint8, device=cuda_device)
+        vals = torch.empty(T, k, device=cuda_device)
+        cols = torch.empty(T, k, dtype=torch.int32, device=cuda_device)
+        st = lib.skyrl_lmhead_topk_logits(h.data_ptr(), H, w.data_ptr(), H, T, H, V, k, 1.0, vals.data_ptr(), cols.data_ptr(), ws.data_ptr(),
+                                          size, torch.cuda.current_stream().cuda_stream)
+        if size < least:
+            assert st == ERR_WORKSPACE
+            continue
+        assert st == 0
+        want = (vals, cols) if want is None else want
+        assert torch.equal(vals, want[0]) and torch.equal(cols, want[1])
+    assert torch.equal(want[0], M.topk_logits(h, w, k, 1.0)[0])
+
+
 def test_topk_ops_opcheck(cuda_device):
     hidden, weight = _operands(96, 64, 700, seed=9)
     h, w = hidden.to(cuda_device), weight.to(cuda_device)
