@@ -1169,8 +1169,9 @@ SplitProblem split_problem(int64_t T, int64_t H, int64_t vc, bool want_dw, int64
 // Slab tiles of dHidden partial sums for at most T tokens and chunks of vc columns.  A launch with 192 dHidden tiles or more keeps
 // three quarters of the CUs busy with them and is not given more; below that there is room for one tile per CU.
 constexpr int64_t kSplitBelowTiles = 192;
+int64_t dh_tiles(int64_t T, int64_t H) { return (T + BM - 1) / BM * ((H + BN - 1) / BN); }
 int64_t slab_slots(int64_t T, int64_t H, int64_t vc) {
-  const int64_t tiles = (T + BM - 1) / BM * ((H + BN - 1) / BN), most = vc / (2 * BK) / kMinSplitPairs;
+  const int64_t tiles = dh_tiles(T, H), most = vc / (2 * BK) / kMinSplitPairs;
   if (tiles >= kSplitBelowTiles || most < 2) return tiles;
   const int64_t room = 2 * tiles > 256 ? 2 * tiles : 256;
   const int64_t used = tiles * (most < kMaxSplits ? most : kMaxSplits);
@@ -1215,6 +1216,21 @@ int64_t default_vocab_chunk(int64_t T, int64_t H, int64_t V) {
     if (vc >= Vpad || !fits) break;
   }
   return best_vc;
+}
+
+// Scratch that is `missing` bytes smaller than the query's.  A width of the library's own choice makes room first, in the dz panel of `rows`
+// rows (2048 columns are the narrowest it chooses), because splits save more than wide chunks; then the slabs: `wanted` floats of them
+// become what fits, but never less than the one per dHidden tile that every call needs.
+int64_t fitting_chunk(int64_t vc, int64_t rows, int64_t V, size_t missing) {
+  const int64_t Vpad = round_up(V, 256), least = Vpad < 2048 ? Vpad : 2048;
+  const int64_t fits = (vc - (int64_t)(missing / (size_t)(2 * rows)) - 1) / 256 * 256;
+  if (fits < least) return least;
+  const int64_t chunks = (Vpad + fits - 1) / fits;
+  return round_up((Vpad + chunks - 1) / chunks, 256);
+}
+int64_t fitting_slabs(int64_t wanted, int64_t T, int64_t H, size_t missing) {
+  const int64_t least = dh_tiles(T, H) * kSlabTileFloats, fits = wanted - (int64_t)((missing + 255) / 256 * 64);
+  return fits > least ? fits : least;
 }
 
 // Forward scratch: three arrays of per-part statistics for `tokens` tokens.
@@ -1339,17 +1355,14 @@ inline int64_t bwd_num_blocks(int64_t T) { return (T + kBwdTokenBlock - 1) / kBw
 
 // vc: chunk width for a block of bwd_block_tokens(T) tokens.  compact: the buffers of the row-compacting entry point.
 // Hk: length of the logits contraction, a multiple of H when the operands are stacked bf16 terms of fp32 values.
-BwdWorkspace carve_bwd(void* ws, int64_t T, int64_t H, int64_t Hk, int64_t V, int64_t vc, bool compact) {
+BwdWorkspace lay_out_bwd(void* ws, int64_t T, int64_t H, int64_t Hk, int64_t V, int64_t vc, bool compact, int64_t slab_floats) {
   const int64_t Tb = bwd_block_tokens(T), Tpad = round_up(Tb, 256), Vpad = round_up(V, 256);
   Carver c(ws);
   BwdWorkspace w{};
   w.Wt = reads_weight_in_place(V) ? nullptr : c.take<uint16_t>((size_t)H * (Vpad + kLdPad));
   w.Ht = c.take<uint16_t>((size_t)H * (Tpad + kLdPad));
-  // dHidden partial sums in accumulator order, whole tiles.  The row-compacting entry point has more room for them: its token
-  // count, and with it the number of tiles, may be far below T.
-  const int64_t slab_floats = slab_slots(Tb, H, vc) * kSlabTileFloats + (compact ? T * H / 2 : 0);
   w.slots = slab_floats / kSlabTileFloats;
-  w.dHacc = c.take<float>((size_t)slab_floats);
+  w.dHacc = c.take<float>((size_t)slab_floats);  // dHidden partial sums in accumulator order, whole tiles
   w.D = c.take<uint16_t>((size_t)Tpad * (vc + kLdPad));
   // Several blocks and a bf16 dW: the sum over the blocks is kept in fp32 here and rounded once, by the last block.
   w.dWsum = bwd_num_blocks(T) > 1 ? c.take<float>((size_t)V * (size_t)H) : nullptr;
@@ -1366,6 +1379,15 @@ BwdWorkspace carve_bwd(void* ws, int64_t T, int64_t H, int64_t Hk, int64_t V, in
   }
   w.bytes = (size_t)round_up((int64_t)c.off, 256);
   return w;
+}
+
+// The row-compacting entry point has more room for slabs: its token count, and with it the number of tiles, may be far below T.
+// A result whose `bytes` exceed ws_bytes does not fit.
+BwdWorkspace carve_bwd(void* ws, int64_t T, int64_t H, int64_t Hk, int64_t V, int64_t vc, bool compact, size_t ws_bytes) {
+  const int64_t Tb = bwd_block_tokens(T), wanted = slab_slots(Tb, H, vc) * kSlabTileFloats + (compact ? T * H / 2 : 0);
+  const BwdWorkspace w = lay_out_bwd(ws, T, H, Hk, V, vc, compact, wanted);
+  if (w.bytes <= ws_bytes) return w;
+  return lay_out_bwd(ws, T, H, Hk, V, vc, compact, fitting_slabs(wanted, Tb, H, w.bytes - ws_bytes));
 }
 
 GemmArgs make_gemm(const uint16_t* A, int64_t lda, int64_t a_rows, const uint16_t* B, int64_t ldb, int64_t b_rows, bool b_kmajor,
@@ -1568,7 +1590,7 @@ size_t bwd_workspace_bytes(int64_t T, int64_t H, int64_t V, int64_t vocab_chunk,
   if (T > kMaxExtent || V > kMaxExtent || H > kMaxExtent / 4 || vocab_chunk > kMaxExtent) return 0;
   int64_t vc = vocab_chunk ? vocab_chunk : default_vocab_chunk(bwd_block_tokens(T), H, V);
   if (vc > round_up(V, 256)) vc = round_up(V, 256);
-  return carve_bwd(nullptr, T, H, terms * H, V, vc, compact).bytes;
+  return carve_bwd(nullptr, T, H, terms * H, V, vc, compact, SIZE_MAX).bytes;
 }
 
 // One token block of the backward: the vocab-chunk loop.  Hk is the contraction length of the logits recompute (H, or a
@@ -1674,10 +1696,12 @@ int bwd_entry(const void* hidden, int64_t ld_hidden, const void* weight, int64_t
   // Row pitches of the scratch matrices (weight^T, hidden^T, the dz panel) under the copy plan's limit; Hk <= ld_hidden is.
   if ((!reads_weight_in_place(V) && Vpad + kLdPad > kMaxRowPitch) || Tbpad + kLdPad > kMaxRowPitch || vc + kLdPad > kMaxRowPitch)
     return SKYRL_LMHEAD_ERR_SHAPE;
-  if (!workspace || workspace_bytes < bwd_workspace_bytes(T, H, V, vc, compact, terms)) return SKYRL_LMHEAD_ERR_WORKSPACE;
+  const size_t full = bwd_workspace_bytes(T, H, V, vc, compact, terms);
+  if (!vocab_chunk && workspace_bytes < full) vc = fitting_chunk(vc, Tbpad, V, full - workspace_bytes);
+  const BwdWorkspace w = carve_bwd(workspace, T, H, Hk, V, vc, compact, workspace_bytes);
+  if (!workspace || workspace_bytes < w.bytes) return SKYRL_LMHEAD_ERR_WORKSPACE;
   if ((uintptr_t)workspace & 255u) return SKYRL_LMHEAD_ERR_ALIGN;
 
-  const BwdWorkspace w = carve_bwd(workspace, T, H, Hk, V, vc, compact);
   const uint16_t* Wp = (const uint16_t*)weight;
   const uint16_t* Hp = (const uint16_t*)hidden;
   const int64_t nblocks = bwd_num_blocks(T);

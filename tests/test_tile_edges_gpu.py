@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from oracle import lmhead_oracle as O
-from skyrl_amd import ops
+from skyrl_amd import _lib, ops
 from skyrl_amd import torch_utils as TU
 from skyrl_amd.model_utils import from_parallel_hidden_to_logprobs
 from skyrl_amd.mtp_soft_ce import soft_ce_from_hidden, topk_logits_from_hidden
@@ -19,6 +19,7 @@ pytestmark = pytest.mark.gpu
 
 GRAD_REL_L2 = 5e-3
 GRAD_ROW_REL_L2 = 2e-2
+ERR_WORKSPACE = -4   # include/skyrl_lmhead.h
 
 
 def _operands(T, H, V, seed, dtype=torch.bfloat16):
@@ -296,3 +297,62 @@ def test_scoring_one_sequence(S, temperature, ids, cuda_device):
     scored = from_parallel_hidden_to_logprobs(h, w, tokens, 0, V, None, inference_only=True, temperature=temperature)
     assert scored.shape == (1, S - 1)
     assert torch.equal(scored, from_parallel_hidden_to_logprobs(h, w, tokens, 0, V, None, temperature=temperature).detach())
+
+
+def _bwd_c_abi(h, w, y, lse, pz, g, q, vc, size, active, want_dw):
+    lib = _lib.load()
+    (T, H), V = h.shape, w.shape[0]
+    ws = torch.empty(size, dtype=torch.uint8, device=h.device)
+    dh = torch.full((T, H), float("nan"), dtype=torch.bfloat16, device=h.device)
+    dw = torch.empty(V, H, device=h.device) if want_dw else None
+    fn = lib.skyrl_lmhead_bwd_active_rows if active else lib.skyrl_lmhead_bwd
+    st = fn(h.data_ptr(), H, w.data_ptr(), H, y.data_ptr(), lse.data_ptr(), pz.data_ptr(), g.data_ptr(), q.data_ptr(), T, H, V, 1.0,
+            dh.data_ptr(), dw.data_ptr() if want_dw else None, 0, vc, ws.data_ptr(), size, torch.cuda.current_stream().cuda_stream)
+    return st, dh, dw
+
+
+# Scratch without room for several slabs of dHidden sums: every size down to one slab per tile, the sum of the documented terms, is taken
+# and only splits the contraction less; one byte less is refused.
+@pytest.mark.parametrize("T,H,V,vc", [(300, 192, 5001, 2048), (137, 320, 5120, 5120), (700, 64, 3000, 2304)])
+@pytest.mark.parametrize("active", [False, True])
+@pytest.mark.parametrize("want_dw", [True, False])
+def test_backward_with_less_scratch(T, H, V, vc, active, want_dw, cuda_device):
+    hidden, weight, labels, g, q = _operands(T, H, V, seed=T)
+    g[1::4], q[1::4] = 0.0, 0.0
+    h, w, y, gd, qd = (x.to(cuda_device) for x in (hidden, weight, labels, g, q))
+    _, _, lse, pz = ops.lmhead_fwd(h, w, y, 1.0, True)
+    lib = _lib.load()
+    query = lib.skyrl_lmhead_bwd_active_rows_workspace_bytes if active else lib.skyrl_lmhead_bwd_workspace_bytes
+    full, up = query(T, H, V, vc), lambda n: -(-n // 256) * 256
+    terms = [2 * H * (up(T) + 64), 4 * up(T) * up(H), 2 * up(T) * (vc + 64)]
+    least = sum(map(up, terms + ([2 * T * H, 8 * T] + [4 * T] * 5 + [12] if active else [])))
+    assert least < full
+    ex = O.exact_fwd_bwd(hidden, weight, labels, 1.0, g, q)
+    for size in (full, full - 1, (full + least) // 2, least):
+        st, dh, dw = _bwd_c_abi(h, w, y, lse, pz, gd, qd, vc, size, active, want_dw)
+        assert st == 0, (size, least, full)
+        _close(dh, ex["d_hidden"], f"dHidden, {size} bytes")
+        if want_dw:
+            _close(dw, ex["d_weight"], f"dW, {size} bytes")
+    assert _bwd_c_abi(h, w, y, lse, pz, gd, qd, vc, least - 1, active, want_dw)[0] == ERR_WORKSPACE
+
+
+# Scratch sized once, for the longest call, serves the shorter ones: with a chunk that is given, and with the library's own.
+@pytest.mark.parametrize("T,longest,H,V,vc", [(3072, 3584, 3584, 8192, 4096), (5000, 16384, 512, 152064, 0)])
+@pytest.mark.parametrize("active", [False, True])
+def test_backward_scratch_of_a_longer_call(T, longest, H, V, vc, active, cuda_device):
+    gen = torch.Generator(device=cuda_device).manual_seed(T)
+    h = torch.randn(T, H, generator=gen, device=cuda_device).to(torch.bfloat16)
+    w = (torch.randn(V, H, generator=gen, device=cuda_device) * 3 / H**0.5).to(torch.bfloat16)
+    y = torch.randint(0, V, (T,), generator=gen, device=cuda_device)
+    g, q = (torch.randn(T, generator=gen, device=cuda_device) for _ in range(2))
+    _, _, lse, pz = ops.lmhead_fwd(h, w, y, 1.0, True)
+    lib = _lib.load()
+    query = lib.skyrl_lmhead_bwd_active_rows_workspace_bytes if active else lib.skyrl_lmhead_bwd_workspace_bytes
+    st, want, _ = _bwd_c_abi(h, w, y, lse, pz, g, q, vc, query(T, H, V, vc), active, False)
+    assert st == 0
+    st, got, _ = _bwd_c_abi(h, w, y, lse, pz, g, q, vc, query(longest, H, V, vc), active, False)
+    assert st == 0
+    # The fp32 sums are added in another order, 1e-5 of a value at most: up to 1e-5 / 2^-8 of the values round to the neighbouring bf16,
+    # 2^-8 away, 2e-4 in the 2-norm.
+    assert float((got.float() - want.float()).norm() / want.float().norm()) < 1e-3
