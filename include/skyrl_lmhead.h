@@ -69,8 +69,8 @@ size_t skyrl_lmhead_fwd_workspace_bytes(int64_t T, int64_t H, int64_t V);
  * (T_b', V', H' = T_b, V, H rounded up to 256; the 64 extra elements keep row pitches off powers of two).
  * The default chunk keeps the panel at or below 1.5 GiB, so nothing here grows with T * V.
  * Less is accepted down to the sums of one dHidden (T_b' x H' values): the contraction is then split less, and with vocab_chunk = 0 the
- * chunk is narrower, down to 2048 columns; only the order of the sums differs.  Scratch sized for the longest call so serves the
- * shorter ones.
+ * chunk is narrower, down to 2048 columns, but the query is exact where the splits take less than 1 MiB; only the order of the sums
+ * differs.  Scratch sized for the longest call so serves the shorter ones.
  * (Stands in for the `d_logits [T, 9504]` scratch of the reference's default backward,
  * fused_linear_logprob_triton.py:1689-1748.) */
 size_t skyrl_lmhead_bwd_workspace_bytes(int64_t T, int64_t H, int64_t V, int64_t vocab_chunk);

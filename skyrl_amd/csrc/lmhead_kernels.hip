@@ -1220,7 +1220,7 @@ int64_t default_vocab_chunk(int64_t T, int64_t H, int64_t V) {
 
 // Scratch that is `missing` bytes smaller than the query's.  A width of the library's own choice makes room first, in the dz panel of `rows`
 // rows (2048 columns are the narrowest it chooses), because splits save more than wide chunks; then the slabs: `wanted` floats of them
-// become what fits, but never less than the one per dHidden tile that every call needs.
+// become what fits, but no fewer than the `least`, one per dHidden tile.
 int64_t fitting_chunk(int64_t vc, int64_t rows, int64_t V, size_t missing) {
   const int64_t Vpad = round_up(V, 256), least = Vpad < 2048 ? Vpad : 2048;
   const int64_t fits = (vc - (int64_t)(missing / (size_t)(2 * rows)) - 1) / 256 * 256;
@@ -1228,8 +1228,8 @@ int64_t fitting_chunk(int64_t vc, int64_t rows, int64_t V, size_t missing) {
   const int64_t chunks = (Vpad + fits - 1) / fits;
   return round_up((Vpad + chunks - 1) / chunks, 256);
 }
-int64_t fitting_slabs(int64_t wanted, int64_t T, int64_t H, size_t missing) {
-  const int64_t least = dh_tiles(T, H) * kSlabTileFloats, fits = wanted - (int64_t)((missing + 255) / 256 * 64);
+int64_t fitting_slabs(int64_t wanted, int64_t least, size_t missing) {
+  const int64_t fits = wanted - (int64_t)((missing + 255) / 256 * 64);
   return fits > least ? fits : least;
 }
 
@@ -1382,12 +1382,14 @@ BwdWorkspace lay_out_bwd(void* ws, int64_t T, int64_t H, int64_t Hk, int64_t V, 
 }
 
 // The row-compacting entry point has more room for slabs: its token count, and with it the number of tiles, may be far below T.
-// A result whose `bytes` exceed ws_bytes does not fit.
-BwdWorkspace carve_bwd(void* ws, int64_t T, int64_t H, int64_t Hk, int64_t V, int64_t vc, bool compact, size_t ws_bytes) {
-  const int64_t Tb = bwd_block_tokens(T), wanted = slab_slots(Tb, H, vc) * kSlabTileFloats + (compact ? T * H / 2 : 0);
+// A result whose `bytes` exceed ws_bytes does not fit.  own_chunk: the library's choice of vc, which leaves a caller nothing to size by
+// but a query, for this call or a longer one; the latter's has at least 1 MiB more, and less than that of slabs stays as it is.
+BwdWorkspace carve_bwd(void* ws, int64_t T, int64_t H, int64_t Hk, int64_t V, int64_t vc, bool compact, size_t ws_bytes, bool own_chunk) {
+  const int64_t Tb = bwd_block_tokens(T), more = compact ? T * H / 2 : 0;
+  const int64_t wanted = slab_slots(Tb, H, vc) * kSlabTileFloats + more, least = dh_tiles(Tb, H) * kSlabTileFloats + more;
   const BwdWorkspace w = lay_out_bwd(ws, T, H, Hk, V, vc, compact, wanted);
-  if (w.bytes <= ws_bytes) return w;
-  return lay_out_bwd(ws, T, H, Hk, V, vc, compact, fitting_slabs(wanted, Tb, H, w.bytes - ws_bytes));
+  if (w.bytes <= ws_bytes || (own_chunk && wanted - least < 4 * kSlabTileFloats)) return w;
+  return lay_out_bwd(ws, T, H, Hk, V, vc, compact, fitting_slabs(wanted, least, w.bytes - ws_bytes));
 }
 
 GemmArgs make_gemm(const uint16_t* A, int64_t lda, int64_t a_rows, const uint16_t* B, int64_t ldb, int64_t b_rows, bool b_kmajor,
@@ -1590,7 +1592,7 @@ size_t bwd_workspace_bytes(int64_t T, int64_t H, int64_t V, int64_t vocab_chunk,
   if (T > kMaxExtent || V > kMaxExtent || H > kMaxExtent / 4 || vocab_chunk > kMaxExtent) return 0;
   int64_t vc = vocab_chunk ? vocab_chunk : default_vocab_chunk(bwd_block_tokens(T), H, V);
   if (vc > round_up(V, 256)) vc = round_up(V, 256);
-  return carve_bwd(nullptr, T, H, terms * H, V, vc, compact, SIZE_MAX).bytes;
+  return carve_bwd(nullptr, T, H, terms * H, V, vc, compact, SIZE_MAX, false).bytes;
 }
 
 // One token block of the backward: the vocab-chunk loop.  Hk is the contraction length of the logits recompute (H, or a
@@ -1698,7 +1700,7 @@ int bwd_entry(const void* hidden, int64_t ld_hidden, const void* weight, int64_t
     return SKYRL_LMHEAD_ERR_SHAPE;
   const size_t full = bwd_workspace_bytes(T, H, V, vc, compact, terms);
   if (!vocab_chunk && workspace_bytes < full) vc = fitting_chunk(vc, Tbpad, V, full - workspace_bytes);
-  const BwdWorkspace w = carve_bwd(workspace, T, H, Hk, V, vc, compact, workspace_bytes);
+  const BwdWorkspace w = carve_bwd(workspace, T, H, Hk, V, vc, compact, workspace_bytes, !vocab_chunk);
   if (!workspace || workspace_bytes < w.bytes) return SKYRL_LMHEAD_ERR_WORKSPACE;
   if ((uintptr_t)workspace & 255u) return SKYRL_LMHEAD_ERR_ALIGN;
 

@@ -311,8 +311,8 @@ def _bwd_c_abi(h, w, y, lse, pz, g, q, vc, size, active, want_dw):
     return st, dh, dw
 
 
-# Scratch without room for several slabs of dHidden sums: every size down to one slab per tile, the sum of the documented terms, is taken
-# and only splits the contraction less; one byte less is refused.
+# Scratch without room for several slabs of dHidden sums: every size down to one slab per tile, the sum of the documented terms (4 * T * H
+# + 28 * T more for the gathered rows), is taken and only splits the contraction less; one byte less is refused.
 @pytest.mark.parametrize("T,H,V,vc", [(300, 192, 5001, 2048), (137, 320, 5120, 5120), (700, 64, 3000, 2304)])
 @pytest.mark.parametrize("active", [False, True])
 @pytest.mark.parametrize("want_dw", [True, False])
@@ -324,7 +324,7 @@ def test_backward_with_less_scratch(T, H, V, vc, active, want_dw, cuda_device):
     lib = _lib.load()
     query = lib.skyrl_lmhead_bwd_active_rows_workspace_bytes if active else lib.skyrl_lmhead_bwd_workspace_bytes
     full, up = query(T, H, V, vc), lambda n: -(-n // 256) * 256
-    terms = [2 * H * (up(T) + 64), 4 * up(T) * up(H), 2 * up(T) * (vc + 64)]
+    terms = [2 * H * (up(T) + 64), 4 * up(T) * up(H) + (2 * T * H if active else 0), 2 * up(T) * (vc + 64)]
     least = sum(map(up, terms + ([2 * T * H, 8 * T] + [4 * T] * 5 + [12] if active else [])))
     assert least < full
     ex = O.exact_fwd_bwd(hidden, weight, labels, 1.0, g, q)
