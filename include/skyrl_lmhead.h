@@ -367,8 +367,9 @@ int skyrl_packed_gather_grad(const float* d_out, const int64_t* cu_seqlens, int6
  * weight[v] (soft_ce.py:146-151 followed by the output layer's input gradient).  Tokens with dloss == 0 (masked ones)
  * take no part and get a zero row (listed on the device, no host synchronisation).  The teacher and the weight get no gradient:
  * the reference detaches both (soft_ce.py:16-19, mtp/adapter.py:51-56).  Workspaces: 256-byte aligned device memory of at
- * least the queried size (0 = bad arguments); vocab_chunk as in skyrl_lmhead_bwd.  Not covered: more than one vocabulary
- * shard.
+ * least the queried size (0 = bad arguments); vocab_chunk and what a smaller backward workspace does as in skyrl_lmhead_bwd, and where it
+ * holds nothing but the stacked rows, the sums of one dHidden and a panel of more than 256 columns, the chunk is 256 columns
+ * narrower than asked for.  Not covered: more than one vocabulary shard.
  */
 size_t skyrl_softce_fwd_workspace_bytes(int64_t T, int64_t H, int64_t V);
 size_t skyrl_softce_bwd_workspace_bytes(int64_t T, int64_t H, int64_t V, int64_t vocab_chunk);

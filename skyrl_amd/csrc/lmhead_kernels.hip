@@ -1508,15 +1508,14 @@ struct SoftCeBwdWorkspace {
   size_t bytes;
 };
 
-SoftCeBwdWorkspace carve_softce_bwd(void* ws, int64_t T, int64_t H, int64_t V, int64_t vc) {
+SoftCeBwdWorkspace lay_out_softce_bwd(void* ws, int64_t T, int64_t H, int64_t V, int64_t vc, int64_t slab_floats) {
   const int64_t Tp = round_up(T, kPairTile), Vpad = round_up(V, 256);
   Carver c(ws);
   SoftCeBwdWorkspace w;
   w.S = c.take<uint16_t>((size_t)(2 * Tp) * (size_t)H);
   w.Wt = reads_weight_in_place(V) ? nullptr : c.take<uint16_t>((size_t)H * (Vpad + kLdPad));
-  w.slots = slab_slots(T, H, vc);  // at least; a quarter more lets a batch with few active tokens split further
-  w.slots += w.slots / 4;
-  w.dHacc = c.take<float>((size_t)(w.slots * kSlabTileFloats));
+  w.slots = slab_floats / kSlabTileFloats;
+  w.dHacc = c.take<float>((size_t)slab_floats);
   w.D = c.take<uint16_t>((size_t)Tp * (vc + kLdPad));
   w.lse_student = c.take<float>((size_t)T);
   w.lse_teacher = c.take<float>((size_t)T);
@@ -1525,6 +1524,14 @@ SoftCeBwdWorkspace carve_softce_bwd(void* ws, int64_t T, int64_t H, int64_t V, i
   w.counts = c.take<int>(3);
   w.bytes = (size_t)round_up((int64_t)c.off, 256);
   return w;
+}
+
+// As carve_bwd; a quarter more slabs let a batch with few active tokens split further.
+SoftCeBwdWorkspace carve_softce_bwd(void* ws, int64_t T, int64_t H, int64_t V, int64_t vc, size_t ws_bytes) {
+  const int64_t slots = slab_slots(T, H, vc), wanted = (slots + slots / 4) * kSlabTileFloats;
+  const SoftCeBwdWorkspace w = lay_out_softce_bwd(ws, T, H, V, vc, wanted);
+  if (w.bytes <= ws_bytes) return w;
+  return lay_out_softce_bwd(ws, T, H, V, vc, fitting_slabs(wanted, dh_tiles(T, H) * kSlabTileFloats, w.bytes - ws_bytes));
 }
 
 int check_softce(const void* student, int64_t lds_, const void* teacher, int64_t ldt, const void* weight, int64_t ldw, int64_t T,
@@ -1904,7 +1911,7 @@ size_t skyrl_softce_bwd_workspace_bytes(int64_t T, int64_t H, int64_t V, int64_t
   if (T > kMaxExtent || V > kMaxExtent || H > kMaxExtent || vocab_chunk > kMaxExtent) return 0;
   int64_t vc = vocab_chunk ? vocab_chunk : default_vocab_chunk(T, H, V);
   if (vc > round_up(V, 256)) vc = round_up(V, 256);
-  return carve_softce_bwd(nullptr, T, H, V, vc).bytes;
+  return carve_softce_bwd(nullptr, T, H, V, vc, SIZE_MAX).bytes;
 }
 
 int skyrl_softce_fwd(const void* student_hidden, int64_t ld_student, const void* teacher_hidden, int64_t ld_teacher,
@@ -1960,11 +1967,19 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
   int64_t vc = vocab_chunk ? vocab_chunk : default_vocab_chunk(T, H, V);
   if (vc > Vpad) vc = Vpad;
   if ((!reads_weight_in_place(V) && Vpad + kLdPad > kMaxRowPitch) || vc + kLdPad > kMaxRowPitch) return SKYRL_LMHEAD_ERR_SHAPE;
-  if (!workspace || workspace_bytes < skyrl_softce_bwd_workspace_bytes(T, H, V, vc)) return SKYRL_LMHEAD_ERR_WORKSPACE;
+  const size_t full = skyrl_softce_bwd_workspace_bytes(T, H, V, vc);
+  if (!vocab_chunk && workspace_bytes < full) vc = fitting_chunk(vc, Tp, V, full - workspace_bytes);
+  SoftCeBwdWorkspace w = carve_softce_bwd(workspace, T, H, V, vc, workspace_bytes);
+  // The inputs of the listed tokens (16 bytes each) came to the sums and the panel: where the scratch holds only those, 256 columns of
+  // the panel (512 bytes per token) make way.
+  if (workspace_bytes < w.bytes && vc > BM) {
+    vc -= BM;
+    w = carve_softce_bwd(workspace, T, H, V, vc, workspace_bytes);
+  }
+  if (!workspace || workspace_bytes < w.bytes) return SKYRL_LMHEAD_ERR_WORKSPACE;
   if ((uintptr_t)workspace & 255u) return SKYRL_LMHEAD_ERR_ALIGN;
 
   hipStream_t s = (hipStream_t)stream;
-  const SoftCeBwdWorkspace w = carve_softce_bwd(workspace, T, H, V, vc);
   const uint16_t* Wp = (const uint16_t*)weight;
   hipError_t e;
   const bool w_in_place = reads_weight_in_place(V);

@@ -13,7 +13,7 @@ from oracle import lmhead_oracle as O
 from skyrl_amd import _lib, ops
 from skyrl_amd import torch_utils as TU
 from skyrl_amd.model_utils import from_parallel_hidden_to_logprobs
-from skyrl_amd.mtp_soft_ce import soft_ce_from_hidden, topk_logits_from_hidden
+from skyrl_amd.mtp_soft_ce import soft_ce_from_hidden, softce_bwd, softce_fwd, topk_logits_from_hidden
 
 pytestmark = pytest.mark.gpu
 
@@ -356,3 +356,40 @@ def test_backward_scratch_of_a_longer_call(T, longest, H, V, vc, active, cuda_de
     # The fp32 sums are added in another order, 1e-5 of a value at most: up to 1e-5 / 2^-8 of the values round to the neighbouring bf16,
     # 2^-8 away, 2e-4 in the 2-norm.
     assert float((got.float() - want.float()).norm() / want.float().norm()) < 1e-3
+
+
+# The draft loss's backward in scratch of the documented terms (stacked rows, one dHidden's sums, the panel), which leave no room for the
+# inputs of the listed tokens, and in scratch that was sized for a longer call; below those terms it is refused.
+@pytest.mark.parametrize("T,H,V,vc", [(300, 192, 5001, 2048), (137, 320, 5120, 5120), (700, 64, 3000, 512), (300, 128, 700, 256)])
+def test_draft_loss_backward_with_less_scratch(T, H, V, vc, cuda_device):
+    student, weight, _, g, _ = _operands(T, H, V, seed=T)
+    teacher = _operands(T, H, V, seed=T + 1)[0]
+    g[1::4] = 0.0
+    hs, ht, w, gd = (x.to(cuda_device) for x in (student, teacher, weight, g))
+    _, lse_s, lse_t = softce_fwd(hs, ht, w, T, 1, 1.0)
+    lib = _lib.load()
+    up, Tp = lambda n, m=256: -(-n // m) * m, -(-T // 128) * 128
+    terms = [4 * Tp * H, 4 * up(T) * up(H), 2 * Tp * (vc + 64)]
+    least = sum(map(up, terms + ([] if V >= 1024 else [2 * H * (up(V) + 64)])))
+    if vc == 256:  # no column to spare
+        least += sum(map(up, [4 * T] * 4 + [12]))
+    full = lib.skyrl_softce_bwd_workspace_bytes(T, H, V, vc)
+    sizes = {full, max(full - 1, least), (full + least) // 2, least, lib.skyrl_softce_bwd_workspace_bytes(2 * T, H, V, vc)}
+    want = softce_bwd(hs, ht, w, lse_s, lse_t, gd, T, 1, 1.0, vc)
+    hd = student.double().requires_grad_(True)
+    ls, lt = hd @ weight.double().T, torch.roll(teacher, -1, 0).double() @ weight.double().T
+    (-(lt.softmax(-1) * ls.log_softmax(-1)).sum(-1) * g.double()).sum().backward()
+    _close(want, hd.grad, "d student")
+
+    def call(size):
+        ws = torch.empty(size, dtype=torch.uint8, device=cuda_device)
+        d = torch.full_like(hs, float("nan"))
+        st = lib.skyrl_softce_bwd(hs.data_ptr(), H, ht.data_ptr(), H, w.data_ptr(), H, lse_s.data_ptr(), lse_t.data_ptr(), gd.data_ptr(), T,
+                                  T, 1, H, V, 1.0, d.data_ptr(), vc, ws.data_ptr(), size, torch.cuda.current_stream().cuda_stream)
+        return st, d
+
+    for size in sizes:
+        st, d = call(size)
+        assert st == 0, (size, least, full)
+        _close(d, hd.grad, f"d student, {size} bytes")
+    assert call(least // 2)[0] == ERR_WORKSPACE and (vc > 256 or call(least - 1)[0] == ERR_WORKSPACE)
