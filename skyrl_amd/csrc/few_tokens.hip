@@ -18,7 +18,11 @@ namespace {
 // of 128 columns whose 32-byte windows are permuted by (row & 3) | (row bit 3) << 2, so that the eight row pieces of half a
 // transposing read fall into different banks.  Tiles along the hidden size first: neighbours share the dz columns in L2.
 // The stores are non-temporal: with ordinary ones the kernels behind this one write dW's dirty lines back while they read the weight
-// (V=151936, H=1536: dHidden 150 -> 106 us, forward 141 -> 128 at T=137, this kernel the same).
+// (V=151936, H=1536: dHidden 150 -> 106 us, forward 141 -> 128 at T=137, this kernel the same).  At every size, although results
+// below 256 MiB would be found in the last-level cache: backward, and forward + backward + the sum of dW into another tensor, ordinary ->
+// non-temporal, 98 MiB (bf16, V=32000, H=1600, T=64; the least that comes here) 102 -> 101 and 202 -> 199 us, 141 MiB (V=128256, H=576)
+// 152 -> 136 and 270 -> 258, 195 MiB (fp32) 122 -> 117 and 281 -> 275, 282 MiB 203 -> 159 and 390 -> 358, 890 MiB (V=151936, H=1536) 469 ->
+// 416 and 1089 -> 1035; T=400 and 768 likewise.  A norm of dW behind it gains too, but for 98 MiB at T=64 (187 -> 192).
 // H=1536, V=151936: 88 us at T=17 (5.3 TB/s), 162 at T=137, 250 at T=400, 419 at T=768.
 // ------------------------------------------------------------------------------------------------------------
 constexpr int kDwK = 32;                          // tokens per step
@@ -109,7 +113,7 @@ __global__ __launch_bounds__(kDwThreads, 4) void lmhead_bwd_dw_few(const DwFewAr
     const uint32_t t = s0;
     s0 = s1, s1 = s2, s2 = t;
   }
-  wait_copies_and_barrier<0>();  // no wave reads the ring any more: it becomes the staging room, a ninth of it per wave
+  wait_copies_and_barrier<0>();  // no wave reads the ring any more: it becomes the staging room, an eighth of it per wave, all of it
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // as behind the other mainloops
 #pragma unroll
   for (int i = 0; i < 4; ++i)

@@ -525,9 +525,9 @@ enum { kTokensOnM = 1, kTokensOnN = 2, kTokensOnK = 3 };
 // tile about a seventeenth of a k-tile of the whole chip).  At least 1024 vocabulary rows per split.  Integer arithmetic: the
 // host and compact_active_rows, which rates one candidate per lane for the token count it found, must agree.
 // Measured, GEMM launches of the backward, one workgroup per tile -> split: 2750 -> 560 us at T=428 (active), H=1536, V=151936
-// (12 tiles x 8 splits); 544 -> 168 us at T=1050, H=1024, V=32000, fp32 weight; 2714 -> 1509 us at T=4096, H=2048, V=151936 and
-// 2304 -> 1317 us at T=1592, H=4096, V=128261, both without dW; 3030 -> 2700 us at T=4096, H=1536, V=151936.  With 192 tiles and
-// more the dW tiles fill the CUs and the launch is not split.
+// (12 tiles x 8 splits beside the dW tiles; alone in the launch, as now, 12 x 21 in 180); 544 -> 168 us at T=1050, H=1024, V=32000,
+// fp32 weight; 2714 -> 1509 us at T=4096, H=2048, V=151936 and 2304 -> 1317 us at T=1592, H=4096, V=128261, both without dW; 3030 ->
+// 2700 us at T=4096, H=1536, V=151936.  What the slabs have room for (slab_slots) bounds the choice.
 constexpr int kMinSplitPairs = 8;
 constexpr int kMaxSplits = 64;
 struct SplitProblem {
@@ -1166,8 +1166,11 @@ SplitProblem split_problem(int64_t T, int64_t H, int64_t vc, bool want_dw, int64
   return SplitProblem{(int)tiles_h, (int)(vc / (2 * BK)), want_dw ? (int)(tiles_h * (vc / BM)) : 0, (int)slots, ncu};
 }
 
-// Slab tiles of dHidden partial sums for at most T tokens and chunks of vc columns.  A launch with 192 dHidden tiles or more keeps
-// three quarters of the CUs busy with them and is not given more; below that there is room for one tile per CU.
+// Slab tiles of dHidden partial sums for at most T tokens and chunks of vc columns: room for one tile per CU, at least two per dHidden
+// tile; none beyond one per dHidden tile from 192 tiles on, where dW tiles in the same launch fill the CUs that dHidden leaves idle.
+// The line is drawn for launches with dW.  Without (a frozen weight, the draft loss, a dW launch of its own) it is not measured, and
+// split_cost would go further: 288 tiles (T=8192, H=2304) are rated 1.6 times as long in one piece as in eight, and 96 tiles (draft loss of
+// 2868 active tokens, H=2048), which room for 320 slabs lets go in two, a quarter longer than in eight.
 constexpr int64_t kSplitBelowTiles = 192;
 int64_t dh_tiles(int64_t T, int64_t H) { return (T + BM - 1) / BM * ((H + BN - 1) / BN); }
 int64_t slab_slots(int64_t T, int64_t H, int64_t vc) {
