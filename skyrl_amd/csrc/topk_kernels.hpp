@@ -104,55 +104,54 @@ __device__ __forceinline__ void topk_tile(const FilterArgs& a, char* lds) {
     const int t = tn * BN + wn * WN + j * MT + lrow;
     if (t >= a.T) th[j] = NAN;  // rows past the last token never pass: every comparison with NaN is false
   }
-  // A lane holds 32 logits of each of its eight tokens.  First sweep: how many of them pass (a wave-wide vote on the largest
-  // of four skips the blocks in which nothing does -- nearly all of them once a threshold exists; rounding is monotone and
-  // s > 0, so the scaled maximum is the maximum of the scaled values).  Then one atomic add per lane and token reserves that
-  // many slots of the token's list -- eight independent atomics in flight, one round trip per tile -- and a second sweep
-  // stores the keys.  The accumulators are only read, so both sweeps see the same values.
-  const bool ragged = vbase + WM > a.vrows;
-  int hits[TN];
-  unsigned long long voted[TN];  // bit i: block i of token column j has a passing logit somewhere in the wave
+  // A lane holds 32 logits of each of its eight tokens.  First sweep: the largest of the 32 against the threshold (rounding is
+  // monotone and s > 0, so the scaled maximum is the maximum of the scaled values); a wave-wide vote skips the tokens of which nothing
+  // passes, and for the others every logit that passes becomes a bit of a word.  Then one atomic add per lane and token reserves
+  // as many slots of the token's list -- eight independent atomics in flight, one round trip per tile -- and a second sweep stores the
+  // keys.  A lane has about one passing logit of its 256 while thresholds are young: it finds them by their bits, and the values,
+  // which cannot be indexed in registers, through its own 128 bytes of LDS (free behind the mainloop; no other lane reads them).
+  // At T=1800, H=2048, k=32, tests and branches block of four by block of four -> bits: 59 -> 48 us for a tile of the chunk behind the
+  // first 8192 columns, 48 -> 46 for one of the chunk behind that.
+  uint32_t exists = 0xffffffffu;  // which of the lane's logits do, as the bits below: the chunk's last rows may end inside the tile
+  if (vbase + WM > a.vrows) {
+#pragma unroll
+    for (int x = 0; x < TM * 4; ++x)
+      if (vbase + (x / 4) * MT + kq * 4 + x % 4 >= a.vrows) exists &= ~(0x80000000u >> x);
+  }
+  uint32_t hit[TN];  // bit 31 - (i * 4 + r)
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    hits[j] = 0;
-    voted[j] = 0;
+    float m = acc[0][j][0];
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const float m4 = fmaxf(fmaxf(acc[i][j][0], acc[i][j][1]), fmaxf(acc[i][j][2], acc[i][j][3])) * s;
-      if (__any(m4 >= th[j])) {
-        voted[j] |= 1ull << i;
+    for (int x = 1; x < TM * 4; ++x) m = fmaxf(m, acc[x / 4][j][x % 4]);
+    hit[j] = 0;
+    if (!__any(m * s >= th[j])) continue;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int vr = vbase + i * MT + kq * 4 + r;
-          hits[j] += (acc[i][j][r] * s >= th[j] && (!ragged || vr < a.vrows)) ? 1 : 0;
-        }
-      }
+    for (int x = 0; x < TM * 4; ++x) {
+      const float z = acc[x / 4][j][x % 4] * s;
+      asm("v_cmp_ge_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(hit[j]) : "v"(z), "v"(th[j]) : "vcc");
     }
+    hit[j] &= exists;
   }
   unsigned base[TN];
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
     const int t = tn * BN + wn * WN + j * MT + lrow;
-    base[j] = hits[j] > 0 ? atomicAdd(a.cnt + t, (unsigned)hits[j]) : 0u;
+    base[j] = hit[j] ? atomicAdd(a.cnt + t, (unsigned)__popc(hit[j])) : 0u;
   }
+  char* const mine = lds + wave * (TM * 4 * 64 * 4) + lane * 16;  // [i][lane] pieces of four values
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    if (voted[j] == 0) continue;  // wave-uniform
-    const int t = tn * BN + wn * WN + j * MT + lrow;
-    key_t* list = a.cand + (size_t)t * (size_t)a.cap;
+    if (hit[j] == 0) continue;
+    key_t* list = a.cand + (size_t)(tn * BN + wn * WN + j * MT + lrow) * (size_t)a.cap;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) *(f32x4*)(mine + i * 1024) = acc[i][j];
     unsigned slot = base[j];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      if (!((voted[j] >> i) & 1)) continue;  // wave-uniform
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float z = acc[i][j][r] * s;
-        const int vr = vbase + i * MT + kq * 4 + r;
-        if (z >= th[j] && (!ragged || vr < a.vrows)) {
-          if (slot < (unsigned)a.cap) list[slot] = make_key(z, a.v0 + vr);
-          ++slot;
-        }
-      }
+    for (uint32_t left = hit[j]; left; ++slot) {
+      const int x = __clz((int)left);
+      left &= ~(0x80000000u >> x);
+      const float z = *(const float*)(mine + (x >> 2) * 1024 + (x & 3) * 4) * s;
+      if (slot < (unsigned)a.cap) list[slot] = make_key(z, a.v0 + vbase + (x >> 2) * MT + kq * 4 + (x & 3));
     }
   }
 }
