@@ -392,7 +392,7 @@ __global__ __launch_bounds__(NTHREADS) void softce_dz_tiles(const SoftCeDzArgs z
   const int tiles_n = (T + BN / 2 - 1) / (BN / 2);
   if ((int)blockIdx.x >= z.tiles_m * tiles_n) return;
   int tm, tn;
-  tile_coords(blockIdx.x, z.tiles_m, tiles_n, kGroupM, tm, tn);
+  tile_coords(z.tiles_m * tiles_n - 1 - (int)blockIdx.x, z.tiles_m, tiles_n, kGroupM, tm, tn);  // as in dz_tile
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;

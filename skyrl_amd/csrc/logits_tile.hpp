@@ -189,8 +189,10 @@ __device__ __forceinline__ void dz_tile(const DzArgs& z, int id, char* lds, Prod
   // round-robin of workgroup ids over the XCDs spreads exactly those; the other workgroups of the (static) grid return at once.
   const int tiles_n = z.T_dev ? (T + TILE_N - 1) / TILE_N : z.tiles_n;
   if (id >= z.tiles_m * tiles_n) return;
+  // The last tiles first: the forward ended with their weight rows, and the last-level cache still holds some of them.  Few tokens, whole
+  // training pass, first to last -> last to first: 778 -> 755 us at T=200, H=2048, V=151936, 469 -> 461 at T=40, H=1536; many: the same.
   int tm, tn;
-  tile_coords(id, z.tiles_m, tiles_n, kGroupM, tm, tn);
+  tile_coords(z.tiles_m * tiles_n - 1 - id, z.tiles_m, tiles_n, kGroupM, tm, tn);
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
