@@ -190,9 +190,11 @@ static_assert(kHalfDzLdsBytes >= kHalfLdsBytes && 2 * kHalfDzLdsBytes <= LDS_BYT
 template <bool ENTGRAD>
 __global__ __launch_bounds__(NTHREADS, 2) void lmhead_bwd_half_dz(const DzArgs z) {
   __shared__ __attribute__((aligned(1024))) char lds[kHalfDzLdsBytes];
+  int T, tm, tn;
+  if (!dz_tile_of(z, blockIdx.x, kHalfBN, T, tm, tn)) return;
   dz_tile<ENTGRAD, kHalfTN>(
-      z, blockIdx.x, lds,
-      [&](const Operand& a, const Operand& b, int, int, half_acc_t& acc) {
+      z, T, tm, tn * kHalfBN, lds,
+      [&](const Operand& a, const Operand& b, half_acc_t& acc) {
         half_tile_product(a, b, z.H / kHalfBK, lds, acc);
         return true;
       },

@@ -88,9 +88,11 @@ typedef f32x4 acc_t[TM][TN];
 // operand that changes alternates A, B, A, B.  With random data the matrix pipe is power-limited and the order is
 // measurable: a loop of nothing but MFMAs runs 2 % faster in this order than in a row-by-row serpentine (the A fragment
 // kept for eight MFMAs), 6 % faster than in an order that changes both operands every time; on zeros all orders tie.
-__host__ __device__ constexpr int mfma_row(int x) { return (x / 16) * 2 + ((x % 16 + 1) / 2) % 2; }
-__host__ __device__ constexpr int mfma_col(int x) { return (x / 16) % 2 ? TN - 1 - (x % 16) / 2 : (x % 16) / 2; }
-static_assert(TM == 8 && TN == 8, "mfma_row / mfma_col walk an 8 x 8 grid");
+// N: columns of the grid, 8 or (narrow tiles) 4.
+template <int N = TN>
+__host__ __device__ constexpr int mfma_row(int x) { return (x / (2 * N)) * 2 + ((x % (2 * N) + 1) / 2) % 2; }
+template <int N = TN>
+__host__ __device__ constexpr int mfma_col(int x) { return (x / (2 * N)) % 2 ? N - 1 - (x % (2 * N)) / 2 : (x % (2 * N)) / 2; }
 
 // The n-th (n = 0, 1, ...) MFMA gap of a 64-MFMA step at or behind x that is odd (the even ones carry fragment reads)
 // and is not a copy gap (x % 8 == 5).
@@ -152,11 +154,12 @@ __device__ __forceinline__ void mfma_16x16x32(f32x4& c, const bf16x8& a, const b
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
 
-__device__ __forceinline__ void zero_acc(acc_t& acc) {
+template <int N>
+__device__ __forceinline__ void zero_acc(f32x4 (&acc)[TM][N]) {
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+    for (int j = 0; j < N; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
   // The other hazard the compiler cannot see: an MFMA must not read an accumulator within a few cycles of the
@@ -166,7 +169,7 @@ __device__ __forceinline__ void zero_acc(acc_t& acc) {
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) asm volatile("" : "+a"(acc[i][j]));
+    for (int j = 0; j < N; ++j) asm volatile("" : "+a"(acc[i][j]));
 }
 
 // Per-lane plan of the global->LDS copies of one output tile: which global 16-byte chunk lands in which LDS chunk.
@@ -182,7 +185,7 @@ struct CopyPlan {
   uint32_t a_src[COPIES_PER_OPERAND], b_src[COPIES_PER_OPERAND];
 };
 
-template <bool BKM>
+template <bool BKM, int N = TN>
 __device__ __forceinline__ void make_plan(CopyPlan& p, const Operand& a, const Operand& b, int k_begin) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -194,6 +197,7 @@ __device__ __forceinline__ void make_plan(CopyPlan& p, const Operand& a, const O
     int ra = row >= BM / 2 ? row - a.upper_back : row;
     ra = a.row0 + ra < a.rows ? ra : a.rows - 1 - a.row0;  // row inside the tile; rows past the end re-read the last one
     p.a_src[j] = (uint32_t)ra * (uint32_t)a.ld * 2u + (uint32_t)(kc * 16);
+    if (j >= N) continue;  // a copy per 32 rows of the operand: a narrow tile has as many fewer
     if (BKM) {
       const int block = j * NWAVES + wave;             // rows 2 * block, 2 * block + 1 of the k-tile
       const int q = (lane >> 2) ^ kmajor_sigma(block);  // the pair whose home is this lane's window
@@ -253,17 +257,17 @@ __device__ __forceinline__ uint32_t wave_copy_base(char* lds) {
 // Put the first k-tiles of an output tile in flight: A(0) B(0) A(1) B(1) into slots 0..3.  All five slots must be free
 // (true at kernel start and after mainloop() returns).  Called before the epilogue of the previous output tile so that
 // the copy path keeps working while the VALU does the epilogue.
-template <bool BKM = false>
+template <bool BKM = false, int N = TN>
 __device__ __forceinline__ void prefetch_first_tiles(const Operand& a, const Operand& b, int k_begin, int nk, char* lds) {
   CopyPlan p;  // rebuilt by mainloop(): keeping it in registers across an epilogue costs more than recomputing it
-  make_plan<BKM>(p, a, b, k_begin);
+  make_plan<BKM, N>(p, a, b, k_begin);
   if (BKM && nk == 2) p.b_bytes -= last_pair_back_bytes<BKM>(b);
   const uint32_t w0 = wave_copy_base(lds);
   copy_part(p.a_bytes, p.a_src, w0 + 0 * OPERAND_BYTES, 0, COPIES_PER_OPERAND);
-  copy_part(p.b_bytes, p.b_src, w0 + 1 * OPERAND_BYTES, 0, COPIES_PER_OPERAND);
+  copy_part(p.b_bytes, p.b_src, w0 + 1 * OPERAND_BYTES, 0, N);
   if (nk > 1) {
     copy_part(p.a_bytes + BK * 2, p.a_src, w0 + 2 * OPERAND_BYTES, 0, COPIES_PER_OPERAND);
-    copy_part(p.b_bytes + b_tile_stride<BKM>(b), p.b_src, w0 + 3 * OPERAND_BYTES, 0, COPIES_PER_OPERAND);
+    copy_part(p.b_bytes + b_tile_stride<BKM>(b), p.b_src, w0 + 3 * OPERAND_BYTES, 0, N);
   }
 }
 
@@ -282,10 +286,16 @@ __device__ __forceinline__ void prefetch_first_tiles(const Operand& a, const Ope
 //                register sets), one copy behind every eighth MFMA, in a gap without a read; sched_barrier pins that order.
 // MFMA order inside a step: mfma_row() / mfma_col() above (every fragment of the step is in registers before the step
 // starts, so the order is free to serve the power budget).
-template <bool BKM = false>
-__device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand& b, int k_begin, int nk, char* lds, acc_t& acc) {
+//
+// N = 4: a narrow tile, B[b.row0 : +128], for the last tokens of a call where they are no more than that: half of the MFMAs, three quarters
+// of the copies, so what bounds it is the copies.  A step is then 32 MFMAs, with a copy of A behind every fourth or one of B behind every
+// eighth.  Forward, V=151936, all tiles square -> the last one narrow: 132 -> 114 us at T=300, H=896, 252 -> 221 at T=384, H=2048, 468 -> 432
+// at T=1100, H=1536; training pass 958 -> 925 at T=611, H=1536.  Beyond 128 tokens in the last tile a square one is made.
+template <bool BKM = false, int N = TN>
+__device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand& b, int k_begin, int nk, char* lds, f32x4 (&acc)[TM][N]) {
+  static_assert(N == TN || (N == 4 && !BKM), "the schedule below is written for these");
   CopyPlan p;
-  make_plan<BKM>(p, a, b, k_begin);
+  make_plan<BKM, N>(p, a, b, k_begin);
   const uint32_t b_stride = b_tile_stride<BKM>(b);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -298,7 +308,7 @@ __device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand&
   const uint32_t w0 = wave_copy_base(lds);
   const int rel = -(wave * 1024);
   const int a_off0 = (wm * WM + lrow) * ROW_BYTES + xsw + rel, a_off1 = (wm * WM + lrow) * ROW_BYTES + (xsw ^ 64) + rel;
-  const int b_off0 = (wn * WN + lrow) * ROW_BYTES + xsw + rel, b_off1 = (wn * WN + lrow) * ROW_BYTES + (xsw ^ 64) + rel;
+  const int b_off0 = (wn * (N * MT) + lrow) * ROW_BYTES + xsw + rel, b_off1 = (wn * (N * MT) + lrow) * ROW_BYTES + (xsw ^ 64) + rel;
   typedef const __attribute__((address_space(3))) bf16x8* frag_ptr;
   typedef __attribute__((address_space(3))) i16x4* half_ptr;
 
@@ -320,8 +330,8 @@ __device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand&
   constexpr int kHalfBytes = 2 * 1024;    // 4 k-rows
 
   // Fragment registers.  A K-major B fragment arrives as two 64-bit halves (k 0-3 and k 4-7 of the lane's eight).
-  bf16x8 af[2][TM], bfr[2][BKM ? 1 : TN];
-  i16x4 bh[2][BKM ? TN : 1][2];
+  bf16x8 af[2][TM], bfr[2][BKM ? 1 : N];
+  i16x4 bh[2][BKM ? N : 1][2];
   auto b_frag = [&](int set, int j) -> bf16x8 {
     if constexpr (BKM) {
       typedef __attribute__((ext_vector_type(8))) short i16x8;
@@ -333,7 +343,7 @@ __device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand&
   };
   // Read instruction y of a 32-k step: y < TM is the A fragment of MFMA row y; then the B fragments, one instruction each
   // (K-contiguous B) or two (K-major B).  pa: LDS address of A fragment 0; pb: NB LDS addresses for B.
-  constexpr int READS_PER_STEP = TM + (BKM ? 2 * TN : TN);
+  constexpr int READS_PER_STEP = TM + (BKM ? 2 * N : N);
   auto read_one = [&](uint32_t pa, const uint32_t (&pb)[NB], int set, int y) {
     if (y < TM) {
       af[set][y] = *(frag_ptr)(uintptr_t)(pa + y * MT * ROW_BYTES);
@@ -354,7 +364,7 @@ __device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand&
     boff1[e] = BKM ? kb_off[e] : b_off1;
   }
 
-  if (nk > 1) wait_copies_and_barrier<2 * COPIES_PER_OPERAND>(); else wait_copies_and_barrier<0>();  // tile 0 has landed
+  if (nk > 1) wait_copies_and_barrier<COPIES_PER_OPERAND + N>(); else wait_copies_and_barrier<0>();  // tile 0 has landed
   {
     uint32_t pb[NB];
 #pragma unroll
@@ -387,10 +397,12 @@ __device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand&
   auto tile_step = [&](auto has_next, auto load2) {
     // The fragment addresses of the next k-tile are formed in place, one add per MFMA shadow, in gaps behind the last
     // read of the step (which still uses the old value) that carry neither a read nor a copy.
+    constexpr int kMfmas = TM * N;
     constexpr int kAddX0 = BKM ? 2 * READS_PER_STEP - 1 : 41;
-    constexpr int kGapA = free_gap(kAddX0, 0);
-    constexpr int kGapB[4] = {free_gap(kAddX0, 1), free_gap(kAddX0, 2), free_gap(kAddX0, 3), free_gap(kAddX0, 4)};
-    static_assert(kGapB[3] < TM * TN, "address adds must fit the step");
+    constexpr int kGapA = N == TN ? free_gap(kAddX0, 0) : 24;
+    constexpr int kGapB[4] = {N == TN ? free_gap(kAddX0, 1) : 26, free_gap(kAddX0, 2), free_gap(kAddX0, 3), free_gap(kAddX0, 4)};
+    static_assert(2 * READS_PER_STEP <= (N == TN ? kMfmas : kGapA) && kGapB[NB - 1] < kMfmas, "reads and address adds must fit the step");
+    constexpr int kAPeriod = kMfmas / COPIES_PER_OPERAND, kAGap = N == TN ? 5 : 1;  // MFMAs between the copies of A, and where
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
       if (ks == 1 && has_next) {
@@ -398,19 +410,18 @@ __device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand&
         else wait_copies_and_barrier<0>();
       }
 #pragma unroll
-      for (int x = 0; x < TM * TN; ++x) {
-        const int i = mfma_row(x), j = mfma_col(x);
+      for (int x = 0; x < kMfmas; ++x) {
+        const int i = mfma_row<N>(x), j = mfma_col<N>(x);
         mfma_16x16x32(acc[i][j], af[ks][i], b_frag(ks, j));
         __builtin_amdgcn_sched_barrier(0);
         if (x % 2 == 0 && x < 2 * READS_PER_STEP) {
           if (ks == 0) read_one(ra1, rb1, 1, x / 2);
           else if (has_next) read_one(ra0, rb0, 0, x / 2);
         }
-        if (load2 && x % 8 == 5) {  // an MFMA gap that carries no fragment read
-          if (ks == 0) copy_part(ga, p.a_src, o4, x / 8, 1);
-          else copy_part(gb, p.b_src, o0, x / 8, 1);
-        }
-        if (load2 && x == 62) {
+        // an MFMA gap that carries no fragment read
+        if (load2 && ks == 0 && x % kAPeriod == kAGap) copy_part(ga, p.a_src, o4, x / kAPeriod, 1);
+        if (load2 && ks == 1 && x % 8 == 5) copy_part(gb, p.b_src, o0, x / 8, 1);
+        if (load2 && x == kMfmas - 2) {
           if (ks == 0) {
             ga += BK * 2;
             asm volatile("" : "+s"(ga));
@@ -450,7 +461,7 @@ __device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand&
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) asm volatile("" : "+a"(acc[i][j]));
+    for (int j = 0; j < N; ++j) asm volatile("" : "+a"(acc[i][j]));
 }
 
 // ---- accumulator-stationary pairs -------------------------------------------------------------------------------------

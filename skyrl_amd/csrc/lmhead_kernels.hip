@@ -54,6 +54,18 @@ __host__ __device__ inline int64_t round_up(int64_t x, int64_t m) { return (x + 
 // An even number of k-tiles selects the accumulator-stationary mainloop (the EVEN instantiation of a tile kernel).
 inline bool even_ktiles(int64_t contraction) { return (contraction / BK) % 2 == 0; }
 
+// Whether the last token tile of a call of T tokens is a narrow one.  The branch to it is compiled into kernels of their own: it costs
+// calls of whole tiles half a percent (T=2048, H=896, V=151936: 485 -> 488 us).
+inline bool has_narrow_tile(int64_t T) { return T % BN > 0 && T % BN <= BN / 2; }
+// pick(x, y, z) for the three flags as compile-time constants.
+template <class Pick>
+auto flagged_kernel(Pick pick, bool x, bool y, bool z) {
+  const std::true_type t;
+  const std::false_type f;
+  if (x) return y ? (z ? pick(t, t, t) : pick(t, t, f)) : (z ? pick(t, f, t) : pick(t, f, f));
+  return y ? (z ? pick(f, t, t) : pick(f, t, f)) : (z ? pick(f, f, t) : pick(f, f, f));
+}
+
 // Scratch of skyrl_lmhead_fwd_static_scratch, the entry point for callers that cannot allocate: one fixed array in every
 // device's memory, held until the process ends.  In host code this name is only a handle for hipGetSymbolAddress (see
 // static_scratch_of_current_device); kernels receive the looked-up address as an ordinary argument.
@@ -67,7 +79,8 @@ static __device__ __align__(256) unsigned char static_scratch[kStaticScratchByte
 // The label-logit gather of that kernel (:364-385) is done in lmhead_fwd_merge instead.
 // ------------------------------------------------------------------------------------------------------------
 // EVEN: H / 64 is even, which selects the accumulator-stationary mainloop (gemm_core.hpp).
-template <bool ENTROPY, bool PAIRED, bool EVEN>
+// NARROW: the last token tile holds no more than 128 tokens and is made half as wide (has_narrow_tile()).
+template <bool ENTROPY, bool PAIRED, bool EVEN, bool NARROW>
 __device__ __forceinline__ void fwd_tile(const uint16_t* __restrict__ W, int ldw, const uint16_t* __restrict__ Hd, int ldh, int T,
                                          int H, int V, float rcp_temp, float* __restrict__ part_max,
                                          float* __restrict__ part_sum, float* __restrict__ part_pz, char* lds) {
@@ -83,6 +96,16 @@ __device__ __forceinline__ void fwd_tile(const uint16_t* __restrict__ W, int ldw
   Operand a{W, ldw, tm * BM, V};
   Operand b{Hd, ldh, tn * BN, T};
 #endif
+  if constexpr (NARROW) {
+    if (narrow_tile(tn, T)) {
+      f32x4 half[TM][TN / 2];
+      prefetch_first_tiles<false, TN / 2>(a, b, 0, H / BK, lds);
+      zero_acc(half);
+      mainloop_ksteps<false, TN / 2>(a, b, 0, H / BK, lds, half);
+      fwd_epilogue<ENTROPY, PAIRED>(half, tm, 2 * tn, tiles_m, T, V, rcp_temp, part_max, part_sum, part_pz);
+      return;
+    }
+  }
   acc_t acc;
   prefetch_first_tiles(a, b, 0, H / BK, lds);  // the first copies travel while the accumulators are cleared
   zero_acc(acc);
@@ -94,13 +117,13 @@ __device__ __forceinline__ void fwd_tile(const uint16_t* __restrict__ W, int ldw
   fwd_epilogue<ENTROPY, PAIRED>(acc, tm, tn, tiles_m, T, V, rcp_temp, part_max, part_sum, part_pz);
 }
 
-template <bool ENTROPY, bool EVEN>
+template <bool ENTROPY, bool EVEN, bool NARROW>
 __global__ __launch_bounds__(NTHREADS) void lmhead_fwd_tiles(const uint16_t* __restrict__ W, int ldw,
                                                              const uint16_t* __restrict__ Hd, int ldh, int T, int H, int V,
                                                              float rcp_temp, float* __restrict__ part_max,
                                                              float* __restrict__ part_sum, float* __restrict__ part_pz) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  fwd_tile<ENTROPY, false, EVEN>(W, ldw, Hd, ldh, T, H, V, rcp_temp, part_max, part_sum, part_pz, lds);
+  fwd_tile<ENTROPY, false, EVEN, NARROW>(W, ldw, Hd, ldh, T, H, V, rcp_temp, part_max, part_sum, part_pz, lds);
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -244,13 +267,34 @@ __global__ __launch_bounds__(kMergeThreads) void lmhead_fwd_merge(const float* _
   if (row_pz) row_pz[t] = RELATIVE ? lse - third : third;
 }
 
-// The dz tiles (logits_tile.hpp) on square products.
-template <bool ENTGRAD, bool EVEN>
+// The dz tiles (logits_tile.hpp) on square products, the last tokens' on narrow ones.
+template <bool ENTGRAD, bool EVEN, bool NARROW>
 __device__ __forceinline__ void dz_square_tile(const DzArgs& z, int id, char* lds) {
   static_assert(NWAVES * WN * (kDzTokRow + kDzTokBytes) <= LDS_BYTES, "dz staging and per-token values do not fit LDS");
+  int T, tm, tn;
+  if (!dz_tile_of(z, id, BN, T, tm, tn)) return;
+  auto store = [](u32x4 v, u32x4* p) {
+#if LMHEAD_ABLATE & 4
+    asm volatile("" ::"v"(v), "v"(p));  // staged and read back, not stored
+#else
+    __builtin_nontemporal_store(v, p);
+#endif
+  };
+  if (NARROW && narrow_tile(tn, T)) {
+    dz_tile<ENTGRAD, TN / 2>(
+        z, T, tm, tn * BN, lds,
+        [&](const Operand& a, const Operand& b, f32x4 (&acc)[TM][TN / 2]) {
+          prefetch_first_tiles<false, TN / 2>(a, b, 0, z.H / BK, lds);
+          zero_acc(acc);
+          mainloop_ksteps<false, TN / 2>(a, b, 0, z.H / BK, lds, acc);
+          return true;
+        },
+        store);
+    return;
+  }
   dz_tile<ENTGRAD, TN>(
-      z, id, lds,
-      [&](Operand a, Operand b, int tm, int tn, acc_t& acc) {
+      z, T, tm, tn * BN, lds,
+      [&](Operand a, Operand b, acc_t& acc) {
 #if LMHEAD_ABLATE & 8
         a.row0 = z.vc0 + (tm % 4) * BM, b.row0 = (tn % 8) * BN;
 #endif
@@ -263,13 +307,7 @@ __device__ __forceinline__ void dz_square_tile(const DzArgs& z, int id, char* ld
         return true;
 #endif
       },
-      [](u32x4 v, u32x4* p) {
-#if LMHEAD_ABLATE & 4
-        asm volatile("" ::"v"(v), "v"(p));  // staged and read back, not stored
-#else
-        __builtin_nontemporal_store(v, p);
-#endif
-      });
+      store);
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -350,7 +388,7 @@ __global__ __launch_bounds__(NTHREADS) void softce_fwd_tiles(const uint16_t* __r
                                                              float rcp_temp, float* __restrict__ part_max,
                                                              float* __restrict__ part_sum, float* __restrict__ part_pz) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  fwd_tile<ENTROPY, true, EVEN>(W, ldw, Hd, ldh, T, H, V, rcp_temp, part_max, part_sum, part_pz, lds);
+  fwd_tile<ENTROPY, true, EVEN, false>(W, ldw, Hd, ldh, T, H, V, rcp_temp, part_max, part_sum, part_pz, lds);
 }
 
 // Per token: the merged statistics of its two stacked rows -> loss and the two log-sum-exps the backward needs.
@@ -695,10 +733,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bid, char* lds)
 
 // The two kinds of backward launch per vocab chunk, as kernels of their own so that a kernel trace tells them apart:
 // the dz tiles of the chunk, then its two gradient GEMMs in one launch (workgroups [0, tiles0) work on p0, the rest on p1).
-template <bool ENTGRAD, bool EVEN>
+template <bool ENTGRAD, bool EVEN, bool NARROW>
 __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_dz(const DzArgs z) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  dz_square_tile<ENTGRAD, EVEN>(z, blockIdx.x, lds);
+  dz_square_tile<ENTGRAD, EVEN, NARROW>(z, blockIdx.x, lds);
 }
 
 __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_gemm(const GemmArgs p0, const GemmArgs p1, int tiles0) {
@@ -782,7 +820,7 @@ __global__ __launch_bounds__(NTHREADS) void mfma_probe(const bf16x8* __restrict_
     for (int ks = 0; ks < KSTEPS; ++ks)
 #pragma unroll
       for (int x = 0; x < TM * TN; ++x) {
-        const int i = mfma_row(x), j = mfma_col(x);
+        const int i = mfma_row<>(x), j = mfma_col<>(x);
         mfma_16x16x32(acc[i][j], af[ks][i], bfr[ks][j]);
       }
   }
@@ -1280,8 +1318,9 @@ int fwd_token_blocks(const void* hidden, int64_t ld_hidden, const void* weight, 
     const dim3 grid((unsigned)(tiles_m * tiles_n)), block(NTHREADS);
     {
       Timed timed(kFwdTiles, s);
-      auto kernel = want_pz ? (even_ktiles(H) ? lmhead_fwd_tiles<true, true> : lmhead_fwd_tiles<true, false>)
-                            : (even_ktiles(H) ? lmhead_fwd_tiles<false, true> : lmhead_fwd_tiles<false, false>);
+      auto kernel = flagged_kernel(
+          [](auto pz, auto even, auto narrow) { return &lmhead_fwd_tiles<pz.value, even.value, narrow.value>; }, want_pz, even_ktiles(H),
+          has_narrow_tile(Tb));
       if (half)
         launch_fwd_half_tiles(s, want_pz, Wp, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)H, (int)V, rcp_temperature, pmax, psum, ppz);
       else
@@ -1432,16 +1471,11 @@ hipError_t launch_bwd_dz(hipStream_t s, bool entgrad, DzArgs z) {
     z.tiles_n = 1;
     return launch_bwd_half_dz(s, entgrad, z);
   }
-  const bool even = even_ktiles(z.H);
   z.tiles_n = (z.T + BN - 1) / BN;
-  const dim3 grid((unsigned)(z.tiles_m * z.tiles_n)), block(NTHREADS);
-  if (entgrad) {
-    if (even) hipLaunchKernelGGL((lmhead_bwd_dz<true, true>), grid, block, 0, s, z);
-    else hipLaunchKernelGGL((lmhead_bwd_dz<true, false>), grid, block, 0, s, z);
-  } else {
-    if (even) hipLaunchKernelGGL((lmhead_bwd_dz<false, true>), grid, block, 0, s, z);
-    else hipLaunchKernelGGL((lmhead_bwd_dz<false, false>), grid, block, 0, s, z);
-  }
+  // A count that only the device knows may leave any remainder.
+  auto kernel = flagged_kernel([](auto ent, auto even, auto narrow) { return &lmhead_bwd_dz<ent.value, even.value, narrow.value>; },
+                               entgrad, even_ktiles(z.H), z.T_dev != nullptr || has_narrow_tile(z.T));
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(z.tiles_m * z.tiles_n)), dim3(NTHREADS), 0, s, z);
   return hipGetLastError();
 }
 
@@ -2065,6 +2099,14 @@ int skyrl_lmhead_topk_logits(const void* hidden, int64_t ld_hidden, const void* 
                               (int)v0, rcp_temperature, (int)((vrows + BM - 1) / BM), tiles_n, kGroupM, w.thr, w.cnt, w.cand,
                               (int)w.cap, (float*)w.cand};
     };
+    auto tiles_kernel = [&](bool first) {
+      return flagged_kernel(
+          [](auto first, auto even, auto narrow) {
+            if constexpr (first.value) return &topk::topk_first_tiles<even.value, narrow.value>;
+            else return &topk::topk_filter_tiles<even.value, narrow.value>;
+          },
+          first, even_ktiles(H), has_narrow_tile(Tb));
+    };
     auto launch_tiles = [&](auto kernel, const topk::FilterArgs& a) {
       Timed timed(kTopkFilter, s);
       hipLaunchKernelGGL(kernel, dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(NTHREADS), 0, s, a);
@@ -2077,7 +2119,7 @@ int skyrl_lmhead_topk_logits(const void* hidden, int64_t ld_hidden, const void* 
     if (dense > V) dense = V;
     {
       const topk::FilterArgs a = chunk_args(0, dense);
-      if ((e = launch_tiles(even_ktiles(H) ? topk::topk_first_tiles<true> : topk::topk_first_tiles<false>, a)) != hipSuccess) return (int)e;
+      if ((e = launch_tiles(tiles_kernel(true), a)) != hipSuccess) return (int)e;
       Timed timed(kTopkSelect, s);
       auto init = dense <= 256 * topk::kInitLogits ? topk::topk_init<256> : topk::topk_init<1024>;
       hipLaunchKernelGGL(init, dim3((unsigned)Tb), dim3(dense <= 256 * topk::kInitLogits ? 256 : 1024), 0, s, (int)k,
@@ -2092,8 +2134,7 @@ int skyrl_lmhead_topk_logits(const void* hidden, int64_t ld_hidden, const void* 
       if (width < BM) width = BM;
       const int64_t vrows = (V - v0) < width ? (V - v0) : width;
       const bool last = v0 + vrows >= V;
-      if (vrows > 0 && (e = launch_tiles(even_ktiles(H) ? topk::topk_filter_tiles<true> : topk::topk_filter_tiles<false>,
-                                         chunk_args(v0, vrows))) != hipSuccess)
+      if (vrows > 0 && (e = launch_tiles(tiles_kernel(false), chunk_args(v0, vrows))) != hipSuccess)
         return (int)e;
       {
         Timed timed(kTopkSelect, s);

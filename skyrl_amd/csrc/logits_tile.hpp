@@ -78,6 +78,9 @@ __device__ __forceinline__ void fwd_tile_stats(const f32x4 (&acc)[TM][N], int j,
   e_out = PAIRED ? e * scale2 * kLn2 : e * kLn2;
 }
 
+// Whether token tile tn of 256, the last one, holds at most 128 of a call's T tokens: it is then made half as wide (N = 4 in gemm_core.hpp).
+__device__ __forceinline__ bool narrow_tile(int tn, int T) { return __builtin_amdgcn_readfirstlane((int)(T - tn * BN <= BN / 2)); }
+
 // Statistics of a tile's accumulators, N token blocks per wave, into the partials.
 template <bool ENTROPY, bool PAIRED, int N>
 __device__ __forceinline__ void fwd_epilogue(const f32x4 (&acc)[TM][N], int tm, int tn, int tiles_m, int T, int V, float rcp_temp,
@@ -168,16 +171,29 @@ __device__ __forceinline__ Operand dz_weight_rows(const uint16_t* W, int ldw, in
   return a;
 }
 
-// NB: token blocks of 16 per wave.  product(a, b, tm, tn, acc) leaves the tile's products in acc, with LDS free and at least
-// NWAVES * NB * 16 * (kDzTokRow + kDzTokBytes) bytes of it, or returns false, which ends the tile; store(v, p) writes one piece.
+// Which tile of `tile_n` tokens workgroup `id` makes, of the tokens in force (T, as dz_tile takes it); false: none.
+// With a device-side count the tiles that hold tokens are numbered 0 .. tiles_m * ceil(T / tile_n) - 1, so that the hardware's
+// round-robin of workgroup ids over the XCDs spreads exactly those; the other workgroups of the (static) grid return at once.
+// The last tiles first: the forward ended with their weight rows, and the last-level cache still holds some of them.  Few tokens, whole
+// training pass, first to last -> last to first: 778 -> 755 us at T=200, H=2048, V=151936, 469 -> 461 at T=40, H=1536; many: the same.
+__device__ __forceinline__ bool dz_tile_of(const DzArgs& z, int id, int tile_n, int& T, int& tm, int& tn) {
+  T = z.T_dev ? __builtin_amdgcn_readfirstlane(*z.T_dev) : z.T;
+  const int tiles_n = z.T_dev ? (T + tile_n - 1) / tile_n : z.tiles_n;
+  if (id >= z.tiles_m * tiles_n) return false;
+  tile_coords(z.tiles_m * tiles_n - 1 - id, z.tiles_m, tiles_n, kGroupM, tm, tn);
+  return true;
+}
+
+// One tile: panel columns tm * 256 .. + 255 of the tokens t0 .. t0 + 32 * NB - 1, of T.  NB: token blocks of 16 per wave.  product(a, b,
+// acc) leaves the tile's products in acc, with LDS free and at least NWAVES * NB * 16 * (kDzTokRow + kDzTokBytes) bytes of it, or returns
+// false, which ends the tile; store(v, p) writes one piece.
 constexpr int kDzTokRow = WM * 2 + 16, kDzTokBytes = 24;
 template <bool ENTGRAD, int NB, class Product, class Store>
-__device__ __forceinline__ void dz_tile(const DzArgs& z, int id, char* lds, Product product, Store store) {
-  constexpr int WAVE_N = NB * MT, TILE_N = WAVES_N * WAVE_N;  // tokens per wave and tile
+__device__ __forceinline__ void dz_tile(const DzArgs& z, int T, int tm, int t0, char* lds, Product product, Store store) {
+  constexpr int WAVE_N = NB * MT;  // tokens per wave
   const uint16_t* __restrict__ W = z.W;
   const uint16_t* __restrict__ Hd = z.Hd;
   const int ldw = z.ldw, ldh = z.ldh, V = z.V, vc0 = z.vc0, ldd = z.ldd;
-  const int T = z.T_dev ? __builtin_amdgcn_readfirstlane(*z.T_dev) : z.T;
   const float rcp_temp = z.rcp_temp;
   const int64_t* __restrict__ labels = z.labels;
   const float* __restrict__ row_lse = z.row_lse;
@@ -185,14 +201,6 @@ __device__ __forceinline__ void dz_tile(const DzArgs& z, int id, char* lds, Prod
   const float* __restrict__ dlogprobs = z.dlogprobs;
   const float* __restrict__ dentropy = z.dentropy;
   uint16_t* __restrict__ D = z.D;
-  // With a device-side count the tiles that hold tokens are numbered 0 .. tiles_m * ceil(T / 256) - 1, so that the hardware's
-  // round-robin of workgroup ids over the XCDs spreads exactly those; the other workgroups of the (static) grid return at once.
-  const int tiles_n = z.T_dev ? (T + TILE_N - 1) / TILE_N : z.tiles_n;
-  if (id >= z.tiles_m * tiles_n) return;
-  // The last tiles first: the forward ended with their weight rows, and the last-level cache still holds some of them.  Few tokens, whole
-  // training pass, first to last -> last to first: 778 -> 755 us at T=200, H=2048, V=151936, 469 -> 461 at T=40, H=1536; many: the same.
-  int tm, tn;
-  tile_coords(z.tiles_m * tiles_n - 1 - id, z.tiles_m, tiles_n, kGroupM, tm, tn);
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
@@ -200,7 +208,7 @@ __device__ __forceinline__ void dz_tile(const DzArgs& z, int id, char* lds, Prod
   const int vloc_base = tm * BM + wm * WM;    // first column of this wave inside the chunk panel
   const WaveRows rows = wave_vocab_rows(vc0 + vloc_base, V, z.tail);
   const int vbase = rows.v0;                  // the vocabulary row of its first column
-  const int tbase = tn * TILE_N + wn * WAVE_N;  // first token of this wave (always inside the padded panels)
+  const int tbase = t0 + wn * WAVE_N;  // first token of this wave (always inside the padded panels)
   const bool full = rows.lo == 0 && rows.hi == WM;
   const float scale2 = rcp_temp * kLog2e;
 
@@ -224,9 +232,9 @@ __device__ __forceinline__ void dz_tile(const DzArgs& z, int id, char* lds, Prod
   }
 
   const Operand a = dz_weight_rows(W, ldw, vc0 + tm * BM, V, z.tail);
-  const Operand b{Hd, ldh, tn * TILE_N, T};
+  const Operand b{Hd, ldh, t0, T};
   f32x4 acc[TM][NB];
-  if (!product(a, b, tm, tn, acc)) return;
+  if (!product(a, b, acc)) return;
 
   constexpr int kTokRow = kDzTokRow;  // dz staging (below): the wave's token rows x (128 vocab x 2 B + pad)
   constexpr int kStage = WAVE_N * kTokRow;

@@ -24,6 +24,7 @@
 #include <stdint.h>
 
 #include "gemm_core.hpp"
+#include "logits_tile.hpp"
 
 namespace topk {
 using namespace lmhead;
@@ -60,29 +61,29 @@ struct FilterArgs {
   float* dense;        // first chunk: its logits [T, tiles_m * 256]
 };
 
-template <bool DENSE, bool EVEN>
-__device__ __forceinline__ void topk_tile(const FilterArgs& a, char* lds) {
-  int tm, tn;
-  tile_coords(blockIdx.x, a.tiles_m, a.tiles_n, a.group_m, tm, tn);
-
+// Tile (tm, tn) of 256 x 256; N: token blocks of 16 per wave, 8 or (a narrow last tile, N = 4 in gemm_core.hpp) 4.
+template <bool DENSE, bool EVEN, int N>
+__device__ __forceinline__ void topk_tile(const FilterArgs& a, int tm, int tn, char* lds) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
   const int lrow = lane & 15, kq = lane >> 4;
   // The tokens' thresholds (fixed for the launch): unconditional loads from a clamped index, issued before the mainloop and
   // first touched behind it -- a load under `t < T` is a branch with its own wait, eight memory round trips in a row.
-  float th[TN];
+  const int tbase = tn * BN + wn * (N * MT) + lrow;  // this lane's token of block j: 16 j further
+  float th[N];
 #pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int t = tn * BN + wn * WN + j * MT + lrow;
+  for (int j = 0; j < N; ++j) {
+    const int t = tbase + j * MT;
     th[j] = DENSE ? 0.f : a.thr[t < a.T ? t : a.T - 1];
   }
 
   Operand oa{a.W, a.ldw, tm * BM, a.vrows};
   Operand ob{a.Hd, a.ldh, tn * BN, a.T};
-  acc_t acc;
-  prefetch_first_tiles(oa, ob, 0, a.H / BK, lds);
+  f32x4 acc[TM][N];
+  prefetch_first_tiles<false, N>(oa, ob, 0, a.H / BK, lds);
   zero_acc(acc);
-  mainloop<false, EVEN>(oa, ob, 0, a.H / BK, lds, acc);
+  if constexpr (N == TN) mainloop<false, EVEN>(oa, ob, 0, a.H / BK, lds, acc);
+  else mainloop_ksteps<false, N>(oa, ob, 0, a.H / BK, lds, acc);
 
   const int vbase = tm * BM + wm * WM;  // first row of this wave inside the chunk
   if (vbase >= a.vrows) return;
@@ -90,8 +91,8 @@ __device__ __forceinline__ void topk_tile(const FilterArgs& a, char* lds) {
   if (DENSE) {  // columns past vrows are stored as they come (copies of the last row) and not read
     const size_t pitch = (size_t)a.tiles_m * BM;
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int t = tn * BN + wn * WN + j * MT + lrow;
+    for (int j = 0; j < N; ++j) {
+      const int t = tbase + j * MT;
       if (t >= a.T) continue;
       float* row = a.dense + (size_t)t * pitch + vbase + kq * 4;
 #pragma unroll
@@ -100,8 +101,8 @@ __device__ __forceinline__ void topk_tile(const FilterArgs& a, char* lds) {
     return;
   }
 #pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int t = tn * BN + wn * WN + j * MT + lrow;
+  for (int j = 0; j < N; ++j) {
+    const int t = tbase + j * MT;
     if (t >= a.T) th[j] = NAN;  // rows past the last token never pass: every comparison with NaN is false
   }
   // A lane holds 32 logits of each of its eight tokens.  First sweep: the largest of the 32 against the threshold (rounding is
@@ -118,9 +119,9 @@ __device__ __forceinline__ void topk_tile(const FilterArgs& a, char* lds) {
     for (int x = 0; x < TM * 4; ++x)
       if (vbase + (x / 4) * MT + kq * 4 + x % 4 >= a.vrows) exists &= ~(0x80000000u >> x);
   }
-  uint32_t hit[TN];  // bit 31 - (i * 4 + r)
+  uint32_t hit[N];  // bit 31 - (i * 4 + r)
 #pragma unroll
-  for (int j = 0; j < TN; ++j) {
+  for (int j = 0; j < N; ++j) {
     float m = acc[0][j][0];
 #pragma unroll
     for (int x = 1; x < TM * 4; ++x) m = fmaxf(m, acc[x / 4][j][x % 4]);
@@ -133,17 +134,17 @@ __device__ __forceinline__ void topk_tile(const FilterArgs& a, char* lds) {
     }
     hit[j] &= exists;
   }
-  unsigned base[TN];
+  unsigned base[N];
 #pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int t = tn * BN + wn * WN + j * MT + lrow;
+  for (int j = 0; j < N; ++j) {
+    const int t = tbase + j * MT;
     base[j] = hit[j] ? atomicAdd(a.cnt + t, (unsigned)__popc(hit[j])) : 0u;
   }
   char* const mine = lds + wave * (TM * 4 * 64 * 4) + lane * 16;  // [i][lane] pieces of four values
 #pragma unroll
-  for (int j = 0; j < TN; ++j) {
+  for (int j = 0; j < N; ++j) {
     if (hit[j] == 0) continue;
-    key_t* list = a.cand + (size_t)(tn * BN + wn * WN + j * MT + lrow) * (size_t)a.cap;
+    key_t* list = a.cand + (size_t)(tbase + j * MT) * (size_t)a.cap;
 #pragma unroll
     for (int i = 0; i < TM; ++i) *(f32x4*)(mine + i * 1024) = acc[i][j];
     unsigned slot = base[j];
@@ -156,16 +157,24 @@ __device__ __forceinline__ void topk_tile(const FilterArgs& a, char* lds) {
   }
 }
 
-template <bool EVEN>
-__global__ __launch_bounds__(NTHREADS) void topk_first_tiles(const FilterArgs a) {
-  __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  topk_tile<true, EVEN>(a, lds);
+template <bool DENSE, bool EVEN, bool NARROW>
+__device__ __forceinline__ void topk_tile_of_workgroup(const FilterArgs& a, char* lds) {
+  int tm, tn;
+  tile_coords(blockIdx.x, a.tiles_m, a.tiles_n, a.group_m, tm, tn);
+  if (NARROW && narrow_tile(tn, a.T)) topk_tile<DENSE, EVEN, TN / 2>(a, tm, tn, lds);
+  else topk_tile<DENSE, EVEN, TN>(a, tm, tn, lds);
 }
 
-template <bool EVEN>
+template <bool EVEN, bool NARROW>
+__global__ __launch_bounds__(NTHREADS) void topk_first_tiles(const FilterArgs a) {
+  __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+  topk_tile_of_workgroup<true, EVEN, NARROW>(a, lds);
+}
+
+template <bool EVEN, bool NARROW>
 __global__ __launch_bounds__(NTHREADS) void topk_filter_tiles(const FilterArgs a) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  topk_tile<false, EVEN>(a, lds);
+  topk_tile_of_workgroup<false, EVEN, NARROW>(a, lds);
 }
 
 // Smallest key of the wave's values, in every lane.

@@ -393,3 +393,32 @@ def test_draft_loss_backward_with_less_scratch(T, H, V, vc, cuda_device):
         assert st == 0, (size, least, full)
         _close(d, hd.grad, f"d student, {size} bytes")
     assert call(least // 2)[0] == ERR_WORKSPACE and (vc > 256 or call(least - 1)[0] == ERR_WORKSPACE)
+
+
+# The last token tile is made half as wide where it holds no more than 128 tokens.  A token's values do not depend on the width of its
+# tile: the last tokens of a call are compared, bit for bit, with those of a longer call in whole tiles.
+@pytest.mark.parametrize("T", [257, 319, 320, 384, 385, 513])
+@pytest.mark.parametrize("H,V", [(64, 1153), (128, 5001), (192, 777), (320, 2304)])
+def test_last_tokens_in_a_narrow_tile(T, H, V, cuda_device):
+    t = 0.8
+    hidden, weight, labels, g, q = _operands(768, H, V, seed=T + H)
+    h, w, y, gd, qd = (x.to(cuda_device) for x in (hidden, weight, labels, g, q))
+    long = ops.lmhead_fwd(h, w, y, 1.0 / t, True)
+    short = ops.lmhead_fwd(h[:T], w, y[:T], 1.0 / t, True)
+    for a, b in zip(short, long):
+        assert torch.equal(a, b[:T])
+    assert torch.equal(ops.lmhead_fwd(h[:T], w, y[:T], 1.0 / t, False)[0], ops.lmhead_fwd(h, w, y, 1.0 / t, False)[0][:T])
+    lse, pz = short[2], short[3]
+    ex = O.exact_fwd_bwd(hidden[:T], weight, labels[:T], t, g[:T], q[:T])
+    dh, dw = ops.lmhead_bwd(h[:T], w, y[:T], lse, pz, gd[:T], qd[:T], 1.0 / t, 0)
+    _close(dh, ex["d_hidden"], f"dHidden T={T}")
+    _close(dw, ex["d_weight"], f"dW T={T}")
+    dropped = gd.clone()  # the same tokens, found by the compaction among others
+    dropped[T:], qd[T:] = 0.0, 0.0
+    dh2, dw2 = ops.lmhead_bwd(h, w, y, long[2], long[3], dropped, qd, 1.0 / t, 0, True)
+    _close(dh2[:T], ex["d_hidden"], f"dHidden of {T} active tokens")
+    _close(dw2, ex["d_weight"], f"dW of {T} active tokens")
+    assert not dh2[T:].any()
+    for k in (5, 200):
+        for a, b in zip(topk_logits_from_hidden(h[:T], w, k), topk_logits_from_hidden(h, w, k)):
+            assert torch.equal(a, b[:T])
