@@ -182,7 +182,9 @@ __global__ __launch_bounds__(NTHREADS, 2) void lmhead_fwd_half_tiles(const uint1
   tile_coords(blockIdx.x, tiles_m, tiles_n, kGroupM, tm, tn);
   half_acc_t acc;
   half_tile_product(Operand{W, ldw, tm * BM, V}, Operand{Hd, ldh, tn * kHalfBN, T}, H / kHalfBK, lds, acc);
-  fwd_epilogue<ENTROPY, false>(acc, tm, tn, tiles_m, T, V, rcp_temp, part_max, part_sum, part_pz);
+  const int wave = threadIdx.x >> 6, wm = wave / WAVES_N, wn = wave % WAVES_N;
+  fwd_epilogue<ENTROPY, false>(acc, tm * WAVES_M + wm, tiles_m * WAVES_M, tn * kHalfBN + wn * kHalfWN, T, V, rcp_temp, part_max, part_sum,
+                               part_pz);
 }
 
 constexpr int kHalfDzLdsBytes = NWAVES * kHalfWN * (kDzTokRow + kDzTokBytes);  // 74 KiB: the epilogue's staging, before it the ring
@@ -190,10 +192,11 @@ static_assert(kHalfDzLdsBytes >= kHalfLdsBytes && 2 * kHalfDzLdsBytes <= LDS_BYT
 template <bool ENTGRAD>
 __global__ __launch_bounds__(NTHREADS, 2) void lmhead_bwd_half_dz(const DzArgs z) {
   __shared__ __attribute__((aligned(1024))) char lds[kHalfDzLdsBytes];
-  int T, tm, tn;
-  if (!dz_tile_of(z, blockIdx.x, kHalfBN, T, tm, tn)) return;
-  dz_tile<ENTGRAD, kHalfTN>(
-      z, T, tm, tn * kHalfBN, lds,
+  int T;
+  Tile tile;
+  if (!dz_tile_of<false>(z, blockIdx.x, kHalfBN, T, tile)) return;
+  dz_tile<ENTGRAD, kHalfTN, false>(
+      z, T, tile.tm * BM, tile.tn * kHalfBN, lds,
       [&](const Operand& a, const Operand& b, half_acc_t& acc) {
         half_tile_product(a, b, z.H / kHalfBK, lds, acc);
         return true;

@@ -101,6 +101,16 @@ constexpr int free_gap(int x, int n) {
     if (g % 8 != 5 && n-- == 0) return g;
 }
 
+// Shapes of a tile.  Narrow, 256 x 128: for the last tokens of a call where they are no more than that.  Short, 128 x 256, the four waves
+// side by side along N: for the last tiles of a launch where they would leave most CUs idle (split_last_round).  Both have half of the MFMAs and three quarters
+// of the copies of a square tile, and a wave's share of them is 128 x 64.
+enum { kSquare = 0, kNarrow = 1, kShort = 2 };
+__host__ __device__ constexpr int waves_n(int shape) { return shape == kShort ? NWAVES : WAVES_N; }
+__host__ __device__ constexpr int wave_cols(int shape) { return shape == kSquare ? TN : TN / 2; }  // blocks of 16 along N per wave
+// Copies per lane and k-tile: one per 32 rows of the operand.
+__host__ __device__ constexpr int a_copies(int shape) { return shape == kShort ? COPIES_PER_OPERAND / 2 : COPIES_PER_OPERAND; }
+__host__ __device__ constexpr int b_copies(int shape) { return shape == kNarrow ? COPIES_PER_OPERAND / 2 : COPIES_PER_OPERAND; }
+
 struct Operand {
   const uint16_t* ptr;  // bf16 bits, row-major, K contiguous
   int ld;               // elements between rows (multiple of 8)
@@ -185,7 +195,7 @@ struct CopyPlan {
   uint32_t a_src[COPIES_PER_OPERAND], b_src[COPIES_PER_OPERAND];
 };
 
-template <bool BKM, int N = TN>
+template <bool BKM, int SHAPE = kSquare>
 __device__ __forceinline__ void make_plan(CopyPlan& p, const Operand& a, const Operand& b, int k_begin) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -194,10 +204,12 @@ __device__ __forceinline__ void make_plan(CopyPlan& p, const Operand& a, const O
     const int c = (j * NWAVES + wave) * 64 + lane;  // chunk index inside the slot
     const int row = c >> 3;
     const int kc = (c & 7) ^ swz(row);
-    int ra = row >= BM / 2 ? row - a.upper_back : row;
-    ra = a.row0 + ra < a.rows ? ra : a.rows - 1 - a.row0;  // row inside the tile; rows past the end re-read the last one
-    p.a_src[j] = (uint32_t)ra * (uint32_t)a.ld * 2u + (uint32_t)(kc * 16);
-    if (j >= N) continue;  // a copy per 32 rows of the operand: a narrow tile has as many fewer
+    if (j < a_copies(SHAPE)) {
+      int ra = row >= BM / 2 ? row - a.upper_back : row;
+      ra = a.row0 + ra < a.rows ? ra : a.rows - 1 - a.row0;  // row inside the tile; rows past the end re-read the last one
+      p.a_src[j] = (uint32_t)ra * (uint32_t)a.ld * 2u + (uint32_t)(kc * 16);
+    }
+    if (j >= b_copies(SHAPE)) continue;
     if (BKM) {
       const int block = j * NWAVES + wave;             // rows 2 * block, 2 * block + 1 of the k-tile
       const int q = (lane >> 2) ^ kmajor_sigma(block);  // the pair whose home is this lane's window
@@ -257,17 +269,17 @@ __device__ __forceinline__ uint32_t wave_copy_base(char* lds) {
 // Put the first k-tiles of an output tile in flight: A(0) B(0) A(1) B(1) into slots 0..3.  All five slots must be free
 // (true at kernel start and after mainloop() returns).  Called before the epilogue of the previous output tile so that
 // the copy path keeps working while the VALU does the epilogue.
-template <bool BKM = false, int N = TN>
+template <bool BKM = false, int SHAPE = kSquare>
 __device__ __forceinline__ void prefetch_first_tiles(const Operand& a, const Operand& b, int k_begin, int nk, char* lds) {
   CopyPlan p;  // rebuilt by mainloop(): keeping it in registers across an epilogue costs more than recomputing it
-  make_plan<BKM, N>(p, a, b, k_begin);
+  make_plan<BKM, SHAPE>(p, a, b, k_begin);
   if (BKM && nk == 2) p.b_bytes -= last_pair_back_bytes<BKM>(b);
   const uint32_t w0 = wave_copy_base(lds);
-  copy_part(p.a_bytes, p.a_src, w0 + 0 * OPERAND_BYTES, 0, COPIES_PER_OPERAND);
-  copy_part(p.b_bytes, p.b_src, w0 + 1 * OPERAND_BYTES, 0, N);
+  copy_part(p.a_bytes, p.a_src, w0 + 0 * OPERAND_BYTES, 0, a_copies(SHAPE));
+  copy_part(p.b_bytes, p.b_src, w0 + 1 * OPERAND_BYTES, 0, b_copies(SHAPE));
   if (nk > 1) {
-    copy_part(p.a_bytes + BK * 2, p.a_src, w0 + 2 * OPERAND_BYTES, 0, COPIES_PER_OPERAND);
-    copy_part(p.b_bytes + b_tile_stride<BKM>(b), p.b_src, w0 + 3 * OPERAND_BYTES, 0, N);
+    copy_part(p.a_bytes + BK * 2, p.a_src, w0 + 2 * OPERAND_BYTES, 0, a_copies(SHAPE));
+    copy_part(p.b_bytes + b_tile_stride<BKM>(b), p.b_src, w0 + 3 * OPERAND_BYTES, 0, b_copies(SHAPE));
   }
 }
 
@@ -287,19 +299,20 @@ __device__ __forceinline__ void prefetch_first_tiles(const Operand& a, const Ope
 // MFMA order inside a step: mfma_row() / mfma_col() above (every fragment of the step is in registers before the step
 // starts, so the order is free to serve the power budget).
 //
-// N = 4: a narrow tile, B[b.row0 : +128], for the last tokens of a call where they are no more than that: half of the MFMAs, three quarters
-// of the copies, so what bounds it is the copies.  A step is then 32 MFMAs, with a copy of A behind every fourth or one of B behind every
-// eighth.  Forward, V=151936, all tiles square -> the last one narrow: 132 -> 114 us at T=300, H=896, 252 -> 221 at T=384, H=2048, 468 -> 432
-// at T=1100, H=1536; training pass 958 -> 925 at T=611, H=1536.  Beyond 128 tokens in the last tile a square one is made.
-template <bool BKM = false, int N = TN>
-__device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand& b, int k_begin, int nk, char* lds, f32x4 (&acc)[TM][N]) {
-  static_assert(N == TN || (N == 4 && !BKM), "the schedule below is written for these");
+// Half shapes: a step is 32 MFMAs, with a copy behind every fourth (of the operand with 256 rows) or every eighth; what bounds them is the
+// copies.  Narrow, forward, V=151936, all tiles square -> the last one narrow: 132 -> 114 us at T=300, H=896, 252 -> 221 at T=384, H=2048,
+// 468 -> 432 at T=1100, H=1536; training pass 958 -> 925 at T=611, H=1536.  Beyond 128 tokens in the last tile a square one is made.
+template <bool BKM = false, int SHAPE = kSquare>
+__device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand& b, int k_begin, int nk, char* lds,
+                                                f32x4 (&acc)[TM][wave_cols(SHAPE)]) {
+  constexpr int N = wave_cols(SHAPE);
+  static_assert(SHAPE == kSquare || !BKM, "the schedule below is written for these");
   CopyPlan p;
-  make_plan<BKM, N>(p, a, b, k_begin);
+  make_plan<BKM, SHAPE>(p, a, b, k_begin);
   const uint32_t b_stride = b_tile_stride<BKM>(b);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+  const int wm = wave / waves_n(SHAPE), wn = wave % waves_n(SHAPE);
   const int lrow = lane & 15;
   const int xsw = ((lane >> 4) ^ swz(lrow)) << 4;  // chunk offset of k-step 0; k-step 1 is xsw ^ 64
   // Per-lane fragment addresses inside a slot, for k-step 0 and 1 of the A and of the B operand.
@@ -364,7 +377,7 @@ __device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand&
     boff1[e] = BKM ? kb_off[e] : b_off1;
   }
 
-  if (nk > 1) wait_copies_and_barrier<COPIES_PER_OPERAND + N>(); else wait_copies_and_barrier<0>();  // tile 0 has landed
+  if (nk > 1) wait_copies_and_barrier<a_copies(SHAPE) + b_copies(SHAPE)>(); else wait_copies_and_barrier<0>();  // tile 0 has landed
   {
     uint32_t pb[NB];
 #pragma unroll
@@ -402,11 +415,13 @@ __device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand&
     constexpr int kGapA = N == TN ? free_gap(kAddX0, 0) : 24;
     constexpr int kGapB[4] = {N == TN ? free_gap(kAddX0, 1) : 26, free_gap(kAddX0, 2), free_gap(kAddX0, 3), free_gap(kAddX0, 4)};
     static_assert(2 * READS_PER_STEP <= (N == TN ? kMfmas : kGapA) && kGapB[NB - 1] < kMfmas, "reads and address adds must fit the step");
-    constexpr int kAPeriod = kMfmas / COPIES_PER_OPERAND, kAGap = N == TN ? 5 : 1;  // MFMAs between the copies of A, and where
+    // MFMAs between the copies of an operand, and where: gaps that carry no fragment read
+    constexpr int kAPeriod = kMfmas / a_copies(SHAPE), kBPeriod = kMfmas / b_copies(SHAPE);
+    constexpr int kAGap = kAPeriod == 8 ? 5 : 1, kBGap = kBPeriod == 8 ? 5 : 1;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
       if (ks == 1 && has_next) {
-        if (load2) wait_copies_and_barrier<COPIES_PER_OPERAND>();  // A(kt+2) may still be in flight
+        if (load2) wait_copies_and_barrier<a_copies(SHAPE)>();  // A(kt+2) may still be in flight
         else wait_copies_and_barrier<0>();
       }
 #pragma unroll
@@ -418,9 +433,8 @@ __device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand&
           if (ks == 0) read_one(ra1, rb1, 1, x / 2);
           else if (has_next) read_one(ra0, rb0, 0, x / 2);
         }
-        // an MFMA gap that carries no fragment read
         if (load2 && ks == 0 && x % kAPeriod == kAGap) copy_part(ga, p.a_src, o4, x / kAPeriod, 1);
-        if (load2 && ks == 1 && x % 8 == 5) copy_part(gb, p.b_src, o0, x / 8, 1);
+        if (load2 && ks == 1 && x % kBPeriod == kBGap) copy_part(gb, p.b_src, o0, x / kBPeriod, 1);
         if (load2 && x == kMfmas - 2) {
           if (ks == 0) {
             ga += BK * 2;
@@ -663,6 +677,15 @@ __device__ __forceinline__ void mainloop(const Operand& a, const Operand& b, int
   else mainloop_ksteps<BKM>(a, b, k_begin, nk, lds, acc);
 }
 
+// acc = the product of a tile of K-contiguous operands over the whole contraction, of nk k-tiles.
+template <int SHAPE, bool EVEN_NK>
+__device__ __forceinline__ void tile_product(const Operand& a, const Operand& b, int nk, char* lds, f32x4 (&acc)[TM][wave_cols(SHAPE)]) {
+  prefetch_first_tiles<false, SHAPE>(a, b, 0, nk, lds);  // the first copies travel while the accumulators are cleared
+  zero_acc(acc);
+  if constexpr (SHAPE == kSquare) mainloop<false, EVEN_NK>(a, b, 0, nk, lds, acc);
+  else mainloop_ksteps<false, SHAPE>(a, b, 0, nk, lds, acc);
+}
+
 // Work item id -> tile coordinates.
 //  1. Hardware hands consecutive workgroup ids to the 8 XCDs round-robin; undo that so each XCD (own L2) owns a
 //     contiguous range of the logical order.  (Persistent workgroups walk ids bid, bid + grid, ...: with a grid that is
@@ -686,6 +709,38 @@ __device__ __forceinline__ void banded_tile(int logical, int tiles_m, int tiles_
 }
 __device__ __forceinline__ void tile_coords(int id, int tiles_m, int tiles_n, int group_m, int& tm, int& tn) {
   banded_tile(xcd_contiguous(id, tiles_m * tiles_n), tiles_m, tiles_n, group_m, tm, tn);
+}
+
+// The tiles of the last round, where they would keep no more than half of the CUs busy, are each made by two workgroups as short tiles: a
+// short tile takes about 0.6 of a square one's time.  How many there are; ncu: CUs, one workgroup each.  594 tiles, 2.3 rounds (forward, T=137,
+// H=896, V=151936): 89 -> 83 us; training pass with 100 of 200 tokens active, H=2048: 768 -> 717; 4.4 and 2.4 rounds (T=2100, 1050 active,
+// H=1024, V=32000, fp32 weight): 654 -> 623.  Beyond half a round the second short tile of some CUs would take longer than one square tile.
+__host__ __device__ inline int split_last_round(int tiles, int ncu) {
+  const int rest = tiles % ncu;
+  return rest <= ncu / 2 ? rest : 0;
+}
+// What workgroup `id` makes of `tiles` tiles, the last `split` of which are made as short ones: ids 0 .. tiles + split - 1.
+struct Tile {
+  int tm, tn;  // place among the square tiles
+  int half;    // short tile: the lower (0) or upper (1) 128 rows of it; -1: all of it
+};
+// REVERSED: the tiles in the opposite order (the short ones still come last).
+template <bool REVERSED, bool SPLIT>
+__device__ __forceinline__ Tile tile_of(int id, int tiles_m, int tiles_n, int group_m, int split) {
+  const int tiles = tiles_m * tiles_n;
+  Tile t;
+  t.half = -1;
+  int logical;
+  if (!SPLIT || id < tiles - split) {
+    logical = xcd_contiguous(id, SPLIT ? tiles - split : tiles);
+  } else {
+    const int s = xcd_contiguous(id - (tiles - split), 2 * split);
+    logical = tiles - split + s / 2;
+    t.half = s & 1;
+  }
+  if (REVERSED) logical = tiles - 1 - logical;
+  banded_tile(logical, tiles_m, tiles_n, group_m, t.tm, t.tn);
+  return t;
 }
 
 // Sum / maximum over the four lanes (l, l^16, l^32, l^48) that hold the same accumulator column, result in all four.

@@ -54,9 +54,9 @@ __host__ __device__ inline int64_t round_up(int64_t x, int64_t m) { return (x + 
 // An even number of k-tiles selects the accumulator-stationary mainloop (the EVEN instantiation of a tile kernel).
 inline bool even_ktiles(int64_t contraction) { return (contraction / BK) % 2 == 0; }
 
-// Whether the last token tile of a call of T tokens is a narrow one.  The branch to it is compiled into kernels of their own: it costs
-// calls of whole tiles half a percent (T=2048, H=896, V=151936: 485 -> 488 us).
-inline bool has_narrow_tile(int64_t T) { return T % BN > 0 && T % BN <= BN / 2; }
+// Whether a launch of tiles_m x ceil(T / 256) tiles has narrow or short ones among them.  The branches to them are compiled into kernels of
+// their own: they cost launches of whole tiles half a percent (T=2048, H=896, V=151936: 485 -> 488 us).
+inline bool has_half_tiles(int64_t T, int split) { return split > 0 || (T % BN > 0 && T % BN <= BN / 2); }
 // pick(x, y, z) for the three flags as compile-time constants.
 template <class Pick>
 auto flagged_kernel(Pick pick, bool x, bool y, bool z) {
@@ -79,51 +79,47 @@ static __device__ __align__(256) unsigned char static_scratch[kStaticScratchByte
 // The label-logit gather of that kernel (:364-385) is done in lmhead_fwd_merge instead.
 // ------------------------------------------------------------------------------------------------------------
 // EVEN: H / 64 is even, which selects the accumulator-stationary mainloop (gemm_core.hpp).
-// NARROW: the last token tile holds no more than 128 tokens and is made half as wide (has_narrow_tile()).
-template <bool ENTROPY, bool PAIRED, bool EVEN, bool NARROW>
+// HALVES: some tiles are narrow or short (has_half_tiles()); split: how many tiles are made as short ones.
+template <bool ENTROPY, bool PAIRED, bool EVEN, bool HALVES>
 __device__ __forceinline__ void fwd_tile(const uint16_t* __restrict__ W, int ldw, const uint16_t* __restrict__ Hd, int ldh, int T,
                                          int H, int V, float rcp_temp, float* __restrict__ part_max,
-                                         float* __restrict__ part_sum, float* __restrict__ part_pz, char* lds) {
+                                         float* __restrict__ part_sum, float* __restrict__ part_pz, int split, char* lds) {
   const int tiles_m = (V + BM - 1) / BM;
   const int tiles_n = (T + BN - 1) / BN;
-  int tm, tn;
-  tile_coords(blockIdx.x, tiles_m, tiles_n, kGroupM, tm, tn);
-
+  const Tile t = tile_of<false, HALVES>(blockIdx.x, tiles_m, tiles_n, kGroupM, split);
+  const int wave = threadIdx.x >> 6;
+  auto tile = [&](auto shape, int v0) {  // the tile of that shape from vocabulary row v0 on
+    constexpr int SHAPE = decltype(shape)::value;
+    const int part = v0 / WM + wave / waves_n(SHAPE), t0 = t.tn * BN + wave % waves_n(SHAPE) * (wave_cols(SHAPE) * MT);
 #if LMHEAD_ABLATE & 8
-  Operand a{W, ldw, (tm % 4) * BM, V};
-  Operand b{Hd, ldh, (tn % 8) * BN, T};
+    const Operand a{W, ldw, (t.tm % 4) * BM, V}, b{Hd, ldh, (t.tn % 8) * BN, T};
 #else
-  Operand a{W, ldw, tm * BM, V};
-  Operand b{Hd, ldh, tn * BN, T};
+    // A part behind the vocabulary (the upper half of the last tile): its statistics are empty whatever row is multiplied.
+    const Operand a{W, ldw, SHAPE == kShort && v0 >= V ? V - 1 : v0, V}, b{Hd, ldh, t.tn * BN, T};
 #endif
-  if constexpr (NARROW) {
-    if (narrow_tile(tn, T)) {
-      f32x4 half[TM][TN / 2];
-      prefetch_first_tiles<false, TN / 2>(a, b, 0, H / BK, lds);
-      zero_acc(half);
-      mainloop_ksteps<false, TN / 2>(a, b, 0, H / BK, lds, half);
-      fwd_epilogue<ENTROPY, PAIRED>(half, tm, 2 * tn, tiles_m, T, V, rcp_temp, part_max, part_sum, part_pz);
+    f32x4 acc[TM][wave_cols(SHAPE)];
+    tile_product<SHAPE, EVEN>(a, b, H / BK, lds, acc);
+#if !(LMHEAD_ABLATE & 1)
+    fwd_epilogue<ENTROPY, PAIRED>(acc, part, tiles_m * WAVES_M, t0, T, V, rcp_temp, part_max, part_sum, part_pz);
+#endif
+  };
+  if constexpr (HALVES) {
+    if (narrow_tile(t.tn, T)) {  // of the two workgroups of a split tile the first makes it
+      if (t.half < 1) tile(std::integral_constant<int, kNarrow>{}, t.tm * BM);
       return;
     }
+    if (t.half >= 0) return tile(std::integral_constant<int, kShort>{}, t.tm * BM + t.half * WM);
   }
-  acc_t acc;
-  prefetch_first_tiles(a, b, 0, H / BK, lds);  // the first copies travel while the accumulators are cleared
-  zero_acc(acc);
-  mainloop<false, EVEN>(a, b, 0, H / BK, lds, acc);
-#if LMHEAD_ABLATE & 1
-  return;
-#endif
-
-  fwd_epilogue<ENTROPY, PAIRED>(acc, tm, tn, tiles_m, T, V, rcp_temp, part_max, part_sum, part_pz);
+  tile(std::integral_constant<int, kSquare>{}, t.tm * BM);
 }
 
-template <bool ENTROPY, bool EVEN, bool NARROW>
+template <bool ENTROPY, bool EVEN, bool HALVES>
 __global__ __launch_bounds__(NTHREADS) void lmhead_fwd_tiles(const uint16_t* __restrict__ W, int ldw,
                                                              const uint16_t* __restrict__ Hd, int ldh, int T, int H, int V,
                                                              float rcp_temp, float* __restrict__ part_max,
-                                                             float* __restrict__ part_sum, float* __restrict__ part_pz) {
+                                                             float* __restrict__ part_sum, float* __restrict__ part_pz, int split) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  fwd_tile<ENTROPY, false, EVEN, NARROW>(W, ldw, Hd, ldh, T, H, V, rcp_temp, part_max, part_sum, part_pz, lds);
+  fwd_tile<ENTROPY, false, EVEN, HALVES>(W, ldw, Hd, ldh, T, H, V, rcp_temp, part_max, part_sum, part_pz, split, lds);
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -267,47 +263,40 @@ __global__ __launch_bounds__(kMergeThreads) void lmhead_fwd_merge(const float* _
   if (row_pz) row_pz[t] = RELATIVE ? lse - third : third;
 }
 
-// The dz tiles (logits_tile.hpp) on square products, the last tokens' on narrow ones.
-template <bool ENTGRAD, bool EVEN, bool NARROW>
+// The dz tiles (logits_tile.hpp) on square, narrow and short products.
+template <bool ENTGRAD, bool EVEN, bool HALVES>
 __device__ __forceinline__ void dz_square_tile(const DzArgs& z, int id, char* lds) {
   static_assert(NWAVES * WN * (kDzTokRow + kDzTokBytes) <= LDS_BYTES, "dz staging and per-token values do not fit LDS");
-  int T, tm, tn;
-  if (!dz_tile_of(z, id, BN, T, tm, tn)) return;
-  auto store = [](u32x4 v, u32x4* p) {
-#if LMHEAD_ABLATE & 4
-    asm volatile("" ::"v"(v), "v"(p));  // staged and read back, not stored
-#else
-    __builtin_nontemporal_store(v, p);
-#endif
-  };
-  if (NARROW && narrow_tile(tn, T)) {
-    dz_tile<ENTGRAD, TN / 2>(
-        z, T, tm, tn * BN, lds,
-        [&](const Operand& a, const Operand& b, f32x4 (&acc)[TM][TN / 2]) {
-          prefetch_first_tiles<false, TN / 2>(a, b, 0, z.H / BK, lds);
-          zero_acc(acc);
-          mainloop_ksteps<false, TN / 2>(a, b, 0, z.H / BK, lds, acc);
-          return true;
-        },
-        store);
-    return;
-  }
-  dz_tile<ENTGRAD, TN>(
-      z, T, tm, tn * BN, lds,
-      [&](Operand a, Operand b, acc_t& acc) {
+  int T;
+  Tile t;
+  if (!dz_tile_of<HALVES>(z, id, BN, T, t)) return;
+  auto tile = [&](auto shape, int col0) {
+    constexpr int SHAPE = decltype(shape)::value;
+    dz_tile<ENTGRAD, wave_cols(SHAPE), SHAPE == kShort>(
+        z, T, col0, t.tn * BN, lds,
+        [&](Operand a, Operand b, f32x4 (&acc)[TM][wave_cols(SHAPE)]) {
 #if LMHEAD_ABLATE & 8
-        a.row0 = z.vc0 + (tm % 4) * BM, b.row0 = (tn % 8) * BN;
+          a.row0 = z.vc0 + (t.tm % 4) * BM, b.row0 = (t.tn % 8) * BN;
 #endif
-        prefetch_first_tiles(a, b, 0, z.H / BK, lds);  // the first copies travel while the accumulators are cleared
-        zero_acc(acc);
-        mainloop<false, EVEN>(a, b, 0, z.H / BK, lds, acc);
-#if LMHEAD_ABLATE & 2
-        return false;
+          tile_product<SHAPE, EVEN>(a, b, z.H / BK, lds, acc);
+          return !(LMHEAD_ABLATE & 2);
+        },
+        [](u32x4 v, u32x4* p) {
+#if LMHEAD_ABLATE & 4
+          asm volatile("" ::"v"(v), "v"(p));  // staged and read back, not stored
 #else
-        return true;
+          __builtin_nontemporal_store(v, p);
 #endif
-      },
-      store);
+        });
+  };
+  if constexpr (HALVES) {
+    if (narrow_tile(t.tn, T)) {  // of the two workgroups of a split tile the first makes it
+      if (t.half < 1) tile(std::integral_constant<int, kNarrow>{}, t.tm * BM);
+      return;
+    }
+    if (t.half >= 0) return tile(std::integral_constant<int, kShort>{}, t.tm * BM + t.half * WM);
+  }
+  tile(std::integral_constant<int, kSquare>{}, t.tm * BM);
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -388,7 +377,7 @@ __global__ __launch_bounds__(NTHREADS) void softce_fwd_tiles(const uint16_t* __r
                                                              float rcp_temp, float* __restrict__ part_max,
                                                              float* __restrict__ part_sum, float* __restrict__ part_pz) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  fwd_tile<ENTROPY, true, EVEN, false>(W, ldw, Hd, ldh, T, H, V, rcp_temp, part_max, part_sum, part_pz, lds);
+  fwd_tile<ENTROPY, true, EVEN, false>(W, ldw, Hd, ldh, T, H, V, rcp_temp, part_max, part_sum, part_pz, 0, lds);
 }
 
 // Per token: the merged statistics of its two stacked rows -> loss and the two log-sum-exps the backward needs.
@@ -733,10 +722,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bid, char* lds)
 
 // The two kinds of backward launch per vocab chunk, as kernels of their own so that a kernel trace tells them apart:
 // the dz tiles of the chunk, then its two gradient GEMMs in one launch (workgroups [0, tiles0) work on p0, the rest on p1).
-template <bool ENTGRAD, bool EVEN, bool NARROW>
+template <bool ENTGRAD, bool EVEN, bool HALVES>
 __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_dz(const DzArgs z) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  dz_square_tile<ENTGRAD, EVEN, NARROW>(z, blockIdx.x, lds);
+  dz_square_tile<ENTGRAD, EVEN, HALVES>(z, blockIdx.x, lds);
 }
 
 __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_gemm(const GemmArgs p0, const GemmArgs p1, int tiles0) {
@@ -1315,17 +1304,18 @@ int fwd_token_blocks(const void* hidden, int64_t ld_hidden, const void* weight, 
     float* psum = c.take<float>(part_elems(nparts, Tb));
     float* ppz = c.take<float>(part_elems(nparts, Tb));
     const uint16_t* Hp = (const uint16_t*)hidden + (size_t)t0 * (size_t)ld_hidden;
-    const dim3 grid((unsigned)(tiles_m * tiles_n)), block(NTHREADS);
+    const int split = split_last_round(tiles_m * tiles_n, compute_units());
+    const dim3 grid((unsigned)(tiles_m * tiles_n + split)), block(NTHREADS);
     {
       Timed timed(kFwdTiles, s);
       auto kernel = flagged_kernel(
-          [](auto pz, auto even, auto narrow) { return &lmhead_fwd_tiles<pz.value, even.value, narrow.value>; }, want_pz, even_ktiles(H),
-          has_narrow_tile(Tb));
+          [](auto pz, auto even, auto halves) { return &lmhead_fwd_tiles<pz.value, even.value, halves.value>; }, want_pz, even_ktiles(H),
+          has_half_tiles(Tb, split));
       if (half)
         launch_fwd_half_tiles(s, want_pz, Wp, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)H, (int)V, rcp_temperature, pmax, psum, ppz);
       else
         hipLaunchKernelGGL(kernel, grid, block, 0, s, Wp, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)H, (int)V,
-                         rcp_temperature, pmax, psum, ppz);
+                         rcp_temperature, pmax, psum, ppz, split);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
@@ -1472,10 +1462,12 @@ hipError_t launch_bwd_dz(hipStream_t s, bool entgrad, DzArgs z) {
     return launch_bwd_half_dz(s, entgrad, z);
   }
   z.tiles_n = (z.T + BN - 1) / BN;
-  // A count that only the device knows may leave any remainder.
-  auto kernel = flagged_kernel([](auto ent, auto even, auto narrow) { return &lmhead_bwd_dz<ent.value, even.value, narrow.value>; },
-                               entgrad, even_ktiles(z.H), z.T_dev != nullptr || has_narrow_tile(z.T));
-  hipLaunchKernelGGL(kernel, dim3((unsigned)(z.tiles_m * z.tiles_n)), dim3(NTHREADS), 0, s, z);
+  const int tiles = z.tiles_m * z.tiles_n;
+  // A count that only the device knows may leave any remainder, and any number of tiles up to these.
+  const int split = z.T_dev ? (tiles < z.ncu / 2 ? tiles : z.ncu / 2) : split_last_round(tiles, z.ncu);
+  auto kernel = flagged_kernel([](auto ent, auto even, auto halves) { return &lmhead_bwd_dz<ent.value, even.value, halves.value>; },
+                               entgrad, even_ktiles(z.H), z.T_dev != nullptr || has_half_tiles(z.T, split));
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles + split)), dim3(NTHREADS), 0, s, z);
   return hipGetLastError();
 }
 
@@ -1679,7 +1671,7 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
     // width, and it needs a second panel.
     const int64_t vc0 = ci * vc, vcw = chunk_width(ci);
     const DzArgs z{Wp, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)Hk, (int)V, rcp_temperature, labels, row_lse, row_pz,
-                   dlogprobs, dentropy, (int)vc0, (int)(vcw / 256), 0, tail, w.D, (int)(vcw + kLdPad), T_dev, resid, p_shift};
+                   dlogprobs, dentropy, (int)vc0, (int)(vcw / 256), 0, tail, w.D, (int)(vcw + kLdPad), T_dev, resid, p_shift, compute_units()};
     e = launch_bwd_dz(s, dentropy != nullptr, z);
     if (e != hipSuccess) return (int)e;
     // dHidden[t, h] (+)= sum_v D[t, v] . weight^T[h, vc0 + v]        (A = weight^T rows at k offset vc0, B = D rows)
@@ -2096,20 +2088,19 @@ int skyrl_lmhead_topk_logits(const void* hidden, int64_t ld_hidden, const void* 
     const uint16_t* Hp = (const uint16_t*)hidden + (size_t)t0 * (size_t)ld_hidden;
     auto chunk_args = [&](int64_t v0, int64_t vrows) {
       return topk::FilterArgs{Wp + (size_t)v0 * (size_t)ld_weight, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)H, (int)vrows,
-                              (int)v0, rcp_temperature, (int)((vrows + BM - 1) / BM), tiles_n, kGroupM, w.thr, w.cnt, w.cand,
-                              (int)w.cap, (float*)w.cand};
+                              (int)v0, rcp_temperature, (int)((vrows + BM - 1) / BM), tiles_n, kGroupM,
+                              split_last_round((int)((vrows + BM - 1) / BM) * tiles_n, compute_units()), w.thr, w.cnt, w.cand, (int)w.cap,
+                              (float*)w.cand};
     };
-    auto tiles_kernel = [&](bool first) {
-      return flagged_kernel(
-          [](auto first, auto even, auto narrow) {
-            if constexpr (first.value) return &topk::topk_first_tiles<even.value, narrow.value>;
-            else return &topk::topk_filter_tiles<even.value, narrow.value>;
+    auto launch_tiles = [&](bool first, const topk::FilterArgs& a) {
+      auto kernel = flagged_kernel(
+          [](auto first, auto even, auto halves) {
+            if constexpr (first.value) return &topk::topk_first_tiles<even.value, halves.value>;
+            else return &topk::topk_filter_tiles<even.value, halves.value>;
           },
-          first, even_ktiles(H), has_narrow_tile(Tb));
-    };
-    auto launch_tiles = [&](auto kernel, const topk::FilterArgs& a) {
+          first, even_ktiles(H), has_half_tiles(Tb, a.split));
       Timed timed(kTopkFilter, s);
-      hipLaunchKernelGGL(kernel, dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(NTHREADS), 0, s, a);
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(a.tiles_m * a.tiles_n + a.split)), dim3(NTHREADS), 0, s, a);
       return hipGetLastError();
     };
     // First chunk: one tile per CU where the stored logits allow it.
@@ -2119,7 +2110,7 @@ int skyrl_lmhead_topk_logits(const void* hidden, int64_t ld_hidden, const void* 
     if (dense > V) dense = V;
     {
       const topk::FilterArgs a = chunk_args(0, dense);
-      if ((e = launch_tiles(tiles_kernel(true), a)) != hipSuccess) return (int)e;
+      if ((e = launch_tiles(true, a)) != hipSuccess) return (int)e;
       Timed timed(kTopkSelect, s);
       auto init = dense <= 256 * topk::kInitLogits ? topk::topk_init<256> : topk::topk_init<1024>;
       hipLaunchKernelGGL(init, dim3((unsigned)Tb), dim3(dense <= 256 * topk::kInitLogits ? 256 : 1024), 0, s, (int)k,
@@ -2134,7 +2125,7 @@ int skyrl_lmhead_topk_logits(const void* hidden, int64_t ld_hidden, const void* 
       if (width < BM) width = BM;
       const int64_t vrows = (V - v0) < width ? (V - v0) : width;
       const bool last = v0 + vrows >= V;
-      if (vrows > 0 && (e = launch_tiles(tiles_kernel(false), chunk_args(v0, vrows))) != hipSuccess)
+      if (vrows > 0 && (e = launch_tiles(false, chunk_args(v0, vrows))) != hipSuccess)
         return (int)e;
       {
         Timed timed(kTopkSelect, s);

@@ -78,19 +78,18 @@ __device__ __forceinline__ void fwd_tile_stats(const f32x4 (&acc)[TM][N], int j,
   e_out = PAIRED ? e * scale2 * kLn2 : e * kLn2;
 }
 
-// Whether token tile tn of 256, the last one, holds at most 128 of a call's T tokens: it is then made half as wide (N = 4 in gemm_core.hpp).
+// Whether token tile tn of 256, the last one, holds at most 128 of a call's T tokens: it is then made half as wide (kNarrow).
 __device__ __forceinline__ bool narrow_tile(int tn, int T) { return __builtin_amdgcn_readfirstlane((int)(T - tn * BN <= BN / 2)); }
 
-// Statistics of a tile's accumulators, N token blocks per wave, into the partials.
+// Statistics of a wave's accumulators, those of part `part` (vocabulary rows 128 * part .. + 127, of nparts parts) and of the N token blocks
+// from token t0 on, into the partials.
 template <bool ENTROPY, bool PAIRED, int N>
-__device__ __forceinline__ void fwd_epilogue(const f32x4 (&acc)[TM][N], int tm, int tn, int tiles_m, int T, int V, float rcp_temp,
+__device__ __forceinline__ void fwd_epilogue(const f32x4 (&acc)[TM][N], int part, int nparts, int t0, int T, int V, float rcp_temp,
                                              float* __restrict__ part_max, float* __restrict__ part_sum,
                                              float* __restrict__ part_pz) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+  const int lane = threadIdx.x & 63;
   const int lrow = lane & 15, kq = lane >> 4;
-  const int vbase = tm * BM + wm * WM;
-  const int part = tm * WAVES_M + wm, nparts = tiles_m * WAVES_M;
+  const int vbase = part * WM;
   const float scale2 = rcp_temp * kLog2e;
   // Whether the wave's 128 vocab rows all exist (0), partly (1: the last vocab tile) or not at all (2) is the same for the
   // whole wave: decided once, outside the unrolled loop over the token blocks.
@@ -99,7 +98,7 @@ __device__ __forceinline__ void fwd_epilogue(const f32x4 (&acc)[TM][N], int tm, 
     constexpr int KIND = decltype(kind)::value;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-      const int t = (tn * WAVES_N + wn) * (N * MT) + j * MT + lrow;
+      const int t = t0 + j * MT + lrow;
       float m = -INFINITY, s = 0.f, e = 0.f;
       if (KIND < 2) fwd_tile_stats<ENTROPY, KIND == 1, PAIRED>(acc, j, vbase, V, scale2, kq, m, s, e);
       if (kq == 0 && t < T) {
@@ -149,6 +148,7 @@ struct DzArgs {
   float* label_resid;
   // 0, or 126 - n: softmax probabilities below 2^-n are treated as zero (SKYRL_BWD_FLUSH_TINY_DZ).
   float p_shift;
+  int ncu;  // CUs of the device
 };
 
 // Which vocabulary rows the 128 panel columns of a wave (columns panel0 .. panel0 + 127 in the full numbering) stand for:
@@ -176,20 +176,24 @@ __device__ __forceinline__ Operand dz_weight_rows(const uint16_t* W, int ldw, in
 // round-robin of workgroup ids over the XCDs spreads exactly those; the other workgroups of the (static) grid return at once.
 // The last tiles first: the forward ended with their weight rows, and the last-level cache still holds some of them.  Few tokens, whole
 // training pass, first to last -> last to first: 778 -> 755 us at T=200, H=2048, V=151936, 469 -> 461 at T=40, H=1536; many: the same.
-__device__ __forceinline__ bool dz_tile_of(const DzArgs& z, int id, int tile_n, int& T, int& tm, int& tn) {
+// SPLIT: the last round may be made of short tiles.
+template <bool SPLIT>
+__device__ __forceinline__ bool dz_tile_of(const DzArgs& z, int id, int tile_n, int& T, Tile& tile) {
   T = z.T_dev ? __builtin_amdgcn_readfirstlane(*z.T_dev) : z.T;
   const int tiles_n = z.T_dev ? (T + tile_n - 1) / tile_n : z.tiles_n;
-  if (id >= z.tiles_m * tiles_n) return false;
-  tile_coords(z.tiles_m * tiles_n - 1 - id, z.tiles_m, tiles_n, kGroupM, tm, tn);
+  const int split = SPLIT ? split_last_round(z.tiles_m * tiles_n, z.ncu) : 0;
+  if (id >= z.tiles_m * tiles_n + split) return false;
+  tile = tile_of<true, SPLIT>(id, z.tiles_m, tiles_n, kGroupM, split);
   return true;
 }
 
-// One tile: panel columns tm * 256 .. + 255 of the tokens t0 .. t0 + 32 * NB - 1, of T.  NB: token blocks of 16 per wave.  product(a, b,
-// acc) leaves the tile's products in acc, with LDS free and at least NWAVES * NB * 16 * (kDzTokRow + kDzTokBytes) bytes of it, or returns
-// false, which ends the tile; store(v, p) writes one piece.
+// One tile: panel columns col0 .. + 255 of the tokens t0 .. t0 + 32 * NB - 1, of T.  NB: token blocks of 16 per wave.  SHORT: the four
+// waves side by side along the tokens, panel columns col0 .. + 127 and twice the tokens.  product(a, b, acc) leaves the tile's products in
+// acc, with LDS free and at least NWAVES * NB * 16 * (kDzTokRow + kDzTokBytes) bytes of it, or returns false, which ends the tile; store(v, p)
+// writes one piece.
 constexpr int kDzTokRow = WM * 2 + 16, kDzTokBytes = 24;
-template <bool ENTGRAD, int NB, class Product, class Store>
-__device__ __forceinline__ void dz_tile(const DzArgs& z, int T, int tm, int t0, char* lds, Product product, Store store) {
+template <bool ENTGRAD, int NB, bool SHORT, class Product, class Store>
+__device__ __forceinline__ void dz_tile(const DzArgs& z, int T, int col0, int t0, char* lds, Product product, Store store) {
   constexpr int WAVE_N = NB * MT;  // tokens per wave
   const uint16_t* __restrict__ W = z.W;
   const uint16_t* __restrict__ Hd = z.Hd;
@@ -203,9 +207,9 @@ __device__ __forceinline__ void dz_tile(const DzArgs& z, int T, int tm, int t0, 
   uint16_t* __restrict__ D = z.D;
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+  const int wm = SHORT ? 0 : wave / WAVES_N, wn = SHORT ? wave : wave % WAVES_N;
   const int lrow = lane & 15, kq = lane >> 4;
-  const int vloc_base = tm * BM + wm * WM;    // first column of this wave inside the chunk panel
+  const int vloc_base = col0 + wm * WM;       // first column of this wave inside the chunk panel
   const WaveRows rows = wave_vocab_rows(vc0 + vloc_base, V, z.tail);
   const int vbase = rows.v0;                  // the vocabulary row of its first column
   const int tbase = t0 + wn * WAVE_N;  // first token of this wave (always inside the padded panels)
@@ -231,7 +235,8 @@ __device__ __forceinline__ void dz_tile(const DzArgs& z, int T, int tm, int t0, 
     y_[u] = labels[tc];
   }
 
-  const Operand a = dz_weight_rows(W, ldw, vc0 + tm * BM, V, z.tail);
+  Operand a = dz_weight_rows(W, ldw, vc0 + col0, V, z.tail);
+  if (SHORT && a.row0 >= V) a.row0 = V - 1;  // the upper half of the last 256 columns may lie behind the vocabulary: zeros, from any row
   const Operand b{Hd, ldh, t0, T};
   f32x4 acc[TM][NB];
   if (!product(a, b, acc)) return;

@@ -54,6 +54,7 @@ struct FilterArgs {
   int v0;              // column number of the chunk's first row
   float rcp_temp;
   int tiles_m, tiles_n, group_m;
+  int split;           // how many of the tiles are made as short ones (split_last_round)
   const float* thr;    // [T] threshold per token, -inf while fewer than k columns have been seen
   unsigned* cnt;       // [T] candidates appended in this launch
   key_t* cand;         // [T, cap]
@@ -61,15 +62,16 @@ struct FilterArgs {
   float* dense;        // first chunk: its logits [T, tiles_m * 256]
 };
 
-// Tile (tm, tn) of 256 x 256; N: token blocks of 16 per wave, 8 or (a narrow last tile, N = 4 in gemm_core.hpp) 4.
-template <bool DENSE, bool EVEN, int N>
-__device__ __forceinline__ void topk_tile(const FilterArgs& a, int tm, int tn, char* lds) {
+// The tile of SHAPE whose first row and token are vtile and ttile.
+template <bool DENSE, bool EVEN, int SHAPE>
+__device__ __forceinline__ void topk_tile(const FilterArgs& a, int vtile, int ttile, char* lds) {
+  constexpr int N = wave_cols(SHAPE);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+  const int wm = wave / waves_n(SHAPE), wn = wave % waves_n(SHAPE);
   const int lrow = lane & 15, kq = lane >> 4;
   // The tokens' thresholds (fixed for the launch): unconditional loads from a clamped index, issued before the mainloop and
   // first touched behind it -- a load under `t < T` is a branch with its own wait, eight memory round trips in a row.
-  const int tbase = tn * BN + wn * (N * MT) + lrow;  // this lane's token of block j: 16 j further
+  const int tbase = ttile + wn * (N * MT) + lrow;  // this lane's token of block j: 16 j further
   float th[N];
 #pragma unroll
   for (int j = 0; j < N; ++j) {
@@ -77,15 +79,13 @@ __device__ __forceinline__ void topk_tile(const FilterArgs& a, int tm, int tn, c
     th[j] = DENSE ? 0.f : a.thr[t < a.T ? t : a.T - 1];
   }
 
-  Operand oa{a.W, a.ldw, tm * BM, a.vrows};
-  Operand ob{a.Hd, a.ldh, tn * BN, a.T};
+  // The upper half of the last tile may lie behind the chunk's rows: multiplied from any row, and dropped below.
+  Operand oa{a.W, a.ldw, SHAPE == kShort && vtile >= a.vrows ? a.vrows - 1 : vtile, a.vrows};
+  Operand ob{a.Hd, a.ldh, ttile, a.T};
   f32x4 acc[TM][N];
-  prefetch_first_tiles<false, N>(oa, ob, 0, a.H / BK, lds);
-  zero_acc(acc);
-  if constexpr (N == TN) mainloop<false, EVEN>(oa, ob, 0, a.H / BK, lds, acc);
-  else mainloop_ksteps<false, N>(oa, ob, 0, a.H / BK, lds, acc);
+  tile_product<SHAPE, EVEN>(oa, ob, a.H / BK, lds, acc);
 
-  const int vbase = tm * BM + wm * WM;  // first row of this wave inside the chunk
+  const int vbase = vtile + wm * WM;  // first row of this wave inside the chunk
   if (vbase >= a.vrows) return;
   const float s = a.rcp_temp;
   if (DENSE) {  // columns past vrows are stored as they come (copies of the last row) and not read
@@ -157,24 +157,30 @@ __device__ __forceinline__ void topk_tile(const FilterArgs& a, int tm, int tn, c
   }
 }
 
-template <bool DENSE, bool EVEN, bool NARROW>
+template <bool DENSE, bool EVEN, bool HALVES>
 __device__ __forceinline__ void topk_tile_of_workgroup(const FilterArgs& a, char* lds) {
-  int tm, tn;
-  tile_coords(blockIdx.x, a.tiles_m, a.tiles_n, a.group_m, tm, tn);
-  if (NARROW && narrow_tile(tn, a.T)) topk_tile<DENSE, EVEN, TN / 2>(a, tm, tn, lds);
-  else topk_tile<DENSE, EVEN, TN>(a, tm, tn, lds);
+  const Tile t = tile_of<false, HALVES>(blockIdx.x, a.tiles_m, a.tiles_n, a.group_m, a.split);
+  const int v = t.tm * BM, n = t.tn * BN;
+  if constexpr (HALVES) {
+    if (narrow_tile(t.tn, a.T)) {
+      if (t.half < 1) topk_tile<DENSE, EVEN, kNarrow>(a, v, n, lds);
+      return;
+    }
+    if (t.half >= 0) return topk_tile<DENSE, EVEN, kShort>(a, v + t.half * WM, n, lds);
+  }
+  topk_tile<DENSE, EVEN, kSquare>(a, v, n, lds);
 }
 
-template <bool EVEN, bool NARROW>
+template <bool EVEN, bool HALVES>
 __global__ __launch_bounds__(NTHREADS) void topk_first_tiles(const FilterArgs a) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  topk_tile_of_workgroup<true, EVEN, NARROW>(a, lds);
+  topk_tile_of_workgroup<true, EVEN, HALVES>(a, lds);
 }
 
-template <bool EVEN, bool NARROW>
+template <bool EVEN, bool HALVES>
 __global__ __launch_bounds__(NTHREADS) void topk_filter_tiles(const FilterArgs a) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  topk_tile_of_workgroup<false, EVEN, NARROW>(a, lds);
+  topk_tile_of_workgroup<false, EVEN, HALVES>(a, lds);
 }
 
 // Smallest key of the wave's values, in every lane.

@@ -422,3 +422,31 @@ def test_last_tokens_in_a_narrow_tile(T, H, V, cuda_device):
     for k in (5, 200):
         for a, b in zip(topk_logits_from_hidden(h[:T], w, k), topk_logits_from_hidden(h, w, k)):
             assert torch.equal(a, b[:T])
+
+
+# The tiles of a last round that fills no more than half of the CUs are made as short ones, the rest as square ones: 133 tile rows give a round
+# of nothing but short tiles for one token tile, 256 square and 10 short ones for two, and none for three, whose values are the measure, bit for
+# bit.  The vocabulary ends in the lower half of its last tile, at its middle, and in the upper half.
+@pytest.mark.parametrize("V", [33900, 33920, 34001])
+@pytest.mark.parametrize("T", [40, 137, 256, 300, 512])
+def test_last_round_in_short_tiles(T, V, cuda_device):
+    H, t = 128, 0.8
+    hidden, weight, labels, g, q = _operands(768, H, V, seed=V)
+    labels[:4] = torch.tensor([V - 1, 132 * 256, 132 * 256 + 107, 0])
+    h, w, y, gd, qd = (x.to(cuda_device) for x in (hidden, weight, labels, g, q))
+    for want_entropy in (False, True):
+        long, short = ops.lmhead_fwd(h, w, y, 1.0 / t, want_entropy), ops.lmhead_fwd(h[:T], w, y[:T], 1.0 / t, want_entropy)
+        for a, b in zip(short, long):
+            assert torch.equal(a, b[:T])
+    for a, b in zip(topk_logits_from_hidden(h[:T], w, 5), topk_logits_from_hidden(h, w, 5)):
+        assert torch.equal(a, b[:T])
+    # d_hidden of the same tokens, alone and found by the compaction, with the whole vocabulary in one chunk and in two
+    gd[T:], qd[T:] = 0.0, 0.0
+    ex = O.exact_fwd_bwd(hidden[:T], weight, labels[:T], t, g[:T], q[:T])
+    for vc in (0, 17408):
+        dh, dw = ops.lmhead_bwd(h[:T], w, y[:T], short[2], short[3], gd[:T], qd[:T], 1.0 / t, vc)
+        _close(dh, ex["d_hidden"], f"dHidden T={T} chunk={vc}")
+        _close(dw, ex["d_weight"], f"dW T={T} chunk={vc}")
+        dh, dw = ops.lmhead_bwd(h, w, y, long[2], long[3], gd, qd, 1.0 / t, vc, True)
+        _close(dh[:T], ex["d_hidden"], f"dHidden of {T} active tokens, chunk={vc}")
+        _close(dw, ex["d_weight"], f"dW of {T} active tokens, chunk={vc}")
