@@ -195,39 +195,52 @@ struct CopyPlan {
   uint32_t a_src[COPIES_PER_OPERAND], b_src[COPIES_PER_OPERAND];
 };
 
+// This runs in front of a tile's first copy, where nothing hides it, so the sixteen offsets are formed from one product per operand: a lane's
+// rows of consecutive copies are 32 apart (8 k-rows of a K-major operand), which is a scalar step, and rows past the end are clamped as
+// offsets.  With a product and a comparison of rows per copy and tile coordinates by integer division (small_quotient) -> this way: forward
+// at T=2048, H=896, V=151936 480 -> 470 us (0.5 us of a tile's 25), at T=700, V=64000 92 -> 89.
 template <bool BKM, int SHAPE = kSquare>
 __device__ __forceinline__ void make_plan(CopyPlan& p, const Operand& a, const Operand& b, int k_begin) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = wave * 8 + (lane >> 3);  // inside the slot, of copy 0; of copy j: 32 j further, with the same swizzle
+  static_assert(NWAVES * 64 / 8 == 32, "32 rows per copy of the workgroup");
+  const uint32_t kc = (uint32_t)(((lane & 7) ^ swz(row)) << 4);
+  const uint32_t a_pitch = (uint32_t)a.ld * 2u, b_pitch = (uint32_t)b.ld * 2u;
+  auto last_row = [](int r) { return (uint32_t)(r < BM ? r : BM); };  // of the tile; rows past the end re-read it
+  const int a_row0 = __builtin_amdgcn_readfirstlane(a.row0), b_row0 = __builtin_amdgcn_readfirstlane(b.row0);
+  {
+    const uint32_t first = (uint32_t)row * a_pitch, last = last_row(a.rows - 1 - a_row0) * a_pitch;
+    const uint32_t back = (uint32_t)__builtin_amdgcn_readfirstlane(a.upper_back) * a_pitch;
 #pragma unroll
-  for (int j = 0; j < COPIES_PER_OPERAND; ++j) {
-    const int c = (j * NWAVES + wave) * 64 + lane;  // chunk index inside the slot
-    const int row = c >> 3;
-    const int kc = (c & 7) ^ swz(row);
-    if (j < a_copies(SHAPE)) {
-      int ra = row >= BM / 2 ? row - a.upper_back : row;
-      ra = a.row0 + ra < a.rows ? ra : a.rows - 1 - a.row0;  // row inside the tile; rows past the end re-read the last one
-      p.a_src[j] = (uint32_t)ra * (uint32_t)a.ld * 2u + (uint32_t)(kc * 16);
-    }
-    if (j >= b_copies(SHAPE)) continue;
-    if (BKM) {
-      const int block = j * NWAVES + wave;             // rows 2 * block, 2 * block + 1 of the k-tile
-      const int q = (lane >> 2) ^ kmajor_sigma(block);  // the pair whose home is this lane's window
-      const int krow = 2 * block + ((lane >> 1) & 1);
-      int n = q * 16 + (lane & 1) * 8;  // column inside the tile
-      n = b.row0 + n < b.rows - 8 ? n : b.rows - 8 - b.row0;
-      p.b_src[j] = (uint32_t)krow * (uint32_t)b.ld * 2u + (uint32_t)(n * 2);
-    } else {
-      int rb = b.row0 + row < b.rows ? row : b.rows - 1 - b.row0;
-      p.b_src[j] = (uint32_t)rb * (uint32_t)b.ld * 2u + (uint32_t)(kc * 16);
+    for (int j = 0; j < a_copies(SHAPE); ++j) {
+      const uint32_t off = first + ((uint32_t)(32 * j) * a_pitch - (32 * j >= BM / 2 ? back : 0u));
+      p.a_src[j] = (off < last ? off : last) + kc;
     }
   }
-  // The tile origins are wave-uniform, but they come out of integer divisions that the compiler runs on the vector unit:
-  // readfirstlane puts them (and with them the two base pointers) back into scalar registers.
-  const size_t a_row0 = (size_t)__builtin_amdgcn_readfirstlane(a.row0), b_row0 = (size_t)__builtin_amdgcn_readfirstlane(b.row0);
-  p.a_bytes = (const char*)a.ptr + (a_row0 * (size_t)a.ld + (size_t)k_begin) * 2;
-  p.b_bytes = (const char*)b.ptr +
-              (BKM ? ((size_t)k_begin * (size_t)b.ld + b_row0) * 2 : (b_row0 * (size_t)b.ld + (size_t)k_begin) * 2);
+  if constexpr (BKM) {
+    const uint32_t first = (uint32_t)(2 * wave + ((lane >> 1) & 1)) * b_pitch;  // block j * NWAVES + wave: its rows 2 * block, 2 * block + 1
+    uint32_t col[2];  // of the copies with an even and an odd j, whose blocks have unlike keys
+#pragma unroll
+    for (int odd = 0; odd < 2; ++odd) {
+      const int q = (lane >> 2) ^ kmajor_sigma(odd * NWAVES + wave);  // the pair whose home is this lane's window
+      const int n = q * 16 + (lane & 1) * 8, end = b.rows - 8 - b_row0;  // column inside the tile
+      col[odd] = (uint32_t)((n < end ? n : end) * 2);
+    }
+#pragma unroll
+    for (int j = 0; j < b_copies(SHAPE); ++j) p.b_src[j] = first + (uint32_t)(2 * NWAVES * j) * b_pitch + col[j & 1];
+  } else {
+    const uint32_t first = (uint32_t)row * b_pitch, last = last_row(b.rows - 1 - b_row0) * b_pitch;
+#pragma unroll
+    for (int j = 0; j < b_copies(SHAPE); ++j) {
+      const uint32_t off = first + (uint32_t)(32 * j) * b_pitch;
+      p.b_src[j] = (off < last ? off : last) + kc;
+    }
+  }
+  // 64-bit addresses of the tile's first row (or column) at k_begin.
+  p.a_bytes = (const char*)a.ptr + ((size_t)a_row0 * (size_t)a.ld + (size_t)k_begin) * 2;
+  p.b_bytes = (const char*)b.ptr + (BKM ? ((size_t)k_begin * (size_t)b.ld + (size_t)b_row0) * 2
+                                        : ((size_t)b_row0 * (size_t)b.ld + (size_t)k_begin) * 2);
 }
 
 // Bytes by which the last pair of k-tiles of the B operand starts earlier than its place in the sequence.
@@ -697,14 +710,22 @@ __device__ __forceinline__ int xcd_contiguous(int id, int total) {
   const int per_xcd = total >> 3;
   return id < (per_xcd << 3) ? (id & 7) * per_xcd + (id >> 3) : id;
 }
+// n / d of wave-uniform n >= 0 and d >= 1 with a quotient below 2^21: in fp32, where its error is below one, and put right.  The compiler's division
+// takes twice as many instructions, five of them multiplications at a quarter of the rate.
+__device__ __forceinline__ int small_quotient(int n, int d) {
+  int q = (int)((float)n * __builtin_amdgcn_rcpf((float)d));
+  int r = n - q * d;
+  q += r < 0 ? -1 : (r >= d ? 1 : 0);
+  return __builtin_amdgcn_readfirstlane(q);
+}
 __device__ __forceinline__ void banded_tile(int logical, int tiles_m, int tiles_n, int group_m, int& tm, int& tn) {
   const int band_sz = group_m * tiles_n;
-  const int band = logical / band_sz;
+  const int band = small_quotient(logical, band_sz);
   const int in_band = logical - band * band_sz;
   const int m_first = band * group_m;
   int gm = tiles_m - m_first;
   gm = gm < group_m ? gm : group_m;
-  tn = in_band / gm;
+  tn = gm == 4 ? in_band >> 2 : small_quotient(in_band, gm);
   tm = m_first + (in_band - tn * gm);
 }
 __device__ __forceinline__ void tile_coords(int id, int tiles_m, int tiles_n, int group_m, int& tm, int& tn) {
