@@ -32,6 +32,7 @@ import torch
 from . import _lib
 from ._launch import call, device_guard, raw_stream, registered_op
 from .ops import _require_device
+from .policy_loss import masked_mean
 
 __all__ = ["soft_ce_from_hidden", "draft_soft_ce_from_hidden", "shift_mask_for_mtp", "softce_fwd", "softce_bwd",
            "topk_logits_from_hidden", "soft_ce_topk_from_hidden", "draft_soft_ce_topk_from_hidden", "topk_logits",
@@ -155,6 +156,18 @@ def soft_ce_from_hidden(student_hidden: torch.Tensor, teacher_hidden: torch.Tens
     return loss.reshape(out_shape)
 
 
+def _masked_loss(per_token: torch.Tensor, mask: torch.Tensor, global_normalization_factor: Optional[torch.Tensor]) -> torch.Tensor:
+    """The masked sum over the mask's own sum (at least 1) or over the given factor.  A mask of the loss's shape goes through the
+    masked-mean kernel, one launch each way instead of five and three; one that is broadcast (its own sum counts every value once) or
+    takes a gradient itself does not."""
+    mask = mask.to(per_token.dtype)
+    if global_normalization_factor is not None:
+        return (per_token * mask).sum() / global_normalization_factor.clamp(min=1.0)
+    if mask.shape == per_token.shape and mask.device == per_token.device and not mask.requires_grad:
+        return masked_mean(per_token, mask)
+    return (per_token * mask).sum() / mask.sum().clamp(min=1.0)
+
+
 def draft_soft_ce_from_hidden(
     student_hidden: torch.Tensor,
     teacher_hidden: torch.Tensor,
@@ -178,10 +191,7 @@ def draft_soft_ce_from_hidden(
             and torch.distributed.get_world_size(vocab_parallel_group) > 1:
         raise NotImplementedError("the fused soft cross-entropy covers one vocabulary shard")
     per_token = soft_ce_from_hidden(student_hidden, teacher_hidden, weight, shift=mtp_layer_number + 1, vocab_chunk=vocab_chunk)
-    mask = mask.to(per_token.dtype)
-    if global_normalization_factor is not None:
-        return (per_token * mask).sum() / global_normalization_factor.clamp(min=1.0)
-    return (per_token * mask).sum() / mask.sum().clamp(min=1.0)
+    return _masked_loss(per_token, mask, global_normalization_factor)
 
 
 @registered_op("skyrl_amd::topk_logits", mutates_args=())
@@ -343,10 +353,7 @@ def draft_soft_ce_topk_from_hidden(
             and torch.distributed.get_world_size(vocab_parallel_group) > 1:
         raise NotImplementedError("the fused top-k soft cross-entropy covers one vocabulary shard")
     per_token = soft_ce_topk_from_hidden(student_hidden, teacher_hidden, weight, k, shift=roll_shift)
-    mask = mask.to(per_token.dtype)
-    if global_normalization_factor is not None:
-        return (per_token * mask).sum() / global_normalization_factor.clamp(min=1.0)
-    return (per_token * mask).sum() / mask.sum().clamp(min=1.0)
+    return _masked_loss(per_token, mask, global_normalization_factor)
 
 
 def shift_mask_for_mtp(mask: torch.Tensor, mtp_layer_number: int = 0, cu_seqlens: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -355,6 +362,9 @@ def shift_mask_for_mtp(mask: torch.Tensor, mtp_layer_number: int = 0, cu_seqlens
     sequence; with ``cu_seqlens`` the ``[1, T]`` mask is one packed row and the roll stays inside each segment."""
     shift = mtp_layer_number + 1
     S = mask.shape[1]
+    if cu_seqlens is None and mask.dim() == 2 and shift >= 0:  # whole rows: three launches instead of nine
+        behind = min(shift, S)
+        return mask * torch.nn.functional.pad(mask[:, behind:], (0, behind))
     pos = torch.arange(S, device=mask.device)
     if cu_seqlens is None:
         end = torch.full((S,), S, device=mask.device, dtype=torch.long)

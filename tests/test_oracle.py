@@ -1218,3 +1218,16 @@ def test_minibatch_rollout_logprob_diff_metrics_by_hand():
     none = torch.zeros(2, 3, dtype=torch.float64)                  # nothing counts: the denominators are clamped at 1
     m = O.minibatch_rollout_logprob_diff_metrics(lp, rollout, none)
     assert (m[f"{pre}_mean"], m[f"{pre}_sq_mean"], m[f"{pre}_max"], m[f"{pre}_min"]) == (0.0, 0.0, 0.0, 0.0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.int64, torch.bool])
+@pytest.mark.parametrize("depth", [-1, 0, 3, 6, 40])
+def test_shift_mask_for_mtp_of_any_type_and_depth(dtype, depth):
+    from skyrl_amd.mtp_soft_ce import shift_mask_for_mtp as product
+
+    mask = (torch.rand(7, 3, generator=torch.Generator().manual_seed(depth + 1)) < 0.7).to(dtype).t()  # strided rows of 7
+    want = torch.zeros_like(mask)
+    for t in range(7 - depth - 1):
+        want[:, t] = mask[:, t] * mask[:, t + depth + 1]
+    got = product(mask, depth)
+    assert got.dtype == dtype and torch.equal(got, want)

@@ -13,7 +13,8 @@ from oracle import lmhead_oracle as O
 from skyrl_amd import _lib, ops
 from skyrl_amd import torch_utils as TU
 from skyrl_amd.model_utils import from_parallel_hidden_to_logprobs
-from skyrl_amd.mtp_soft_ce import soft_ce_from_hidden, softce_bwd, softce_fwd, topk_logits_from_hidden
+from skyrl_amd.mtp_soft_ce import (draft_soft_ce_from_hidden, draft_soft_ce_topk_from_hidden, soft_ce_from_hidden, soft_ce_topk_from_hidden,
+                                   softce_bwd, softce_fwd, topk_logits_from_hidden)
 
 pytestmark = pytest.mark.gpu
 
@@ -450,3 +451,26 @@ def test_last_round_in_short_tiles(T, V, cuda_device):
         dh, dw = ops.lmhead_bwd(h, w, y, long[2], long[3], gd, qd, 1.0 / t, vc, True)
         _close(dh[:T], ex["d_hidden"], f"dHidden of {T} active tokens, chunk={vc}")
         _close(dw, ex["d_weight"], f"dW of {T} active tokens, chunk={vc}")
+
+
+# The draft loss's masked mean: the mask's own sum counts, once per value where it is broadcast over the sequences, and is at least one.
+@pytest.mark.parametrize("shape", [(3, 41), (1, 41)])
+@pytest.mark.parametrize("share", [0.0, 0.01, 0.6])
+def test_masked_mean_of_the_draft_loss(shape, share, cuda_device):
+    B, S, H, V = 3, 41, 64, 1500
+    hidden, weight, *_ = _operands(2 * B * S, H, V, seed=S)
+    student, teacher = (x.reshape(B, S, H).to(cuda_device) for x in hidden.split(B * S))
+    mask = (torch.rand(shape, generator=torch.Generator().manual_seed(7)) < share).to(cuda_device)
+    up = torch.tensor(0.7, device=cuda_device)
+    for loss_of, per_token_of in (
+            (lambda s: draft_soft_ce_from_hidden(s, teacher, weight.to(cuda_device), mask),
+             lambda s: soft_ce_from_hidden(s, teacher, weight.to(cuda_device), shift=1)),
+            (lambda s: draft_soft_ce_topk_from_hidden(s, teacher, weight.to(cuda_device), mask, 9, roll_shift=1),
+             lambda s: soft_ce_topk_from_hidden(s, teacher, weight.to(cuda_device), 9, shift=1))):
+        s, r = (student.clone().requires_grad_(True) for _ in range(2))
+        loss, per_token = loss_of(s), per_token_of(r)
+        want = (per_token.double() * mask).sum() / mask.double().sum().clamp(min=1.0)
+        assert loss.shape == () and abs(float(loss.detach()) - float(want.detach())) <= 1e-6 * max(1.0, abs(float(want.detach())))
+        (loss * up).backward()
+        (want * up).backward()  # the upstream per token differs in fp32 roundings only, which d_hidden's bf16 rounding may turn into an ulp
+        assert torch.allclose(s.grad.float(), r.grad.float(), rtol=2**-7, atol=1e-7)
