@@ -127,9 +127,10 @@ __global__ __launch_bounds__(NTHREADS) void lmhead_fwd_tiles(const uint16_t* __r
 // every 64th of them (a load is 64 contiguous bytes of four parts), the running triples meet in shuffles and in LDS.  Wave w
 // also takes the label logit of token w, 64 lanes to the dot product.
 // What bounds it: 12 bytes per part and token and two rows per label from HBM for many tokens, the chain of load and merge steps
-// for few.  Sixty-four streams per token and 24 loads in flight per lane keep that chain at three steps for 1188 parts (16
-// streams of 64-token blocks: 19), and one exponential per part instead of two.  V=151936: 35 -> 11 us at T=137, 40 -> 13 at
-// T=611, 39 -> 14 at T=2048 with entropy, 50 -> 34 at T=8192 with entropy; 83 -> 81 us at T=16384, H=3584 (5.8 TB/s).
+// for few.  Sixty-four streams per token and 30 loads in flight per lane keep that chain at two steps for 1188 parts (16
+// streams of 64-token blocks: 19), with one exponential per part, and the label's rows are loaded with the first step.  V=151936: 7 us
+// at T=137, 8 at T=611, 9 at T=2048 with entropy, 30 at T=8192 with entropy, 78 at T=16384, H=3584 (6 TB/s); eight parts a step and the
+// label's rows behind them: 7, 10, 10, 30, 77.
 // Merge algebra as in efficient_entropy_triton_kernel_epilogue (fused_linear_logprob_triton.py:417-467) except that
 // the running max starts at -inf (that kernel starts it at 0, which loses rows whose logits are all << 0).
 // Out-of-range labels give logprob 0 (model_utils.py:337; fused_linear_logprob_triton.py:1898-1905).
@@ -190,34 +191,23 @@ __global__ __launch_bounds__(kMergeThreads) void lmhead_fwd_merge(const float* _
   // Four consecutive workgroups read the same cache lines (16 of a block's 64 tokens each): keep them on one XCD.
   const int t0 = xcd_contiguous(blockIdx.x, gridDim.x) * kMergeTokens;
   const int64_t y = (labels && t0 + wave < T) ? labels[t0 + wave] : (int64_t)-1;
-  {
-    const int t = t0 + (lane & 15);
-    const size_t base = part_index(0, t, nparts);
-    float M = -INFINITY, S = 0.f, E = 0.f;
-    if (t < T) {
-      constexpr int kBatch = 8, kStreams = kMergeWaves * 4;  // loads in flight per array before the dependent merge chain
-      for (int p0 = wave * 4 + (lane >> 4); p0 < nparts; p0 += kStreams * kBatch) {
-        float m[kBatch], sv[kBatch], ev[kBatch];
+  const int t = t0 + (lane & 15);
+  const size_t base = part_index(0, t < T ? t : T - 1, nparts);
+  constexpr int kBatch = 10, kStreams = kMergeWaves * 4;  // loads in flight per array before the dependent merge chain
+  const int first = wave * 4 + (lane >> 4);
+  float m[kBatch], sv[kBatch], ev[kBatch];
+  auto load_batch = [&](int p0) {  // parts p0, p0 + kStreams, ...; behind the last one: part 0, dropped below
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u) {
-          const int p = p0 + u * kStreams;
-          const bool in = p < nparts;
-          const size_t idx = base + (size_t)(in ? p : p0) * kPartTokens;
-          m[u] = part_max[idx];
-          sv[u] = part_sum[idx];
-          ev[u] = part_pz ? part_pz[idx] : 0.f;
-        }
-#pragma unroll
-        for (int u = 0; u < kBatch; ++u)
-          if (p0 + u * kStreams >= nparts || sv[u] == 0.f) m[u] = -INFINITY, sv[u] = 0.f, ev[u] = 0.f;
-        merge_partials<RELATIVE>(M, S, E, m, sv, ev);
-      }
+    for (int u = 0; u < kBatch; ++u) {
+      const int p = p0 + u * kStreams;
+      const size_t idx = base + (size_t)(p < nparts ? p : 0) * kPartTokens;
+      m[u] = part_max[idx];
+      sv[u] = part_sum[idx];
+      ev[u] = part_pz ? part_pz[idx] : 0.f;
     }
-    merge_lanes<RELATIVE>(M, S, E, 16);
-    merge_lanes<RELATIVE>(M, S, E, 32);
-    if (lane < kMergeTokens) sm_m[wave][lane] = M, sm_s[wave][lane] = S, sm_e[wave][lane] = E;
-  }
-  // Label logit: 16-byte loads, fp32 accumulation.
+  };
+  load_batch(first);
+  // Label logit: 16-byte loads, fp32 accumulation.  Its two rows travel together with the first batch of the partials.
   float dot = 0.f;
   const bool has_label = y >= 0 && y < (int64_t)V;
   if (has_label) {
@@ -236,12 +226,26 @@ __global__ __launch_bounds__(kMergeThreads) void lmhead_fwd_merge(const float* _
       }
     }
   }
+  {
+    float M = -INFINITY, S = 0.f, E = 0.f;
+    for (int p0 = first; p0 < nparts;) {
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u)
+        if (p0 + u * kStreams >= nparts || sv[u] == 0.f) m[u] = -INFINITY, sv[u] = 0.f, ev[u] = 0.f;
+      merge_partials<RELATIVE>(M, S, E, m, sv, ev);
+      p0 += kStreams * kBatch;
+      if (p0 < nparts) load_batch(p0);
+    }
+    merge_lanes<RELATIVE>(M, S, E, 16);
+    merge_lanes<RELATIVE>(M, S, E, 32);
+    if (lane < kMergeTokens) sm_m[wave][lane] = M, sm_s[wave][lane] = S, sm_e[wave][lane] = E;
+  }
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) dot += __shfl_xor(dot, o, 64);
   if (lane == 0) sm_dot[wave] = dot, sm_has_label[wave] = has_label;
   __syncthreads();
   if (wave != 0) return;
-  const int tl = lane & 15, t = t0 + tl;
+  const int tl = lane & 15;
   float M = -INFINITY, S = 0.f, E = 0.f;
   float wm[kMergeWaves / 4], ws[kMergeWaves / 4], we[kMergeWaves / 4];
 #pragma unroll
