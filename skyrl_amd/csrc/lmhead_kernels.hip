@@ -128,9 +128,9 @@ __global__ __launch_bounds__(NTHREADS) void lmhead_fwd_tiles(const uint16_t* __r
 // also takes the label logit of token w, 64 lanes to the dot product.
 // What bounds it: 12 bytes per part and token and two rows per label from HBM for many tokens, the chain of load and merge steps
 // for few.  Sixty-four streams per token and 30 loads in flight per lane keep that chain at two steps for 1188 parts (16
-// streams of 64-token blocks: 19), with one exponential per part, and the label's rows are loaded with the first step.  V=151936: 7 us
-// at T=137, 8 at T=611, 9 at T=2048 with entropy, 30 at T=8192 with entropy, 78 at T=16384, H=3584 (6 TB/s); eight parts a step and the
-// label's rows behind them: 7, 10, 10, 30, 77.
+// streams of 64-token blocks: 19), with one exponential per part, and the label's rows are loaded with the first step.  Between HIP events
+// (which add about 4 us), V=151936, eight parts a step and the label's rows behind them -> this way: 11.2 -> 10.8 us at T=137, 14.0 -> 12.3 at
+// T=611, 14.4 -> 13.3 at T=2048 with entropy, 34 and 34 at T=8192, 81 and 82 at T=16384, H=3584 (5.8 TB/s).
 // Merge algebra as in efficient_entropy_triton_kernel_epilogue (fused_linear_logprob_triton.py:417-467) except that
 // the running max starts at -inf (that kernel starts it at 0, which loses rows whose logits are all << 0).
 // Out-of-range labels give logprob 0 (model_utils.py:337; fused_linear_logprob_triton.py:1898-1905).
