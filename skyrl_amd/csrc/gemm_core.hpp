@@ -88,7 +88,7 @@ typedef f32x4 acc_t[TM][TN];
 // operand that changes alternates A, B, A, B.  With random data the matrix pipe is power-limited and the order is
 // measurable: a loop of nothing but MFMAs runs 2 % faster in this order than in a row-by-row serpentine (the A fragment
 // kept for eight MFMAs), 6 % faster than in an order that changes both operands every time; on zeros all orders tie.
-// N: columns of the grid, 8 or (narrow tiles) 4.
+// N: columns of the grid, 8 or (the other shapes of a tile) 4 or 6.
 template <int N = TN>
 __host__ __device__ constexpr int mfma_row(int x) { return (x / (2 * N)) * 2 + ((x % (2 * N) + 1) / 2) % 2; }
 template <int N = TN>
@@ -101,15 +101,18 @@ constexpr int free_gap(int x, int n) {
     if (g % 8 != 5 && n-- == 0) return g;
 }
 
-// Shapes of a tile.  Narrow, 256 x 128: for the last tokens of a call where they are no more than that.  Short, 128 x 256, the four waves
-// side by side along N: for the last tiles of a launch where they would leave most CUs idle (split_last_round).  Both have half of the MFMAs and three quarters
-// of the copies of a square tile, and a wave's share of them is 128 x 64.
-enum { kSquare = 0, kNarrow = 1, kShort = 2 };
+// Shapes of a tile.  Narrow, 256 x 128, and medium, 256 x 192: for the last tokens of a call where they are no more than that.  Short, 128 x 256,
+// the four waves side by side along N: for the last tiles of a launch where they would leave most CUs idle (split_last_round).  Narrow and short
+// ones have half of the MFMAs and three quarters of the copies of a square tile, and a wave's share of them is 128 x 64; medium ones three
+// quarters and seven eighths, and 128 x 96.
+enum { kSquare = 0, kNarrow = 1, kShort = 2, kMedium = 3 };
 __host__ __device__ constexpr int waves_n(int shape) { return shape == kShort ? NWAVES : WAVES_N; }
-__host__ __device__ constexpr int wave_cols(int shape) { return shape == kSquare ? TN : TN / 2; }  // blocks of 16 along N per wave
+__host__ __device__ constexpr int wave_cols(int shape) { return shape == kSquare ? TN : shape == kMedium ? TN * 3 / 4 : TN / 2; }  // blocks of 16 along N per wave
 // Copies per lane and k-tile: one per 32 rows of the operand.
 __host__ __device__ constexpr int a_copies(int shape) { return shape == kShort ? COPIES_PER_OPERAND / 2 : COPIES_PER_OPERAND; }
-__host__ __device__ constexpr int b_copies(int shape) { return shape == kNarrow ? COPIES_PER_OPERAND / 2 : COPIES_PER_OPERAND; }
+__host__ __device__ constexpr int b_copies(int shape) {
+  return shape == kNarrow ? COPIES_PER_OPERAND / 2 : shape == kMedium ? COPIES_PER_OPERAND * 3 / 4 : COPIES_PER_OPERAND;
+}
 
 struct Operand {
   const uint16_t* ptr;  // bf16 bits, row-major, K contiguous
@@ -312,9 +315,10 @@ __device__ __forceinline__ void prefetch_first_tiles(const Operand& a, const Ope
 // MFMA order inside a step: mfma_row() / mfma_col() above (every fragment of the step is in registers before the step
 // starts, so the order is free to serve the power budget).
 //
-// Half shapes: a step is 32 MFMAs, with a copy behind every fourth (of the operand with 256 rows) or every eighth; what bounds them is the
-// copies.  Narrow, forward, V=151936, all tiles square -> the last one narrow: 132 -> 114 us at T=300, H=896, 252 -> 221 at T=384, H=2048,
-// 468 -> 432 at T=1100, H=1536; training pass 958 -> 925 at T=611, H=1536.  Beyond 128 tokens in the last tile a square one is made.
+// Other shapes: a step is 32 or 48 MFMAs, with a copy behind every fourth, sixth or eighth; what bounds them is the copies.  Narrow, forward,
+// V=151936, all tiles square -> the last one narrow: 132 -> 114 us at T=300, H=896, 252 -> 221 at T=384, H=2048, 468 -> 432 at T=1100, H=1536;
+// training pass 958 -> 925 at T=611, H=1536.  Medium, square -> medium: 84 -> 75 us at T=137, H=896, 461 -> 445 at T=1200, H=1536, training
+// pass 778 -> 751 at T=440, H=2048, V=100000.
 template <bool BKM = false, int SHAPE = kSquare>
 __device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand& b, int k_begin, int nk, char* lds,
                                                 f32x4 (&acc)[TM][wave_cols(SHAPE)]) {
@@ -425,8 +429,8 @@ __device__ __forceinline__ void mainloop_ksteps(const Operand& a, const Operand&
     // read of the step (which still uses the old value) that carry neither a read nor a copy.
     constexpr int kMfmas = TM * N;
     constexpr int kAddX0 = BKM ? 2 * READS_PER_STEP - 1 : 41;
-    constexpr int kGapA = N == TN ? free_gap(kAddX0, 0) : 24;
-    constexpr int kGapB[4] = {N == TN ? free_gap(kAddX0, 1) : 26, free_gap(kAddX0, 2), free_gap(kAddX0, 3), free_gap(kAddX0, 4)};
+    constexpr int kGapA = N == TN ? free_gap(kAddX0, 0) : 2 * READS_PER_STEP;
+    constexpr int kGapB[4] = {N == TN ? free_gap(kAddX0, 1) : 2 * READS_PER_STEP + 2, free_gap(kAddX0, 2), free_gap(kAddX0, 3), free_gap(kAddX0, 4)};
     static_assert(2 * READS_PER_STEP <= (N == TN ? kMfmas : kGapA) && kGapB[NB - 1] < kMfmas, "reads and address adds must fit the step");
     // MFMAs between the copies of an operand, and where: gaps that carry no fragment read
     constexpr int kAPeriod = kMfmas / a_copies(SHAPE), kBPeriod = kMfmas / b_copies(SHAPE);

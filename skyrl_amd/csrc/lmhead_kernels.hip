@@ -54,9 +54,9 @@ __host__ __device__ inline int64_t round_up(int64_t x, int64_t m) { return (x + 
 // An even number of k-tiles selects the accumulator-stationary mainloop (the EVEN instantiation of a tile kernel).
 inline bool even_ktiles(int64_t contraction) { return (contraction / BK) % 2 == 0; }
 
-// Whether a launch of tiles_m x ceil(T / 256) tiles has narrow or short ones among them.  The branches to them are compiled into kernels of
+// Whether a launch of tiles_m x ceil(T / 256) tiles has others than square ones among them.  The branches to them are compiled into kernels of
 // their own: they cost launches of whole tiles half a percent (T=2048, H=896, V=151936: 485 -> 488 us).
-inline bool has_half_tiles(int64_t T, int split) { return split > 0 || (T % BN > 0 && T % BN <= BN / 2); }
+inline bool has_other_shapes(int64_t T, int split) { return split > 0 || (T % BN > 0 && T % BN <= BN * 3 / 4); }
 // pick(x, y, z) for the three flags as compile-time constants.
 template <class Pick>
 auto flagged_kernel(Pick pick, bool x, bool y, bool z) {
@@ -79,14 +79,14 @@ static __device__ __align__(256) unsigned char static_scratch[kStaticScratchByte
 // The label-logit gather of that kernel (:364-385) is done in lmhead_fwd_merge instead.
 // ------------------------------------------------------------------------------------------------------------
 // EVEN: H / 64 is even, which selects the accumulator-stationary mainloop (gemm_core.hpp).
-// HALVES: some tiles are narrow or short (has_half_tiles()); split: how many tiles are made as short ones.
-template <bool ENTROPY, bool PAIRED, bool EVEN, bool HALVES>
+// SHAPES: some tiles are not square (has_other_shapes()); split: how many of them are made as short ones.
+template <bool ENTROPY, bool PAIRED, bool EVEN, bool SHAPES>
 __device__ __forceinline__ void fwd_tile(const uint16_t* __restrict__ W, int ldw, const uint16_t* __restrict__ Hd, int ldh, int T,
                                          int H, int V, float rcp_temp, float* __restrict__ part_max,
                                          float* __restrict__ part_sum, float* __restrict__ part_pz, int split, char* lds) {
   const int tiles_m = (V + BM - 1) / BM;
   const int tiles_n = (T + BN - 1) / BN;
-  const Tile t = tile_of<false, HALVES>(blockIdx.x, tiles_m, tiles_n, kGroupM, split);
+  const Tile t = tile_of<false, SHAPES>(blockIdx.x, tiles_m, tiles_n, kGroupM, split);
   const int wave = threadIdx.x >> 6;
   auto tile = [&](auto shape, int v0) {  // the tile of that shape from vocabulary row v0 on
     constexpr int SHAPE = decltype(shape)::value;
@@ -103,23 +103,25 @@ __device__ __forceinline__ void fwd_tile(const uint16_t* __restrict__ W, int ldw
     fwd_epilogue<ENTROPY, PAIRED>(acc, part, tiles_m * WAVES_M, t0, T, V, rcp_temp, part_max, part_sum, part_pz);
 #endif
   };
-  if constexpr (HALVES) {
-    if (narrow_tile(t.tn, T)) {  // of the two workgroups of a split tile the first makes it
+  if constexpr (SHAPES) {
+    const int shape = shape_of_tile(t.tn, T);
+    if (shape == kNarrow) {  // of the two workgroups of a split tile the first makes it
       if (t.half < 1) tile(std::integral_constant<int, kNarrow>{}, t.tm * BM);
       return;
     }
     if (t.half >= 0) return tile(std::integral_constant<int, kShort>{}, t.tm * BM + t.half * WM);
+    if (shape == kMedium) return tile(std::integral_constant<int, kMedium>{}, t.tm * BM);
   }
   tile(std::integral_constant<int, kSquare>{}, t.tm * BM);
 }
 
-template <bool ENTROPY, bool EVEN, bool HALVES>
+template <bool ENTROPY, bool EVEN, bool SHAPES>
 __global__ __launch_bounds__(NTHREADS) void lmhead_fwd_tiles(const uint16_t* __restrict__ W, int ldw,
                                                              const uint16_t* __restrict__ Hd, int ldh, int T, int H, int V,
                                                              float rcp_temp, float* __restrict__ part_max,
                                                              float* __restrict__ part_sum, float* __restrict__ part_pz, int split) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  fwd_tile<ENTROPY, false, EVEN, HALVES>(W, ldw, Hd, ldh, T, H, V, rcp_temp, part_max, part_sum, part_pz, split, lds);
+  fwd_tile<ENTROPY, false, EVEN, SHAPES>(W, ldw, Hd, ldh, T, H, V, rcp_temp, part_max, part_sum, part_pz, split, lds);
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -267,13 +269,13 @@ __global__ __launch_bounds__(kMergeThreads) void lmhead_fwd_merge(const float* _
   if (row_pz) row_pz[t] = RELATIVE ? lse - third : third;
 }
 
-// The dz tiles (logits_tile.hpp) on square, narrow and short products.
-template <bool ENTGRAD, bool EVEN, bool HALVES>
+// The dz tiles (logits_tile.hpp) on products of any shape.
+template <bool ENTGRAD, bool EVEN, bool SHAPES>
 __device__ __forceinline__ void dz_square_tile(const DzArgs& z, int id, char* lds) {
   static_assert(NWAVES * WN * (kDzTokRow + kDzTokBytes) <= LDS_BYTES, "dz staging and per-token values do not fit LDS");
   int T;
   Tile t;
-  if (!dz_tile_of<HALVES>(z, id, BN, T, t)) return;
+  if (!dz_tile_of<SHAPES>(z, id, BN, T, t)) return;
   auto tile = [&](auto shape, int col0) {
     constexpr int SHAPE = decltype(shape)::value;
     dz_tile<ENTGRAD, wave_cols(SHAPE), SHAPE == kShort>(
@@ -293,12 +295,14 @@ __device__ __forceinline__ void dz_square_tile(const DzArgs& z, int id, char* ld
 #endif
         });
   };
-  if constexpr (HALVES) {
-    if (narrow_tile(t.tn, T)) {  // of the two workgroups of a split tile the first makes it
+  if constexpr (SHAPES) {
+    const int shape = shape_of_tile(t.tn, T);
+    if (shape == kNarrow) {  // of the two workgroups of a split tile the first makes it
       if (t.half < 1) tile(std::integral_constant<int, kNarrow>{}, t.tm * BM);
       return;
     }
     if (t.half >= 0) return tile(std::integral_constant<int, kShort>{}, t.tm * BM + t.half * WM);
+    if (shape == kMedium) return tile(std::integral_constant<int, kMedium>{}, t.tm * BM);
   }
   tile(std::integral_constant<int, kSquare>{}, t.tm * BM);
 }
@@ -726,10 +730,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bid, char* lds)
 
 // The two kinds of backward launch per vocab chunk, as kernels of their own so that a kernel trace tells them apart:
 // the dz tiles of the chunk, then its two gradient GEMMs in one launch (workgroups [0, tiles0) work on p0, the rest on p1).
-template <bool ENTGRAD, bool EVEN, bool HALVES>
+template <bool ENTGRAD, bool EVEN, bool SHAPES>
 __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_dz(const DzArgs z) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  dz_square_tile<ENTGRAD, EVEN, HALVES>(z, blockIdx.x, lds);
+  dz_square_tile<ENTGRAD, EVEN, SHAPES>(z, blockIdx.x, lds);
 }
 
 __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_gemm(const GemmArgs p0, const GemmArgs p1, int tiles0) {
@@ -1313,8 +1317,8 @@ int fwd_token_blocks(const void* hidden, int64_t ld_hidden, const void* weight, 
     {
       Timed timed(kFwdTiles, s);
       auto kernel = flagged_kernel(
-          [](auto pz, auto even, auto halves) { return &lmhead_fwd_tiles<pz.value, even.value, halves.value>; }, want_pz, even_ktiles(H),
-          has_half_tiles(Tb, split));
+          [](auto pz, auto even, auto shapes) { return &lmhead_fwd_tiles<pz.value, even.value, shapes.value>; }, want_pz, even_ktiles(H),
+          has_other_shapes(Tb, split));
       if (half)
         launch_fwd_half_tiles(s, want_pz, Wp, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)H, (int)V, rcp_temperature, pmax, psum, ppz);
       else
@@ -1469,8 +1473,8 @@ hipError_t launch_bwd_dz(hipStream_t s, bool entgrad, DzArgs z) {
   const int tiles = z.tiles_m * z.tiles_n;
   // A count that only the device knows may leave any remainder, and any number of tiles up to these.
   const int split = z.T_dev ? (tiles < z.ncu / 2 ? tiles : z.ncu / 2) : split_last_round(tiles, z.ncu);
-  auto kernel = flagged_kernel([](auto ent, auto even, auto halves) { return &lmhead_bwd_dz<ent.value, even.value, halves.value>; },
-                               entgrad, even_ktiles(z.H), z.T_dev != nullptr || has_half_tiles(z.T, split));
+  auto kernel = flagged_kernel([](auto ent, auto even, auto shapes) { return &lmhead_bwd_dz<ent.value, even.value, shapes.value>; },
+                               entgrad, even_ktiles(z.H), z.T_dev != nullptr || has_other_shapes(z.T, split));
   hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles + split)), dim3(NTHREADS), 0, s, z);
   return hipGetLastError();
 }
@@ -2098,11 +2102,11 @@ int skyrl_lmhead_topk_logits(const void* hidden, int64_t ld_hidden, const void* 
     };
     auto launch_tiles = [&](bool first, const topk::FilterArgs& a) {
       auto kernel = flagged_kernel(
-          [](auto first, auto even, auto halves) {
-            if constexpr (first.value) return &topk::topk_first_tiles<even.value, halves.value>;
-            else return &topk::topk_filter_tiles<even.value, halves.value>;
+          [](auto first, auto even, auto shapes) {
+            if constexpr (first.value) return &topk::topk_first_tiles<even.value, shapes.value>;
+            else return &topk::topk_filter_tiles<even.value, shapes.value>;
           },
-          first, even_ktiles(H), has_half_tiles(Tb, a.split));
+          first, even_ktiles(H), has_other_shapes(Tb, a.split));
       Timed timed(kTopkFilter, s);
       hipLaunchKernelGGL(kernel, dim3((unsigned)(a.tiles_m * a.tiles_n + a.split)), dim3(NTHREADS), 0, s, a);
       return hipGetLastError();

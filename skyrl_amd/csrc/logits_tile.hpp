@@ -78,8 +78,11 @@ __device__ __forceinline__ void fwd_tile_stats(const f32x4 (&acc)[TM][N], int j,
   e_out = PAIRED ? e * scale2 * kLn2 : e * kLn2;
 }
 
-// Whether token tile tn of 256, the last one, holds at most 128 of a call's T tokens: it is then made half as wide (kNarrow).
-__device__ __forceinline__ bool narrow_tile(int tn, int T) { return __builtin_amdgcn_readfirstlane((int)(T - tn * BN <= BN / 2)); }
+// The shape of token tile tn of 256, by how many of a call's T tokens it holds.
+__device__ __forceinline__ int shape_of_tile(int tn, int T) {
+  const int rest = __builtin_amdgcn_readfirstlane(T - tn * BN);
+  return rest <= BN / 2 ? kNarrow : rest <= BN * 3 / 4 ? kMedium : kSquare;
+}
 
 // Statistics of a wave's accumulators, those of part `part` (vocabulary rows 128 * part .. + 127, of nparts parts) and of the N token blocks
 // from token t0 on, into the partials.
@@ -221,7 +224,7 @@ __device__ __forceinline__ void dz_tile(const DzArgs& z, int T, int col0, int t0
   // `t < T` becomes a branch with its own wait: one memory round trip per token block before the first copy is issued).  Lane
   // l loads tokens l and (square tiles) 64 + l of the wave's -- twelve registers to carry through the mainloop -- and the values reach
   // the lanes that need them (token j * 16 + lrow for every token block j) through LDS afterwards.
-  constexpr int NU = WAVE_N / 64;
+  constexpr int NU = (WAVE_N + 63) / 64;
   float g_[NU], q_[NU], lse_[NU], pz_[NU];
   int64_t y_[NU];
 #pragma unroll
@@ -249,6 +252,7 @@ __device__ __forceinline__ void dz_tile(const DzArgs& z, int T, int col0, int t0
   char* tokv = lds + NWAVES * kStage + wave * kTokBytes;  // float4 {g, q, lse, pz} per token, then the int64 labels
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
+    if (u * 64 + lane >= WAVE_N) break;
     const f32x4 v = {g_[u], q_[u], lse_[u], pz_[u]};
     *(f32x4*)(tokv + (u * 64 + lane) * 16) = v;
     *(int64_t*)(tokv + WAVE_N * 16 + (u * 64 + lane) * 8) = y_[u];
@@ -359,6 +363,17 @@ __device__ __forceinline__ void dz_tile(const DzArgs& z, int T, int col0, int t0
     for (int j = 0; j < NB; ++j) token_block(j, yes, yes);
   }
   flush_block(NB - 1);
+  // The products behind the panel run over whole groups of 128 tokens: a medium tile, whose tokens end in its second group, leaves zeros in
+  // what remains of that.
+  constexpr int kRest = WAVE_N * WAVES_N % 128 > 0 ? 128 - WAVE_N * WAVES_N % 128 : 0;
+  if constexpr (kRest > 0) {
+    uint16_t* zero_row = D + (size_t)(t0 + WAVES_N * WAVE_N + wn * (kRest / WAVES_N) + (lane >> 4)) * (size_t)ldd + vloc_base + (lane & 15) * 8;
+#pragma unroll
+    for (int it = 0; it < kRest / WAVES_N / 4; ++it) {
+      store(u32x4{0u, 0u, 0u, 0u}, (u32x4*)zero_row);
+      zero_row += d_step;
+    }
+  }
 }
 
 }  // namespace lmhead

@@ -157,30 +157,32 @@ __device__ __forceinline__ void topk_tile(const FilterArgs& a, int vtile, int tt
   }
 }
 
-template <bool DENSE, bool EVEN, bool HALVES>
+template <bool DENSE, bool EVEN, bool SHAPES>
 __device__ __forceinline__ void topk_tile_of_workgroup(const FilterArgs& a, char* lds) {
-  const Tile t = tile_of<false, HALVES>(blockIdx.x, a.tiles_m, a.tiles_n, a.group_m, a.split);
+  const Tile t = tile_of<false, SHAPES>(blockIdx.x, a.tiles_m, a.tiles_n, a.group_m, a.split);
   const int v = t.tm * BM, n = t.tn * BN;
-  if constexpr (HALVES) {
-    if (narrow_tile(t.tn, a.T)) {
+  if constexpr (SHAPES) {
+    const int shape = shape_of_tile(t.tn, a.T);
+    if (shape == kNarrow) {  // of the two workgroups of a split tile the first makes it
       if (t.half < 1) topk_tile<DENSE, EVEN, kNarrow>(a, v, n, lds);
       return;
     }
     if (t.half >= 0) return topk_tile<DENSE, EVEN, kShort>(a, v + t.half * WM, n, lds);
+    if (shape == kMedium) return topk_tile<DENSE, EVEN, kMedium>(a, v, n, lds);
   }
   topk_tile<DENSE, EVEN, kSquare>(a, v, n, lds);
 }
 
-template <bool EVEN, bool HALVES>
+template <bool EVEN, bool SHAPES>
 __global__ __launch_bounds__(NTHREADS) void topk_first_tiles(const FilterArgs a) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  topk_tile_of_workgroup<true, EVEN, HALVES>(a, lds);
+  topk_tile_of_workgroup<true, EVEN, SHAPES>(a, lds);
 }
 
-template <bool EVEN, bool HALVES>
+template <bool EVEN, bool SHAPES>
 __global__ __launch_bounds__(NTHREADS) void topk_filter_tiles(const FilterArgs a) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  topk_tile_of_workgroup<false, EVEN, HALVES>(a, lds);
+  topk_tile_of_workgroup<false, EVEN, SHAPES>(a, lds);
 }
 
 // Smallest key of the wave's values, in every lane.

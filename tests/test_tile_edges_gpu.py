@@ -396,9 +396,9 @@ def test_draft_loss_backward_with_less_scratch(T, H, V, vc, cuda_device):
     assert call(least // 2)[0] == ERR_WORKSPACE and (vc > 256 or call(least - 1)[0] == ERR_WORKSPACE)
 
 
-# The last token tile is made half as wide where it holds no more than 128 tokens.  A token's values do not depend on the width of its
+# The last token tile is made narrower where it holds no more than 128 or 192 tokens.  A token's values do not depend on the width of its
 # tile: the last tokens of a call are compared, bit for bit, with those of a longer call in whole tiles.
-@pytest.mark.parametrize("T", [257, 319, 320, 384, 385, 513])
+@pytest.mark.parametrize("T", [257, 319, 320, 384, 385, 447, 448, 449, 513])
 @pytest.mark.parametrize("H,V", [(64, 1153), (128, 5001), (192, 777), (320, 2304)])
 def test_last_tokens_in_a_narrow_tile(T, H, V, cuda_device):
     t = 0.8
