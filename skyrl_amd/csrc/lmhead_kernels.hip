@@ -54,9 +54,22 @@ __host__ __device__ inline int64_t round_up(int64_t x, int64_t m) { return (x + 
 // An even number of k-tiles selects the accumulator-stationary mainloop (the EVEN instantiation of a tile kernel).
 inline bool even_ktiles(int64_t contraction) { return (contraction / BK) % 2 == 0; }
 
-// Whether a launch of tiles_m x ceil(T / 256) tiles has others than square ones among them.  The branches to them are compiled into kernels of
-// their own: they cost launches of whole tiles half a percent (T=2048, H=896, V=151936: 485 -> 488 us).
-inline bool has_other_shapes(int64_t T, int split) { return split > 0 || (T % BN > 0 && T % BN <= BN * 3 / 4); }
+// Whether a launch of tiles_m x ceil(T / 256) tiles makes others than square ones, and how many of them as short ones.  The branches to them
+// are compiled into kernels of their own, because they cost every tile about half a k-tile's time (V=151936; T=8192, H=896, where they save
+// 0.4 of 75 rounds: 1768 us without them, 1796 with; T=20608, H=1536: 6688 and 6692 to 6724).  What they save, 0.4 or 0.2 of a tile in the
+// last token column (128 or 192 tokens) and 0.4 of a round at the end, has to be more than that; a square tile takes H / 64 + 5 k-tiles' time.
+struct TileShapes {
+  bool used;
+  int split;
+};
+inline bool shapes_pay(int64_t tenths_saved, int64_t H, int64_t tiles) { return tenths_saved * (H / BK + 5) > 5 * tiles; }
+inline TileShapes tile_shapes(int64_t T, int64_t H, int tiles_m, int ncu) {
+  const int64_t tiles = (T + BN - 1) / BN * tiles_m, rest = T % BN;
+  const int split = split_last_round((int)tiles, ncu);
+  const int64_t tenths = (rest == 0 || rest > BN * 3 / 4 ? 0 : rest > BN / 2 ? 2 : 4) * tiles_m + (split > 0 ? 4 * ncu : 0);
+  const bool used = shapes_pay(tenths, H, tiles);
+  return TileShapes{used, used ? split : 0};
+}
 // pick(x, y, z) for the three flags as compile-time constants.
 template <class Pick>
 auto flagged_kernel(Pick pick, bool x, bool y, bool z) {
@@ -79,7 +92,7 @@ static __device__ __align__(256) unsigned char static_scratch[kStaticScratchByte
 // The label-logit gather of that kernel (:364-385) is done in lmhead_fwd_merge instead.
 // ------------------------------------------------------------------------------------------------------------
 // EVEN: H / 64 is even, which selects the accumulator-stationary mainloop (gemm_core.hpp).
-// SHAPES: some tiles are not square (has_other_shapes()); split: how many of them are made as short ones.
+// SHAPES: some tiles are not square (tile_shapes()); split: how many of them are made as short ones.
 template <bool ENTROPY, bool PAIRED, bool EVEN, bool SHAPES>
 __device__ __forceinline__ void fwd_tile(const uint16_t* __restrict__ W, int ldw, const uint16_t* __restrict__ Hd, int ldh, int T,
                                          int H, int V, float rcp_temp, float* __restrict__ part_max,
@@ -1312,18 +1325,18 @@ int fwd_token_blocks(const void* hidden, int64_t ld_hidden, const void* weight, 
     float* psum = c.take<float>(part_elems(nparts, Tb));
     float* ppz = c.take<float>(part_elems(nparts, Tb));
     const uint16_t* Hp = (const uint16_t*)hidden + (size_t)t0 * (size_t)ld_hidden;
-    const int split = split_last_round(tiles_m * tiles_n, compute_units());
-    const dim3 grid((unsigned)(tiles_m * tiles_n + split)), block(NTHREADS);
+    const TileShapes shapes = tile_shapes(Tb, H, tiles_m, compute_units());
+    const dim3 grid((unsigned)(tiles_m * tiles_n + shapes.split)), block(NTHREADS);
     {
       Timed timed(kFwdTiles, s);
       auto kernel = flagged_kernel(
-          [](auto pz, auto even, auto shapes) { return &lmhead_fwd_tiles<pz.value, even.value, shapes.value>; }, want_pz, even_ktiles(H),
-          has_other_shapes(Tb, split));
+          [](auto pz, auto even, auto others) { return &lmhead_fwd_tiles<pz.value, even.value, others.value>; }, want_pz, even_ktiles(H),
+          shapes.used);
       if (half)
         launch_fwd_half_tiles(s, want_pz, Wp, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)H, (int)V, rcp_temperature, pmax, psum, ppz);
       else
         hipLaunchKernelGGL(kernel, grid, block, 0, s, Wp, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)H, (int)V,
-                         rcp_temperature, pmax, psum, ppz, split);
+                         rcp_temperature, pmax, psum, ppz, shapes.split);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
@@ -1471,11 +1484,16 @@ hipError_t launch_bwd_dz(hipStream_t s, bool entgrad, DzArgs z) {
   }
   z.tiles_n = (z.T + BN - 1) / BN;
   const int tiles = z.tiles_m * z.tiles_n;
-  // A count that only the device knows may leave any remainder, and any number of tiles up to these.
-  const int split = z.T_dev ? (tiles < z.ncu / 2 ? tiles : z.ncu / 2) : split_last_round(tiles, z.ncu);
-  auto kernel = flagged_kernel([](auto ent, auto even, auto shapes) { return &lmhead_bwd_dz<ent.value, even.value, shapes.value>; },
-                               entgrad, even_ktiles(z.H), z.T_dev != nullptr || has_other_shapes(z.T, split));
-  hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles + split)), dim3(NTHREADS), 0, s, z);
+  TileShapes shapes = tile_shapes(z.T, z.H, z.tiles_m, z.ncu);
+  if (z.T_dev) {
+    // A count that only the device knows may leave any remainder, and any number of tiles up to these: on the average over the remainders a
+    // quarter of a tile is saved in the last token column.
+    shapes.used = shapes_pay(10 * z.tiles_m / 4, z.H, tiles);
+    shapes.split = !shapes.used ? 0 : (tiles < z.ncu / 2 ? tiles : z.ncu / 2);
+  }
+  auto kernel = flagged_kernel([](auto ent, auto even, auto others) { return &lmhead_bwd_dz<ent.value, even.value, others.value>; },
+                               entgrad, even_ktiles(z.H), shapes.used);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles + shapes.split)), dim3(NTHREADS), 0, s, z);
   return hipGetLastError();
 }
 
@@ -2094,11 +2112,11 @@ int skyrl_lmhead_topk_logits(const void* hidden, int64_t ld_hidden, const void* 
     const int64_t Tb = (T - t0) < block_tokens ? (T - t0) : block_tokens;
     const int tiles_n = (int)((Tb + BN - 1) / BN);
     const uint16_t* Hp = (const uint16_t*)hidden + (size_t)t0 * (size_t)ld_hidden;
+    auto chunk_shapes = [&](int64_t vrows) { return tile_shapes(Tb, H, (int)((vrows + BM - 1) / BM), compute_units()); };
     auto chunk_args = [&](int64_t v0, int64_t vrows) {
       return topk::FilterArgs{Wp + (size_t)v0 * (size_t)ld_weight, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)H, (int)vrows,
                               (int)v0, rcp_temperature, (int)((vrows + BM - 1) / BM), tiles_n, kGroupM,
-                              split_last_round((int)((vrows + BM - 1) / BM) * tiles_n, compute_units()), w.thr, w.cnt, w.cand, (int)w.cap,
-                              (float*)w.cand};
+                              chunk_shapes(vrows).split, w.thr, w.cnt, w.cand, (int)w.cap, (float*)w.cand};
     };
     auto launch_tiles = [&](bool first, const topk::FilterArgs& a) {
       auto kernel = flagged_kernel(
@@ -2106,7 +2124,7 @@ int skyrl_lmhead_topk_logits(const void* hidden, int64_t ld_hidden, const void* 
             if constexpr (first.value) return &topk::topk_first_tiles<even.value, shapes.value>;
             else return &topk::topk_filter_tiles<even.value, shapes.value>;
           },
-          first, even_ktiles(H), has_other_shapes(Tb, a.split));
+          first, even_ktiles(H), chunk_shapes(a.vrows).used);
       Timed timed(kTopkFilter, s);
       hipLaunchKernelGGL(kernel, dim3((unsigned)(a.tiles_m * a.tiles_n + a.split)), dim3(NTHREADS), 0, s, a);
       return hipGetLastError();

@@ -54,7 +54,7 @@ struct FilterArgs {
   int v0;              // column number of the chunk's first row
   float rcp_temp;
   int tiles_m, tiles_n, group_m;
-  int split;           // how many of the tiles are made as short ones (split_last_round)
+  int split;           // how many of the tiles are made as short ones (tile_shapes)
   const float* thr;    // [T] threshold per token, -inf while fewer than k columns have been seen
   unsigned* cnt;       // [T] candidates appended in this launch
   key_t* cand;         // [T, cap]
