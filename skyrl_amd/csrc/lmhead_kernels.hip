@@ -70,6 +70,12 @@ inline TileShapes tile_shapes(int64_t T, int64_t H, int tiles_m, int ncu) {
   const bool used = shapes_pay(tenths, H, tiles);
   return TileShapes{used, used ? split : 0};
 }
+// The same for a count of tokens that only the device knows: it may leave any remainder, and any number of tiles up to these.  On the average
+// over the remainders a quarter of a tile is saved in the last token column.
+inline TileShapes tile_shapes_of_any_count(int64_t H, int tiles_m, int tiles, int ncu) {
+  const bool used = shapes_pay(10 * tiles_m / 4, H, tiles);
+  return TileShapes{used, !used ? 0 : tiles < ncu / 2 ? tiles : ncu / 2};
+}
 // pick(x, y, z) for the three flags as compile-time constants.
 template <class Pick>
 auto flagged_kernel(Pick pick, bool x, bool y, bool z) {
@@ -325,18 +331,21 @@ __device__ __forceinline__ void dz_square_tile(const DzArgs& z, int id, char* ld
 // soft_ce.py:200-240):  loss[t] = -sum_v softmax(z_teacher[t])_v * log_softmax(z_student[t])_v = lse_student - E_teacher[z_student],
 // both logits rows being products with the same (detached) output weight.  The reference materialises both [T, V] logits
 // tensors and their fp32 softmaxes; here the two hidden rows of a token sit in one "stacked" operand so that one lane
-// holds z_student and z_teacher of the same (token, vocab) pair, TN / 2 accumulator blocks apart:
-//   stacked row of token t:   student  (t / 64) * 128 + t % 64,   teacher  (t / 64) * 128 + 64 + t % 64
-// i.e. each wave's 128 token rows are 64 student rows followed by the 64 teacher rows of the same tokens.  The forward
-// is the ordinary tile kernel on the stacked rows with the paired third statistic; the backward recomputes a tile and
-// writes  d loss / d z_student = g * (softmax(z_student) - softmax(z_teacher))  (soft_ce.py:146-151) for the student rows
+// holds z_student and z_teacher of the same (token, vocab) pair, one accumulator block apart:
+//   stacked row of token t:   student  (t / 16) * 32 + t % 16,   teacher  (t / 16) * 32 + 16 + t % 16
+// i.e. a wave's token blocks are in turn 16 student rows and the 16 teacher rows of the same tokens, so that a tile of any shape
+// holds whole pairs and calls of few tokens use them (V=151936, forward and backward, square tiles -> this: 389 -> 341 us at T=16, H=1536;
+// 557 -> 521 at T=137, H=2048; 7.27 -> 7.23 ms at T=4096, where all tiles are square).  The forward
+// is the ordinary tile kernel on the stacked rows with the paired third statistic; the backward recomputes a tile and writes
+//   d loss / d z_student = g * (softmax(z_student) - softmax(z_teacher))  (soft_ce.py:146-151) for the student rows
 // into the token-major dz panel, from which the ordinary dHidden GEMM runs.  The weight gets no gradient (it is detached
 // in the reference, mtp/adapter.py:51-56), neither does the teacher.
 // ------------------------------------------------------------------------------------------------------------
-constexpr int kPairRows = WN / 2;  // 64 tokens per wave
+constexpr int kPairRows = MT;
+__host__ __device__ inline int stacked_rows(int T) { return (T + kPairRows - 1) / kPairRows * (2 * kPairRows); }
 
 __host__ __device__ inline int64_t stacked_row(int64_t t, bool teacher) {
-  return (t / kPairRows) * WN + (teacher ? kPairRows : 0) + t % kPairRows;
+  return (t / kPairRows) * (2 * kPairRows) + (teacher ? kPairRows : 0) + t % kPairRows;
 }
 
 // One workgroup per stacked row: copies the student's or the teacher's hidden row, zeros for the padding tokens.
@@ -354,7 +363,7 @@ __global__ __launch_bounds__(256) void softce_pack_rows(const uint16_t* __restri
                                                         int shift, int H, uint16_t* __restrict__ stacked) {
   const int r = blockIdx.x;
   const bool is_teacher = (r / kPairRows) & 1;
-  const int t = (r / WN) * kPairRows + r % kPairRows;
+  const int t = r / (2 * kPairRows) * kPairRows + r % kPairRows;
   const uint16_t* src = t < T ? softce_source_row(t, is_teacher, student, lds_, teacher, ldt, seq_len, shift) : nullptr;
   uint16_t* dst = stacked + (size_t)r * (size_t)H;
   for (int c = threadIdx.x * 8; c < H; c += 256 * 8)
@@ -362,7 +371,7 @@ __global__ __launch_bounds__(256) void softce_pack_rows(const uint16_t* __restri
 }
 
 // The same for the backward, which runs on the tokens with an upstream gradient only (compact_active_rows: idx, counts): stacked
-// rows and per-token inputs of compacted token t are those of token idx[t].  Rows beyond the last tile that holds a token are
+// rows and per-token inputs of compacted token t are those of token idx[t].  Rows beyond the last 16 tokens that hold one are
 // not written.  As student row, token t also clears d_student[t]; active tokens get their row from the dHidden GEMM.
 __global__ __launch_bounds__(256) void softce_gather_rows(const uint16_t* __restrict__ student, int lds_,
                                                           const uint16_t* __restrict__ teacher, int ldt, int T, int seq_len,
@@ -374,12 +383,12 @@ __global__ __launch_bounds__(256) void softce_gather_rows(const uint16_t* __rest
                                                           uint16_t* __restrict__ d_student) {
   const int r = blockIdx.x;
   const bool is_teacher = (r / kPairRows) & 1;
-  const int t = (r / WN) * kPairRows + r % kPairRows, n = counts[0];
+  const int t = r / (2 * kPairRows) * kPairRows + r % kPairRows, n = counts[0];
   if (!is_teacher && t < T) {
     uint16_t* zero_row = d_student + (size_t)t * (size_t)H;
     for (int c = threadIdx.x * 8; c < H; c += 256 * 8) *(uint4*)(zero_row + c) = make_uint4(0, 0, 0, 0);
   }
-  if (t >= (n + BN / 2 - 1) / (BN / 2) * (BN / 2)) return;
+  if (r >= stacked_rows(n)) return;
   const uint16_t* src = nullptr;
   if (t < n) {
     const int token = idx[t];
@@ -392,13 +401,13 @@ __global__ __launch_bounds__(256) void softce_gather_rows(const uint16_t* __rest
     *(uint4*)(dst + c) = src ? *(const uint4*)(src + c) : make_uint4(0, 0, 0, 0);
 }
 
-template <bool ENTROPY, bool EVEN>
+template <bool EVEN, bool SHAPES>
 __global__ __launch_bounds__(NTHREADS) void softce_fwd_tiles(const uint16_t* __restrict__ W, int ldw,
                                                              const uint16_t* __restrict__ Hd, int ldh, int T, int H, int V,
                                                              float rcp_temp, float* __restrict__ part_max,
-                                                             float* __restrict__ part_sum, float* __restrict__ part_pz) {
+                                                             float* __restrict__ part_sum, float* __restrict__ part_pz, int split) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
-  fwd_tile<ENTROPY, true, EVEN, false>(W, ldw, Hd, ldh, T, H, V, rcp_temp, part_max, part_sum, part_pz, 0, lds);
+  fwd_tile<true, true, EVEN, SHAPES>(W, ldw, Hd, ldh, T, H, V, rcp_temp, part_max, part_sum, part_pz, split, lds);
 }
 
 // Per token: the merged statistics of its two stacked rows -> loss and the two log-sum-exps the backward needs.
@@ -417,69 +426,65 @@ __global__ __launch_bounds__(256) void softce_finish(const float* __restrict__ r
 struct SoftCeDzArgs {
   const uint16_t* W;
   int ldw;
-  const uint16_t* S;  // stacked hidden rows [2 * Tp, H], Tp = T rounded up to whole 128-token tiles
-  int Tp, H, V;
-  const int* T_dev;   // the number of tokens, <= Tp, counted on the device; token tiles beyond it return at once
+  const uint16_t* S;  // stacked hidden rows [stacked_rows(tokens), H]
+  int H, V;
+  const int* T_dev;   // the number of tokens, counted on the device; token tiles beyond it return at once
   float rcp_temp;
   const float* lse_student;
   const float* lse_teacher;
   const float* dloss;
   int vc0, tiles_m, tiles_n;  // first vocab row of the chunk; tiles along the chunk's vocab rows and the stacked rows
   VocabTail tail;
-  uint16_t* D;                // [Tp, ldd]  dz of the student rows, token-major
+  uint16_t* D;                // [tokens rounded up to 128, ldd]  dz of the student rows, token-major; rows behind the last tile are not written
   int ldd;
+  int ncu;
 };
 
-template <bool EVEN>
-__global__ __launch_bounds__(NTHREADS) void softce_dz_tiles(const SoftCeDzArgs z) {
-  __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+// The tile of SHAPE from panel column col0 and token tok0 on, of T >= 1.
+template <bool EVEN, int SHAPE>
+__device__ __forceinline__ void softce_dz_tile(const SoftCeDzArgs& z, int T, int col0, int tok0, char* lds) {
+  constexpr int N = wave_cols(SHAPE), PAIRS = N / 2;  // a wave's token blocks, and those of its student rows
   const uint16_t* __restrict__ W = z.W;
-  const uint16_t* __restrict__ S = z.S;
-  const int T = __builtin_amdgcn_readfirstlane(*z.T_dev), H = z.H, V = z.V, vc0 = z.vc0, ldd = z.ldd;
+  const int V = z.V, vc0 = z.vc0, ldd = z.ldd;
   uint16_t* __restrict__ D = z.D;
-  const int tiles_n = (T + BN / 2 - 1) / (BN / 2);
-  if ((int)blockIdx.x >= z.tiles_m * tiles_n) return;
-  int tm, tn;
-  tile_coords(z.tiles_m * tiles_n - 1 - (int)blockIdx.x, z.tiles_m, tiles_n, kGroupM, tm, tn);  // as in dz_tile
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+  const int wm = wave / waves_n(SHAPE), wn = wave % waves_n(SHAPE);
   const int lrow = lane & 15, kq = lane >> 4;
-  const int vloc_base = tm * BM + wm * WM;
+  const int vloc_base = col0 + wm * WM;
   const WaveRows rows = wave_vocab_rows(vc0 + vloc_base, V, z.tail);
-  const int tokbase = (tn * WAVES_N + wn) * kPairRows;  // first token of this wave
+  const int tokbase = tok0 + wn * (PAIRS * MT);  // first token of this wave
   const bool full = rows.lo == 0 && rows.hi == WM;
   const float scale2 = z.rcp_temp * kLog2e;
 
   // Per-token inputs: unconditional loads from a clamped index, issued before the mainloop and first touched behind it (as
   // in dz_tile: a load under `t < T` is a branch with its own wait in front of the first copy).
-  float gs_[TN / 2], ls2_[TN / 2], lt2_[TN / 2];
+  float gs_[PAIRS], ls2_[PAIRS], lt2_[PAIRS];
 #pragma unroll
-  for (int j = 0; j < TN / 2; ++j) {
+  for (int j = 0; j < PAIRS; ++j) {
     const int t = tokbase + j * MT + lrow;
-    const int tc = t < T ? t : T - 1;  // T >= 1 here: a tile without a token has returned above
+    const int tc = t < T ? t : T - 1;
     gs_[j] = z.dloss[tc];
     ls2_[j] = z.lse_student[tc];
     lt2_[j] = z.lse_teacher[tc];
   }
 
-  const Operand a = dz_weight_rows(W, z.ldw, vc0 + tm * BM, V, z.tail);
-  Operand b{S, H, tn * BN, 2 * z.Tp};
-  acc_t acc;
-  prefetch_first_tiles(a, b, 0, H / BK, lds);  // the first copies travel while the accumulators are cleared
-  zero_acc(acc);
-  mainloop<false, EVEN>(a, b, 0, H / BK, lds, acc);
+  Operand a = dz_weight_rows(W, z.ldw, vc0 + col0, V, z.tail);
+  if (SHAPE == kShort && a.row0 >= V) a.row0 = V - 1;  // as in dz_tile
+  const Operand b{z.S, z.H, 2 * tok0, stacked_rows(T)};
+  f32x4 acc[TM][N];
+  tile_product<SHAPE, EVEN>(a, b, z.H / BK, lds, acc);
 #pragma unroll
-  for (int j = 0; j < TN / 2; ++j) {
+  for (int j = 0; j < PAIRS; ++j) {
     const bool valid = tokbase + j * MT + lrow < T;
     gs_[j] = valid ? gs_[j] * z.rcp_temp : 0.f;
     ls2_[j] = valid ? ls2_[j] * kLog2e : INFINITY;
     lt2_[j] = valid ? lt2_[j] * kLog2e : INFINITY;
   }
 
-  // Staging as in dz_tile: a private region per wave, 64 token rows of 128 vocab columns, then 16-byte non-temporal stores.
+  // Staging as in dz_tile: a private region per wave, its token rows of 128 vocab columns, then 16-byte non-temporal stores.
   constexpr int kTokRow = WM * 2 + 16;
-  constexpr int kStage = WN * kTokRow;
+  constexpr int kStage = PAIRS * MT * kTokRow;
   char* stage = lds + wave * kStage;
   auto flush_block = [&](int j) {  // as in dz_tile: a finished token block leaves while the next one is computed
 #pragma unroll
@@ -491,15 +496,15 @@ __global__ __launch_bounds__(NTHREADS) void softce_dz_tiles(const SoftCeDzArgs z
     }
   };
 #pragma unroll
-  for (int j = 0; j < TN / 2; ++j) {
+  for (int j = 0; j < PAIRS; ++j) {
     const float gs = gs_[j], ls2 = ls2_[j], lt2 = lt2_[j];
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       float d[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float q = __builtin_amdgcn_exp2f(fmaf(acc[i][j][r], scale2, -ls2));
-        const float p = __builtin_amdgcn_exp2f(fmaf(acc[i][j + TN / 2][r], scale2, -lt2));
+        const float q = __builtin_amdgcn_exp2f(fmaf(acc[i][2 * j][r], scale2, -ls2));
+        const float p = __builtin_amdgcn_exp2f(fmaf(acc[i][2 * j + 1][r], scale2, -lt2));
         d[r] = gs * (q - p);
       }
       const int vl = i * MT + kq * 4;
@@ -514,7 +519,28 @@ __global__ __launch_bounds__(NTHREADS) void softce_dz_tiles(const SoftCeDzArgs z
       if (i == TM / 2 - 1 && j > 0) flush_block(j - 1);
     }
   }
-  flush_block(TN / 2 - 1);
+  flush_block(PAIRS - 1);
+}
+
+template <bool EVEN, bool SHAPES>
+__global__ __launch_bounds__(NTHREADS) void softce_dz_tiles(const SoftCeDzArgs z) {
+  __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+  const int T = __builtin_amdgcn_readfirstlane(*z.T_dev);
+  const int tiles_n = (T + BN / 2 - 1) / (BN / 2);
+  const int split = SHAPES ? split_last_round(z.tiles_m * tiles_n, z.ncu) : 0;
+  if ((int)blockIdx.x >= z.tiles_m * tiles_n + split) return;
+  const Tile t = tile_of<true, SHAPES>(blockIdx.x, z.tiles_m, tiles_n, kGroupM, split);  // as in dz_tile_of
+  const int tok0 = t.tn * (BN / 2);
+  if constexpr (SHAPES) {
+    const int shape = shape_of_tile(t.tn, stacked_rows(T));
+    if (shape == kNarrow) {  // of the two workgroups of a split tile the first makes it
+      if (t.half < 1) softce_dz_tile<EVEN, kNarrow>(z, T, t.tm * BM, tok0, lds);
+      return;
+    }
+    if (t.half >= 0) return softce_dz_tile<EVEN, kShort>(z, T, t.tm * BM + t.half * WM, tok0, lds);
+    if (shape == kMedium) return softce_dz_tile<EVEN, kMedium>(z, T, t.tm * BM, tok0, lds);
+  }
+  softce_dz_tile<EVEN, kSquare>(z, T, t.tm * BM, tok0, lds);
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -1484,13 +1510,7 @@ hipError_t launch_bwd_dz(hipStream_t s, bool entgrad, DzArgs z) {
   }
   z.tiles_n = (z.T + BN - 1) / BN;
   const int tiles = z.tiles_m * z.tiles_n;
-  TileShapes shapes = tile_shapes(z.T, z.H, z.tiles_m, z.ncu);
-  if (z.T_dev) {
-    // A count that only the device knows may leave any remainder, and any number of tiles up to these: on the average over the remainders a
-    // quarter of a tile is saved in the last token column.
-    shapes.used = shapes_pay(10 * z.tiles_m / 4, z.H, tiles);
-    shapes.split = !shapes.used ? 0 : (tiles < z.ncu / 2 ? tiles : z.ncu / 2);
-  }
+  const TileShapes shapes = z.T_dev ? tile_shapes_of_any_count(z.H, z.tiles_m, tiles, z.ncu) : tile_shapes(z.T, z.H, z.tiles_m, z.ncu);
   auto kernel = flagged_kernel([](auto ent, auto even, auto others) { return &lmhead_bwd_dz<ent.value, even.value, others.value>; },
                                entgrad, even_ktiles(z.H), shapes.used);
   hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles + shapes.split)), dim3(NTHREADS), 0, s, z);
@@ -1604,7 +1624,7 @@ int check_softce(const void* student, int64_t lds_, const void* teacher, int64_t
 hipError_t launch_softce_pack(hipStream_t s, const void* student, int64_t lds_, const void* teacher, int64_t ldt, int64_t T,
                               int64_t seq_len, int64_t shift, int64_t H, uint16_t* S) {
   Timed timed(kSoftCePack, s);
-  hipLaunchKernelGGL(softce_pack_rows, dim3((unsigned)(2 * round_up(T, kPairTile))), dim3(256), 0, s, (const uint16_t*)student,
+  hipLaunchKernelGGL(softce_pack_rows, dim3((unsigned)stacked_rows((int)T)), dim3(256), 0, s, (const uint16_t*)student,
                      (int)lds_, (const uint16_t*)teacher, (int)ldt, (int)T, (int)seq_len, (int)(shift % seq_len), (int)H, S);
   return hipGetLastError();
 }
@@ -1983,16 +2003,18 @@ int skyrl_softce_fwd(const void* student_hidden, int64_t ld_student, const void*
 
   hipStream_t s = (hipStream_t)stream;
   const SoftCeFwdWorkspace w = carve_softce_fwd(workspace, T, H, V);
-  const int64_t rows = 2 * round_up(T, kPairTile);
+  const int64_t rows = stacked_rows((int)T);
   const uint16_t* Wp = (const uint16_t*)weight;
   hipError_t e = launch_softce_pack(s, student_hidden, ld_student, teacher_hidden, ld_teacher, T, seq_len, shift, H, w.S);
   if (e != hipSuccess) return (int)e;
-  const int tiles_m = (int)((V + BM - 1) / BM), tiles_n = (int)(rows / BN);
+  const int tiles_m = (int)((V + BM - 1) / BM), tiles_n = (int)((rows + BN - 1) / BN);
+  const TileShapes shapes = tile_shapes(rows, H, tiles_m, compute_units());
   {
     Timed timed(kSoftCeFwdTiles, s);
-    auto kernel = even_ktiles(H) ? softce_fwd_tiles<true, true> : softce_fwd_tiles<true, false>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(NTHREADS), 0, s, Wp, (int)ld_weight, w.S, (int)H,
-                       (int)rows, (int)H, (int)V, rcp_temperature, w.pmax, w.psum, w.ppz);
+    auto kernel = flagged_kernel([](auto, auto even, auto others) { return &softce_fwd_tiles<even.value, others.value>; }, true,
+                                 even_ktiles(H), shapes.used);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles_m * tiles_n + shapes.split)), dim3(NTHREADS), 0, s, Wp, (int)ld_weight, w.S, (int)H,
+                       (int)rows, (int)H, (int)V, rcp_temperature, w.pmax, w.psum, w.ppz, shapes.split);
   }
   if ((e = hipGetLastError()) != hipSuccess) return (int)e;
   {
@@ -2048,7 +2070,7 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
   if ((e = hipGetLastError()) != hipSuccess) return (int)e;
   {
     Timed timed(kSoftCePack, s);
-    hipLaunchKernelGGL(softce_gather_rows, dim3((unsigned)(2 * Tp)), dim3(256), 0, s, (const uint16_t*)student_hidden, (int)ld_student,
+    hipLaunchKernelGGL(softce_gather_rows, dim3((unsigned)stacked_rows((int)T)), dim3(256), 0, s, (const uint16_t*)student_hidden, (int)ld_student,
                        (const uint16_t*)teacher_hidden, (int)ld_teacher, (int)T, (int)seq_len, (int)(shift % seq_len), (int)H,
                        (const int*)w.idx, (const int*)w.counts, lse_student, lse_teacher, dloss, w.S, w.lse_student, w.lse_teacher,
                        w.dloss, (uint16_t*)d_student_hidden);
@@ -2064,12 +2086,15 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
   const GemmArgs none{};
   for (int64_t ci = 0; ci < nchunks; ++ci) {
     const int64_t vc0 = ci * vc, vcw = (Vpad - vc0) < vc ? (Vpad - vc0) : vc;
-    const SoftCeDzArgs z{Wp, (int)ld_weight, w.S, (int)Tp, (int)H, (int)V, w.counts + 1, rcp_temperature, w.lse_student,
-                         w.lse_teacher, w.dloss, (int)vc0, (int)(vcw / 256), (int)(2 * Tp / BN), tail, w.D, (int)(vcw + kLdPad)};
+    const SoftCeDzArgs z{Wp, (int)ld_weight, w.S, (int)H, (int)V, w.counts + 1, rcp_temperature, w.lse_student,
+                         w.lse_teacher, w.dloss, (int)vc0, (int)(vcw / 256), (int)(2 * Tp / BN), tail, w.D, (int)(vcw + kLdPad),
+                         compute_units()};
     {
       Timed timed(kSoftCeDz, s);
-      auto kernel = even_ktiles(H) ? softce_dz_tiles<true> : softce_dz_tiles<false>;
-      hipLaunchKernelGGL(kernel, dim3((unsigned)(z.tiles_m * z.tiles_n)), dim3(NTHREADS), 0, s, z);
+      const TileShapes shapes = tile_shapes_of_any_count(H, z.tiles_m, z.tiles_m * z.tiles_n, z.ncu);
+      auto kernel = flagged_kernel([](auto, auto even, auto others) { return &softce_dz_tiles<even.value, others.value>; }, true,
+                                   even_ktiles(H), shapes.used);
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(z.tiles_m * z.tiles_n + shapes.split)), dim3(NTHREADS), 0, s, z);
     }
     if ((e = hipGetLastError()) != hipSuccess) return (int)e;
     // d student hidden [t, h] (+)= sum_v D[t, v] . weight[vc0 + v, h]: the dHidden GEMM of the log-probability backward,

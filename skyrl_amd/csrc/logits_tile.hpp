@@ -29,12 +29,12 @@ __host__ __device__ inline size_t part_elems(size_t nparts, int64_t T) {
 }
 
 // N: token blocks per wave, 8 on square tiles, 4 on half tiles (half_tile.hpp).
-// PAIRED (the soft cross-entropy, below): token blocks j >= TN / 2 hold teacher rows, and their third statistic weighs the
-// *student's* logit -- the same lane's accumulator TN / 2 blocks earlier -- with the teacher's exp: sum z_student e^(z_teacher - m).
+// PAIRED (the soft cross-entropy, below): odd token blocks hold teacher rows, and their third statistic weighs the
+// *student's* logit -- the same lane's accumulator one block earlier -- with the teacher's exp: sum z_student e^(z_teacher - m).
 template <bool ENTROPY, bool MASKED, bool PAIRED, int N>
 __device__ __forceinline__ void fwd_tile_stats(const f32x4 (&acc)[TM][N], int j, int vbase, int V, float scale2, int kq, float& m_out,
                                                float& s_out, float& e_out) {
-  const int jy = (PAIRED && j >= TN / 2) ? j - TN / 2 : j;  // j is a constant of the caller's unrolled loop
+  const int jy = (PAIRED && j % 2) ? j - 1 : j;  // j is a constant of the caller's unrolled loop
   // Two read-only passes over the accumulators (they live in AGPRs; writing scaled values back would cost a move each
   // way).  scale2 > 0, so the maximum commutes with the scaling.  The third statistic of an ordinary row is taken relative
   // to the tile's maximum, sum (z - m) e^(z - m): the exponent is at hand, and the entropy ln s - e / s then comes out of two

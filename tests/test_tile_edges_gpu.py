@@ -474,3 +474,26 @@ def test_masked_mean_of_the_draft_loss(shape, share, cuda_device):
         (loss * up).backward()
         (want * up).backward()  # the upstream per token differs in fp32 roundings only, which d_hidden's bf16 rounding may turn into an ulp
         assert torch.allclose(s.grad.float(), r.grad.float(), rtol=2**-7, atol=1e-7)
+
+
+# The draft loss stacks a student's and a teacher's row per token, so its last tile is made narrower where it holds no more than 64 or 96
+# tokens, and a last round (133 tile rows, V=34001) in short tiles.  Values do not depend on the tile's shape: the first tokens of a longer
+# call in whole tiles are the measure, bit for bit.
+@pytest.mark.parametrize("T", [1, 16, 17, 64, 65, 96, 97, 128, 129, 208, 300])
+@pytest.mark.parametrize("H,V", [(64, 1153), (320, 5001), (128, 34001)])
+def test_last_tokens_of_the_draft_loss(T, H, V, cuda_device):
+    hidden, weight, _, g, _ = _operands(384, H, V, seed=T + H)
+    teacher = torch.randn(384, H, generator=torch.Generator().manual_seed(V)).to(torch.bfloat16)
+    h, ht, w, gd = (x.to(cuda_device) for x in (hidden, teacher, weight, g))
+    long = softce_fwd(h, ht, w, 384, 0, 1.0)
+    short = softce_fwd(h[:T], ht[:T], w, T, 0, 1.0)
+    for a, b in zip(short, long):
+        assert torch.equal(a, b[:T])
+    zs, zt = hidden[:T].double() @ weight.double().t(), teacher[:T].double() @ weight.double().t()
+    want = (g[:T].double()[:, None] * (zs.softmax(-1) - zt.softmax(-1))) @ weight.double()
+    gd[T:] = 0.0
+    for vc in (0, 1024):
+        _close(softce_bwd(h[:T], ht[:T], w, short[1], short[2], gd[:T], T, 0, 1.0, vc), want, f"d student T={T}")
+        d = softce_bwd(h, ht, w, long[1], long[2], gd, 384, 0, 1.0, vc)  # the same tokens, found by the compaction among others
+        _close(d[:T], want, f"d student of {T} active tokens")
+        assert not d[T:].any()
