@@ -128,9 +128,17 @@ __device__ __forceinline__ void topk_tile(const FilterArgs& a, int vtile, int tt
     hit[j] = 0;
     if (!__any(m * s >= th[j])) continue;
 #pragma unroll
-    for (int x = 0; x < TM * 4; ++x) {
-      const float z = acc[x / 4][j][x % 4] * s;
-      asm("v_cmp_ge_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(hit[j]) : "v"(z), "v"(th[j]) : "vcc");
+    for (int i = 0; i < TM; ++i) {
+      const f32x4 z = acc[i][j] * s;
+      // A comparison's result is a carry two wait states later at the earliest, which the compiler cannot keep inside an assembly
+      // statement: four comparisons, then four additions, so that three instructions lie between the two of a pair.
+      uint64_t p0, p1, p2, p3;
+      asm("v_cmp_ge_f32_e64 %1, %5, %9\n\tv_cmp_ge_f32_e64 %2, %6, %9\n\tv_cmp_ge_f32_e64 %3, %7, %9\n\tv_cmp_ge_f32_e64 %4, %8, %9\n\t"
+          "v_addc_co_u32_e64 %0, vcc, %0, %0, %1\n\tv_addc_co_u32_e64 %0, vcc, %0, %0, %2\n\t"
+          "v_addc_co_u32_e64 %0, vcc, %0, %0, %3\n\tv_addc_co_u32_e64 %0, vcc, %0, %0, %4"
+          : "+v"(hit[j]), "=&s"(p0), "=&s"(p1), "=&s"(p2), "=&s"(p3)
+          : "v"(z[0]), "v"(z[1]), "v"(z[2]), "v"(z[3]), "v"(th[j])
+          : "vcc");
     }
     hit[j] &= exists;
   }

@@ -7,7 +7,9 @@ every kernel that contains MFMAs and check the properties the source relies on:
 * every ``v_accvgpr_read`` comes after the explicit wait states that follow the last MFMA before it, and no
   ``v_accvgpr_write`` sits right in front of an MFMA;
 * every MFMA accumulates in place, in AGPRs (no rotation of accumulators through the loop);
-* the steady-state loop (the block with MFMAs and global->LDS copies) has no scratch (spill) traffic and no accumulator moves.
+* the steady-state loop (the block with MFMAs and global->LDS copies) has no scratch (spill) traffic and no accumulator moves;
+* no scalar register that a vector instruction writes is read by another one less than two wait states later (the compiler keeps that
+  distance in its own code, but cannot see into an assembly statement).
 """
 
 from __future__ import annotations
@@ -73,6 +75,60 @@ def test_no_accumulator_write_right_before_an_mfma(kernels):
             if ln.startswith("v_mfma"):
                 near = [p for p in lines[max(0, k - 3):k] if p.startswith("v_accvgpr_write")]
                 assert not near, f"{name}: {near[0]} within three instructions of '{ln}'"
+
+
+def _scalars(operands):
+    """The scalar registers that the operands name, VCC as one of them."""
+    found = {"vcc"} if "vcc" in operands else set()
+    for lo, hi in re.findall(r"\bs\[(\d+):(\d+)\]", operands):
+        found |= {f"s{i}" for i in range(int(lo), int(hi) + 1)}
+    return found | set(re.findall(r"\bs\d+\b", operands))
+
+
+def _scalars_written_and_read(line):
+    """Of a vector instruction; what stands unwritten (the VCC of the 32-bit encodings) included."""
+    op, _, rest = line.split(";")[0].partition(" ")
+    operands = [x.strip() for x in re.split(r",(?![^\[]*\])", rest)]
+    outputs = 2 if re.match(r"v_(add|addc|sub|subb|subrev|subbrev)_co_|v_mad_[ui]64_[ui]32|v_div_scale", op) else 1
+    written, read = _scalars(" ".join(operands[:outputs])), _scalars(" ".join(operands[outputs:]))
+    if op.startswith("v_cmp") and len(operands) == 2:
+        written, read = {"vcc"}, _scalars(" ".join(operands))
+    if op.startswith("v_cndmask") and len(operands) == 3 or op.startswith("v_div_fmas"):
+        read.add("vcc")
+    return written, read
+
+
+def _too_close(lines):
+    """Pairs of vector instructions of which the second reads a scalar register that the first wrote less than two wait states before."""
+    pairs, since = [], []  # since: (wait states passed, scalars written, line) of the last vector instructions
+    for ln in lines:
+        if re.match(r"^\.?\w+:", ln) or ln.startswith("."):
+            since = []
+            continue
+        states = int(ln.split()[1]) + 1 if ln.startswith("s_nop") else 1
+        written, read = _scalars_written_and_read(ln) if ln.startswith("v_") else (set(), set())
+        pairs += [(before, ln) for passed, scalars, before in since if passed < 2 and scalars & read]
+        since = [(passed + states, scalars, before) for passed, scalars, before in since if passed + states < 2]
+        if written:
+            since.append((0, written, ln))
+    return pairs
+
+
+def test_the_distance_check_sees_what_it_claims():
+    pair = ["v_cmp_ge_f32 vcc, v1, v2", "v_addc_co_u32 v0, vcc, v0, v0, vcc"]
+    assert _too_close(pair) and _too_close([pair[0], "v_mov_b32_e32 v7, v8", pair[1]])
+    assert _too_close([pair[0], "s_nop 0", pair[1]]) and not _too_close([pair[0], "s_nop 1", pair[1]])
+    assert _too_close(["v_cmp_lt_f32_e64 s[4:5], v1, v2", "v_cndmask_b32_e64 v0, v1, v2, s[4:5]"])
+    assert _too_close(["v_cmp_lt_f32_e32 vcc, v1, v2", "v_cndmask_b32_e32 v0, v1, v2"])
+    assert _too_close(["v_readfirstlane_b32 s6, v1", "v_add_u32_e32 v0, s6, v2"])
+    assert not _too_close(["v_cmp_lt_f32_e64 s[4:5], v1, v2", "v_cndmask_b32_e64 v0, v1, v2, s[6:7]"])
+    assert not _too_close(["v_add_co_u32_e32 v0, vcc, v1, v2", "s_nop 1", "v_addc_co_u32_e32 v3, vcc, v4, v5, vcc"])
+
+
+def test_vector_reads_keep_their_distance_from_scalar_writes(kernels):
+    for name, lines in kernels.items():
+        bad = _too_close(lines)
+        assert not bad, f"{name}: {len(bad)} pairs, the first {bad[0]}"
 
 
 def test_every_lds_copy_sets_m0_first(kernels):
