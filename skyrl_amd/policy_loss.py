@@ -33,7 +33,7 @@ per-token decision to the same fused kernel (``compute_policy_loss_clip_cov``, `
 
 from __future__ import annotations
 
-from typing import Any, Dict, Optional, Tuple
+from typing import Any, Dict, Optional, Sequence, Tuple
 
 import torch
 
@@ -513,11 +513,12 @@ def approx_kl_loss(
 
 
 @registered_op("skyrl_amd::masked_mean", mutates_args=())
-def _masked_mean(values: torch.Tensor, mask: Optional[torch.Tensor], want_grad: bool) -> Tuple[torch.Tensor, torch.Tensor]:
-    """``(means [rows], dvalues [rows, cols] or empty)`` for contiguous fp32 ``[rows, cols]`` inputs."""
+def _masked_mean(values: torch.Tensor, mask: Optional[torch.Tensor], shape: Sequence[int],
+                 want_grad: bool) -> Tuple[torch.Tensor, torch.Tensor]:
+    """``(means of the given shape, one per row, dvalues [rows, cols] or empty)`` for contiguous fp32 ``[rows, cols]`` inputs."""
     dev = _require_device(values)
     rows, cols = values.shape
-    means = torch.empty(rows, dtype=torch.float32, device=dev)
+    means = torch.empty(shape, dtype=torch.float32, device=dev)
     dv = torch.empty_like(values) if want_grad else torch.empty(0, dtype=torch.float32, device=dev)
     with device_guard(dev):
         st = _lib.load().skyrl_masked_mean(values.data_ptr(), None if mask is None else mask.data_ptr(), rows, cols,
@@ -528,8 +529,8 @@ def _masked_mean(values: torch.Tensor, mask: Optional[torch.Tensor], want_grad: 
 
 
 @_masked_mean.register_fake
-def _(values, mask, want_grad):
-    return values.new_empty(values.shape[0]), torch.empty_like(values) if want_grad else values.new_empty(0)
+def _(values, mask, shape, want_grad):
+    return values.new_empty(shape), torch.empty_like(values) if want_grad else values.new_empty(0)
 
 
 class _MaskedMean(torch.autograd.Function):
@@ -537,10 +538,10 @@ class _MaskedMean(torch.autograd.Function):
     def forward(ctx, tensor, mask, rows, cols, out_shape):
         v = tensor.detach().to(torch.float32).contiguous().reshape(rows, cols)
         m = None if mask is None else mask.detach().to(torch.float32).expand_as(tensor).contiguous().reshape(rows, cols)
-        means, dv = call(_masked_mean, v, m, bool(ctx.needs_input_grad[0]))
+        means, dv = call(_masked_mean, v, m, out_shape, bool(ctx.needs_input_grad[0]))
         ctx.save_for_backward(dv)
         ctx.shape, ctx.dtype, ctx.rows = tensor.shape, tensor.dtype, rows
-        return means.reshape(out_shape)
+        return means  # as it was allocated: a view made here could not be changed in place
 
     @staticmethod
     def backward(ctx, grad_out):

@@ -301,6 +301,28 @@ def test_public_entry_points_give_shapes_on_the_meta_device():
         assert dh.shape == (S, H) and dw.shape == (V, H) and dh.device == meta
 
 
+def test_means_and_draft_losses_can_be_scaled_in_place():
+    """``loss *= coef`` before the backward, whatever the shape of the mask."""
+    from skyrl_amd import mtp_soft_ce as M
+    from skyrl_amd import policy_loss as PL
+
+    B, S, H, V, meta = 3, 8, 64, 300, torch.device("meta")
+    hidden = torch.empty(B, S, H, dtype=torch.bfloat16, device=meta, requires_grad=True)
+    weight = torch.empty(V, H, dtype=torch.bfloat16, device=meta)
+    values = torch.empty(B, S, device=meta, requires_grad=True)
+    mask = torch.empty(B, S, device=meta)
+    draft = [loss_of(m) for m in (mask, mask[:1])
+             for loss_of in (lambda m: M.draft_soft_ce_from_hidden(hidden, hidden.detach(), weight, m),
+                             lambda m: M.draft_soft_ce_topk_from_hidden(hidden, hidden.detach(), weight, m, 8))]
+    means = [PL.masked_mean(values, m, dim) for m in (mask, None) for dim in (None, -1)]
+    for x, leaf in [(loss, hidden) for loss in draft] + [(mean, values) for mean in means]:
+        x *= 0.5
+        x /= 3
+        x.add_(1.0)
+        (g,) = torch.autograd.grad(x.sum(), leaf)
+        assert g.shape == leaf.shape and g.dtype == leaf.dtype
+
+
 def test_losses_of_fake_tensors_outside_their_mode():
     from types import SimpleNamespace
 

@@ -476,6 +476,22 @@ def test_masked_mean_of_the_draft_loss(shape, share, cuda_device):
         assert torch.allclose(s.grad.float(), r.grad.float(), rtol=2**-7, atol=1e-7)
 
 
+@pytest.mark.parametrize("shape", [(2, 41), (1, 41)])
+@pytest.mark.parametrize("topk", [False, True])
+def test_draft_loss_scaled_in_place(shape, topk, cuda_device):
+    B, S, H, V = 2, 41, 64, 1500
+    hidden, weight, *_ = _operands(2 * B * S, H, V, seed=S)
+    student, teacher = (x.reshape(B, S, H).to(cuda_device) for x in hidden.split(B * S))
+    mask, w = torch.ones(shape, device=cuda_device), weight.to(cuda_device)
+    loss_of = (lambda s: draft_soft_ce_topk_from_hidden(s, teacher, w, mask, 9)) if topk else (lambda s: draft_soft_ce_from_hidden(s, teacher, w, mask))
+    s, r = (student.clone().requires_grad_(True) for _ in range(2))
+    loss, whole = loss_of(s), loss_of(r)
+    loss *= 0.5
+    loss.backward()
+    whole.backward()
+    assert torch.equal(loss.detach(), 0.5 * whole.detach()) and torch.equal(s.grad, 0.5 * r.grad)  # halves are exact
+
+
 # The draft loss stacks a student's and a teacher's row per token, so its last tile is made narrower where it holds no more than 64 or 96
 # tokens, and a last round (133 tile rows, V=34001) in short tiles.  Values do not depend on the tile's shape: the first tokens of a longer
 # call in whole tiles are the measure, bit for bit.
