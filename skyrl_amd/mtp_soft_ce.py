@@ -28,6 +28,7 @@ from __future__ import annotations
 from typing import Optional, Tuple
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 from ._launch import call, device_guard, raw_stream, registered_op
@@ -158,12 +159,13 @@ def soft_ce_from_hidden(student_hidden: torch.Tensor, teacher_hidden: torch.Tens
 
 def _masked_loss(per_token: torch.Tensor, mask: torch.Tensor, global_normalization_factor: Optional[torch.Tensor]) -> torch.Tensor:
     """The masked sum over the mask's own sum (at least 1) or over the given factor.  A mask of the loss's shape goes through the
-    masked-mean kernel, one launch each way instead of five and three; one that is broadcast (its own sum counts every value once) or
-    takes a gradient itself does not."""
+    masked-mean kernel, one launch each way instead of five and three; one that is broadcast (its own sum counts every value once), or
+    is differentiated itself, backward or forward, does not: the kernel knows the derivative with respect to the loss only."""
     mask = mask.to(per_token.dtype)
     if global_normalization_factor is not None:
         return (per_token * mask).sum() / global_normalization_factor.clamp(min=1.0)
-    if mask.shape == per_token.shape and mask.device == per_token.device and not mask.requires_grad:
+    constant = not mask.requires_grad and (torch.compiler.is_compiling() or forward_ad.unpack_dual(mask).tangent is None)
+    if constant and mask.shape == per_token.shape and mask.device == per_token.device:
         return masked_mean(per_token, mask)
     return (per_token * mask).sum() / mask.sum().clamp(min=1.0)
 

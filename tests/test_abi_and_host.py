@@ -323,6 +323,23 @@ def test_means_and_draft_losses_can_be_scaled_in_place():
         assert g.shape == leaf.shape and g.dtype == leaf.dtype
 
 
+def test_draft_losses_carry_the_tangent_of_their_mask():
+    from torch.autograd import forward_ad
+
+    from skyrl_amd import mtp_soft_ce as M
+
+    B, S, H, V, meta = 3, 8, 64, 300, torch.device("meta")
+    hidden = torch.empty(B, S, H, dtype=torch.bfloat16, device=meta)
+    weight = torch.empty(V, H, dtype=torch.bfloat16, device=meta)
+    mask = torch.empty(B, S, device=meta)
+    with forward_ad.dual_level():
+        dual = forward_ad.make_dual(mask, mask.clone())
+        for loss in (M.draft_soft_ce_from_hidden(hidden, hidden, weight, dual),
+                     M.draft_soft_ce_topk_from_hidden(hidden, hidden, weight, dual, 8)):
+            assert forward_ad.unpack_dual(loss).tangent.shape == ()
+        assert forward_ad.unpack_dual(M.draft_soft_ce_from_hidden(hidden, hidden, weight, mask)).tangent is None
+
+
 def test_losses_of_fake_tensors_outside_their_mode():
     from types import SimpleNamespace
 
