@@ -157,15 +157,21 @@ def soft_ce_from_hidden(student_hidden: torch.Tensor, teacher_hidden: torch.Tens
     return loss.reshape(out_shape)
 
 
+# The masked-mean kernel is one workgroup, plain torch sums over the whole chip: forward and backward together 8.1 against 20.6 us at 4096
+# tokens, 26.7 against 33.0 at 65536, 36.5 against 38.1 at 98304, 46 against 33 at 131072, 633 against 37 at 2^20.
+_MASKED_MEAN_TOKENS = 1 << 16
+
+
 def _masked_loss(per_token: torch.Tensor, mask: torch.Tensor, global_normalization_factor: Optional[torch.Tensor]) -> torch.Tensor:
     """The masked sum over the mask's own sum (at least 1) or over the given factor.  A mask of the loss's shape goes through the
-    masked-mean kernel, one launch each way instead of five and three; one that is broadcast (its own sum counts every value once), or
-    is differentiated itself, backward or forward, does not: the kernel knows the derivative with respect to the loss only."""
+    masked-mean kernel, one launch each way instead of five and three, up to the size where its one workgroup takes longer than those; one
+    that is broadcast (its own sum counts every value once), or is differentiated itself, backward or forward, does not: the kernel knows
+    the derivative with respect to the loss only."""
     mask = mask.to(per_token.dtype)
     if global_normalization_factor is not None:
         return (per_token * mask).sum() / global_normalization_factor.clamp(min=1.0)
     constant = not mask.requires_grad and (torch.compiler.is_compiling() or forward_ad.unpack_dual(mask).tangent is None)
-    if constant and mask.shape == per_token.shape and mask.device == per_token.device:
+    if constant and per_token.numel() <= _MASKED_MEAN_TOKENS and mask.shape == per_token.shape and mask.device == per_token.device:
         return masked_mean(per_token, mask)
     return (per_token * mask).sum() / mask.sum().clamp(min=1.0)
 

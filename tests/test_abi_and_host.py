@@ -340,6 +340,18 @@ def test_draft_losses_carry_the_tangent_of_their_mask():
         assert forward_ad.unpack_dual(M.draft_soft_ce_from_hidden(hidden, hidden, weight, mask)).tangent is None
 
 
+def test_masked_mean_of_many_tokens_is_left_to_torch(monkeypatch):
+    from skyrl_amd import mtp_soft_ce as M
+
+    taken = []
+    monkeypatch.setattr(M, "masked_mean", lambda v, m: taken.append(v.numel()))
+    for n in (64, 1 << 16, (1 << 16) + 1, 1 << 20):
+        v = torch.linspace(0.0, 1.0, n, dtype=torch.float64)
+        loss = M._masked_loss(v, torch.ones(n), None)
+        assert taken[-1:] == [n] if n <= 1 << 16 else abs(float(loss) - 0.5) < 1e-9
+    assert taken == [64, 1 << 16]
+
+
 def test_losses_of_fake_tensors_outside_their_mode():
     from types import SimpleNamespace
 
