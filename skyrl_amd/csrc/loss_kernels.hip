@@ -397,7 +397,8 @@ __global__ __launch_bounds__(kRowThreads) void masked_mean_rows_kernel(const flo
     sm += m;
   }
   const float total = block_sum(sv, red);
-  const float denom = mask ? fmaxf(block_sum(sm, red), 1.f) : (float)cols;
+  const float count = mask ? block_sum(sm, red) : (float)cols;
+  const float denom = count < 1.f ? 1.f : count;  // a NaN stays one, as torch's clamp leaves it
   if (threadIdx.x == 0) means[blockIdx.x] = total / denom;
   if (dv) {
     const float r = 1.f / denom;

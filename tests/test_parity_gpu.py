@@ -1105,6 +1105,21 @@ def test_masked_mean_matches_oracle(cuda_device):
         masked_mean(v.to(cuda_device), None, 0)
 
 
+@pytest.mark.parametrize("special", [float("nan"), float("inf"), float("-inf"), -3.0])
+@pytest.mark.parametrize("dim", [None, -1])
+def test_masked_mean_of_special_masks(special, dim, cuda_device):
+    from skyrl_amd.policy_loss import masked_mean
+
+    v, mask = torch.linspace(0.5, 2.0, 24).reshape(3, 8), torch.ones(3, 8)
+    mask[1, 3], mask[2] = special, 0.0
+    want_v, got_v = v.double().requires_grad_(True), v.to(cuda_device).requires_grad_(True)
+    want, got = O.masked_mean(want_v, mask.double(), dim), masked_mean(got_v, mask.to(cuda_device), dim)
+    want.sum().backward()
+    got.sum().backward()
+    torch.testing.assert_close(got.detach().cpu().double(), want.detach(), rtol=1e-6, atol=0.0, equal_nan=True)
+    torch.testing.assert_close(got_v.grad.cpu().double(), want_v.grad, rtol=1e-6, atol=0.0, equal_nan=True)
+
+
 def test_loss_argument_errors(cuda_device):
     lib = _lib.load()
     x = torch.zeros(16, dtype=torch.float32, device=cuda_device)
