@@ -289,13 +289,14 @@ __global__ __launch_bounds__(64) void logprob_diff_finish_kernel(const float* __
 constexpr int kRowThreads = 1024;  // one workgroup per row of [B, S]: rows are few and long
 
 // Sum of one value per thread over the workgroup, in a fixed order; every thread receives it.
-__device__ __forceinline__ float block_sum(float v, float* red) {
+template <class X>
+__device__ __forceinline__ X block_sum(X v, X* red) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   __syncthreads();  // red may still be read from an earlier call
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  float s = 0.f;
+  X s = 0;
   for (int k = 0; k < kRowThreads / 64; ++k) s += red[k];
   return s;
 }
@@ -384,24 +385,32 @@ __global__ __launch_bounds__(kRowThreads) void scaled_sum_kernel(const float* __
 // ------------------------------------------------------------------------------------------------------------
 // masked_mean (torch_utils.py:180-184).  Per row: means[b] = sum_s v * mask / max(sum_s mask, 1) (mask NULL: plain mean),
 // dvalues = d means[b] / d v = mask / max(sum mask, 1).  The global form is the same kernel on one row of rows * cols.
+// A thread's values go into four sums in turn and these over the workgroup in 64 bits: one 32-bit sum per thread and 32-bit sums of those are
+// further off than torch's tree of sums (mean error over 100 draws, one sum -> this, torch: 5.4e-8 -> 1.8e-8, 4.7e-8 at 2048 tokens; 4.6e-8 -> 1.9e-8, 3.0e-8 at 49152).
 // ------------------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(kRowThreads) void masked_mean_rows_kernel(const float* __restrict__ v, const float* __restrict__ mask,
                                                                        int64_t cols, float* __restrict__ means,
                                                                        float* __restrict__ dv) {
-  __shared__ float red[kRowThreads / 64];
+  __shared__ double red[kRowThreads / 64];
   const int64_t row0 = (int64_t)blockIdx.x * cols;
-  float sv = 0.f, sm = 0.f;
-  for (int64_t c = threadIdx.x; c < cols; c += kRowThreads) {
-    const float m = mask ? mask[row0 + c] : 1.f;
-    sv += v[row0 + c] * m;
-    sm += m;
+  float v4[4] = {0.f, 0.f, 0.f, 0.f}, m4[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int64_t c0 = threadIdx.x; c0 < cols; c0 += 4 * kRowThreads) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t c = c0 + u * kRowThreads;
+      if (c >= cols) break;
+      const float m = mask ? mask[row0 + c] : 1.f;
+      v4[u] += v[row0 + c] * m;
+      m4[u] += m;
+    }
   }
-  const float total = block_sum(sv, red);
-  const float count = mask ? block_sum(sm, red) : (float)cols;
-  const float denom = count < 1.f ? 1.f : count;  // a NaN stays one, as torch's clamp leaves it
-  if (threadIdx.x == 0) means[blockIdx.x] = total / denom;
+  const double sv = ((double)v4[0] + v4[1]) + ((double)v4[2] + v4[3]), sm = ((double)m4[0] + m4[1]) + ((double)m4[2] + m4[3]);
+  const double total = block_sum(sv, red);
+  const double count = mask ? block_sum(sm, red) : (double)cols;
+  const double denom = count < 1.0 ? 1.0 : count;  // a NaN stays one, as torch's clamp leaves it
+  if (threadIdx.x == 0) means[blockIdx.x] = (float)(total / denom);
   if (dv) {
-    const float r = 1.f / denom;
+    const float r = 1.f / (float)denom;
     for (int64_t c = threadIdx.x; c < cols; c += kRowThreads) dv[row0 + c] = mask ? mask[row0 + c] * r : r;
   }
 }

@@ -157,8 +157,8 @@ def soft_ce_from_hidden(student_hidden: torch.Tensor, teacher_hidden: torch.Tens
     return loss.reshape(out_shape)
 
 
-# The masked-mean kernel is one workgroup, plain torch sums over the whole chip: forward and backward together 8.1 against 20.6 us at 4096
-# tokens, 26.7 against 33.0 at 65536, 36.5 against 38.1 at 98304, 46 against 33 at 131072, 633 against 37 at 2^20.
+# The masked-mean kernel is one workgroup, plain torch sums over the whole chip: forward and backward together 9.4 against 21.3 us at 4096
+# tokens, 27.3 against 33.0 at 65536, 36.5 against 38.2 at 98304, 46 against 34 at 131072, 523 against 37 at 2^20.
 _MASKED_MEAN_TOKENS = 1 << 16
 
 

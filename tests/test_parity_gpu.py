@@ -1120,6 +1120,20 @@ def test_masked_mean_of_special_masks(special, dim, cuda_device):
     torch.testing.assert_close(got_v.grad.cpu().double(), want_v.grad, rtol=1e-6, atol=0.0, equal_nan=True)
 
 
+@pytest.mark.parametrize("n", [1, 1023, 1024, 1025, 4095, 4097, 16384, 60001])
+def test_masked_mean_is_as_good_as_its_rounding(n, cuda_device):
+    """The quotient is rounded to fp32 once (2^-24); what the threads' own sums add, of independent roundings of a thousandth of the total
+    each, is far below that."""
+    from skyrl_amd.policy_loss import masked_mean
+
+    for seed in range(20):
+        gen = torch.Generator().manual_seed(seed)
+        v, mask = torch.rand(n, generator=gen) * 12, (torch.rand(n, generator=gen) > 0.3).float()
+        want = O.masked_mean(v.double(), mask.double()).item()
+        got = masked_mean(v.to(cuda_device), mask.to(cuda_device)).double().item()
+        assert abs(got - want) <= 1.1 * 2.0**-24 * abs(want), (n, seed)
+
+
 def test_loss_argument_errors(cuda_device):
     lib = _lib.load()
     x = torch.zeros(16, dtype=torch.float32, device=cuda_device)
