@@ -148,10 +148,10 @@ __global__ __launch_bounds__(NTHREADS) void lmhead_fwd_tiles(const uint16_t* __r
 // every 64th of them (a load is 64 contiguous bytes of four parts), the running triples meet in shuffles and in LDS.  Wave w
 // also takes the label logit of token w, 64 lanes to the dot product.
 // What bounds it: 12 bytes per part and token and two rows per label from HBM for many tokens, the chain of load and merge steps
-// for few.  Sixty-four streams per token and 30 loads in flight per lane keep that chain at two steps for 1188 parts (16
-// streams of 64-token blocks: 19), with one exponential per part, and the label's rows are loaded with the first step.  Between HIP events
-// (which add about 4 us), V=151936, eight parts a step and the label's rows behind them -> this way: 11.2 -> 10.8 us at T=137, 14.0 -> 12.3 at
-// T=611, 14.4 -> 13.3 at T=2048 with entropy, 34 and 34 at T=8192, 81 and 82 at T=16384, H=3584 (5.8 TB/s).
+// for few.  Sixty-four streams per token and BATCH parts a step, 24 or 30 loads in flight per lane, keep that chain at two steps for 1188
+// parts (16 streams of 64-token blocks: 19), with one exponential per part, and the label's rows are loaded with the first step.  Between
+// HIP events (which add about 4 us), V=151936, eight parts a step and the label's rows behind them -> this way: 11.2 -> 10.6 us at T=137, 14.0
+// -> 12.3 at T=611, 14.5 -> 13.2 at T=2048 with entropy, 34 and 34 at T=8192, 81 and 82 at T=16384, H=3584 (5.8 TB/s).
 // Merge algebra as in efficient_entropy_triton_kernel_epilogue (fused_linear_logprob_triton.py:417-467) except that
 // the running max starts at -inf (that kernel starts it at 0, which loses rows whose logits are all << 0).
 // Out-of-range labels give logprob 0 (model_utils.py:337; fused_linear_logprob_triton.py:1898-1905).
@@ -159,6 +159,7 @@ __global__ __launch_bounds__(NTHREADS) void lmhead_fwd_tiles(const uint16_t* __r
 constexpr int kMergeTokens = 16;
 constexpr int kMergeThreads = 1024;
 constexpr int kMergeWaves = kMergeThreads / 64;
+constexpr int kMergeStreams = kMergeWaves * 4;  // of parts per token
 static_assert(kMergeWaves == kMergeTokens && kPartTokens % kMergeTokens == 0, "one wave per token for the label logit");
 
 // Partial triples (maximum, sum e^(z - max), third statistic) of one token become one.  RELATIVE: the third statistic is
@@ -196,7 +197,7 @@ __device__ __forceinline__ void merge_lanes(float& M, float& S, float& E, int o)
   merge_partials<RELATIVE>(M, S, E, m, s, e);
 }
 
-template <bool RELATIVE>
+template <bool RELATIVE, int BATCH>
 __global__ __launch_bounds__(kMergeThreads) void lmhead_fwd_merge(const float* __restrict__ part_max,
                                                                   const float* __restrict__ part_sum,
                                                                   const float* __restrict__ part_pz, int nparts, int T,
@@ -214,13 +215,12 @@ __global__ __launch_bounds__(kMergeThreads) void lmhead_fwd_merge(const float* _
   const int64_t y = (labels && t0 + wave < T) ? labels[t0 + wave] : (int64_t)-1;
   const int t = t0 + (lane & 15);
   const size_t base = part_index(0, t < T ? t : T - 1, nparts);
-  constexpr int kBatch = 10, kStreams = kMergeWaves * 4;  // loads in flight per array before the dependent merge chain
   const int first = wave * 4 + (lane >> 4);
-  float m[kBatch], sv[kBatch], ev[kBatch];
-  auto load_batch = [&](int p0) {  // parts p0, p0 + kStreams, ...; behind the last one: part 0, dropped below
+  float m[BATCH], sv[BATCH], ev[BATCH];
+  auto load_batch = [&](int p0) {  // parts p0, p0 + kMergeStreams, ...; behind the last one: part 0, dropped below
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int p = p0 + u * kStreams;
+    for (int u = 0; u < BATCH; ++u) {
+      const int p = p0 + u * kMergeStreams;
       const size_t idx = base + (size_t)(p < nparts ? p : 0) * kPartTokens;
       m[u] = part_max[idx];
       sv[u] = part_sum[idx];
@@ -251,10 +251,10 @@ __global__ __launch_bounds__(kMergeThreads) void lmhead_fwd_merge(const float* _
     float M = -INFINITY, S = 0.f, E = 0.f;
     for (int p0 = first; p0 < nparts;) {
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u)
-        if (p0 + u * kStreams >= nparts || sv[u] == 0.f) m[u] = -INFINITY, sv[u] = 0.f, ev[u] = 0.f;
+      for (int u = 0; u < BATCH; ++u)
+        if (p0 + u * kMergeStreams >= nparts || sv[u] == 0.f) m[u] = -INFINITY, sv[u] = 0.f, ev[u] = 0.f;
       merge_partials<RELATIVE>(M, S, E, m, sv, ev);
-      p0 += kStreams * kBatch;
+      p0 += kMergeStreams * BATCH;
       if (p0 < nparts) load_batch(p0);
     }
     merge_lanes<RELATIVE>(M, S, E, 16);
@@ -286,6 +286,16 @@ __global__ __launch_bounds__(kMergeThreads) void lmhead_fwd_merge(const float* _
   if (entropy) entropy[t] = RELATIVE ? third : lse - third;
   if (row_lse) row_lse[t] = lse;
   if (row_pz) row_pz[t] = RELATIVE ? lse - third : third;
+}
+
+// Ten parts a step where that saves the first or the second of the steps that eight take (lanes without a part of their own load and drop
+// one): with ten instead of eight 8.5 -> 7.7 us at 137 tokens of V=80000 (ten parts per stream), 11.5 -> 10.6 at V=151936 (19), but 8.5 -> 9.2
+// at V=100000 (13), 10.2 -> 10.8 at V=200064 (25), and 29 -> 38 at 32768 tokens of V=32000 (4).  The same for every number of tokens, so that
+// a token's sums do not depend on it.
+template <bool RELATIVE>
+auto merge_kernel(int64_t nparts) {
+  const int64_t n = (nparts + kMergeStreams - 1) / kMergeStreams;
+  return n <= 20 && (n + 9) / 10 < (n + 7) / 8 ? &lmhead_fwd_merge<RELATIVE, 10> : &lmhead_fwd_merge<RELATIVE, 8>;
 }
 
 // The dz tiles (logits_tile.hpp) on products of any shape.
@@ -1367,7 +1377,7 @@ int fwd_token_blocks(const void* hidden, int64_t ld_hidden, const void* weight, 
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
     Timed timed(kFwdMerge, s);
-    hipLaunchKernelGGL(lmhead_fwd_merge<true>, dim3((unsigned)((Tb + kMergeTokens - 1) / kMergeTokens)), dim3(kMergeThreads), 0, s, pmax,
+    hipLaunchKernelGGL(merge_kernel<true>(nparts), dim3((unsigned)((Tb + kMergeTokens - 1) / kMergeTokens)), dim3(kMergeThreads), 0, s, pmax,
                        psum, want_pz ? ppz : (float*)nullptr, (int)nparts, (int)Tb, Hp, (int)ld_hidden, Wp, (int)ld_weight,
                        labels + t0, (int)H, (int)V, rcp_temperature, logprobs + t0, entropy ? entropy + t0 : (float*)nullptr,
                        row_lse ? row_lse + t0 : (float*)nullptr, row_pz ? row_pz + t0 : (float*)nullptr);
@@ -2019,7 +2029,7 @@ int skyrl_softce_fwd(const void* student_hidden, int64_t ld_student, const void*
   if ((e = hipGetLastError()) != hipSuccess) return (int)e;
   {
     Timed timed(kFwdMerge, s);
-    hipLaunchKernelGGL(lmhead_fwd_merge<false>, dim3((unsigned)((rows + kMergeTokens - 1) / kMergeTokens)), dim3(kMergeThreads), 0, s, w.pmax,
+    hipLaunchKernelGGL(merge_kernel<false>(w.nparts), dim3((unsigned)((rows + kMergeTokens - 1) / kMergeTokens)), dim3(kMergeThreads), 0, s, w.pmax,
                        w.psum, w.ppz, (int)w.nparts, (int)rows, w.S, (int)H, Wp, (int)ld_weight, (const int64_t*)nullptr, (int)H,
                        (int)V, rcp_temperature, (float*)nullptr, (float*)nullptr, w.row_lse, w.row_pz);
   }

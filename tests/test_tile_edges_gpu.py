@@ -425,6 +425,20 @@ def test_last_tokens_in_a_narrow_tile(T, H, V, cuda_device):
             assert torch.equal(a, b[:T])
 
 
+# The merge takes eight or ten parts (128 vocabulary rows each) a step, by how many there are per stream: both sides of every line of that
+# rule.  fp32 statistics of bf16 products: 1e-5 relative covers their summation orders.
+@pytest.mark.parametrize("streams", [1, 8, 10, 16, 20])
+@pytest.mark.parametrize("more", [0, 1])
+def test_parts_of_the_forward_merge(streams, more, cuda_device):
+    T, H, V = 17, 64, streams * 64 * 128 + more
+    hidden, weight, labels, _, _ = _operands(T, H, V, seed=V)
+    labels[:3] = torch.tensor([V - 1, 0, V // 2])
+    ex = O.exact_fwd_bwd(hidden, weight, labels, 0.9)
+    lp, ent, *_ = ops.lmhead_fwd(hidden.to(cuda_device), weight.to(cuda_device), labels.to(cuda_device), 1.0 / 0.9, True)
+    torch.testing.assert_close(lp.double().cpu(), ex["logprobs"], rtol=1e-5, atol=1e-5)
+    torch.testing.assert_close(ent.double().cpu(), ex["entropy"], rtol=1e-5, atol=1e-5)
+
+
 # The tiles of a last round that fills no more than half of the CUs are made as short ones, the rest as square ones: 133 tile rows give a round
 # of nothing but short tiles for one token tile, 256 square and 10 short ones for two, and none for three, whose values are the measure, bit for
 # bit.  The vocabulary ends in the lower half of its last tile, at its middle, and in the upper half.
