@@ -640,7 +640,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bid, char* lds)
     const int count = __builtin_amdgcn_readfirstlane(*p.T_dev);
     if (p.t_role == kTokensOnM) M = count;
     else if (p.t_role == kTokensOnN) N = count;
-    else nk = (count + 2 * BK - 1) / (2 * BK) * 2;  // whole pairs of k-tiles: the rows up to the next multiple of 256 are zeros
+    else nk = (count + kTokenGroup - 1) / kTokenGroup * 2;  // whole pairs of k-tiles: the panel's rows up to the next kTokenGroup are zeros
     // Nothing to contract: C += 0 needs no work; a C that is overwritten or converted still goes through the epilogue.
     if (nk == 0 && !p.Cb && p.Cin == p.Cf) return;
   }

@@ -139,7 +139,7 @@ struct DzArgs {
   const float* dentropy;
   int vc0, tiles_m, tiles_n;  // first vocab row of the chunk; tiles of the chunk panel along vocab and tokens
   VocabTail tail;
-  uint16_t* D;                // [T rounded up to 256, ldd]  dz, token-major; rows behind the last tile are not written
+  uint16_t* D;                // [T rounded up to 256, ldd]  dz, token-major; behind the tokens zeros up to the next kTokenGroup
   int ldd;
   // When not NULL: the number of tokens, <= T, as a value in device memory (what a compaction kernel counted).  T then
   // only sizes the grid: token tiles at or beyond the device-side count return at once.
@@ -189,6 +189,11 @@ __device__ __forceinline__ bool dz_tile_of(const DzArgs& z, int id, int tile_n, 
   tile = tile_of<true, SPLIT>(id, z.tiles_m, tiles_n, kGroupM, split);
   return true;
 }
+
+// Tokens that the products behind the panel contract at once, two k-tiles.  A tile of whatever width writes its tokens' rows up to the next
+// multiple (dz_tile's end); what lies behind that in the panel is whatever the scratch held.
+constexpr int kTokenGroup = 2 * BK;
+static_assert(BN % kTokenGroup == 0, "tiles begin at whole groups");
 
 // One tile: panel columns col0 .. + 255 of the tokens t0 .. t0 + 32 * NB - 1, of T.  NB: token blocks of 16 per wave.  SHORT: the four
 // waves side by side along the tokens, panel columns col0 .. + 127 and twice the tokens.  product(a, b, acc) leaves the tile's products in
@@ -363,9 +368,10 @@ __device__ __forceinline__ void dz_tile(const DzArgs& z, int T, int col0, int t0
     for (int j = 0; j < NB; ++j) token_block(j, yes, yes);
   }
   flush_block(NB - 1);
-  // The products behind the panel run over whole groups of 128 tokens: a medium tile, whose tokens end in its second group, leaves zeros in
+  // The products behind the panel run over whole groups of tokens: a medium tile, whose tokens end in its second group, leaves zeros in
   // what remains of that.
-  constexpr int kRest = WAVE_N * WAVES_N % 128 > 0 ? 128 - WAVE_N * WAVES_N % 128 : 0;
+  constexpr int kTokens = WAVE_N * (SHORT ? NWAVES : WAVES_N), kRest = (kTokens + kTokenGroup - 1) / kTokenGroup * kTokenGroup - kTokens;
+  static_assert(!SHORT || kRest == 0, "the rows below are those of two waves side by side");
   if constexpr (kRest > 0) {
     uint16_t* zero_row = D + (size_t)(t0 + WAVES_N * WAVE_N + wn * (kRest / WAVES_N) + (lane >> 4)) * (size_t)ldd + vloc_base + (lane & 15) * 8;
 #pragma unroll
