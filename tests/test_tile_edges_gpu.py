@@ -397,7 +397,8 @@ def test_draft_loss_backward_with_less_scratch(T, H, V, vc, cuda_device):
 
 
 # The last token tile is made narrower where it holds no more than 128 or 192 tokens.  A token's values do not depend on the width of its
-# tile: the last tokens of a call are compared, bit for bit, with those of a longer call in whole tiles.
+# tile: the last tokens of a call are compared, bit for bit, with those of a longer call.  (These vocabularies give no more than 128 tiles,
+# which the longer call makes as short ones; test_shapes_against_square_tiles compares with square ones.)
 @pytest.mark.parametrize("T", [257, 319, 320, 384, 385, 447, 448, 449, 513])
 @pytest.mark.parametrize("H,V", [(64, 1153), (128, 5001), (192, 777), (320, 2304)])
 def test_last_tokens_in_a_narrow_tile(T, H, V, cuda_device):
@@ -439,9 +440,9 @@ def test_parts_of_the_forward_merge(streams, more, cuda_device):
     torch.testing.assert_close(ent.double().cpu(), ex["entropy"], rtol=1e-5, atol=1e-5)
 
 
-# The tiles of a last round that fills no more than half of the CUs are made as short ones, the rest as square ones: 133 tile rows give a round
-# of nothing but short tiles for one token tile, 256 square and 10 short ones for two, and none for three, whose values are the measure, bit for
-# bit.  The vocabulary ends in the lower half of its last tile, at its middle, and in the upper half.
+# The tiles of a last round that fills no more than half of the CUs are made as short ones, the rest as square ones: 133 tile rows give
+# none for one token tile (T=40: half tiles, 137: medium ones, 256: square ones), 256 square and 10 short ones for two, and none for three,
+# whose values are the measure, bit for bit.  The vocabulary ends in the lower half of its last tile, at its middle, and in the upper half.
 @pytest.mark.parametrize("V", [33900, 33920, 34001])
 @pytest.mark.parametrize("T", [40, 137, 256, 300, 512])
 def test_last_round_in_short_tiles(T, V, cuda_device):
@@ -506,9 +507,36 @@ def test_draft_loss_scaled_in_place(shape, topk, cuda_device):
     assert torch.equal(loss.detach(), 0.5 * whole.detach()) and torch.equal(s.grad, 0.5 * r.grad)  # halves are exact
 
 
+# Square tiles are the measure of all other shapes, bit for bit and behind the first k-tiles too (three, four and five of them): 50 tile rows
+# make 150 tiles of 768 tokens, more than half of the CUs and no remainder, so all square; for one and two token tiles no more than 128,
+# so all short or, where the last column is narrow, that; and for three a last column of its own width beside square ones.  The vocabulary ends
+# in the lower half of its last tile, at its middle, and in the upper half.  Top-k: 1024 tokens of 128 tile rows are two chunks of 256 tiles.
+@pytest.mark.parametrize("H", [192, 256, 320])
+@pytest.mark.parametrize("rest", [100, 128, 200])
+def test_shapes_against_square_tiles(H, rest, cuda_device):
+    V, wide = 49 * 256 + rest, 127 * 256 + rest
+    hidden, weight, labels, *_ = _operands(1024, H, wide, seed=H + rest)
+    h, w, y = hidden.to(cuda_device), weight.to(cuda_device), labels.remainder(V).to(cuda_device)
+    whole = [ops.lmhead_fwd(h[:768], w[:V], y[:768], 1.25, ent) for ent in (False, True)]
+    first = [topk_logits_from_hidden(h, w, k) for k in (5, 200)]
+    for T in (137, 256, 300, 512, 513, 640, 641, 700, 704):
+        for ent in (False, True):
+            for a, b in zip(ops.lmhead_fwd(h[:T], w[:V], y[:T], 1.25, ent), whole[ent]):
+                assert torch.equal(a, b[:T]), (T, ent)
+        for k, want in zip((5, 200), first):
+            for a, b in zip(topk_logits_from_hidden(h[:T], w, k), want):
+                assert torch.equal(a, b[:T]), (T, k)
+    # the draft loss: two rows per token
+    ht = h.flip(0)[:384].contiguous()
+    pairs = softce_fwd(h[:384], ht, w[:V], 384, 0, 1.25)
+    for T in (69, 128, 150, 256, 257, 320, 321, 340, 352):
+        for a, b in zip(softce_fwd(h[:T], ht[:T], w[:V], T, 0, 1.25), pairs):
+            assert torch.equal(a, b[:T]), T
+
+
 # The draft loss stacks a student's and a teacher's row per token, so its last tile is made narrower where it holds no more than 64 or 96
-# tokens, and a last round (133 tile rows, V=34001) in short tiles.  Values do not depend on the tile's shape: the first tokens of a longer
-# call in whole tiles are the measure, bit for bit.
+# tokens, and a last round in short tiles.  Values do not depend on the tile's shape: the first tokens of a longer call are the measure, bit
+# for bit (square tiles with 133 tile rows, V=34001; short ones with fewer).
 @pytest.mark.parametrize("T", [1, 16, 17, 64, 65, 96, 97, 128, 129, 208, 300])
 @pytest.mark.parametrize("H,V", [(64, 1153), (320, 5001), (128, 34001)])
 def test_last_tokens_of_the_draft_loss(T, H, V, cuda_device):
