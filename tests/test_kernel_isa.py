@@ -159,7 +159,15 @@ def test_mfma_accumulates_in_place_in_agprs(kernels):
                 assert m and m.group(1) == m.group(2), f"{name}: unexpected MFMA form '{ln}'"
 
 
+# MFMAs and copies of a k-tile in the steady state, 16 copies per 128 MFMAs on square tiles (one or two k-tiles per loop body), and fewer of
+# either on the other shapes.
+SQUARE_LOOPS, NARROW_OR_SHORT_LOOP, MEDIUM_LOOP = ((128, 16), (256, 32)), (64, 12), (96, 14)
+# The instantiations that make tiles of all shapes: the last of the kernel's flags.
+ALL_SHAPES = re.compile(r"(lmhead_fwd_tiles|lmhead_bwd_dz|softce_fwd_tiles|softce_dz_tiles|topk_first_tiles|topk_filter_tiles)I(Lb[01]E)+Lb1EE")
+
+
 def test_steady_state_loop_is_clean(kernels):
+    of_all_shapes = set()
     for name, lines in kernels.items():
         # split into basic blocks at labels
         blocks, cur = [], []
@@ -169,16 +177,25 @@ def test_steady_state_loop_is_clean(kernels):
                 cur = []
             cur.append(ln)
         blocks.append(cur)
-        matched = 0
+        matched = []
         for b in blocks:
-            n_mfma = sum(ln.startswith("v_mfma") for ln in b)
-            n_copy = sum(ln.startswith("global_load_lds") for ln in b)
-            if n_mfma and n_mfma % 128 == 0 and n_copy * 8 == n_mfma:  # steady-state k-tile steps: 16 copies per 128 MFMAs
-                matched += 1
-                bad = [ln for ln in b if ln.startswith(("scratch_", "v_accvgpr_"))]
-                assert not bad, f"{name}: steady-state loop has spill / accumulator traffic: {bad[:4]}"
+            work = sum(ln.startswith("v_mfma") for ln in b), sum(ln.startswith("global_load_lds") for ln in b)
+            if not all(work):
+                continue
+            assert work in (*SQUARE_LOOPS, NARROW_OR_SHORT_LOOP, MEDIUM_LOOP), f"{name}: a loop of {work} MFMAs and copies"
+            matched.append(work)
+            bad = [ln for ln in b if ln.startswith(("scratch_", "v_accvgpr_"))]
+            assert not bad, f"{name}: steady-state loop has spill / accumulator traffic: {bad[:4]}"
+        square = [work for work in matched if work in SQUARE_LOOPS]
         if any(ln.startswith("global_load_lds") for ln in lines):
-            assert matched >= 1, f"{name}: no steady-state loop block recognised"
+            assert len(square) >= 1, f"{name}: no steady-state loop block recognised"
+        others = sorted(work for work in matched if work not in SQUARE_LOOPS)
+        if ALL_SHAPES.search(name):
+            of_all_shapes.add(ALL_SHAPES.search(name).group(1))
+            assert others == [NARROW_OR_SHORT_LOOP, NARROW_OR_SHORT_LOOP, MEDIUM_LOOP], f"{name}: {others} beside the square loop"
+        else:
+            assert not others, f"{name}: {others} in a kernel of square tiles"
+    assert len(of_all_shapes) == 6, of_all_shapes
 
 
 def test_even_kernels_issue_both_k_steps_of_an_accumulator_back_to_back(kernels):
