@@ -166,11 +166,13 @@ def _masked_loss(per_token: torch.Tensor, mask: torch.Tensor, global_normalizati
     """The masked sum over the mask's own sum (at least 1) or over the given factor.  A mask of the loss's shape goes through the
     masked-mean kernel, one launch each way instead of five and three, up to the size where its one workgroup takes longer than those; one
     that is broadcast (its own sum counts every value once), or is differentiated itself, backward or forward, does not: the kernel knows
-    the derivative with respect to the loss only."""
+    the derivative with respect to the loss only.  Nor does a call that is traced, compiled or exported: what that records is to hold for
+    other numbers of tokens too."""
     mask = mask.to(per_token.dtype)
     if global_normalization_factor is not None:
         return (per_token * mask).sum() / global_normalization_factor.clamp(min=1.0)
-    constant = not mask.requires_grad and (torch.compiler.is_compiling() or forward_ad.unpack_dual(mask).tangent is None)
+    traced = torch.compiler.is_compiling() or torch.jit.is_tracing()
+    constant = not (traced or mask.requires_grad) and forward_ad.unpack_dual(mask).tangent is None
     if constant and per_token.numel() <= _MASKED_MEAN_TOKENS and mask.shape == per_token.shape and mask.device == per_token.device:
         return masked_mean(per_token, mask)
     return (per_token * mask).sum() / mask.sum().clamp(min=1.0)

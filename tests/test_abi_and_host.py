@@ -352,6 +352,24 @@ def test_masked_mean_of_many_tokens_is_left_to_torch(monkeypatch):
     assert taken == [64, 1 << 16]
 
 
+def test_recorded_draft_losses_hold_for_other_numbers_of_tokens():
+    from skyrl_amd import mtp_soft_ce as M
+
+    class Loss(torch.nn.Module):
+        def forward(self, values, mask):
+            return M._masked_loss(values, mask, None)
+
+    inputs = lambda n: (torch.linspace(0.0, 1.0, 5 * n).reshape(n, 5), torch.arange(5 * n).reshape(n, 5) % 3 != 0)  # noqa: E731
+    n = torch.export.Dim("n")
+    recorded = (torch.jit.trace(Loss(), inputs(2), check_trace=False),
+                torch.export.export(Loss(), inputs(2), dynamic_shapes=({0: n}, {0: n})).module(),
+                torch.compile(Loss(), backend="eager", dynamic=True, fullgraph=True))
+    for rows in (2, 3, 20000):
+        values, mask = inputs(rows)
+        for loss in recorded:
+            assert torch.allclose(loss(values, mask), values[mask].mean(), rtol=1e-5)
+
+
 def test_losses_of_fake_tensors_outside_their_mode():
     from types import SimpleNamespace
 
