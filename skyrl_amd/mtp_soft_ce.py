@@ -372,9 +372,11 @@ def shift_mask_for_mtp(mask: torch.Tensor, mtp_layer_number: int = 0, cu_seqlens
     sequence; with ``cu_seqlens`` the ``[1, T]`` mask is one packed row and the roll stays inside each segment."""
     shift = mtp_layer_number + 1
     S = mask.shape[1]
-    if cu_seqlens is None and mask.dim() == 2 and shift >= 0:  # whole rows: three launches instead of nine
-        behind = min(shift, S)
-        return mask * torch.nn.functional.pad(mask[:, behind:], (0, behind))
+    # Whole rows: three launches instead of nine, and nothing in them depends on the row's length, so that a recorded call holds for others.
+    # Only for what is known while it runs: a symbolic mask or depth decides nothing here.
+    if cu_seqlens is None and isinstance(mask, torch.Tensor) and isinstance(mtp_layer_number, int):
+        if mask.dim() == 2 and shift >= 0:
+            return mask * torch.nn.functional.pad(mask, (0, shift))[:, shift:]
     pos = torch.arange(S, device=mask.device)
     if cu_seqlens is None:
         end = torch.full((S,), S, device=mask.device, dtype=torch.long)

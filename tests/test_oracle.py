@@ -1231,3 +1231,22 @@ def test_shift_mask_for_mtp_of_any_type_and_depth(dtype, depth):
         want[:, t] = mask[:, t] * mask[:, t + depth + 1]
     got = product(mask, depth)
     assert got.dtype == dtype and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("depth", [0, 2, 40])
+def test_recorded_shift_mask_holds_for_other_lengths(depth):
+    from skyrl_amd.mtp_soft_ce import shift_mask_for_mtp as product
+
+    class Shift(torch.nn.Module):
+        def forward(self, mask):
+            return product(mask, depth)
+
+    mask = lambda n: (torch.arange(3 * n).reshape(3, n) % 5 != 0).float()  # noqa: E731
+    n = torch.export.Dim("n")
+    recorded = (torch.jit.trace(Shift(), mask(2)), torch.jit.trace(Shift(), mask(9)),
+                torch.export.export(Shift(), (mask(9),), dynamic_shapes=({1: n},)).module(),
+                torch.fx.symbolic_trace(Shift()), lambda m: torch.jit.script(product)(m, depth))
+    for length in (2, 3, 9, 50):
+        want = O.shift_mask_for_mtp(mask(length), depth)
+        for shift in recorded:
+            assert torch.equal(shift(mask(length)), want)
