@@ -513,12 +513,12 @@ def approx_kl_loss(
 
 
 @registered_op("skyrl_amd::masked_mean", mutates_args=())
-def _masked_mean(values: torch.Tensor, mask: Optional[torch.Tensor], shape: Sequence[int],
-                 want_grad: bool) -> Tuple[torch.Tensor, torch.Tensor]:
-    """``(means of the given shape, one per row, dvalues [rows, cols] or empty)`` for contiguous fp32 ``[rows, cols]`` inputs."""
+def _masked_mean(values: torch.Tensor, mask: Optional[torch.Tensor], want_grad: bool,
+                 shape: Optional[Sequence[int]] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+    """``(means, one per row, of the given shape or [rows], dvalues [rows, cols] or empty)`` for contiguous fp32 ``[rows, cols]`` inputs."""
     dev = _require_device(values)
     rows, cols = values.shape
-    means = torch.empty(shape, dtype=torch.float32, device=dev)
+    means = torch.empty(rows if shape is None else shape, dtype=torch.float32, device=dev)
     dv = torch.empty_like(values) if want_grad else torch.empty(0, dtype=torch.float32, device=dev)
     with device_guard(dev):
         st = _lib.load().skyrl_masked_mean(values.data_ptr(), None if mask is None else mask.data_ptr(), rows, cols,
@@ -529,8 +529,9 @@ def _masked_mean(values: torch.Tensor, mask: Optional[torch.Tensor], shape: Sequ
 
 
 @_masked_mean.register_fake
-def _(values, mask, shape, want_grad):
-    return values.new_empty(shape), torch.empty_like(values) if want_grad else values.new_empty(0)
+def _(values, mask, want_grad, shape=None):
+    means = values.new_empty(values.shape[0] if shape is None else shape)
+    return means, torch.empty_like(values) if want_grad else values.new_empty(0)
 
 
 class _MaskedMean(torch.autograd.Function):
@@ -538,7 +539,7 @@ class _MaskedMean(torch.autograd.Function):
     def forward(ctx, tensor, mask, rows, cols, out_shape):
         v = tensor.detach().to(torch.float32).contiguous().reshape(rows, cols)
         m = None if mask is None else mask.detach().to(torch.float32).expand_as(tensor).contiguous().reshape(rows, cols)
-        means, dv = call(_masked_mean, v, m, out_shape, bool(ctx.needs_input_grad[0]))
+        means, dv = call(_masked_mean, v, m, bool(ctx.needs_input_grad[0]), out_shape)
         ctx.save_for_backward(dv)
         ctx.shape, ctx.dtype, ctx.rows = tensor.shape, tensor.dtype, rows
         return means  # as it was allocated: a view made here could not be changed in place

@@ -323,6 +323,15 @@ def test_means_and_draft_losses_can_be_scaled_in_place():
         assert g.shape == leaf.shape and g.dtype == leaf.dtype
 
 
+def test_masked_mean_op_takes_the_calls_that_saved_programs_hold():
+    from skyrl_amd import policy_loss  # noqa: F401  (registers the op)
+
+    values = torch.empty(3, 8, device="meta")
+    for mask, want_grad in ((values, True), (None, False)):
+        means, dv = torch.ops.skyrl_amd.masked_mean(values, mask, want_grad)
+        assert means.shape == (3,) and dv.shape == ((3, 8) if want_grad else (0,))
+
+
 def test_draft_losses_carry_the_tangent_of_their_mask():
     from torch.autograd import forward_ad
 
