@@ -8,6 +8,7 @@
 namespace lmhead {
 
 constexpr int kDwH = 128, kDwV = 256;  // tile of the weight gradient: hidden columns, vocabulary rows
+constexpr int kDwUnitH = 64;           // hidden columns of what the kernel for more tokens makes at once
 
 struct DwFewArgs {
   const uint16_t* Hd;  // hidden [T, ldh], the first H columns
@@ -22,8 +23,13 @@ struct DwFewArgs {
   int N, n_tail, n_back;
   float* Cf;
   uint16_t* Cb;        // dW rows of the chunk [.., H]: one of the two
+  int ncu;             // CUs of the device
 };
 
+// Up to this many tokens, of which any number may have a gradient, dW is made in those tiles, behind it with dz in registers, which takes 118 to 122 us
+// for whatever is below 130 tokens (H=1536, V=151936): 88 -> 121 at 20, 123 -> 119 at 64, 144 -> 118 at 96, 152 -> 118 at 128.  Not at the sizes
+// of the tie, because half of the tokens and more are often masked.
+constexpr int64_t kDwTileTokens = 96;
 inline int64_t dw_few_tiles(int64_t H, int64_t N) { return (N + kDwV - 1) / kDwV * ((H + kDwH - 1) / kDwH); }
 
 hipError_t launch_bwd_dw_few(hipStream_t s, const DwFewArgs& a);

@@ -1752,7 +1752,7 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
     if (few) {
       Timed timed(kBwdDwFew, s);
       e = launch_bwd_dw_few(s, DwFewArgs{Hp, (int)ld_hidden, w.D, (int)(vcw + kLdPad), (int)Tb, T_dev, (int)H, (int)n_rows,
-                                         moved ? gw.n_tail : 0x7fffffff, gw.n_back, cf, cb});
+                                         moved ? gw.n_tail : 0x7fffffff, gw.n_back, cf, cb, compute_units()});
       if (e != hipSuccess) return (int)e;
     }
     e = launch_bwd_gemm(s, gh, gw, w.slots);

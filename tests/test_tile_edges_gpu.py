@@ -258,6 +258,28 @@ def test_weight_gradient_of_few_tokens(T, vc, cuda_device):
     assert not any(t.any() for t in ops.lmhead_bwd_bf16(h, w, y, lse, pz, zero, zero, 1.0, vc, True))
 
 
+# Behind 96 tokens dz stays in registers, in code of its own for every 64 tokens: the tokens with a gradient at the ends of these, more and
+# fewer hidden columns than a workgroup's share of units, a last vocabulary group moved back.  Both sides are fp32 sums of the same dz panel in
+# another order, sqrt(768) 2^-24 = 2e-6.
+@pytest.mark.parametrize("active", [1, 64, 65, 128, 129, 193, 256, 257, 321, 385, 449, 513, 577, 640, 641, 705, 767])
+@pytest.mark.parametrize("H,V", [(4160, 12100), (256, 196741)])
+def test_weight_gradient_with_resident_dz(active, H, V, cuda_device):
+    T = 97 if active < 96 else 768
+    hidden, weight, labels, g, q = _operands(T, H, V, seed=active)
+    labels[0], labels[T - 1] = V - 1, -1
+    rest = torch.randperm(T, generator=torch.Generator().manual_seed(active))[active:]
+    g[rest], q[rest] = 0.0, 0.0
+    h, w, y, gd, qd = (x.to(cuda_device) for x in (hidden, weight, labels, g, q))
+    _, _, lse, pz = ops.lmhead_fwd(h, w, y, 1.0, True)
+    want = torch.zeros(V, H, device=cuda_device)
+    ops.lmhead_bwd_accumulate(h, w, y, lse, pz, gd, qd, 1.0, want, 0)
+    dh32, dw32 = ops.lmhead_bwd(h, w, y, lse, pz, gd, qd, 1.0, 0, True)
+    dh16, dw16 = ops.lmhead_bwd_bf16(h, w, y, lse, pz, gd, qd, 1.0, 0, True)
+    assert float((dw32 - want).norm() / want.norm()) < 1e-5
+    assert float((dw32 - want).abs().max() / want.abs().max()) < 1e-5
+    assert torch.equal(dw16, dw32.to(torch.bfloat16)) and torch.equal(dh16, dh32)
+
+
 # Logits of at most 128 tokens come from 256 x 128 tiles (two steps of 32 k at H=64, the shortest): one token, a wave's 64 and one
 # more, the last size of the rule and the first behind it; a vocabulary that ends inside a tile, its last group moved back (V >= 1024) or
 # not, chunks of one tile, a fp32 weight with its label residual.  The forward accumulates every logit in the same order as the square
