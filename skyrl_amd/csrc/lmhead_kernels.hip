@@ -585,7 +585,7 @@ struct GemmArgs {
   float* P;
   int p_first, p_last;
   // Number of splits of the contraction: workgroups per C tile, each with its share of the k-tile pairs and its own slab of P,
-  // summed by lmhead_dh_reduce.  splits_dev, when not NULL, replaces it (what compact_active_rows chose for its token count).
+  // summed by lmhead_dh_reduce; in lmhead_bwd_dh_shares a code of Shares.  splits_dev, when not NULL, replaces it (what compact_active_rows chose for its token count).
   int splits;
   const int* splits_dev;
   // When not NULL: row m of the bf16 output is row row_map[m] of C.
@@ -631,8 +631,57 @@ __host__ __device__ inline int64_t split_cost(const SplitProblem& p, int tokens,
   return (alone > spread ? alone : spread) + (splits > 1 ? items * 15 + 4 * p.ncu : 0);
 }
 
+// Shares.  Where dHidden is alone in its launch, a whole number of workgroups per tile leaves CUs idle: 96 tiles go in two splits on 192 of 256.  So
+// the tiles may also be taken in groups of b, u workgroups each, and every workgroup takes an equal share of its group's k-tile pairs, laid end to
+// end: the end of one tile, whole tiles, the beginning of another.  Splits are groups of one tile.  Group g holds tiles g, g + G, g + 2 G, ... of the
+// launch's order, G groups in all: the workgroups at one place j of their groups read the same range of the vocabulary for G neighbouring tiles
+// and come one behind the other, on one XCD.  Splits -> shares, the GEMM launch: 1437 -> 1251 us at 96 tiles (draft loss of 2868 tokens, H=2048,
+// V=151936), one round and a part -> shares 2457 -> 1582 at 288 tiles (draft loss of 8192, H=2304, V=64000; pass 9135 -> 8282) and 2580 -> 2311 at
+// 400 (5120 tokens, H=5120, V=64000), three quarters of a round 1877 -> 1578 at 192 (2868 of 4096 tokens, H=4096, V=100000).  112 tiles in two splits, 224
+// CUs, draw the power that 256 do: 1261 and 1290, hence the term for it in share_cost().
+struct Shares {
+  int b, u, groups;
+  __host__ __device__ int workgroups() const { return groups * u; }
+  __host__ __device__ int slots() const { return groups * (u + b - 1); }
+  // Group g: its tiles, and the first and last of them that workgroup j shares in, the first and last workgroup of its i-th tile.
+  __host__ __device__ int tiles_of(int g, int tiles) const { return (tiles - g + groups - 1) / groups; }
+  __host__ __device__ int first_tile(int j, int bg) const { return j * bg / u; }
+  __host__ __device__ int last_tile(int j, int bg) const { return ((j + 1) * bg + u - 1) / u - 1; }
+  __host__ __device__ int first_workgroup(int i, int bg) const { return i * u / bg; }
+  __host__ __device__ int last_workgroup(int i, int bg) const { return ((i + 1) * u + bg - 1) / bg - 1; }
+  // The slab of workgroup j's sums for the i-th tile: j + i differs along a group, because each step goes on to the next of either.
+  __host__ __device__ int slot(int g, int i, int j) const { return (j + i) * groups + g; }
+};
+constexpr int kMaxGroup = 32;
+// code: u, and b above its lowest eight bits where it is not 1.
+__host__ __device__ inline Shares shares_of(int code, int tiles) {
+  const int b = code < 256 ? 1 : code >> 8;
+  return Shares{b, code & 255, b == 1 ? tiles : (tiles + b - 1) / b};
+}
+// Groups of b >= 2 tiles, as many workgroups each as the CUs hold at once, rated as above.  A workgroup's further tiles cost it an epilogue and
+// another beginning each.  `code` is set where the answer is below INT64_MAX.
+__host__ __device__ inline int64_t share_cost(const SplitProblem& p, int tokens, int b, int& code) {
+  const int tiles = (tokens + BM - 1) / BM * p.tiles_h;
+  if (p.dw_tiles || b > tiles) return INT64_MAX;
+  const int groups = (tiles + b - 1) / b;
+  int u = p.ncu / groups;
+  u = u < kMaxSplits ? u : kMaxSplits;
+  if (u < 1) return INT64_MAX;
+  const Shares s{b, u, groups};
+  const int64_t pairs = ((int64_t)p.pairs * b + u - 1) / u;
+  if (s.slots() > p.slots || pairs < kMinSplitPairs) return INT64_MAX;
+  code = b << 8 | u;
+  const int64_t len = 2 * pairs + 10 * ((b + u - 1) / u + (b % u && u % b ? 1 : 0));
+  const int64_t busy = (int64_t)s.workgroups() * 7 / 6;  // behind six sevenths of the CUs the power is what limits
+  return len * (busy > p.ncu ? busy : p.ncu) + (int64_t)s.slots() * 15 + 4 * p.ncu;
+}
+
 // BKM: the B operand is K-major.  The two variants are separate instantiations of the whole tile (mainloop and
 // epilogue) so that their accumulators never meet at a join, where the register allocator would shuffle all 256 of them.
+// Tile (tm, tn), its k-tiles k0 .. k0 + nk - 1, the slab `slot` of P; partial: the sum stays there.
+template <bool BKM>
+__device__ __forceinline__ void gemm_tile_at(const GemmArgs& p, int M, int N, int tm, int tn, int k0, int nk, int k_back, size_t slot, bool partial, char* lds);
+
 template <bool BKM>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bid, char* lds) {
   int M = p.M, N = p.N, nk = p.nk;
@@ -663,6 +712,11 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bid, char* lds)
     if (nk == 0 && !p.p_first) return;  // a narrow last chunk: this split adds nothing to its slab
   }
   banded_tile(logical, tiles_m, tiles_n, kGroupM, tm, tn);
+  gemm_tile_at<BKM>(p, M, N, tm, tn, k0, nk, k_back, (size_t)(split * tiles + logical), !p.p_last || splits > 1, lds);
+}
+
+template <bool BKM>
+__device__ __forceinline__ void gemm_tile_at(const GemmArgs& p, int M, int N, int tm, int tn, int k0, int nk, int k_back, size_t slot, bool partial, char* lds) {
 #if LMHEAD_ABLATE & 16
   Operand a{p.A, p.lda, (tm % 4) * BM, p.a_rows};
   Operand b{p.B, p.ldb, (tn % 8) * BN, p.b_rows};
@@ -686,7 +740,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bid, char* lds)
   const int lrow = lane & 15, kq = lane >> 4;
 
   if (p.P) {
-    float* part = p.P + ((size_t)(split * tiles + tm * tiles_n + tn) * NWAVES + wave) * kSlabWaveFloats + (size_t)lane * 4;
+    float* part = p.P + (slot * NWAVES + wave) * kSlabWaveFloats + (size_t)lane * 4;
     if (!p.p_first) {  // sixteen loads in flight at a time: one at a time costs a round trip to HBM each (36 us per tile)
 #pragma unroll
       for (int i = 0; i < TM; i += 2) {
@@ -697,7 +751,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bid, char* lds)
         for (int x = 0; x < 2 * TN; ++x) acc[i + x / TN][x % TN] += t[x];
       }
     }
-    if (!p.p_last || splits > 1) {
+    if (partial) {
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -803,6 +857,36 @@ __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_gemm(const GemmArgs p0, c
   else gemm_tile<false>(p0, id, lds);
 }
 
+// dHidden alone (a frozen weight, the draft loss, a dW launch of its own): its tiles in equal shares (Shares; B K-major, tokens along M).
+__global__ __launch_bounds__(NTHREADS) void lmhead_bwd_dh_shares(const GemmArgs p) {
+  __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+  const int M = p.T_dev ? __builtin_amdgcn_readfirstlane(*p.T_dev) : p.M;
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN, tiles = tiles_m * tiles_n;
+  Shares s = shares_of(p.splits_dev ? __builtin_amdgcn_readfirstlane(*p.splits_dev) : p.splits, tiles);
+  s.groups = __builtin_amdgcn_readfirstlane(s.groups);
+  if ((int)blockIdx.x >= s.workgroups()) return;
+  const int id = xcd_contiguous(blockIdx.x, s.workgroups());
+  // All of this in scalar registers: the mainloop leaves no vector register to hold it.
+  const int j = __builtin_amdgcn_readfirstlane(id / s.groups), g = id - j * s.groups, bg = __builtin_amdgcn_readfirstlane(s.tiles_of(g, tiles));
+  const int pairs = p.nk / 2, all = bg * pairs;  // below 2^20, and times u below 2^26
+  const int from = __builtin_amdgcn_readfirstlane(all * j / s.u), to = __builtin_amdgcn_readfirstlane(all * (j + 1) / s.u);
+  const int first = __builtin_amdgcn_readfirstlane(s.first_tile(j, bg)), last = __builtin_amdgcn_readfirstlane(s.last_tile(j, bg));
+  for (int i = first; i <= last; ++i) {
+    const int k0 = from > i * pairs ? from - i * pairs : 0, k1 = to < (i + 1) * pairs ? to - i * pairs : pairs;
+    const int nk = 2 * (k1 - k0);
+    if (nk == 0 && !p.p_first) continue;  // a narrow last chunk: nothing to add to this slab
+    if (i > first) __syncthreads();  // every wave has taken its rows of the tile before from LDS
+    int tm, tn;
+    banded_tile(i * s.groups + g, tiles_m, tiles_n, kGroupM, tm, tn);
+    const bool alone = __builtin_amdgcn_readfirstlane(s.first_workgroup(i, bg)) == __builtin_amdgcn_readfirstlane(s.last_workgroup(i, bg));
+    // The lanes' copy offsets and LDS addresses formed once for all tiles would be vector registers that the mainloop does not have.
+    GemmArgs q = p;
+    int lds_at = 0;
+    asm volatile("" : "+s"(q.lda), "+s"(q.ldb), "+s"(q.ldc), "+s"(lds_at));
+    gemm_tile_at<true>(q, M, p.N, tm, tn, 2 * k0, nk, k1 == pairs ? p.k_back : 0, (size_t)s.slot(g, i, j), !p.p_last || !alone, lds + lds_at);
+  }
+}
+
 // dHidden rows from the slabs of a split contraction: C[m, n] = bf16(sum of the slabs), added in split order.  One workgroup per
 // 16 tokens x 128 columns (an MFMA row block of a wave): 16-byte loads of contiguous slab pieces, 16-byte row pieces out
 // through LDS.  HBM-bound, splits x tokens x H x 4 bytes: 8 us at 240 slab tiles (60 MB).
@@ -817,20 +901,30 @@ constexpr int kReduceGroups = NWAVES * TM;  // workgroups per tile
 
 __global__ __launch_bounds__(256) void lmhead_dh_reduce(const DhReduceArgs a) {
   __shared__ __attribute__((aligned(16))) uint16_t rows[MT][WN + 8];
-  const int splits = a.splits_dev ? *a.splits_dev : a.splits;
-  const int M = a.T_dev ? *a.T_dev : a.M;
-  const int tiles_n = (a.H + BN - 1) / BN, tiles = (M + BM - 1) / BM * tiles_n;
+  const int splits = __builtin_amdgcn_readfirstlane(a.splits_dev ? *a.splits_dev : a.splits);
+  const int M = __builtin_amdgcn_readfirstlane(a.T_dev ? *a.T_dev : a.M);
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (a.H + BN - 1) / BN, tiles = tiles_m * tiles_n;
   const int tile = blockIdx.x / kReduceGroups, wave = blockIdx.x / TM % NWAVES, i = blockIdx.x % TM;
-  if (splits < 2 || tile >= tiles) return;  // without splits the GEMM epilogue has written C
-  const int m0 = tile / tiles_n * BM + wave / WAVES_N * WM + i * MT;
-  const int n0 = tile % tiles_n * BN + wave % WAVES_N * WN;
+  if (tile >= tiles) return;
+  const Shares sh = shares_of(splits, tiles);
+  int in_group = 0, g = tile, first = 0, last = sh.u - 1;
+  if (sh.b > 1) {  // splits need none of these divisions
+    in_group = tile / sh.groups, g = tile - in_group * sh.groups;
+    const int bg = sh.tiles_of(g, tiles);
+    first = sh.first_workgroup(in_group, bg), last = sh.last_workgroup(in_group, bg);
+  }
+  if (first == last) return;  // one workgroup made the tile, and its epilogue has written C
+  int tm, tn;
+  banded_tile(tile, tiles_m, tiles_n, kGroupM, tm, tn);
+  const int m0 = tm * BM + wave / WAVES_N * WM + i * MT;
+  const int n0 = tn * BN + wave % WAVES_N * WN;
   if (m0 >= M || n0 >= a.H) return;
   const int tid = threadIdx.x;
-  const float* part = a.P + ((size_t)tile * NWAVES + wave) * kSlabWaveFloats + (size_t)(i * TN) * (64 * 4) + (size_t)tid * 4;
-  const size_t slab = (size_t)tiles * kSlabTileFloats;
+  const float* part = a.P + ((size_t)sh.slot(g, in_group, first) * NWAVES + wave) * kSlabWaveFloats + (size_t)(i * TN) * (64 * 4) + (size_t)tid * 4;
+  const size_t slab = (size_t)sh.groups * kSlabTileFloats;
   f32x4 sum[2] = {*(const f32x4*)part, *(const f32x4*)(part + 1024)};
 #pragma unroll 4
-  for (int s = 1; s < splits; ++s) {
+  for (int s = 1; s <= last - first; ++s) {
     sum[0] += *(const f32x4*)(part + (size_t)s * slab);
     sum[1] += *(const f32x4*)(part + (size_t)s * slab + 1024);
   }
@@ -1048,11 +1142,13 @@ __global__ __launch_bounds__(kCompactThreads) void compact_active_rows(const flo
       counts[b] = left < 0 ? 0 : (left > block ? block : (int)left);
     }
   }
-  for (int b = wave; b < nblocks; b += kCompactThreads / 64) {  // lane l rates l + 1 splits; the cheapest, of equals the fewest, wins
+  for (int b = wave; b < nblocks; b += kCompactThreads / 64) {  // lane l rates l + 1 splits and groups of l + 2 tiles; the cheapest, of equals the fewest, wins
     const long long left = (long long)n - (long long)b * block;
     const int tokens = left < 0 ? 0 : (left > block ? block : (int)left);
     long long best = split_cost(split, tokens, lane + 1);
-    int splits = lane + 1;
+    int splits = lane + 1, code = 0;
+    const long long shared = lane < kMaxGroup - 1 ? share_cost(split, tokens, lane + 2, code) : INT64_MAX;
+    if (shared < best) best = shared, splits = code;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       const long long c = __shfl_xor(best, o, 64);
@@ -1252,9 +1348,8 @@ SplitProblem split_problem(int64_t T, int64_t H, int64_t vc, bool want_dw, int64
 
 // Slab tiles of dHidden partial sums for at most T tokens and chunks of vc columns: room for one tile per CU, at least two per dHidden
 // tile; none beyond one per dHidden tile from 192 tiles on, where dW tiles in the same launch fill the CUs that dHidden leaves idle.
-// The line is drawn for launches with dW.  Without (a frozen weight, the draft loss, a dW launch of its own) it is not measured, and
-// split_cost would go further: 288 tiles (T=8192, H=2304) are rated 1.6 times as long in one piece as in eight, and 96 tiles (draft loss of
-// 2868 active tokens, H=2048), which room for 320 slabs lets go in two, a quarter longer than in eight.
+// The line is drawn for launches with dW.  Without (a frozen weight, the draft loss, a dW launch of its own) shares would go further where there is
+// room for them: the draft loss always has it, a frozen weight from the room that row compaction brings (carve_bwd).
 constexpr int64_t kSplitBelowTiles = 192;
 int64_t dh_tiles(int64_t T, int64_t H) { return (T + BM - 1) / BM * ((H + BN - 1) / BN); }
 int64_t slab_slots(int64_t T, int64_t H, int64_t vc) {
@@ -1271,6 +1366,11 @@ int best_splits(const SplitProblem& p, int64_t tokens) {
   for (int k = 2; k <= kMaxSplits; ++k) {
     const int64_t c = split_cost(p, (int)tokens, k);
     if (c < best_cost) best = k, best_cost = c;
+  }
+  for (int b = 2; b <= kMaxGroup; ++b) {
+    int code = 0;
+    const int64_t c = share_cost(p, (int)tokens, b, code);
+    if (c < best_cost) best = code, best_cost = c;
   }
   return best;
 }
@@ -1530,12 +1630,18 @@ hipError_t launch_bwd_dz(hipStream_t s, bool entgrad, DzArgs z) {
 // Both problems (p1 may be empty) must have an even number of k-tiles: every caller contracts over padded extents that
 // are multiples of 256, or over vocabulary rows that reads_weight_in_place() admits.
 // slots: slab tiles there is room for, which bounds splits * tiles when the splits are chosen on the device.
-hipError_t launch_bwd_gemm(hipStream_t s, const GemmArgs& p0, const GemmArgs& p1, int64_t slots) {
+hipError_t launch_bwd_gemm(hipStream_t s, const GemmArgs& p0, const GemmArgs& p1, int64_t slots, int ncu) {
   if ((p0.nk & 1) || (p1.nk & 1)) return hipErrorInvalidValue;
-  unsigned t0 = gemm_tiles(p0) * (unsigned)p0.splits;
-  if (p0.splits_dev && (int64_t)t0 < slots) t0 = (unsigned)slots;
   const unsigned t1 = gemm_tiles(p1);
+  const int tiles0 = (int)gemm_tiles(p0);
+  unsigned t0 = (unsigned)shares_of(p0.splits, tiles0).workgroups();
+  if (p0.splits_dev && (int64_t)t0 < slots) t0 = (unsigned)slots;
   Timed timed(kBwdChunkGemm, s);
+  if (t1 == 0 && p0.b_kmajor) {
+    if (p0.splits_dev && (int)t0 < ncu) t0 = (unsigned)ncu;
+    hipLaunchKernelGGL(lmhead_bwd_dh_shares, dim3(t0), dim3(NTHREADS), 0, s, p0);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(lmhead_bwd_gemm, dim3(t0 + t1), dim3(NTHREADS), 0, s, p0, p1, (int)t0);
   return hipGetLastError();
 }
@@ -1553,8 +1659,8 @@ inline bool few_token_dw(bool want_dw, bool adds, int64_t T, int64_t H, int64_t 
 // The sum over the slabs of a split dHidden contraction; g is the GEMM of the last chunk.
 hipError_t launch_dh_reduce(hipStream_t s, const GemmArgs& g, int64_t slots) {
   if (!g.splits_dev && g.splits < 2) return hipSuccess;
-  // only a problem with at most half as many tiles as slots is ever split
-  const int64_t tiles = gemm_tiles(g), most = g.splits_dev && slots / 2 < tiles ? slots / 2 : tiles;
+  // a problem with more tiles than slots is never split
+  const int64_t tiles = gemm_tiles(g), most = g.splits_dev && slots < tiles ? slots : tiles;
   if (most < 1) return hipSuccess;
   Timed timed(kDhReduce, s);
   hipLaunchKernelGGL(lmhead_dh_reduce, dim3((unsigned)(most * kReduceGroups)), dim3(256), 0, s,
@@ -1612,9 +1718,11 @@ SoftCeBwdWorkspace lay_out_softce_bwd(void* ws, int64_t T, int64_t H, int64_t V,
   return w;
 }
 
-// As carve_bwd; a quarter more slabs let a batch with few active tokens split further.
+// As carve_bwd; a quarter more slabs let a batch with few active tokens split further, and 64 MiB at least of more lets dHidden tiles that fill
+// whole rounds and a part of one go in equal shares.
 SoftCeBwdWorkspace carve_softce_bwd(void* ws, int64_t T, int64_t H, int64_t V, int64_t vc, size_t ws_bytes) {
-  const int64_t slots = slab_slots(T, H, vc), wanted = (slots + slots / 4) * kSlabTileFloats;
+  const int64_t slots = slab_slots(T, H, vc), more = dh_tiles(T, H) >= kSplitBelowTiles && slots < 4 * 256 ? 256 : slots / 4;
+  const int64_t wanted = (slots + more) * kSlabTileFloats;
   const SoftCeBwdWorkspace w = lay_out_softce_bwd(ws, T, H, V, vc, wanted);
   if (w.bytes <= ws_bytes) return w;
   return lay_out_softce_bwd(ws, T, H, V, vc, fitting_slabs(wanted, dh_tiles(T, H) * kSlabTileFloats, w.bytes - ws_bytes));
@@ -1699,6 +1807,7 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
                     const float* dw_in, float* dw_f32, uint16_t* dw_bf16, int64_t vc, const BwdWorkspace& w, float p_shift,
                     hipStream_t s) {
   const int64_t Tpad = round_up(Tb, 256), Vpad = round_up(V, 256);
+  const int ncu = compute_units();
   const bool w_in_place = reads_weight_in_place(V);
   hipError_t e;
   const bool few = few_token_dw(want_dw, dw_in != nullptr, Tb, H, V);
@@ -1717,7 +1826,7 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
   const VocabTail tail = vocab_tail(V);
   // The splits are those of a full chunk: the slabs are carried from chunk to chunk.
   const int splits =
-      !T_dev && w_in_place ? best_splits(split_problem(Tb, H, vc < Vpad ? vc : Vpad, want_dw && !few, w.slots, compute_units()), Tb) : 1;
+      !T_dev && w_in_place ? best_splits(split_problem(Tb, H, vc < Vpad ? vc : Vpad, want_dw && !few, w.slots, ncu), Tb) : 1;
   const int64_t nchunks = (Vpad + vc - 1) / vc;
   auto chunk_width = [&](int64_t ci) { return (Vpad - ci * vc) < vc ? (Vpad - ci * vc) : vc; };  // multiple of 256
   const GemmArgs none{};
@@ -1727,7 +1836,7 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
     // width, and it needs a second panel.
     const int64_t vc0 = ci * vc, vcw = chunk_width(ci);
     const DzArgs z{Wp, (int)ld_weight, Hp, (int)ld_hidden, (int)Tb, (int)Hk, (int)V, rcp_temperature, labels, row_lse, row_pz,
-                   dlogprobs, dentropy, (int)vc0, (int)(vcw / 256), 0, tail, w.D, (int)(vcw + kLdPad), T_dev, resid, p_shift, compute_units()};
+                   dlogprobs, dentropy, (int)vc0, (int)(vcw / 256), 0, tail, w.D, (int)(vcw + kLdPad), T_dev, resid, p_shift, ncu};
     e = launch_bwd_dz(s, dentropy != nullptr, z);
     if (e != hipSuccess) return (int)e;
     // dHidden[t, h] (+)= sum_v D[t, v] . weight^T[h, vc0 + v]        (A = weight^T rows at k offset vc0, B = D rows)
@@ -1752,10 +1861,10 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
     if (few) {
       Timed timed(kBwdDwFew, s);
       e = launch_bwd_dw_few(s, DwFewArgs{Hp, (int)ld_hidden, w.D, (int)(vcw + kLdPad), (int)Tb, T_dev, (int)H, (int)n_rows,
-                                         moved ? gw.n_tail : 0x7fffffff, gw.n_back, cf, cb, compute_units()});
+                                         moved ? gw.n_tail : 0x7fffffff, gw.n_back, cf, cb, ncu});
       if (e != hipSuccess) return (int)e;
     }
-    e = launch_bwd_gemm(s, gh, gw, w.slots);
+    e = launch_bwd_gemm(s, gh, gw, w.slots, ncu);
     if (e == hipSuccess && last) e = launch_dh_reduce(s, gh, w.slots);
     if (e != hipSuccess) return (int)e;
   }
@@ -2072,10 +2181,11 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
   hipError_t e;
   const bool w_in_place = reads_weight_in_place(V);
   const VocabTail tail = vocab_tail(V);
+  const int ncu = compute_units();
   {  // tokens without an upstream gradient (what the supervision mask removes) have a zero row and take no part
     Timed timed(kCompactRows, s);
     hipLaunchKernelGGL(compact_active_rows, dim3(1), dim3(kCompactThreads), 0, s, dloss, (const float*)nullptr, (int)T, (int)T, 1,
-                       split_problem(T, H, vc, false, w.slots, compute_units()), w.idx, w.counts);
+                       split_problem(T, H, vc, false, w.slots, ncu), w.idx, w.counts);
   }
   if ((e = hipGetLastError()) != hipSuccess) return (int)e;
   {
@@ -2098,7 +2208,7 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
     const int64_t vc0 = ci * vc, vcw = (Vpad - vc0) < vc ? (Vpad - vc0) : vc;
     const SoftCeDzArgs z{Wp, (int)ld_weight, w.S, (int)H, (int)V, w.counts + 1, rcp_temperature, w.lse_student,
                          w.lse_teacher, w.dloss, (int)vc0, (int)(vcw / 256), (int)(2 * Tp / BN), tail, w.D, (int)(vcw + kLdPad),
-                         compute_units()};
+                         ncu};
     {
       Timed timed(kSoftCeDz, s);
       const TileShapes shapes = tile_shapes_of_any_count(H, z.tiles_m, z.tiles_m * z.tiles_n, z.ncu);
@@ -2113,7 +2223,7 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
     GemmArgs gh = dhidden_gemm(w.D, vcw + kLdPad, Tp, Wp, ld_weight, w_in_place ? nullptr : w.Wt, Vpad + kLdPad, vc0, vcw, V, T, H,
                                (uint16_t*)d_student_hidden, w.dHacc, first, last, w.counts + 1);
     gh.splits_dev = w_in_place ? w.counts + 2 : nullptr, gh.row_map = w.idx;
-    e = launch_bwd_gemm(s, gh, none, w.slots);
+    e = launch_bwd_gemm(s, gh, none, w.slots, ncu);
     if (e == hipSuccess && last) e = launch_dh_reduce(s, gh, w.slots);
     if (e != hipSuccess) return (int)e;
   }

@@ -97,6 +97,33 @@ def test_split_hidden_gradient(T, H, V, vc, keep, cuda_device):
     assert torch.equal(active[0], ops.lmhead_bwd_bf16(h, w, y, lse, pz, gd, qd, 1.0, vc, True)[0])   # a fixed order of addition
 
 
+# Alone in its launch, dHidden goes in equal shares of its tiles where whole workgroups per tile leave CUs idle: a round of 256 tiles and a
+# part of one, with tiles of one workgroup among them, three tiles for eight workgroups, both in one chunk and in several of which the last is
+# narrow and ends in a moved group, and token counts that the host does not know.  Beside dW the same sums run whole or in splits: fp32 sums of
+# V <= 2^15 products in another order, rounded to bf16 once: an element in some 200 falls to the other side, sqrt(1 / 200) 2^-8 = 3e-4.
+@pytest.mark.parametrize("T,H,V,vc", [(4500, 4160, 8000, 0), (4500, 4160, 9300, 4096), (1500, 4096, 32000, 0), (1400, 4096, 32001, 20480)])
+@pytest.mark.parametrize("keep", [1.0, 0.7])
+def test_hidden_gradient_in_shares(T, H, V, vc, keep, cuda_device):
+    hidden, weight, labels, g, q = _operands(T, H, V, seed=T + V)
+    keep_rows = torch.rand(T, generator=torch.Generator().manual_seed(T)) < keep
+    h, w, y, gd, qd = (x.to(cuda_device) for x in (hidden, weight, labels, g * keep_rows, q * keep_rows))
+    _, _, lse, pz = ops.lmhead_fwd(h, w, y, 1.0, True)
+    want = ops.lmhead_bwd_bf16(h, w, y, lse, pz, gd, qd, 1.0, vc)[0].float()
+    for active in (False, True):
+        dh = ops.lmhead_bwd_hidden(h, w, y, lse, pz, gd, qd, 1.0, vc, active)
+        assert float((dh.float() - want).norm() / want.norm()) < 1e-3
+        assert float((dh.float() - want).abs().max() / want.abs().max()) < 2**-7  # no tile is missing, none added twice
+        assert not dh[(~keep_rows).to(cuda_device)].any()
+        assert torch.equal(dh, ops.lmhead_bwd_hidden(h, w, y, lse, pz, gd, qd, 1.0, vc, active))  # a fixed order of addition
+    s, teacher = h.clone().requires_grad_(True), h.roll(1, 0)
+    per_token = soft_ce_from_hidden(s.reshape(1, T, H), teacher.reshape(1, T, H), w)
+    per_token.backward(gd.reshape(1, T))
+    probs = [torch.softmax(x.float() @ w.t().float(), dim=-1) for x in (h, teacher)]
+    dz = (gd.unsqueeze(1) * (probs[0] - probs[1])).to(torch.bfloat16).float()
+    ref = dz @ w.float()  # dz rounded to bf16 from probabilities that differ in fp32 roundings, dHidden rounded to bf16: 2^-8 / sqrt(3) each
+    assert float((s.grad.float() - ref).norm() / ref.norm()) < 5e-3
+
+
 # The first vocabulary chunk of the top-k search is stored and searched: its width follows the number of tokens, the later ones the
 # room for candidate lists and k.  One chunk only, one column behind the first, many equal logits at the k-th rank, k = V.
 @pytest.mark.parametrize("T,H,V,k", [(3, 64, 8192, 5), (300, 64, 32769, 32), (260, 64, 33025, 1000), (2050, 64, 8449, 64), (5, 64, 40, 40)])
