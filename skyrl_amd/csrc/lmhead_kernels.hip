@@ -1110,30 +1110,41 @@ constexpr int kCompactThreads = 1024;
 __global__ __launch_bounds__(kCompactThreads) void compact_active_rows(const float* __restrict__ g, const float* __restrict__ q,
                                                                        int T, int block, int nblocks, SplitProblem split,
                                                                        int* __restrict__ idx, int* __restrict__ counts) {
-  __shared__ int wave_sum[kCompactThreads / 64];
-  __shared__ int carry;
+  // A step takes four tokens per thread: their loads travel together, and every wave scans the 64 counts of the step by itself, so that one
+  // barrier stands between the counts and the list.  What bounds it is that chain: with a token per thread and the counts added up by one thread
+  // 12.1 -> 7.7 us at T=8192, 6.7 -> 5.4 at 4096, 6.6 -> 5.2 at 2100.
+  constexpr int kTokens = 4;
+  static_assert(kTokens * kCompactThreads / 64 == 64, "one lane per count");
+  __shared__ int count[2][64];  // of tokens t0 + k * kCompactThreads + wave * 64 .. + 63: k * 16 + wave; steps take turns
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (tid == 0) carry = 0;
-  __syncthreads();
-  for (int t0 = 0; t0 < T; t0 += kCompactThreads) {
-    const int t = t0 + tid;
-    const bool active = t < T && (g[t] != 0.f || (q && q[t] != 0.f));
-    const unsigned long long ballot = __ballot(active);
-    const int before = __popcll(ballot & ((1ull << lane) - 1ull));
-    if (lane == 0) wave_sum[wave] = __popcll(ballot);
-    __syncthreads();
-    int base = carry;
-    for (int w = 0; w < wave; ++w) base += wave_sum[w];
-    if (active) idx[base + before] = t;
-    __syncthreads();
-    if (tid == 0) {
-      int total = 0;
-      for (int w = 0; w < kCompactThreads / 64; ++w) total += wave_sum[w];
-      carry += total;
+  int n = 0;
+  for (int t0 = 0, turn = 0; t0 < T; t0 += kTokens * kCompactThreads, turn ^= 1) {
+    unsigned long long ballot[kTokens];
+#pragma unroll
+    for (int k = 0; k < kTokens; ++k) {
+      const int t = t0 + k * kCompactThreads + tid;
+      const int tc = t < T ? t : T - 1;
+      const float gv = g[tc], qv = q ? q[tc] : 0.f;
+      ballot[k] = __ballot(t < T && (gv != 0.f || qv != 0.f));
     }
+#pragma unroll
+    for (int k = 0; k < kTokens; ++k)
+      if (lane == 0) count[turn][k * (kCompactThreads / 64) + wave] = __popcll(ballot[k]);
     __syncthreads();
+    const int mine = count[turn][lane];
+    int upto = mine;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int below = __shfl_up(upto, o, 64);
+      upto += lane >= o ? below : 0;
+    }
+#pragma unroll
+    for (int k = 0; k < kTokens; ++k) {
+      const int base = n + __shfl(upto - mine, k * (kCompactThreads / 64) + wave, 64);
+      if (ballot[k] >> lane & 1) idx[base + __popcll(ballot[k] & ((1ull << lane) - 1ull))] = t0 + k * kCompactThreads + tid;
+    }
+    n += __shfl(upto, 63, 64);
   }
-  const int n = carry;
   for (int b = tid; b <= nblocks; b += kCompactThreads) {
     if (b == 0) {
       counts[0] = n;
