@@ -210,36 +210,77 @@ constexpr int kMaxK = 1024;
 // rewritten.
 __device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
+constexpr int kInRegisters = 512;  // keys that keep_largest() takes into registers
+
 // The k largest of the M > k keys in `list` (LDS, unique keys), moved to its front by the calling wave: a bisection over the key
-// bits finds a threshold that exactly k keys reach (a pass over the keys per bit, usually 20 to 30 bits until the count is exact).
-__device__ __forceinline__ void keep_largest(key_t* list, int M, int k, int lane) {
-  key_t reach = 0;  // grows bit by bit while at least k keys reach it; done when exactly k do
-  for (int b = 63; b >= 0; --b) {
-    const key_t trial = reach | ((key_t)1 << b);
-    int c = 0;
-    for (int e = lane; e < M; e += 64) c += list[e] >= trial ? 1 : 0;
+// bits finds a threshold that exactly k keys reach (a count of the keys per bit, usually 20 to 30 bits until it is exact).  BATCHES: M <= 64 BATCHES,
+// and a lane holds its keys in registers, so that a count is a few comparisons and votes; 0: any M, from LDS, with a sum over the lanes per bit.  What
+// bounds it is that chain, a wave per token.  From LDS -> registers, T=1800, k=32: topk_init (33 keys a token) 28 -> 22 us,
+// topk_select (300) 20 -> 10; pass 1032 -> 1013, at k=128, T=600, H=1024, V=128000 421 -> 405.
+template <int BATCHES>
+__device__ __forceinline__ void keep_largest_of(key_t* list, int M, int k, int lane) {
+  if constexpr (BATCHES == 0) {
+    key_t reach = 0;  // grows bit by bit while at least k keys reach it; done when exactly k do
+    for (int b = 63; b >= 0; --b) {
+      const key_t trial = reach | ((key_t)1 << b);
+      int c = 0;
+      for (int e = lane; e < M; e += 64) c += list[e] >= trial ? 1 : 0;
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) c += __shfl_xor(c, o, 64);
-    if (c >= k) {
-      reach = trial;
-      if (c == k) break;
+      for (int o = 32; o >= 1; o >>= 1) c += __shfl_xor(c, o, 64);
+      if (c >= k) {
+        reach = trial;
+        if (c == k) break;
+      }
     }
-  }
-  int w = 0;  // in-place compaction: a step reads 64 entries and writes at or below where it read
-  for (int base = 0; base < M; base += 64) {
-    const int e = base + lane;
-    const key_t x = e < M ? list[e] : 0;
-    const bool keep = e < M && x >= reach;
-    const unsigned long long mask = __ballot(keep);
+    int w = 0;  // in-place compaction: a step reads 64 entries and writes at or below where it read
+    for (int base = 0; base < M; base += 64) {
+      const int e = base + lane;
+      const key_t x = e < M ? list[e] : 0;
+      const bool keep = e < M && x >= reach;
+      const unsigned long long mask = __ballot(keep);
+      wave_lds_fence();
+      if (keep) list[w + __popcll(mask & (((key_t)1 << lane) - 1))] = x;
+      w += (int)__popcll(mask);
+      wave_lds_fence();
+    }
+  } else {
+    key_t x[BATCHES];
+#pragma unroll
+    for (int u = 0; u < BATCHES; ++u) x[u] = u * 64 + lane < M ? list[u * 64 + lane] : 0;  // 0 reaches no trial
+    key_t reach = 0;
+    for (int b = 63; b >= 0; --b) {
+      const key_t trial = reach | ((key_t)1 << b);
+      int c = 0;
+#pragma unroll
+      for (int u = 0; u < BATCHES; ++u) c += (int)__popcll(__ballot(x[u] >= trial));
+      if (c >= k) {
+        reach = trial;
+        if (c == k) break;
+      }
+    }
     wave_lds_fence();
-    if (keep) list[w + __popcll(mask & (((key_t)1 << lane) - 1))] = x;
-    w += (int)__popcll(mask);
+    int w = 0;
+#pragma unroll
+    for (int u = 0; u < BATCHES; ++u) {
+      const bool keep = u * 64 + lane < M && x[u] >= reach;
+      const unsigned long long mask = __ballot(keep);
+      if (keep) list[w + __popcll(mask & (((key_t)1 << lane) - 1))] = x[u];
+      w += (int)__popcll(mask);
+    }
     wave_lds_fence();
   }
 }
+__device__ __forceinline__ void keep_largest(key_t* list, int M, int k, int lane) {
+  if (M <= 64) keep_largest_of<1>(list, M, k, lane);
+  else if (M <= 256) keep_largest_of<4>(list, M, k, lane);
+  else if (M <= kInRegisters) keep_largest_of<8>(list, M, k, lane);
+  else keep_largest_of<0>(list, M, k, lane);
+}
 
 constexpr int kSelectStage = 1024;   // candidates one bulk round takes into LDS, behind the list
-constexpr int kSelectBulkMin = 96;   // fewer candidates than this are inserted one by one
+// Fewer candidates than this are inserted one by one, each of which costs a search for the worst entry: where a bulk round works in registers
+// (keep_largest) it is the cheaper from four on (topk_select with 27 candidates, k=32, T=1800: 22.9 -> 7.0 us; pass 969 -> 953, at k=128 392 -> 372), else from 96.
+constexpr int kSelectBulkMin = 96, kSelectBulkMinInRegisters = 4;
 
 // best: [T, k] running lists (unordered), have: [T] entries of the list that are filled.  One wave per token; the list lives
 // in LDS while the wave works on it.  Many candidates (the first chunks, a large k, adversarial data) are merged in bulk: up to
@@ -277,7 +318,8 @@ __global__ __launch_bounds__(64 * kSelectWaves) void topk_select(int T, int k, k
   };
   const key_t* cl = cand + (size_t)t * (size_t)cap;
   int done = 0;
-  while (n - done >= kSelectBulkMin) {
+  const int bulk_min = n_have + n <= kInRegisters ? kSelectBulkMinInRegisters : kSelectBulkMin;
+  while (n - done >= bulk_min) {
     const int take = (n - done) < kSelectStage ? (n - done) : kSelectStage;
     for (int e = lane; e < take; e += 64) list[n_have + e] = cl[done + e];
     lds_fence();
@@ -352,7 +394,7 @@ __global__ __launch_bounds__(64 * kSelectWaves) void topk_select(int T, int k, k
 //   larger k, or so many equal logits that the list overflows: a bisection over the bits of the values (all threads count, one
 //     barrier per bit, fewer when the count comes out exact), and among equal values one over the columns.
 // Bound by the read of the logits.  Filling the lists through the candidate path instead (every logit passes while there is no
-// threshold) took 93 us for 32 tiles of 1024 columns at T=1800; first tiles of 8192 columns and this kernel take 61 + 31 us (the bisection alone: 61 + 45).
+// threshold) took 93 us for 32 tiles of 1024 columns at T=1800; first tiles of 8192 columns and this kernel take 61 + 22 us (the bisection alone: 61 + 45).
 constexpr int kInitLogits = 32;  // per thread
 constexpr int kInitList = 1024;
 constexpr int kInitListK = 128;

@@ -97,6 +97,24 @@ def test_split_hidden_gradient(T, H, V, vc, keep, cuda_device):
     assert torch.equal(active[0], ops.lmhead_bwd_bf16(h, w, y, lse, pz, gd, qd, 1.0, vc, True)[0])   # a fixed order of addition
 
 
+# Candidates of a later chunk that all beat the first chunk's 31 best: inserted one by one, or merged from 35 keys on in registers of one, four and
+# eight keys a lane, and from LDS behind 512; exact sums of two terms, so any order of the keys but torch's would show.
+@pytest.mark.parametrize("n", [1, 3, 4, 33, 34, 225, 226, 481, 482, 700])
+def test_topk_candidates_that_all_pass(n, cuda_device):
+    first, H, k, T = 32768, 64, 31, 3  # the first chunk of so few tokens
+    gen = torch.Generator().manual_seed(n)
+    weight = torch.zeros(first + n, H)
+    weight[:first, 0] = torch.randint(-64, 64, (first,), generator=gen).float()
+    late = torch.randperm(n, generator=gen).float()
+    weight[first:, 0], weight[first:, 1] = 64 + late // 8, (late % 8) / 8
+    hidden = torch.zeros(T, H)
+    hidden[:, :2] = 1.0
+    values, columns = topk_logits_from_hidden(hidden.to(torch.bfloat16).to(cuda_device), weight.to(torch.bfloat16).to(cuda_device), k)
+    logits = weight[:, 0] + weight[:, 1]
+    order = sorted(range(first + n), key=lambda v: (-float(logits[v]), v))[:k]  # higher first, lower column first among equals
+    assert values.cpu().tolist() == [[float(logits[v]) for v in order]] * T and columns.cpu().tolist() == [order] * T
+
+
 # Alone in its launch, dHidden goes in equal shares of its tiles where whole workgroups per tile leave CUs idle: a round of 256 tiles and a
 # part of one, with tiles of one workgroup among them, three tiles for eight workgroups, both in one chunk and in several of which the last is
 # narrow and ends in a moved group, and token counts that the host does not know.  Beside dW the same sums run whole or in splits: fp32 sums of
