@@ -619,6 +619,7 @@ struct SplitProblem {
   int pairs;      // k-tile pairs of a chunk's vocabulary
   int dw_tiles;   // dW tiles of the same launch (0: frozen weight)
   int slots;      // slab tiles there is room for
+  int shares;     // whether the launch may go in Shares
   int ncu;
 };
 __host__ __device__ inline int64_t split_cost(const SplitProblem& p, int tokens, int splits) {
@@ -653,6 +654,9 @@ struct Shares {
   __host__ __device__ int slot(int g, int i, int j) const { return (j + i) * groups + g; }
 };
 constexpr int kMaxGroup = 32;
+// Launches that may have more tiles than this: up to 64 tiles in four splits and more already fill nine tenths of the CUs, and calls of few tokens
+// notice what finding a share takes (draft loss of 20 tokens, H=896, V=246016, four tiles in 64 splits: GEMM 109 -> 111 us, their sum 11.6 -> 12.9).
+constexpr int64_t kSharesFromTiles = 65;
 // code: u, and b above its lowest eight bits where it is not 1.
 __host__ __device__ inline Shares shares_of(int code, int tiles) {
   const int b = code < 256 ? 1 : code >> 8;
@@ -662,17 +666,17 @@ __host__ __device__ inline Shares shares_of(int code, int tiles) {
 // another beginning each.  `code` is set where the answer is below INT64_MAX.
 __host__ __device__ inline int64_t share_cost(const SplitProblem& p, int tokens, int b, int& code) {
   const int tiles = (tokens + BM - 1) / BM * p.tiles_h;
-  if (p.dw_tiles || b > tiles) return INT64_MAX;
+  if (!p.shares || b > tiles) return INT64_MAX;
   const int groups = (tiles + b - 1) / b;
   int u = p.ncu / groups;
   u = u < kMaxSplits ? u : kMaxSplits;
   if (u < 1) return INT64_MAX;
   const Shares s{b, u, groups};
-  const int64_t pairs = ((int64_t)p.pairs * b + u - 1) / u;
+  const int pairs = (p.pairs * b + u - 1) / u;  // chunks have fewer than 2^15 pairs
   if (s.slots() > p.slots || pairs < kMinSplitPairs) return INT64_MAX;
   code = b << 8 | u;
   const int64_t len = 2 * pairs + 10 * ((b + u - 1) / u + (b % u && u % b ? 1 : 0));
-  const int64_t busy = (int64_t)s.workgroups() * 7 / 6;  // behind six sevenths of the CUs the power is what limits
+  const int64_t busy = s.workgroups() * 7 / 6;  // behind six sevenths of the CUs the power is what limits
   return len * (busy > p.ncu ? busy : p.ncu) + (int64_t)s.slots() * 15 + 4 * p.ncu;
 }
 
@@ -712,7 +716,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bid, char* lds)
     if (nk == 0 && !p.p_first) return;  // a narrow last chunk: this split adds nothing to its slab
   }
   banded_tile(logical, tiles_m, tiles_n, kGroupM, tm, tn);
-  gemm_tile_at<BKM>(p, M, N, tm, tn, k0, nk, k_back, (size_t)(split * tiles + logical), !p.p_last || splits > 1, lds);
+  gemm_tile_at<BKM>(p, M, N, tm, tn, k0, nk, k_back, (size_t)(split * tiles + tm * tiles_n + tn), !p.p_last || splits > 1, lds);
 }
 
 template <bool BKM>
@@ -867,10 +871,14 @@ __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_dh_shares(const GemmArgs 
   if ((int)blockIdx.x >= s.workgroups()) return;
   const int id = xcd_contiguous(blockIdx.x, s.workgroups());
   // All of this in scalar registers: the mainloop leaves no vector register to hold it.
-  const int j = __builtin_amdgcn_readfirstlane(id / s.groups), g = id - j * s.groups, bg = __builtin_amdgcn_readfirstlane(s.tiles_of(g, tiles));
+  const int j = __builtin_amdgcn_readfirstlane(id / s.groups), g = id - j * s.groups;
+  int bg = 1, first = 0, last = 0;
+  if (s.b > 1) {  // splits need none of these divisions, and calls of few tokens would notice them
+    bg = __builtin_amdgcn_readfirstlane(s.tiles_of(g, tiles));
+    first = __builtin_amdgcn_readfirstlane(s.first_tile(j, bg)), last = __builtin_amdgcn_readfirstlane(s.last_tile(j, bg));
+  }
   const int pairs = p.nk / 2, all = bg * pairs;  // below 2^20, and times u below 2^26
   const int from = __builtin_amdgcn_readfirstlane(all * j / s.u), to = __builtin_amdgcn_readfirstlane(all * (j + 1) / s.u);
-  const int first = __builtin_amdgcn_readfirstlane(s.first_tile(j, bg)), last = __builtin_amdgcn_readfirstlane(s.last_tile(j, bg));
   for (int i = first; i <= last; ++i) {
     const int k0 = from > i * pairs ? from - i * pairs : 0, k1 = to < (i + 1) * pairs ? to - i * pairs : pairs;
     const int nk = 2 * (k1 - k0);
@@ -878,12 +886,13 @@ __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_dh_shares(const GemmArgs 
     if (i > first) __syncthreads();  // every wave has taken its rows of the tile before from LDS
     int tm, tn;
     banded_tile(i * s.groups + g, tiles_m, tiles_n, kGroupM, tm, tn);
-    const bool alone = __builtin_amdgcn_readfirstlane(s.first_workgroup(i, bg)) == __builtin_amdgcn_readfirstlane(s.last_workgroup(i, bg));
+    bool alone = s.u == 1;
+    if (s.b > 1) alone = __builtin_amdgcn_readfirstlane(s.first_workgroup(i, bg)) == __builtin_amdgcn_readfirstlane(s.last_workgroup(i, bg));
     // The lanes' copy offsets and LDS addresses formed once for all tiles would be vector registers that the mainloop does not have.
     GemmArgs q = p;
     int lds_at = 0;
     asm volatile("" : "+s"(q.lda), "+s"(q.ldb), "+s"(q.ldc), "+s"(lds_at));
-    gemm_tile_at<true>(q, M, p.N, tm, tn, 2 * k0, nk, k1 == pairs ? p.k_back : 0, (size_t)s.slot(g, i, j), !p.p_last || !alone, lds + lds_at);
+    gemm_tile_at<true>(q, M, p.N, tm, tn, 2 * k0, nk, k1 == pairs ? p.k_back : 0, (size_t)(s.b > 1 ? s.slot(g, i, j) : j * tiles + tm * tiles_n + tn), !p.p_last || !alone, lds + lds_at);
   }
 }
 
@@ -906,25 +915,27 @@ __global__ __launch_bounds__(256) void lmhead_dh_reduce(const DhReduceArgs a) {
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (a.H + BN - 1) / BN, tiles = tiles_m * tiles_n;
   const int tile = blockIdx.x / kReduceGroups, wave = blockIdx.x / TM % NWAVES, i = blockIdx.x % TM;
   if (tile >= tiles) return;
-  const Shares sh = shares_of(splits, tiles);
-  int in_group = 0, g = tile, first = 0, last = sh.u - 1;
-  if (sh.b > 1) {  // splits need none of these divisions
-    in_group = tile / sh.groups, g = tile - in_group * sh.groups;
-    const int bg = sh.tiles_of(g, tiles);
-    first = sh.first_workgroup(in_group, bg), last = sh.last_workgroup(in_group, bg);
+  // Splits: the slabs of a tile stand `tiles` apart, in row order; shares: `groups` apart, in the launch's order.
+  int tm, tn, count = splits, step = tiles, slot = tile;
+  if (splits < 256) {
+    tm = tile / tiles_n, tn = tile - tm * tiles_n;
+  } else {
+    const Shares sh = shares_of(splits, tiles);
+    const int in_group = tile / sh.groups, g = tile - in_group * sh.groups, bg = sh.tiles_of(g, tiles), first = sh.first_workgroup(in_group, bg);
+    count = sh.last_workgroup(in_group, bg) - first + 1, step = sh.groups, slot = sh.slot(g, in_group, first);
+    banded_tile(tile, tiles_m, tiles_n, kGroupM, tm, tn);
   }
-  if (first == last) return;  // one workgroup made the tile, and its epilogue has written C
-  int tm, tn;
-  banded_tile(tile, tiles_m, tiles_n, kGroupM, tm, tn);
+  count = __builtin_amdgcn_readfirstlane(count), step = __builtin_amdgcn_readfirstlane(step), slot = __builtin_amdgcn_readfirstlane(slot);
+  if (count < 2) return;  // one workgroup made the tile, and its epilogue has written C
   const int m0 = tm * BM + wave / WAVES_N * WM + i * MT;
   const int n0 = tn * BN + wave % WAVES_N * WN;
   if (m0 >= M || n0 >= a.H) return;
   const int tid = threadIdx.x;
-  const float* part = a.P + ((size_t)sh.slot(g, in_group, first) * NWAVES + wave) * kSlabWaveFloats + (size_t)(i * TN) * (64 * 4) + (size_t)tid * 4;
-  const size_t slab = (size_t)sh.groups * kSlabTileFloats;
+  const float* part = a.P + ((size_t)slot * NWAVES + wave) * kSlabWaveFloats + (size_t)(i * TN) * (64 * 4) + (size_t)tid * 4;
+  const size_t slab = (size_t)step * kSlabTileFloats;
   f32x4 sum[2] = {*(const f32x4*)part, *(const f32x4*)(part + 1024)};
 #pragma unroll 4
-  for (int s = 1; s <= last - first; ++s) {
+  for (int s = 1; s < count; ++s) {
     sum[0] += *(const f32x4*)(part + (size_t)s * slab);
     sum[1] += *(const f32x4*)(part + (size_t)s * slab + 1024);
   }
@@ -1345,6 +1356,9 @@ int64_t list_schedule(int64_t count_a, int64_t len_a, int64_t count_b, int64_t l
   return best > t_late ? best : t_late;
 }
 
+// dHidden tiles of T tokens.
+int64_t dh_tiles(int64_t T, int64_t H) { return (T + BM - 1) / BM * ((H + BN - 1) / BN); }
+
 // Width of the dz panel in vocab columns when the caller does not choose one.  Wider chunks mean fewer launches (every
 // launch ends with CUs idling for part of a tile), fewer read-modify-write passes over the dHidden partial sums and a
 // larger panel; what matters most is whether the tiles of a launch divide evenly over the CUs.  The candidates
@@ -1354,7 +1368,8 @@ int64_t list_schedule(int64_t count_a, int64_t len_a, int64_t count_b, int64_t l
 // that is 49152 columns: 4096 x 3 dz tiles and 896 + 2688 GEMM tiles per launch, both multiples of 256 CUs.
 SplitProblem split_problem(int64_t T, int64_t H, int64_t vc, bool want_dw, int64_t slots, int ncu) {
   const int64_t tiles_h = (H + BN - 1) / BN;
-  return SplitProblem{(int)tiles_h, (int)(vc / (2 * BK)), want_dw ? (int)(tiles_h * (vc / BM)) : 0, (int)slots, ncu};
+  return SplitProblem{(int)tiles_h, (int)(vc / (2 * BK)), want_dw ? (int)(tiles_h * (vc / BM)) : 0, (int)slots,
+                      !want_dw && dh_tiles(T, H) >= kSharesFromTiles, ncu};
 }
 
 // Slab tiles of dHidden partial sums for at most T tokens and chunks of vc columns: room for one tile per CU, at least two per dHidden
@@ -1362,7 +1377,6 @@ SplitProblem split_problem(int64_t T, int64_t H, int64_t vc, bool want_dw, int64
 // The line is drawn for launches with dW.  Without (a frozen weight, the draft loss, a dW launch of its own) shares would go further where there is
 // room for them: the draft loss always has it, a frozen weight from the room that row compaction brings (carve_bwd).
 constexpr int64_t kSplitBelowTiles = 192;
-int64_t dh_tiles(int64_t T, int64_t H) { return (T + BM - 1) / BM * ((H + BN - 1) / BN); }
 int64_t slab_slots(int64_t T, int64_t H, int64_t vc) {
   const int64_t tiles = dh_tiles(T, H), most = vc / (2 * BK) / kMinSplitPairs;
   if (tiles >= kSplitBelowTiles || most < 2) return tiles;
@@ -1648,7 +1662,7 @@ hipError_t launch_bwd_gemm(hipStream_t s, const GemmArgs& p0, const GemmArgs& p1
   unsigned t0 = (unsigned)shares_of(p0.splits, tiles0).workgroups();
   if (p0.splits_dev && (int64_t)t0 < slots) t0 = (unsigned)slots;
   Timed timed(kBwdChunkGemm, s);
-  if (t1 == 0 && p0.b_kmajor) {
+  if (t1 == 0 && p0.b_kmajor && tiles0 >= kSharesFromTiles) {
     if (p0.splits_dev && (int)t0 < ncu) t0 = (unsigned)ncu;
     hipLaunchKernelGGL(lmhead_bwd_dh_shares, dim3(t0), dim3(NTHREADS), 0, s, p0);
     return hipGetLastError();
