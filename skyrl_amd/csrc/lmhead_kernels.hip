@@ -29,6 +29,7 @@
 
 #include "../../include/skyrl_lmhead.h"
 #include "../../include/skyrl_lmhead_bench.h"
+#include "dh_split.hpp"
 #include "few_tokens.hpp"
 #include "gemm_core.hpp"
 #include "logits_tile.hpp"
@@ -37,6 +38,8 @@
 using namespace lmhead;
 
 namespace {
+
+static_assert(BM == kSplitTile && BN == kSplitTile && 2 * BK == kSplitPair, "the tiles that dh_split.hpp rates");
 
 // Timing-only ablations for skyrl_amd/bench_ablations.py (results are wrong with any of them; 0 in the product build):
 //   1  forward tiles skip their statistics epilogue        2  dz tiles skip their epilogue (arithmetic, staging, stores)
@@ -601,84 +604,6 @@ struct GemmArgs {
   int k_back, n_tail, n_back;
 };
 enum { kTokensOnM = 1, kTokensOnN = 2, kTokensOnK = 3 };
-
-// How many workgroups share the vocabulary of one dHidden tile.  There are tokens/256 x H/256 such tiles with a contraction of a
-// whole chunk of the vocabulary: 18 tiles of 2374 k-tiles at T=611, H=1536, V=151936, which one workgroup each leaves on 18
-// of 256 CUs for 2.5 ms.  Rated in k-tiles of mainloop: the dHidden tiles alone in whole rounds of the CUs, or everything the
-// launch carries spread evenly plus half a dW tile of tail, plus what the slabs cost to write, read and add (a 256 KiB slab
-// tile about a seventeenth of a k-tile of the whole chip).  At least 1024 vocabulary rows per split.  Integer arithmetic: the
-// host and compact_active_rows, which rates one candidate per lane for the token count it found, must agree.
-// Measured, GEMM launches of the backward, one workgroup per tile -> split: 2750 -> 560 us at T=428 (active), H=1536, V=151936
-// (12 tiles x 8 splits beside the dW tiles; alone in the launch, as now, 12 x 21 in 180); 544 -> 168 us at T=1050, H=1024, V=32000,
-// fp32 weight; 2714 -> 1509 us at T=4096, H=2048, V=151936 and 2304 -> 1317 us at T=1592, H=4096, V=128261, both without dW; 3030 ->
-// 2700 us at T=4096, H=1536, V=151936.  What the slabs have room for (slab_slots) bounds the choice.
-constexpr int kMinSplitPairs = 8;
-constexpr int kMaxSplits = 64;
-struct SplitProblem {
-  int tiles_h;    // dHidden tiles per 256 tokens
-  int pairs;      // k-tile pairs of a chunk's vocabulary
-  int dw_tiles;   // dW tiles of the same launch (0: frozen weight)
-  int slots;      // slab tiles there is room for
-  int shares;     // whether the launch may go in Shares
-  int ncu;
-};
-__host__ __device__ inline int64_t split_cost(const SplitProblem& p, int tokens, int splits) {
-  const int tiles = (tokens + BM - 1) / BM * p.tiles_h;
-  if (splits > 1 && ((int64_t)tiles * splits > p.slots || p.pairs / splits < kMinSplitPairs)) return INT64_MAX;
-  const int64_t len = 2 * ((p.pairs + splits - 1) / splits) + (splits > 1 ? 10 : 8);
-  const int64_t items = (int64_t)tiles * splits, dw_len = (tokens + 2 * BK - 1) / (2 * BK) * 2 + 6;
-  const int64_t alone = (int64_t)(((int)items + p.ncu - 1) / p.ncu) * len * p.ncu;
-  const int64_t spread = items * len + p.dw_tiles * dw_len + (p.dw_tiles ? dw_len * p.ncu / 2 : 0);
-  return (alone > spread ? alone : spread) + (splits > 1 ? items * 15 + 4 * p.ncu : 0);
-}
-
-// Shares.  Where dHidden is alone in its launch, a whole number of workgroups per tile leaves CUs idle: 96 tiles go in two splits on 192 of 256.  So
-// the tiles may also be taken in groups of b, u workgroups each, and every workgroup takes an equal share of its group's k-tile pairs, laid end to
-// end: the end of one tile, whole tiles, the beginning of another.  Splits are groups of one tile.  Group g holds tiles g, g + G, g + 2 G, ... of the
-// launch's order, G groups in all: the workgroups at one place j of their groups read the same range of the vocabulary for G neighbouring tiles
-// and come one behind the other, on one XCD.  Splits -> shares, the GEMM launch: 1437 -> 1251 us at 96 tiles (draft loss of 2868 tokens, H=2048,
-// V=151936), one round and a part -> shares 2457 -> 1582 at 288 tiles (draft loss of 8192, H=2304, V=64000; pass 9135 -> 8282) and 2580 -> 2311 at
-// 400 (5120 tokens, H=5120, V=64000), three quarters of a round 1877 -> 1578 at 192 (2868 of 4096 tokens, H=4096, V=100000).  112 tiles in two splits, 224
-// CUs, draw the power that 256 do: 1261 and 1290, hence the term for it in share_cost().
-struct Shares {
-  int b, u, groups;
-  __host__ __device__ int workgroups() const { return groups * u; }
-  __host__ __device__ int slots() const { return groups * (u + b - 1); }
-  // Group g: its tiles, and the first and last of them that workgroup j shares in, the first and last workgroup of its i-th tile.
-  __host__ __device__ int tiles_of(int g, int tiles) const { return (tiles - g + groups - 1) / groups; }
-  __host__ __device__ int first_tile(int j, int bg) const { return j * bg / u; }
-  __host__ __device__ int last_tile(int j, int bg) const { return ((j + 1) * bg + u - 1) / u - 1; }
-  __host__ __device__ int first_workgroup(int i, int bg) const { return i * u / bg; }
-  __host__ __device__ int last_workgroup(int i, int bg) const { return ((i + 1) * u + bg - 1) / bg - 1; }
-  // The slab of workgroup j's sums for the i-th tile: j + i differs along a group, because each step goes on to the next of either.
-  __host__ __device__ int slot(int g, int i, int j) const { return (j + i) * groups + g; }
-};
-constexpr int kMaxGroup = 32;
-// Launches that may have more tiles than this: up to 64 tiles in four splits and more already fill nine tenths of the CUs, and calls of few tokens
-// notice what finding a share takes (draft loss of 20 tokens, H=896, V=246016, four tiles in 64 splits: GEMM 109 -> 111 us, their sum 11.6 -> 12.9).
-constexpr int64_t kSharesFromTiles = 65;
-// code: u, and b above its lowest eight bits where it is not 1.
-__host__ __device__ inline Shares shares_of(int code, int tiles) {
-  const int b = code < 256 ? 1 : code >> 8;
-  return Shares{b, code & 255, b == 1 ? tiles : (tiles + b - 1) / b};
-}
-// Groups of b >= 2 tiles, as many workgroups each as the CUs hold at once, rated as above.  A workgroup's further tiles cost it an epilogue and
-// another beginning each.  `code` is set where the answer is below INT64_MAX.
-__host__ __device__ inline int64_t share_cost(const SplitProblem& p, int tokens, int b, int& code) {
-  const int tiles = (tokens + BM - 1) / BM * p.tiles_h;
-  if (!p.shares || b > tiles) return INT64_MAX;
-  const int groups = (tiles + b - 1) / b;
-  int u = p.ncu / groups;
-  u = u < kMaxSplits ? u : kMaxSplits;
-  if (u < 1) return INT64_MAX;
-  const Shares s{b, u, groups};
-  const int pairs = (p.pairs * b + u - 1) / u;  // chunks have fewer than 2^15 pairs
-  if (s.slots() > p.slots || pairs < kMinSplitPairs) return INT64_MAX;
-  code = b << 8 | u;
-  const int64_t len = 2 * pairs + 10 * ((b + u - 1) / u + (b % u && u % b ? 1 : 0));
-  const int64_t busy = s.workgroups() * 7 / 6;  // behind six sevenths of the CUs the power is what limits
-  return len * (busy > p.ncu ? busy : p.ncu) + (int64_t)s.slots() * 15 + 4 * p.ncu;
-}
 
 // BKM: the B operand is K-major.  The two variants are separate instantiations of the whole tile (mainloop and
 // epilogue) so that their accumulators never meet at a join, where the register allocator would shuffle all 256 of them.
@@ -1356,9 +1281,6 @@ int64_t list_schedule(int64_t count_a, int64_t len_a, int64_t count_b, int64_t l
   return best > t_late ? best : t_late;
 }
 
-// dHidden tiles of T tokens.
-int64_t dh_tiles(int64_t T, int64_t H) { return (T + BM - 1) / BM * ((H + BN - 1) / BN); }
-
 // Width of the dz panel in vocab columns when the caller does not choose one.  Wider chunks mean fewer launches (every
 // launch ends with CUs idling for part of a tile), fewer read-modify-write passes over the dHidden partial sums and a
 // larger panel; what matters most is whether the tiles of a launch divide evenly over the CUs.  The candidates
@@ -1366,40 +1288,6 @@ int64_t dh_tiles(int64_t T, int64_t H) { return (T + BM - 1) / BM * ((H + BN - 1
 // chunk -- dz tiles of H/64 k-tiles plus an epilogue, then dHidden tiles of chunk/64 and dW tiles of T'/64 k-tiles,
 // list-scheduled over the CUs, plus a fixed cost per launch -- and the cheapest wins.  At the 7B shape (T = 16384, H = 3584)
 // that is 49152 columns: 4096 x 3 dz tiles and 896 + 2688 GEMM tiles per launch, both multiples of 256 CUs.
-SplitProblem split_problem(int64_t T, int64_t H, int64_t vc, bool want_dw, int64_t slots, int ncu) {
-  const int64_t tiles_h = (H + BN - 1) / BN;
-  return SplitProblem{(int)tiles_h, (int)(vc / (2 * BK)), want_dw ? (int)(tiles_h * (vc / BM)) : 0, (int)slots,
-                      !want_dw && dh_tiles(T, H) >= kSharesFromTiles, ncu};
-}
-
-// Slab tiles of dHidden partial sums for at most T tokens and chunks of vc columns: room for one tile per CU, at least two per dHidden
-// tile; none beyond one per dHidden tile from 192 tiles on, where dW tiles in the same launch fill the CUs that dHidden leaves idle.
-// The line is drawn for launches with dW.  Without (a frozen weight, the draft loss, a dW launch of its own) shares would go further where there is
-// room for them: the draft loss always has it, a frozen weight from the room that row compaction brings (carve_bwd).
-constexpr int64_t kSplitBelowTiles = 192;
-int64_t slab_slots(int64_t T, int64_t H, int64_t vc) {
-  const int64_t tiles = dh_tiles(T, H), most = vc / (2 * BK) / kMinSplitPairs;
-  if (tiles >= kSplitBelowTiles || most < 2) return tiles;
-  const int64_t room = 2 * tiles > 256 ? 2 * tiles : 256;
-  const int64_t used = tiles * (most < kMaxSplits ? most : kMaxSplits);
-  return room < used ? room : used;
-}
-
-int best_splits(const SplitProblem& p, int64_t tokens) {
-  int best = 1;
-  int64_t best_cost = split_cost(p, (int)tokens, 1);
-  for (int k = 2; k <= kMaxSplits; ++k) {
-    const int64_t c = split_cost(p, (int)tokens, k);
-    if (c < best_cost) best = k, best_cost = c;
-  }
-  for (int b = 2; b <= kMaxGroup; ++b) {
-    int code = 0;
-    const int64_t c = share_cost(p, (int)tokens, b, code);
-    if (c < best_cost) best = code, best_cost = c;
-  }
-  return best;
-}
-
 int64_t default_vocab_chunk(int64_t T, int64_t H, int64_t V) {
   const int64_t Tpad = round_up(T, 256), Vpad = round_up(V, 256), Hpad = round_up(H, 256);
   const int ncu = compute_units();
