@@ -63,6 +63,8 @@ struct Shares {
   LMHEAD_HD int last_tile(int j, int bg) const { return ((j + 1) * bg + u - 1) / u - 1; }
   LMHEAD_HD int first_workgroup(int i, int bg) const { return i * u / bg; }
   LMHEAD_HD int last_workgroup(int i, int bg) const { return ((i + 1) * u + bg - 1) / bg - 1; }
+  // Where workgroup j's share of the group's bg * pairs k-tile pairs begins, and the one before it ends.  Below 2^26: chunks have fewer than 2^15 pairs.
+  LMHEAD_HD int begin(int j, int bg, int pairs) const { return bg * pairs * j / u; }
   // The slab of workgroup j's sums for the i-th tile: j + i differs along a group, because each step goes on to the next of either.
   LMHEAD_HD int slot(int g, int i, int j) const { return (j + i) * groups + g; }
 };
@@ -127,6 +129,20 @@ inline int best_splits(const SplitProblem& p, int64_t tokens) {
     if (c < best_cost) best = code, best_cost = c;
   }
   return best;
+}
+
+// The launch of a block of at most `tiles` dHidden tiles: whether it goes to lmhead_bwd_dh_shares, which alone understands codes of Shares, and the
+// workgroups for dHidden.  p is what rates the block, here or on the device (the code is then not known yet): with row compaction that is one
+// problem for all blocks of a call, and the last of them may have far fewer tiles than it was made for.
+struct DhLaunch {
+  bool shares;
+  int workgroups;
+};
+inline DhLaunch dh_launch(const SplitProblem& p, int tiles, int code, bool code_on_device) {
+  int n = shares_of(code, tiles).workgroups();
+  if (code_on_device && n < p.slots) n = p.slots;             // splits: a slab each
+  if (code_on_device && p.shares && n < p.ncu) n = p.ncu;  // shares: at most a workgroup per CU
+  return DhLaunch{(bool)p.shares, n};
 }
 
 }  // namespace lmhead

@@ -802,8 +802,8 @@ __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_dh_shares(const GemmArgs 
     bg = __builtin_amdgcn_readfirstlane(s.tiles_of(g, tiles));
     first = __builtin_amdgcn_readfirstlane(s.first_tile(j, bg)), last = __builtin_amdgcn_readfirstlane(s.last_tile(j, bg));
   }
-  const int pairs = p.nk / 2, all = bg * pairs;  // below 2^20, and times u below 2^26
-  const int from = __builtin_amdgcn_readfirstlane(all * j / s.u), to = __builtin_amdgcn_readfirstlane(all * (j + 1) / s.u);
+  const int pairs = p.nk / 2;
+  const int from = __builtin_amdgcn_readfirstlane(s.begin(j, bg, pairs)), to = __builtin_amdgcn_readfirstlane(s.begin(j + 1, bg, pairs));
   for (int i = first; i <= last; ++i) {
     const int k0 = from > i * pairs ? from - i * pairs : 0, k1 = to < (i + 1) * pairs ? to - i * pairs : pairs;
     const int nk = 2 * (k1 - k0);
@@ -1036,7 +1036,8 @@ __global__ __launch_bounds__(256) void split_operand_rows(const void* __restrict
 // learning how many there are (no synchronisation, so the call can be captured in a HIP graph):
 //   compact_active_rows   one workgroup: idx[i] = i-th token with g != 0 or q != 0 (ascending), counts[0] = their number n,
 //                         counts[1 + b] = how many of them fall into block b of `block` compacted rows,
-//                         counts[1 + nblocks + b] = the splits of that block's dHidden contraction (split_cost)
+//                         counts[1 + nblocks + b] = how that block's dHidden contraction is cut: the number of splits, or, where
+//                         SplitProblem::shares admits it, a code of Shares, which only lmhead_bwd_dh_shares and lmhead_dh_reduce read
 //   gather_active_rows    compacted copies of hidden rows and of the per-token inputs; zero dHidden rows for the inactive
 // The GEMM kernels take the counts from device memory (T_dev), run on the static upper-bound grid and write the dHidden rows
 // through the index list.
@@ -1542,16 +1543,15 @@ hipError_t launch_bwd_dz(hipStream_t s, bool entgrad, DzArgs z) {
 
 // Both problems (p1 may be empty) must have an even number of k-tiles: every caller contracts over padded extents that
 // are multiples of 256, or over vocabulary rows that reads_weight_in_place() admits.
-// slots: slab tiles there is room for, which bounds splits * tiles when the splits are chosen on the device.
-hipError_t launch_bwd_gemm(hipStream_t s, const GemmArgs& p0, const GemmArgs& p1, int64_t slots, int ncu) {
+// split: the problem that p0's splits are chosen with, here or on the device.
+hipError_t launch_bwd_gemm(hipStream_t s, const GemmArgs& p0, const GemmArgs& p1, const SplitProblem& split) {
   if ((p0.nk & 1) || (p1.nk & 1)) return hipErrorInvalidValue;
   const unsigned t1 = gemm_tiles(p1);
-  const int tiles0 = (int)gemm_tiles(p0);
-  unsigned t0 = (unsigned)shares_of(p0.splits, tiles0).workgroups();
-  if (p0.splits_dev && (int64_t)t0 < slots) t0 = (unsigned)slots;
+  const DhLaunch launch = dh_launch(split, (int)gemm_tiles(p0), p0.splits, p0.splits_dev != nullptr);
+  const unsigned t0 = (unsigned)launch.workgroups;
   Timed timed(kBwdChunkGemm, s);
-  if (t1 == 0 && p0.b_kmajor && tiles0 >= kSharesFromTiles) {
-    if (p0.splits_dev && (int)t0 < ncu) t0 = (unsigned)ncu;
+  if (launch.shares && p0.b_kmajor) {  // a transposed copy of the weight (b_kmajor 0) is never split
+    if (t1 != 0) return hipErrorInvalidValue;
     hipLaunchKernelGGL(lmhead_bwd_dh_shares, dim3(t0), dim3(NTHREADS), 0, s, p0);
     return hipGetLastError();
   }
@@ -1711,11 +1711,11 @@ size_t bwd_workspace_bytes(int64_t T, int64_t H, int64_t V, int64_t vocab_chunk,
 
 // One token block of the backward: the vocab-chunk loop.  Hk is the contraction length of the logits recompute (H, or a
 // multiple of it for stacked bf16 terms, in which case the two gradient GEMMs use the leading H columns: the hi terms).  `Tb` tokens (an upper bound when `T_dev` points at the block's
-// count in device memory), per-token inputs and d_hidden already offset to the block.  dW of every chunk leaves the GEMM
+// count in device memory and `splits_dev` at what `rated` made of it), per-token inputs and d_hidden already offset to the block.  dW of every chunk leaves the GEMM
 // epilogue as  (Cin ? Cin : 0) + product  ->  Cf (fp32) and / or Cb (bf16), each a [V, H] matrix or NULL.
 int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, int64_t ld_weight, const int64_t* labels,
                     const float* row_lse, const float* row_pz, const float* dlogprobs, const float* dentropy, int64_t Tb,
-                    const int* T_dev, const int* splits_dev, const int* row_map, int64_t H, int64_t Hk, int64_t V,
+                    const int* T_dev, const int* splits_dev, const SplitProblem& rated, const int* row_map, int64_t H, int64_t Hk, int64_t V,
                     float rcp_temperature, uint16_t* d_hidden, bool want_dw,
                     const float* dw_in, float* dw_f32, uint16_t* dw_bf16, int64_t vc, const BwdWorkspace& w, float p_shift,
                     hipStream_t s) {
@@ -1738,8 +1738,8 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
   }
   const VocabTail tail = vocab_tail(V);
   // The splits are those of a full chunk: the slabs are carried from chunk to chunk.
-  const int splits =
-      !T_dev && w_in_place ? best_splits(split_problem(Tb, H, vc < Vpad ? vc : Vpad, want_dw && !few, w.slots, ncu), Tb) : 1;
+  const SplitProblem split = T_dev ? rated : split_problem(Tb, H, vc < Vpad ? vc : Vpad, want_dw && !few, w.slots, ncu);
+  const int splits = !T_dev && w_in_place ? best_splits(split, Tb) : 1;
   const int64_t nchunks = (Vpad + vc - 1) / vc;
   auto chunk_width = [&](int64_t ci) { return (Vpad - ci * vc) < vc ? (Vpad - ci * vc) : vc; };  // multiple of 256
   const GemmArgs none{};
@@ -1777,7 +1777,7 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
                                          moved ? gw.n_tail : 0x7fffffff, gw.n_back, cf, cb, ncu});
       if (e != hipSuccess) return (int)e;
     }
-    e = launch_bwd_gemm(s, gh, gw, w.slots, ncu);
+    e = launch_bwd_gemm(s, gh, gw, split);
     if (e == hipSuccess && last) e = launch_dh_reduce(s, gh, w.slots);
     if (e != hipSuccess) return (int)e;
   }
@@ -1826,10 +1826,11 @@ int bwd_entry(const void* hidden, int64_t ld_hidden, const void* weight, int64_t
 
   // dW in the launch of the dHidden tiles (bwd_token_block decides the same way)
   const bool dw_in_gemm = d_weight && !few_token_dw(true, dw_mode == SKYRL_DW_FP32_ACCUMULATE || nblocks > 1, Tb, H, V);
+  const SplitProblem rated = split_problem(Tb, H, vc, dw_in_gemm, w.slots, compute_units());
   if (compact) {
     Timed timed(kCompactRows, s);
     hipLaunchKernelGGL(compact_active_rows, dim3(1), dim3(kCompactThreads), 0, s, dlogprobs, dentropy, (int)T, (int)Tb,
-                       (int)nblocks, split_problem(Tb, H, vc, dw_in_gemm, w.slots, compute_units()), w.idx, w.counts);
+                       (int)nblocks, rated, w.idx, w.counts);
     hipLaunchKernelGGL(gather_active_rows, dim3((unsigned)T), dim3(256), 0, s, (const int*)w.idx, (const int*)w.counts, Hp,
                        (int)ld_hidden, (int)Hk, (int)H, labels, row_lse, row_pz, dlogprobs, dentropy, w.hidden_c, w.labels_c,
                        w.lse_c, w.pz_c, w.g_c, w.q_c, (uint16_t*)d_hidden);
@@ -1867,12 +1868,12 @@ int bwd_entry(const void* hidden, int64_t ld_hidden, const void* weight, int64_t
     if (compact) {
       st = bwd_token_block(w.hidden_c + (size_t)t0 * (size_t)Hk, Hk, Wp, ld_weight, w.labels_c + t0, w.lse_c + t0,
                            dentropy ? w.pz_c + t0 : nullptr, w.g_c + t0, dentropy ? w.q_c + t0 : nullptr, Tcur,
-                           w.counts + 1 + b, w.counts + 1 + nblocks + b, w.idx + t0, H, Hk, V, rcp_temperature, (uint16_t*)d_hidden,
+                           w.counts + 1 + b, w.counts + 1 + nblocks + b, rated, w.idx + t0, H, Hk, V, rcp_temperature, (uint16_t*)d_hidden,
                            d_weight != nullptr, dw_in, dw_f32, dw_bf16, vc, w, p_shift, s);
     } else {
       st = bwd_token_block(Hp + (size_t)t0 * (size_t)ld_hidden, ld_hidden, Wp, ld_weight, labels + t0, row_lse + t0,
                            row_pz ? row_pz + t0 : nullptr, dlogprobs + t0, dentropy ? dentropy + t0 : nullptr, Tcur, nullptr,
-                           nullptr, nullptr, H, Hk, V, rcp_temperature, (uint16_t*)d_hidden + (size_t)t0 * (size_t)H, d_weight != nullptr, dw_in, dw_f32,
+                           nullptr, rated, nullptr, H, Hk, V, rcp_temperature, (uint16_t*)d_hidden + (size_t)t0 * (size_t)H, d_weight != nullptr, dw_in, dw_f32,
                            dw_bf16, vc, w, p_shift, s);
     }
     if (st) return st;
@@ -2095,10 +2096,11 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
   const bool w_in_place = reads_weight_in_place(V);
   const VocabTail tail = vocab_tail(V);
   const int ncu = compute_units();
+  const SplitProblem split = split_problem(T, H, vc, false, w.slots, ncu);
   {  // tokens without an upstream gradient (what the supervision mask removes) have a zero row and take no part
     Timed timed(kCompactRows, s);
     hipLaunchKernelGGL(compact_active_rows, dim3(1), dim3(kCompactThreads), 0, s, dloss, (const float*)nullptr, (int)T, (int)T, 1,
-                       split_problem(T, H, vc, false, w.slots, ncu), w.idx, w.counts);
+                       split, w.idx, w.counts);
   }
   if ((e = hipGetLastError()) != hipSuccess) return (int)e;
   {
@@ -2136,7 +2138,7 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
     GemmArgs gh = dhidden_gemm(w.D, vcw + kLdPad, Tp, Wp, ld_weight, w_in_place ? nullptr : w.Wt, Vpad + kLdPad, vc0, vcw, V, T, H,
                                (uint16_t*)d_student_hidden, w.dHacc, first, last, w.counts + 1);
     gh.splits_dev = w_in_place ? w.counts + 2 : nullptr, gh.row_map = w.idx;
-    e = launch_bwd_gemm(s, gh, none, w.slots, ncu);
+    e = launch_bwd_gemm(s, gh, none, split);
     if (e == hipSuccess && last) e = launch_dh_reduce(s, gh, w.slots);
     if (e != hipSuccess) return (int)e;
   }

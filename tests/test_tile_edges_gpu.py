@@ -119,7 +119,11 @@ def test_topk_candidates_that_all_pass(n, cuda_device):
 # part of one, with tiles of one workgroup among them, three tiles for eight workgroups, both in one chunk and in several of which the last is
 # narrow and ends in a moved group, and token counts that the host does not know.  Beside dW the same sums run whole or in splits: fp32 sums of
 # V <= 2^15 products in another order, rounded to bf16 once: an element in some 200 falls to the other side, sqrt(1 / 200) 2^-8 = 3e-4.
-@pytest.mark.parametrize("T,H,V,vc", [(4500, 4160, 8000, 0), (4500, 4160, 9300, 4096), (1500, 4096, 32000, 0), (1400, 4096, 32001, 20480)])
+SHARES = [(4500, 4160, 8000, 0), (4500, 4160, 12300, 8192), (1500, 4096, 32000, 0), (1400, 4096, 32001, 20480)]
+NO_ROOM_FOR_SHARES = (4500, 4160, 9300, 4096)  # but for the draft loss
+
+
+@pytest.mark.parametrize("T,H,V,vc", [*SHARES, NO_ROOM_FOR_SHARES])
 @pytest.mark.parametrize("keep", [1.0, 0.7])
 def test_hidden_gradient_in_shares(T, H, V, vc, keep, cuda_device):
     hidden, weight, labels, g, q = _operands(T, H, V, seed=T + V)
@@ -140,6 +144,30 @@ def test_hidden_gradient_in_shares(T, H, V, vc, keep, cuda_device):
     dz = (gd.unsqueeze(1) * (probs[0] - probs[1])).to(torch.bfloat16).float()
     ref = dz @ w.float()  # dz rounded to bf16 from probabilities that differ in fp32 roundings, dHidden rounded to bf16: 2^-8 / sqrt(3) each
     assert float((s.grad.float() - ref).norm() / ref.norm()) < 5e-3
+
+
+# Several blocks of tokens whose contractions the device cuts by one rule, the last with few tiles: 8 and 4 of them in groups of four, cut for 64
+# workgroups each.  Tokens without a gradient are moved out of the way, so the last block holds the same number with them.  Against the blocks by
+# themselves: the bounds of test_hidden_gradient_in_shares.
+SHARES_OF_A_SHORT_LAST_BLOCK = [(33024, 2048, 16000, 0), (33792, 256, 32000, 0)]
+
+
+@pytest.mark.parametrize("T,H,V,vc", SHARES_OF_A_SHORT_LAST_BLOCK)
+@pytest.mark.parametrize("masked", [0, 300])
+def test_hidden_gradient_of_a_short_last_block(T, H, V, vc, masked, cuda_device):
+    T += masked
+    hidden, weight, labels, g, q = _operands(T, H, V, seed=T)
+    rest = torch.randperm(T, generator=torch.Generator().manual_seed(T))[:masked]
+    g[rest], q[rest] = 0.0, 0.0
+    h, w, y, gd, qd = (x.to(cuda_device) for x in (hidden, weight, labels, g, q))
+    _, _, lse, pz = ops.lmhead_fwd(h, w, y, 1.0, True)
+    dh = ops.lmhead_bwd_hidden(h, w, y, lse, pz, gd, qd, 1.0, vc, True)
+    assert not dh[rest.to(cuda_device)].any()
+    for first in range(0, T, 4096):
+        b = slice(first, first + 4096)
+        want = ops.lmhead_bwd_hidden(h[b], w, y[b], lse[b], pz[b], gd[b], qd[b], 1.0, vc, False).float()
+        assert float((dh[b].float() - want).norm() / want.norm()) < 1e-3, first
+        assert float((dh[b].float() - want).abs().max() / want.abs().max()) < 2**-7, first
 
 
 # The first vocabulary chunk of the top-k search is stored and searched: its width follows the number of tokens, the later ones the
