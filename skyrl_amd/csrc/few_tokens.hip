@@ -39,11 +39,8 @@ __device__ __forceinline__ void copy_to_lds(const uint16_t* g, uint32_t lds_addr
 }
 
 template <bool F32>
-__global__ __launch_bounds__(kDwThreads, 4) void lmhead_bwd_dw_few(const DwFewArgs a) {
-  __shared__ __attribute__((aligned(1024))) char lds[kDwSlots * kDwSlotBytes];
-  const int n = a.T_dev ? __builtin_amdgcn_readfirstlane(*a.T_dev) : a.T;
+__device__ __forceinline__ void dw_few_tile(const DwFewArgs& a, int n, int logical, char* lds) {
   const int tiles_h = (a.H + kDwH - 1) / kDwH;
-  const int logical = xcd_contiguous(blockIdx.x, gridDim.x);
   const int tv = logical / tiles_h;
   const int h0 = __builtin_amdgcn_readfirstlane((logical - tv * tiles_h) * kDwH), v0 = __builtin_amdgcn_readfirstlane(tv * kDwV);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -170,6 +167,29 @@ __global__ __launch_bounds__(kDwThreads, 4) void lmhead_bwd_dw_few(const DwFewAr
   }
 }
 
+// A tile per workgroup.
+template <bool F32>
+__global__ __launch_bounds__(kDwThreads, 4) void lmhead_bwd_dw_few(const DwFewArgs a) {
+  __shared__ __attribute__((aligned(1024))) char lds[kDwSlots * kDwSlotBytes];
+  const int n = a.T_dev ? __builtin_amdgcn_readfirstlane(*a.T_dev) : a.T;
+  dw_few_tile<F32>(a, n, xcd_contiguous(blockIdx.x, gridDim.x), lds);
+}
+
+// The tiles of a call for more tokens, of which up to kDwTileActive turn out to have a gradient.  Two workgroups per CU make all of them, because
+// those of a launch that finds more have to end before the next one begins (a workgroup per tile: 7128 at H=1536, V=151936, training pass with 137 of 137
+// tokens 505 -> 507 us, with 428 of 611 865 -> 870).  A tile begins when the stores of the one before have left: with 20 tokens 457 -> 463 us, but with
+// 40 492 -> 474.  Four per CU: 462 and 476.
+template <bool F32>
+__global__ __launch_bounds__(kDwThreads, 4) void lmhead_bwd_dw_few_active(const DwFewArgs a, int tiles) {
+  __shared__ __attribute__((aligned(1024))) char lds[kDwSlots * kDwSlotBytes];
+  const int n = __builtin_amdgcn_readfirstlane(*a.T_dev);
+  if (n > kDwTileActive) return;
+  for (int id = blockIdx.x; id < tiles; id += gridDim.x) {
+    if (id != (int)blockIdx.x) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave has taken its rows of the tile before from LDS
+    dw_few_tile<F32>(a, n, xcd_contiguous(id, tiles), lds);
+  }
+}
+
 // ------------------------------------------------------------------------------------------------------------
 // Weight gradient of a chunk for few tokens: dW[v, h] = sum_t D[t, v] . hidden[t, h], a contraction of up to 24 32-token steps that
 // writes V x H values, with the dz values of 256 vocabulary rows resident in registers.
@@ -271,8 +291,8 @@ __device__ __forceinline__ void dw_resident_units(const DwFewArgs& a, int n, cha
   const int share = __builtin_amdgcn_readfirstlane(units / (int)gridDim.x), more = units - share * (int)gridDim.x;
   const int u0 = id * share + (id < more ? id : more), u1 = u0 + share + (id < more ? 1 : 0);  // at least one: the grid has no more workgroups
 
-  // Copies of a slot: copy j of wave w brings tokens 16 (4 j + w) .. + 15, four lanes a token.  Tokens behind the last one repeat it: in the
-  // last copy, or, of 64 tokens and fewer, in both.
+  // Copies of a slot: copy j of wave w brings tokens 16 (4 j + w) .. + 15, four lanes a token.  Tokens behind the last one repeat it, in the
+  // last copy.
   const uint32_t c_row = (uint32_t)(lane >> 2);
   const uint32_t c_col = (uint32_t)((((lane & 3) ^ (((lane >> 5) & 1) << 1))) * 16);
   const uint32_t h_pitch = (uint32_t)a.ldh * 2u, d_pitch = (uint32_t)a.ldd * 2u;
@@ -280,11 +300,8 @@ __device__ __forceinline__ void dw_resident_units(const DwFewArgs& a, int n, cha
     const int t = 16 * (4 * j + wave);
     return t < n ? t : n - 1;
   };
-  auto hidden_offset = [&](int j) {
-    const uint32_t last = (uint32_t)(n - 1 - first_token(j));
-    return (c_row < last ? c_row : last) * h_pitch + c_col;
-  };
-  const uint32_t h_off[2] = {hidden_offset(0), hidden_offset(PT - 1)};
+  const uint32_t behind = (uint32_t)(n - 1 - first_token(PT - 1));
+  const uint32_t h_off[2] = {c_row * h_pitch + c_col, (c_row < behind ? c_row : behind) * h_pitch + c_col};
   auto copy_hidden = [&](int j, int h, uint32_t slot) {
     dw_copy((const char*)(a.Hd + (size_t)first_token(j) * (size_t)a.ldh + h), h_off[j == PT - 1], slot + (uint32_t)((4 * j + wave) * 1024));
   };
@@ -464,22 +481,13 @@ __device__ __forceinline__ void dw_resident_units(const DwFewArgs& a, int n, cha
   for (int it = 0; it < 8; ++it) store(out, F32 ? 128 : 0, it, staged(it));
 }
 
-// No token: zeros.
-template <bool F32>
-__device__ __forceinline__ void dw_resident_zeros(const DwFewArgs& a) {
-  const size_t bytes = (size_t)(a.N > a.n_tail ? a.N - a.n_back : a.N) * (size_t)a.H * (F32 ? 4 : 2);  // a multiple of 128
-  char* c = F32 ? (char*)a.Cf : (char*)a.Cb;
-  for (size_t o = ((size_t)blockIdx.x * kDwResidentThreads + threadIdx.x) * 16; o < bytes; o += (size_t)gridDim.x * kDwResidentThreads * 16)
-    *(u32x4*)(c + o) = u32x4{0u, 0u, 0u, 0u};
-}
-
 template <bool F32>
 __global__ __launch_bounds__(kDwResidentThreads, 1) void lmhead_bwd_dw_resident(const DwFewArgs a) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
   const int n = a.T_dev ? __builtin_amdgcn_readfirstlane(*a.T_dev) : a.T;
+  static_assert(kDwTileActive == 64 && kDwTileTokens >= 64, "at least 65 tokens");
+  if (n <= kDwTileActive) return;  // made in tiles, by the launch before
   switch ((n + 63) / 64) {
-    case 0: return dw_resident_zeros<F32>(a);
-    case 1:
     case 2: return dw_resident_units<F32, 4>(a, n, lds);
     case 3: return dw_resident_units<F32, 6>(a, n, lds);
     case 4: return dw_resident_units<F32, 8>(a, n, lds);
@@ -535,6 +543,13 @@ __global__ __launch_bounds__(NTHREADS, 2) void lmhead_bwd_half_dz(const DzArgs z
 
 hipError_t launch_bwd_dw_few(hipStream_t s, const DwFewArgs& a) {
   if (a.T > kDwTileTokens) {
+    if (a.T_dev) {  // either kernel returns at once where the other one makes dW
+      const int64_t tiles = dw_few_tiles(a.H, a.N), most = 2 * (int64_t)a.ncu;
+      hipLaunchKernelGGL(a.Cf ? lmhead_bwd_dw_few_active<true> : lmhead_bwd_dw_few_active<false>, dim3((unsigned)(tiles < most ? tiles : most)),
+                         dim3(kDwThreads), 0, s, a, (int)tiles);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+    }
     const int64_t units = (a.N + kDwV - 1) / kDwV * (a.H / kDwUnitH);
     hipLaunchKernelGGL(a.Cf ? lmhead_bwd_dw_resident<true> : lmhead_bwd_dw_resident<false>, dim3((unsigned)(units < a.ncu ? units : a.ncu)),
                        dim3(kDwResidentThreads), 0, s, a);

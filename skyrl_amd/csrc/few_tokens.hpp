@@ -30,6 +30,11 @@ struct DwFewArgs {
 // for whatever is below 130 tokens (H=1536, V=151936): 88 -> 121 at 20, 123 -> 119 at 64, 144 -> 118 at 96, 152 -> 118 at 128.  Not at the sizes
 // of the tie, because half of the tokens and more are often masked.
 constexpr int64_t kDwTileTokens = 96;
+// Behind it, where the device finds out how many tokens have a gradient, it also chooses: up to this many are made in the tiles, by a launch in front
+// that returns at once if there are more.  Training pass, H=1536, V=151936, dz in registers -> the device's choice: 480 -> 463 us with 20 tokens of
+// 137, 482 -> 474 with 40, 481 -> 478 with 60; 490 -> 473, 490 -> 484, 492 -> 488 of 200; 610 -> 592 with 20 of 611, 611 -> 606 with 60.  With 20 known
+// to the host it would be 448.  What the choice costs a call that has more: 502 -> 504 with 137 of 137, 865 -> 865 with 428 of 611.
+constexpr int kDwTileActive = 64;
 inline int64_t dw_few_tiles(int64_t H, int64_t N) { return (N + kDwV - 1) / kDwV * ((H + kDwH - 1) / kDwH); }
 
 hipError_t launch_bwd_dw_few(hipStream_t s, const DwFewArgs& a);

@@ -331,7 +331,7 @@ def test_weight_gradient_of_few_tokens(T, vc, cuda_device):
     assert not any(t.any() for t in ops.lmhead_bwd_bf16(h, w, y, lse, pz, zero, zero, 1.0, vc, True))
 
 
-# Behind 96 tokens dz stays in registers, in code of its own for every 64 tokens: the tokens with a gradient at the ends of these, more and
+# Behind 96 tokens dz stays in registers, in code of its own for every 64 tokens, unless the device finds 64 and fewer: the tokens with a gradient at the ends of these, more and
 # fewer hidden columns than a workgroup's share of units, a last vocabulary group moved back.  Both sides are fp32 sums of the same dz panel in
 # another order, sqrt(768) 2^-24 = 2e-6.
 @pytest.mark.parametrize("active", [1, 64, 65, 128, 129, 193, 256, 257, 321, 385, 449, 513, 577, 640, 641, 705, 767])
