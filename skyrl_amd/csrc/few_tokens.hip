@@ -485,7 +485,7 @@ template <bool F32>
 __global__ __launch_bounds__(kDwResidentThreads, 1) void lmhead_bwd_dw_resident(const DwFewArgs a) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
   const int n = a.T_dev ? __builtin_amdgcn_readfirstlane(*a.T_dev) : a.T;
-  static_assert(kDwTileActive == 64 && kDwTileTokens >= 64, "at least 65 tokens");
+  static_assert(kDwTileActive == 64 && kDwTileTokens >= 64, "below 65 tokens there is no code here");
   if (n <= kDwTileActive) return;  // made in tiles, by the launch before
   switch ((n + 63) / 64) {
     case 2: return dw_resident_units<F32, 4>(a, n, lds);
@@ -542,7 +542,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void lmhead_bwd_half_dz(const DzArgs z
 }  // namespace
 
 hipError_t launch_bwd_dw_few(hipStream_t s, const DwFewArgs& a) {
-  if (a.T > kDwTileTokens) {
+  if (dw_resident(a.T, a.H)) {
     if (a.T_dev) {  // either kernel returns at once where the other one makes dW
       const int64_t tiles = dw_few_tiles(a.H, a.N), most = 2 * (int64_t)a.ncu;
       hipLaunchKernelGGL(a.Cf ? lmhead_bwd_dw_few_active<true> : lmhead_bwd_dw_few_active<false>, dim3((unsigned)(tiles < most ? tiles : most)),

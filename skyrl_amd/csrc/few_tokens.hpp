@@ -35,6 +35,11 @@ constexpr int64_t kDwTileTokens = 96;
 // 137, 482 -> 474 with 40, 481 -> 478 with 60; 490 -> 473, 490 -> 484, 492 -> 488 of 200; 610 -> 592 with 20 of 611, 611 -> 606 with 60.  With 20 known
 // to the host it would be 448.  What the choice costs a call that has more: 502 -> 504 with 137 of 137, 865 -> 865 with 428 of 611.
 constexpr int kDwTileActive = 64;
+// Whether the call is one for resident dz.  A workgroup's new dz rows cost it 6 us, for a row of H / 64 units: with short rows that is more than is
+// saved.  Tiles -> resident dz, us, 137, 300 and 768 tokens: H=256, V=248320 48 -> 59, 66 -> 77, 124 -> 143 (fp32 result 73 -> 83 and 148 -> 169 at
+// 137 and 768); V=151936, 120, 300, 500 and 768 tokens: H=512 56 -> 50, 81 -> 80, 105 -> 109, 136 -> 144; H=576 64 -> 51, 95 -> 84, 123 -> 114, 161 -> 151;
+// H=384 42 -> 39, 60 -> 65 at 300, 88 -> 99 at 600; H=448 52 -> 45, 101 -> 102 at 500.  Of what stands here 2 to 4 us go to the device's choice.
+inline bool dw_resident(int64_t T, int64_t H) { return T > kDwTileTokens && (H > 512 || (H > 384 && T <= 128)); }
 inline int64_t dw_few_tiles(int64_t H, int64_t N) { return (N + kDwV - 1) / kDwV * ((H + kDwH - 1) / kDwH); }
 
 hipError_t launch_bwd_dw_few(hipStream_t s, const DwFewArgs& a);

@@ -331,13 +331,14 @@ def test_weight_gradient_of_few_tokens(T, vc, cuda_device):
     assert not any(t.any() for t in ops.lmhead_bwd_bf16(h, w, y, lse, pz, zero, zero, 1.0, vc, True))
 
 
-# Behind 96 tokens dz stays in registers, in code of its own for every 64 tokens, unless the device finds 64 and fewer: the tokens with a gradient at the ends of these, more and
-# fewer hidden columns than a workgroup's share of units, a last vocabulary group moved back.  Both sides are fp32 sums of the same dz panel in
+# Behind 96 tokens dz stays in registers, in code of its own for every 64 tokens, unless the device finds 64 and fewer or rows of hidden columns are
+# short (256): the tokens with a gradient at the ends of these, more (4160) and fewer (640) hidden columns than a workgroup's share of units, the
+# shortest rows (448, up to 128 tokens), a last vocabulary group moved back.  Both sides are fp32 sums of the same dz panel in
 # another order, sqrt(768) 2^-24 = 2e-6.
-@pytest.mark.parametrize("active", [1, 64, 65, 128, 129, 193, 256, 257, 321, 385, 449, 513, 577, 640, 641, 705, 767])
-@pytest.mark.parametrize("H,V", [(4160, 12100), (256, 196741)])
+@pytest.mark.parametrize("active", [1, 64, 65, 127, 128, 129, 193, 256, 257, 321, 385, 449, 513, 577, 640, 641, 705, 767])
+@pytest.mark.parametrize("H,V", [(4160, 12100), (640, 98341), (448, 98341), (256, 196741)])
 def test_weight_gradient_with_resident_dz(active, H, V, cuda_device):
-    T = 97 if active < 96 else 768
+    T = 97 if active < 96 else 128 if active == 127 else 768
     hidden, weight, labels, g, q = _operands(T, H, V, seed=active)
     labels[0], labels[T - 1] = V - 1, -1
     rest = torch.randperm(T, generator=torch.Generator().manual_seed(active))[active:]
