@@ -823,7 +823,9 @@ __global__ __launch_bounds__(NTHREADS) void lmhead_bwd_dh_shares(const GemmArgs 
 
 // dHidden rows from the slabs of a split contraction: C[m, n] = bf16(sum of the slabs), added in split order.  One workgroup per
 // 16 tokens x 128 columns (an MFMA row block of a wave): 16-byte loads of contiguous slab pieces, 16-byte row pieces out
-// through LDS.  HBM-bound, splits x tokens x H x 4 bytes: 8 us at 240 slab tiles (60 MB).
+// through LDS.  HBM-bound, splits x tokens x H x 4 bytes: 8 us at 240 slab tiles (60 MB).  SHARES: of a launch that may have been cut in shares; the
+// code for these costs calls of few tokens, which bring it from memory each time: 6.9 -> 8.4 us at 20 tokens, H=1536, 10.0 -> 12.1 at 300, H=512,
+// 8.6 -> 11.4 in the draft loss of 20 tokens, H=896, V=246016.
 struct DhReduceArgs {
   const float* P;
   int M, H, splits;
@@ -833,25 +835,24 @@ struct DhReduceArgs {
 };
 constexpr int kReduceGroups = NWAVES * TM;  // workgroups per tile
 
+template <bool SHARES>
 __global__ __launch_bounds__(256) void lmhead_dh_reduce(const DhReduceArgs a) {
   __shared__ __attribute__((aligned(16))) uint16_t rows[MT][WN + 8];
-  const int splits = __builtin_amdgcn_readfirstlane(a.splits_dev ? *a.splits_dev : a.splits);
-  const int M = __builtin_amdgcn_readfirstlane(a.T_dev ? *a.T_dev : a.M);
+  const int splits = a.splits_dev ? *a.splits_dev : a.splits;
+  const int M = a.T_dev ? *a.T_dev : a.M;
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (a.H + BN - 1) / BN, tiles = tiles_m * tiles_n;
   const int tile = blockIdx.x / kReduceGroups, wave = blockIdx.x / TM % NWAVES, i = blockIdx.x % TM;
-  if (tile >= tiles) return;
+  if (splits < 2 || tile >= tiles) return;  // without splits the GEMM epilogue has written C
   // Splits: the slabs of a tile stand `tiles` apart, in row order; shares: `groups` apart, in the launch's order.
-  int tm, tn, count = splits, step = tiles, slot = tile;
-  if (splits < 256) {
-    tm = tile / tiles_n, tn = tile - tm * tiles_n;
-  } else {
+  int tm = tile / tiles_n, tn = tile % tiles_n, count = splits, step = tiles, slot = tile;
+  if (SHARES && splits >= 256) {
     const Shares sh = shares_of(splits, tiles);
     const int in_group = tile / sh.groups, g = tile - in_group * sh.groups, bg = sh.tiles_of(g, tiles), first = sh.first_workgroup(in_group, bg);
-    count = sh.last_workgroup(in_group, bg) - first + 1, step = sh.groups, slot = sh.slot(g, in_group, first);
+    count = __builtin_amdgcn_readfirstlane(sh.last_workgroup(in_group, bg) - first + 1), step = __builtin_amdgcn_readfirstlane(sh.groups);
+    slot = __builtin_amdgcn_readfirstlane(sh.slot(g, in_group, first));
+    if (count < 2) return;  // one workgroup made the tile, and its epilogue has written C
     banded_tile(tile, tiles_m, tiles_n, kGroupM, tm, tn);
   }
-  count = __builtin_amdgcn_readfirstlane(count), step = __builtin_amdgcn_readfirstlane(step), slot = __builtin_amdgcn_readfirstlane(slot);
-  if (count < 2) return;  // one workgroup made the tile, and its epilogue has written C
   const int m0 = tm * BM + wave / WAVES_N * WM + i * MT;
   const int n0 = tn * BN + wave % WAVES_N * WN;
   if (m0 >= M || n0 >= a.H) return;
@@ -1569,14 +1570,14 @@ inline bool few_token_dw(bool want_dw, bool adds, int64_t T, int64_t H, int64_t 
   return want_dw && !adds && T <= kDwFewTokens && dw_few_tiles(H, V) >= kDwFewTiles;
 }
 
-// The sum over the slabs of a split dHidden contraction; g is the GEMM of the last chunk.
-hipError_t launch_dh_reduce(hipStream_t s, const GemmArgs& g, int64_t slots) {
+// The sum over the slabs of a split dHidden contraction; g is the GEMM of the last chunk, split the problem that its splits are chosen with.
+hipError_t launch_dh_reduce(hipStream_t s, const GemmArgs& g, const SplitProblem& split) {
   if (!g.splits_dev && g.splits < 2) return hipSuccess;
-  // a problem with more tiles than slots is never split
-  const int64_t tiles = gemm_tiles(g), most = g.splits_dev && slots < tiles ? slots : tiles;
+  // a problem with more tiles than slots is never split, and without shares none with more than half as many
+  const int64_t tiles = gemm_tiles(g), slots = split.shares ? split.slots : split.slots / 2, most = g.splits_dev && slots < tiles ? slots : tiles;
   if (most < 1) return hipSuccess;
   Timed timed(kDhReduce, s);
-  hipLaunchKernelGGL(lmhead_dh_reduce, dim3((unsigned)(most * kReduceGroups)), dim3(256), 0, s,
+  hipLaunchKernelGGL(split.shares ? lmhead_dh_reduce<true> : lmhead_dh_reduce<false>, dim3((unsigned)(most * kReduceGroups)), dim3(256), 0, s,
                      DhReduceArgs{g.P, g.M, g.N, g.splits, g.T_dev, g.splits_dev, g.row_map, g.Cb, g.ldc});
   return hipGetLastError();
 }
@@ -1778,7 +1779,7 @@ int bwd_token_block(const uint16_t* Hp, int64_t ld_hidden, const uint16_t* Wp, i
       if (e != hipSuccess) return (int)e;
     }
     e = launch_bwd_gemm(s, gh, gw, split);
-    if (e == hipSuccess && last) e = launch_dh_reduce(s, gh, w.slots);
+    if (e == hipSuccess && last) e = launch_dh_reduce(s, gh, split);
     if (e != hipSuccess) return (int)e;
   }
   if (resid) {
@@ -2139,7 +2140,7 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
                                (uint16_t*)d_student_hidden, w.dHacc, first, last, w.counts + 1);
     gh.splits_dev = w_in_place ? w.counts + 2 : nullptr, gh.row_map = w.idx;
     e = launch_bwd_gemm(s, gh, none, split);
-    if (e == hipSuccess && last) e = launch_dh_reduce(s, gh, w.slots);
+    if (e == hipSuccess && last) e = launch_dh_reduce(s, gh, split);
     if (e != hipSuccess) return (int)e;
   }
   return SKYRL_LMHEAD_OK;
