@@ -1045,43 +1045,45 @@ __global__ __launch_bounds__(256) void split_operand_rows(const void* __restrict
 // ------------------------------------------------------------------------------------------------------------
 constexpr int kCompactThreads = 1024;
 
+template <int TOKENS>  // per thread and step
 __global__ __launch_bounds__(kCompactThreads) void compact_active_rows(const float* __restrict__ g, const float* __restrict__ q,
                                                                        int T, int block, int nblocks, SplitProblem split,
                                                                        int* __restrict__ idx, int* __restrict__ counts) {
   // A step takes four tokens per thread: their loads travel together, and every wave scans the 64 counts of the step by itself, so that one
   // barrier stands between the counts and the list.  What bounds it is that chain: with a token per thread and the counts added up by one thread
-  // 12.1 -> 7.7 us at T=8192, 6.7 -> 5.4 at 4096, 6.6 -> 5.2 at 2100.
-  constexpr int kTokens = 4;
-  static_assert(kTokens * kCompactThreads / 64 == 64, "one lane per count");
-  __shared__ int count[2][64];  // of tokens t0 + k * kCompactThreads + wave * 64 .. + 63: k * 16 + wave; steps take turns
+  // 12.1 -> 7.7 us at T=8192, 6.7 -> 5.4 at 4096, 6.6 -> 5.2 at 2100.  Up to 1024 tokens, where it is the code that has to be fetched first, a
+  // token per thread: 4.1 -> 3.6 us at T=137, 4.3 -> 3.7 at 300.
+  constexpr int kCounts = TOKENS * kCompactThreads / 64;
+  static_assert(kCounts <= 64, "one lane per count");
+  __shared__ int count[2][kCounts];  // of tokens t0 + k * kCompactThreads + wave * 64 .. + 63: k * 16 + wave; steps take turns
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int n = 0;
-  for (int t0 = 0, turn = 0; t0 < T; t0 += kTokens * kCompactThreads, turn ^= 1) {
-    unsigned long long ballot[kTokens];
+  for (int t0 = 0, turn = 0; t0 < T; t0 += TOKENS * kCompactThreads, turn ^= 1) {
+    unsigned long long ballot[TOKENS];
 #pragma unroll
-    for (int k = 0; k < kTokens; ++k) {
+    for (int k = 0; k < TOKENS; ++k) {
       const int t = t0 + k * kCompactThreads + tid;
       const int tc = t < T ? t : T - 1;
       const float gv = g[tc], qv = q ? q[tc] : 0.f;
       ballot[k] = __ballot(t < T && (gv != 0.f || qv != 0.f));
     }
 #pragma unroll
-    for (int k = 0; k < kTokens; ++k)
+    for (int k = 0; k < TOKENS; ++k)
       if (lane == 0) count[turn][k * (kCompactThreads / 64) + wave] = __popcll(ballot[k]);
     __syncthreads();
-    const int mine = count[turn][lane];
+    const int mine = lane < kCounts ? count[turn][lane] : 0;
     int upto = mine;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
+    for (int o = 1; o < kCounts; o <<= 1) {
       const int below = __shfl_up(upto, o, 64);
       upto += lane >= o ? below : 0;
     }
 #pragma unroll
-    for (int k = 0; k < kTokens; ++k) {
+    for (int k = 0; k < TOKENS; ++k) {
       const int base = n + __shfl(upto - mine, k * (kCompactThreads / 64) + wave, 64);
       if (ballot[k] >> lane & 1) idx[base + __popcll(ballot[k] & ((1ull << lane) - 1ull))] = t0 + k * kCompactThreads + tid;
     }
-    n += __shfl(upto, 63, 64);
+    n += __shfl(upto, kCounts - 1, 64);
   }
   for (int b = tid; b <= nblocks; b += kCompactThreads) {
     if (b == 0) {
@@ -1095,9 +1097,12 @@ __global__ __launch_bounds__(kCompactThreads) void compact_active_rows(const flo
     const long long left = (long long)n - (long long)b * block;
     const int tokens = left < 0 ? 0 : (left > block ? block : (int)left);
     long long best = split_cost(split, tokens, lane + 1);
-    int splits = lane + 1, code = 0;
-    const long long shared = lane < kMaxGroup - 1 ? share_cost(split, tokens, lane + 2, code) : INT64_MAX;
-    if (shared < best) best = shared, splits = code;
+    int splits = lane + 1;
+    if (split.shares) {
+      int code = 0;
+      const long long shared = lane < kMaxGroup - 1 ? share_cost(split, tokens, lane + 2, code) : INT64_MAX;
+      if (shared < best) best = shared, splits = code;
+    }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       const long long c = __shfl_xor(best, o, 64);
@@ -1107,6 +1112,8 @@ __global__ __launch_bounds__(kCompactThreads) void compact_active_rows(const flo
     if (lane == 0) counts[1 + nblocks + b] = splits;
   }
 }
+
+inline auto compact_kernel(int64_t T) { return T <= kCompactThreads ? compact_active_rows<1> : compact_active_rows<4>; }
 
 // One workgroup per row r < T: as compacted row r (when r < n) it copies the inputs of token idx[r]; as token r it clears
 // d_hidden[r] -- active tokens get their row from the dHidden GEMM (or the sum over its splits) afterwards.
@@ -1830,7 +1837,7 @@ int bwd_entry(const void* hidden, int64_t ld_hidden, const void* weight, int64_t
   const SplitProblem rated = split_problem(Tb, H, vc, dw_in_gemm, w.slots, compute_units());
   if (compact) {
     Timed timed(kCompactRows, s);
-    hipLaunchKernelGGL(compact_active_rows, dim3(1), dim3(kCompactThreads), 0, s, dlogprobs, dentropy, (int)T, (int)Tb,
+    hipLaunchKernelGGL(compact_kernel(T), dim3(1), dim3(kCompactThreads), 0, s, dlogprobs, dentropy, (int)T, (int)Tb,
                        (int)nblocks, rated, w.idx, w.counts);
     hipLaunchKernelGGL(gather_active_rows, dim3((unsigned)T), dim3(256), 0, s, (const int*)w.idx, (const int*)w.counts, Hp,
                        (int)ld_hidden, (int)Hk, (int)H, labels, row_lse, row_pz, dlogprobs, dentropy, w.hidden_c, w.labels_c,
@@ -2100,7 +2107,7 @@ int skyrl_softce_bwd(const void* student_hidden, int64_t ld_student, const void*
   const SplitProblem split = split_problem(T, H, vc, false, w.slots, ncu);
   {  // tokens without an upstream gradient (what the supervision mask removes) have a zero row and take no part
     Timed timed(kCompactRows, s);
-    hipLaunchKernelGGL(compact_active_rows, dim3(1), dim3(kCompactThreads), 0, s, dloss, (const float*)nullptr, (int)T, (int)T, 1,
+    hipLaunchKernelGGL(compact_kernel(T), dim3(1), dim3(kCompactThreads), 0, s, dloss, (const float*)nullptr, (int)T, (int)T, 1,
                        split, w.idx, w.counts);
   }
   if ((e = hipGetLastError()) != hipSuccess) return (int)e;
