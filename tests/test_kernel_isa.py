@@ -8,6 +8,7 @@ every kernel that contains MFMAs and check the properties the source relies on:
   ``v_accvgpr_write`` sits right in front of an MFMA;
 * every MFMA accumulates in place, in AGPRs (no rotation of accumulators through the loop);
 * the steady-state loop (the block with MFMAs and global->LDS copies) has no scratch (spill) traffic and no accumulator moves;
+* in the one kernel that accumulates in VGPRs, everything keeps its distance from the MFMAs;
 * no scalar register that a vector instruction writes is read by another one less than two wait states later (the compiler keeps that
   distance in its own code, but cannot see into an assembly statement).
 """
@@ -28,12 +29,11 @@ pytestmark = pytest.mark.skipif(
 )
 
 
-@pytest.fixture(scope="module")
-def kernels(tmp_path_factory):
+def _kernels_of(source, tmp_path_factory):
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
-    out = tmp_path_factory.mktemp("isa") / "lmhead.s"
+    out = tmp_path_factory.mktemp("isa") / "kernels.s"
     flags = [f for f in B.HIPCC_FLAGS if f not in ("-shared", "-fPIC")]
-    cmd = [hipcc, *flags, "-S", "--cuda-device-only", "-o", str(out), os.path.join(B.HERE, B.SOURCES[0])]
+    cmd = [hipcc, *flags, "-S", "--cuda-device-only", "-o", str(out), os.path.join(B.HERE, source)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     assert proc.returncode == 0, proc.stderr[-2000:]
     text = out.read_text()
@@ -51,14 +51,32 @@ def kernels(tmp_path_factory):
     return found
 
 
-def test_mfma_kernels_found(kernels):
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    return _kernels_of("lmhead_kernels.hip", tmp_path_factory)
+
+
+@pytest.fixture(scope="module")
+def few_token_kernels(tmp_path_factory):
+    return _kernels_of("few_tokens.hip", tmp_path_factory)
+
+
+@pytest.fixture(scope="module")
+def all_kernels(kernels, few_token_kernels):
+    return {**kernels, **few_token_kernels}
+
+
+def test_mfma_kernels_found(kernels, few_token_kernels):
+    names = " ".join(few_token_kernels)
+    for expect in ("lmhead_bwd_dw_few", "lmhead_bwd_dw_resident", "lmhead_fwd_half_tiles", "lmhead_bwd_half_dz"):
+        assert expect in names, f"no MFMA kernel named *{expect}* in the assembly: {list(few_token_kernels)}"
     names = " ".join(kernels)
     for expect in ("lmhead_fwd_tiles", "lmhead_bwd_dz", "lmhead_bwd_gemm", "mfma_probe"):
         assert expect in names, f"no MFMA kernel named *{expect}* in the assembly: {list(kernels)}"
 
 
-def test_accumulator_reads_follow_the_wait_states(kernels):
-    for name, lines in kernels.items():
+def test_accumulator_reads_follow_the_wait_states(all_kernels):
+    for name, lines in all_kernels.items():
         waited = False
         for ln in lines:
             if ln.startswith("v_mfma"):
@@ -69,8 +87,8 @@ def test_accumulator_reads_follow_the_wait_states(kernels):
                 assert waited, f"{name}: '{ln}' is not behind the wait states that follow the last MFMA"
 
 
-def test_no_accumulator_write_right_before_an_mfma(kernels):
-    for name, lines in kernels.items():
+def test_no_accumulator_write_right_before_an_mfma(all_kernels):
+    for name, lines in all_kernels.items():
         for k, ln in enumerate(lines):
             if ln.startswith("v_mfma"):
                 near = [p for p in lines[max(0, k - 3):k] if p.startswith("v_accvgpr_write")]
@@ -125,16 +143,16 @@ def test_the_distance_check_sees_what_it_claims():
     assert not _too_close(["v_add_co_u32_e32 v0, vcc, v1, v2", "s_nop 1", "v_addc_co_u32_e32 v3, vcc, v4, v5, vcc"])
 
 
-def test_vector_reads_keep_their_distance_from_scalar_writes(kernels):
-    for name, lines in kernels.items():
+def test_vector_reads_keep_their_distance_from_scalar_writes(all_kernels):
+    for name, lines in all_kernels.items():
         bad = _too_close(lines)
         assert not bad, f"{name}: {len(bad)} pairs, the first {bad[0]}"
 
 
-def test_every_lds_copy_sets_m0_first(kernels):
+def test_every_lds_copy_sets_m0_first(all_kernels):
     """global_load_lds takes its LDS destination from M0: each one must be preceded, within a few instructions and with no
     other copy in between, by a write of M0."""
-    for name, lines in kernels.items():
+    for name, lines in all_kernels.items():
         for k, ln in enumerate(lines):
             if ln.startswith("global_load_lds"):
                 window = lines[max(0, k - 4):k]
@@ -143,20 +161,85 @@ def test_every_lds_copy_sets_m0_first(kernels):
                 assert not any(p.startswith("global_load_lds") for p in window[writes[-1]:]), f"{name}: stale M0 before '{ln}'"
 
 
-def test_no_packed_fp32_arithmetic(kernels):
+def test_no_packed_fp32_arithmetic(all_kernels):
     """The build switches the packed fp32 instructions off (``-packed-fp32-ops``); none may appear in the MFMA kernels."""
-    for name, lines in kernels.items():
+    for name, lines in all_kernels.items():
         bad = [ln for ln in lines if ln.startswith(("v_pk_add_f32", "v_pk_mul_f32", "v_pk_fma_f32"))]
         assert not bad, f"{name}: {bad[:3]}"
 
 
-def test_mfma_accumulates_in_place_in_agprs(kernels):
+def test_mfma_accumulates_in_place_in_agprs(all_kernels):
     pat = re.compile(r"v_mfma_f32_16x16x32_bf16 (a\[\d+:\d+\]), v\[\d+:\d+\], v\[\d+:\d+\], (a\[\d+:\d+\])$")
-    for name, lines in kernels.items():
+    for name, lines in all_kernels.items():
+        if "bwd_dw_resident" in name:
+            continue  # accumulates in VGPRs, below
         for ln in lines:
             if ln.startswith("v_mfma"):
                 m = pat.match(ln)
                 assert m and m.group(1) == m.group(2), f"{name}: unexpected MFMA form '{ln}'"
+
+
+def _vectors(operands):
+    """The vector and accumulator registers that the operands name."""
+    found = set()
+    for kind, lo, hi in re.findall(r"\b([va])\[(\d+):(\d+)\]", operands):
+        found |= {f"{kind}{i}" for i in range(int(lo), int(hi) + 1)}
+    return found | set(re.findall(r"\b[va]\d+\b", operands))
+
+
+# Wait states between a product of 16 x 16 x 32 bf16 values (eight passes) and what is not a product and names a register of its result, and
+# between a vector instruction and a product that reads what it writes.
+BEHIND_A_PRODUCT, IN_FRONT_OF_A_PRODUCT = 11, 2
+
+
+def _unsettled(lines):
+    """Pairs of instructions nearer to each other than these, in the order of the text."""
+    pairs, products, writes = [], [], []  # (wait states passed, registers, line)
+    for ln in lines:
+        op, _, rest = ln.split(";")[0].partition(" ")
+        if not re.match(r"[vs]_|ds_|global_|buffer_|scratch_", op):
+            continue
+        operands = [x.strip() for x in re.split(r",(?![^\[]*\])", rest)]
+        states = int(operands[0]) + 1 if op == "s_nop" else 1
+        if op.startswith("v_mfma"):
+            sources = _vectors(" ".join(operands[1:]))
+            pairs += [(before, ln) for passed, regs, before in writes if passed < IN_FRONT_OF_A_PRODUCT and regs & sources]
+            # an accumulator may go on at once, but is no operand of the next product and not begun anew
+            reads = _vectors(" ".join(operands[1:3])) | (_vectors(operands[0]) if operands[3] == "0" else set())
+            pairs += [(before, ln) for passed, regs, before in products if passed < BEHIND_A_PRODUCT and regs & reads]
+        else:
+            pairs += [(before, ln) for passed, regs, before in products if passed < BEHIND_A_PRODUCT and regs & _vectors(rest)]
+        products = [(passed + states, regs, before) for passed, regs, before in products if passed + states < BEHIND_A_PRODUCT]
+        writes = [(passed + states, regs, before) for passed, regs, before in writes if passed + states < IN_FRONT_OF_A_PRODUCT]
+        if op.startswith("v_"):
+            (products if op.startswith("v_mfma") else writes).append((0, _vectors(operands[0]), ln))
+    return pairs
+
+
+def test_the_product_distance_check_sees_what_it_claims():
+    mfma = "v_mfma_f32_16x16x32_bf16 v[0:3], v[8:11], a[0:3], v[0:3]"
+    assert _unsettled([mfma, "s_nop 9", "v_add_f32_e32 v9, v3, v4"]) and not _unsettled([mfma, "s_nop 10", "v_add_f32_e32 v9, v3, v4"])
+    assert _unsettled([mfma, "ds_write_b128 v20, v[0:3] offset:16"]) and _unsettled([mfma, "v_mov_b32_e32 v2, 0"])
+    assert _unsettled(["v_mov_b32_e32 v11, v20", "s_nop 0", mfma]) and not _unsettled(["v_mov_b32_e32 v11, v20", "s_nop 1", mfma])
+    assert _unsettled(["v_accvgpr_write_b32 a3, v20", mfma]) and not _unsettled([mfma, mfma])
+    assert _unsettled([mfma, mfma.replace(", v[0:3]", ", 0")]) and _unsettled([mfma, mfma.replace("v[0:3]", "v[4:7]").replace("v[8:11]", "v[0:3]")])
+
+
+def test_products_with_resident_dz_keep_their_distance(few_token_kernels):
+    """lmhead_bwd_dw_resident accumulates in VGPRs and keeps dz in AGPRs and VGPRs: the compiler, which cannot see into the products, neither moves
+    the one next to them nor reads the other too early, and spills no vector register."""
+    pat = re.compile(r"v_mfma_f32_16x16x32_bf16 (v\[\d+:\d+\]), v\[\d+:\d+\], [va]\[\d+:\d+\], (v\[\d+:\d+\]|0)$")
+    checked = 0
+    for name, lines in few_token_kernels.items():
+        if "bwd_dw_resident" not in name:
+            continue
+        bad = _unsettled(lines)
+        assert not bad, f"{name}: {len(bad)} pairs, the first {bad[0]}"
+        forms = [pat.match(ln) for ln in lines if ln.startswith("v_mfma")]
+        assert forms and all(m and m.group(2) in (m.group(1), "0") for m in forms), name
+        assert not any(ln.startswith("scratch_") for ln in lines), name
+        checked += 1
+    assert checked == 2
 
 
 # MFMAs and copies of a k-tile in the steady state, 16 copies per 128 MFMAs on square tiles (one or two k-tiles per loop body), and fewer of
