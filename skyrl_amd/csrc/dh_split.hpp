@@ -69,8 +69,9 @@ struct Shares {
   LMHEAD_HD int slot(int g, int i, int j) const { return (j + i) * groups + g; }
 };
 constexpr int kMaxGroup = 32;
-// Launches that may have more tiles than this: up to 64 tiles in four splits and more already fill nine tenths of the CUs, and calls of few tokens
-// notice what finding a share takes (draft loss of 20 tokens, H=896, V=246016, four tiles in 64 splits: GEMM 109 -> 111 us, their sum 11.6 -> 12.9).
+// Blocks that may have this many tiles and more.  Below it splits leave little: from 64000 columns on shares are rated at most 2.7 % shorter (52 tiles, whose
+// four splits keep 208 of 256 CUs busy), with narrower chunks up to 4 % of launches of some 30 us.  And calls of few tokens notice what finding a
+// share takes: draft loss of 20 tokens, H=896, V=246016, four tiles in 64 splits, GEMM 109 -> 111 us, their sum 8.6 -> 11.4.
 constexpr int64_t kSharesFromTiles = 65;
 // code: u, and b above its lowest eight bits where it is not 1.
 LMHEAD_HD inline Shares shares_of(int code, int tiles) {
@@ -79,6 +80,10 @@ LMHEAD_HD inline Shares shares_of(int code, int tiles) {
 }
 // Groups of b >= 2 tiles, as many workgroups each as the CUs hold at once, rated as above.  A workgroup's further tiles cost it an epilogue and
 // another beginning each.  `code` is set where the answer is below INT64_MAX.
+// Behind six sevenths of the CUs the power is what limits, so that a workgroup more makes the others slower.  Draft loss, V=151936, rated
+// without that -> with it: 6 tiles x 23 workgroups -> 2 x 7 at 66 tiles, GEMM 951 -> 897 us, pass 4.91 -> 4.77 ms; 9 x 32 -> three splits at 72, 977 -> 989 and
+// 5.12 -> 4.99; 5 x 16 -> three splits at 80, 1014 -> 1017 and 5.56 -> 5.49; no difference at 120.  split_cost() has no such term, which
+// prefers splits that keep six sevenths busy to shares of the same length.
 LMHEAD_HD inline int64_t share_cost(const SplitProblem& p, int tokens, int b, int& code) {
   const int tiles = (tokens + kSplitTile - 1) / kSplitTile * p.tiles_h;
   if (!p.shares || b > tiles) return INT64_MAX;
@@ -91,7 +96,7 @@ LMHEAD_HD inline int64_t share_cost(const SplitProblem& p, int tokens, int b, in
   if (s.slots() > p.slots || pairs < kMinSplitPairs) return INT64_MAX;
   code = b << 8 | u;
   const int64_t len = 2 * pairs + 10 * ((b + u - 1) / u + (b % u && u % b ? 1 : 0));
-  const int64_t busy = s.workgroups() * 7 / 6;  // behind six sevenths of the CUs the power is what limits
+  const int64_t busy = s.workgroups() * 7 / 6;
   return len * (busy > p.ncu ? busy : p.ncu) + (int64_t)s.slots() * 15 + 4 * p.ncu;
 }
 

@@ -25,7 +25,7 @@ namespace {
 // below 256 MiB would be found in the last-level cache: backward, and forward + backward + the sum of dW into another tensor, ordinary ->
 // non-temporal, 98 MiB (bf16, V=32000, H=1600, T=64; the least that comes here) 102 -> 101 and 202 -> 199 us, 141 MiB (V=128256, H=576)
 // 152 -> 136 and 270 -> 258, 195 MiB (fp32) 122 -> 117 and 281 -> 275, 282 MiB 203 -> 159 and 390 -> 358, 890 MiB (V=151936, H=1536) 469 ->
-// 416 and 1089 -> 1035; T=400 and 768 likewise.  A norm of dW behind it gains too, but for 98 MiB at T=64 (187 -> 192).
+// 416 and 1089 -> 1035.  A norm of dW behind it gains too, but for 98 MiB at T=64 (187 -> 192).
 // H=1536, V=151936: 88 us at T=17 (5.3 TB/s), 123 at T=64, 144 at T=96.
 // ------------------------------------------------------------------------------------------------------------
 constexpr int kDwK = 32;                          // tokens per step

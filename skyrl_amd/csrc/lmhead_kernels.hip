@@ -1174,6 +1174,8 @@ __global__ __launch_bounds__(256) void zero_f32(float* __restrict__ p, int n) {
 // ------------------------------------------------------------------------------------------------------------
 // Optional per-kernel timing: while a profile is open on the calling thread every launch below is bracketed by a pair of
 // HIP events on the launch stream.  Closed profiles cost one thread-local load per launch.
+// A kind is a task: lmhead_bwd_gemm the gradient products of a chunk, in the kernel of that name or in lmhead_bwd_dh_shares; lmhead_bwd_dw_few dW of few
+// tokens, in tiles or with resident dz.
 enum KernelKind {
   kFwdTiles = 0, kFwdMerge, kTranspose, kBwdChunkDz, kBwdChunkGemm, kSoftCePack, kSoftCeFwdTiles, kSoftCeFinish, kSoftCeDz,
   kCompactRows, kSplitOperand, kTopkFilter, kTopkSelect, kTopkRows, kTopkBwdRows, kDhReduce, kBwdDwFew,
@@ -1567,7 +1569,7 @@ hipError_t launch_bwd_gemm(hipStream_t s, const GemmArgs& p0, const GemmArgs& p1
   return hipGetLastError();
 }
 
-// Whether dW of a call has a launch of its own, lmhead_bwd_dw_few, rather than 256 x 256 tiles next to the dHidden tiles.  Both sides of
+// Whether dW of a call has a launch of its own, launch_bwd_dw_few(), rather than 256 x 256 tiles next to the dHidden tiles.  Both sides of
 // the line, all launches behind the dz tiles, tiles in one launch -> own launch: T=137 248 -> 177 us at H=896, 375 -> 276 at H=1536
 // (V=151936), 860 -> 604 at H=4096, V=128261; T=400 554 -> 451 and 1315 -> 1080; T=768, H=3584, V=152064 1760 -> 1630; T=1024 947 -> 883
 // and 2017 -> 2037; T=1400, H=4096 2776 -> 3074.  Below three rounds of two tiles per CU the second launch costs what it gains: 1000
