@@ -177,16 +177,22 @@ __global__ __launch_bounds__(kDwThreads, 4) void lmhead_bwd_dw_few(const DwFewAr
 
 // The tiles of a call for more tokens, of which up to kDwTileActive turn out to have a gradient.  Two workgroups per CU make all of them, because
 // those of a launch that finds more have to end before the next one begins (a workgroup per tile: 7128 at H=1536, V=151936, training pass with 137 of 137
-// tokens 505 -> 507 us, with 428 of 611 865 -> 870).  A tile begins when the stores of the one before have left: with 20 tokens 457 -> 463 us, but with
-// 40 492 -> 474.  Four per CU: 462 and 476.
+// tokens 505 -> 507 us, with 428 of 611 865 -> 870).  A tile begins when the stores of the one before have left, which costs 6 us of a pass with 20 tokens;
+// with its copies in front of those stores it is no faster (459 -> 456 us with 20 tokens, 469 -> 476 with 40), and neither are four workgroups per CU.
+// Tokens of one step: the workgroups go through the tiles side by side, 512 at a time; of two: each has neighbours, which read the same dz columns.  dW in
+// us, 24 and 40 tokens, side by side / neighbours: H=1536, V=151936 101 / 106 and 111 / 112; H=2048, V=100000 80 / 95 and 112 / 97; H=4096, V=128256 196 / 226 and
+// 254 / 226 (dz in registers 244 and 243, a workgroup per tile 222 and 260 with no launch beside it).
 template <bool F32>
 __global__ __launch_bounds__(kDwThreads, 4) void lmhead_bwd_dw_few_active(const DwFewArgs a, int tiles) {
   __shared__ __attribute__((aligned(1024))) char lds[kDwSlots * kDwSlotBytes];
   const int n = __builtin_amdgcn_readfirstlane(*a.T_dev);
   if (n > kDwTileActive) return;
-  for (int id = blockIdx.x; id < tiles; id += gridDim.x) {
-    if (id != (int)blockIdx.x) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave has taken its rows of the tile before from LDS
-    dw_few_tile<F32>(a, n, xcd_contiguous(id, tiles), lds);
+  const bool neighbours = n > kDwK;
+  const int groups = gridDim.x, group = neighbours ? xcd_contiguous(blockIdx.x, groups) : (int)blockIdx.x;
+  const int first = neighbours ? (int)((int64_t)tiles * group / groups) : group, end = neighbours ? (int)((int64_t)tiles * (group + 1) / groups) : tiles;
+  for (int id = first; id < end; id += neighbours ? 1 : groups) {
+    if (id != first) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave has taken its rows of the tile before from LDS
+    dw_few_tile<F32>(a, n, neighbours ? id : xcd_contiguous(id, tiles), lds);
   }
 }
 

@@ -30,10 +30,11 @@ struct DwFewArgs {
 // for whatever is below 130 tokens (H=1536, V=151936): 88 -> 121 at 20, 123 -> 119 at 64, 144 -> 118 at 96, 152 -> 118 at 128.  Not at the sizes
 // of the tie, because half of the tokens and more are often masked.
 constexpr int64_t kDwTileTokens = 96;
-// Behind it, where the device finds out how many tokens have a gradient, it also chooses: up to this many are made in the tiles, by a launch in front
-// that returns at once if there are more.  Training pass, H=1536, V=151936, dz in registers -> the device's choice: 480 -> 463 us with 20 tokens of
-// 137, 482 -> 474 with 40, 481 -> 478 with 60; 490 -> 473, 490 -> 484, 492 -> 488 of 200; 610 -> 592 with 20 of 611, 611 -> 606 with 60.  With 20 known
-// to the host it would be 448.  What the choice costs a call that has more: 502 -> 504 with 137 of 137, 865 -> 865 with 428 of 611.
+// Behind it, where the device finds out how many tokens have a gradient, it also chooses: up to this many, two steps of the tiles, are made in tiles, by
+// a launch in front that returns at once if there are more.  Training pass, H=1536, V=151936, dz in registers -> the device's choice: 478 -> 459 us with 20
+// tokens of 137, 479 -> 469 with 40 and with 60; 490 -> 468, 488 -> 477 and 491 -> 480 of 200; 599 -> 578 with 20 of 611, 601 -> 591 with 60; 994 -> 981
+// with 50 of 300 at H=4096, V=128261.  With 20 known to the host it would be 444.  What the choice costs a call that has more: 493 -> 495 with 137 of 137, 848 ->
+// 846 with 428 of 611.
 constexpr int kDwTileActive = 64;
 // Whether the call is one for resident dz.  A workgroup's new dz rows cost it 6 us, for a row of H / 64 units: with short rows that is more than is
 // saved.  Tiles -> resident dz, us, 137, 300 and 768 tokens: H=256, V=248320 48 -> 59, 66 -> 77, 124 -> 143 (fp32 result 73 -> 83 and 148 -> 169 at
